@@ -3,6 +3,8 @@
 #include "sl_device.h"
 #include "sl_internal.h"
 
+#include <algorithm>
+
 namespace sl {
 using namespace dev;
 
@@ -458,9 +460,9 @@ __global__ void __launch_bounds__(256) k_monotone(SceneDev sc, const float2 *__r
     }
 }
 
-// Work lists.  Pieces (curve << 3 | piece) with nx + ny + 1 >= 128 cuts are "long": their
-// two solve chains (curve << 4 | piece << 1 | side, non-empty only) are listed for one
-// thread each, and the piece for the wave-parallel merge.  Shorter pieces are listed for
+// Work lists.  Pieces (curve << 3 | piece) with nx + ny + 1 >= 128 cuts (cubic ones from
+// cubic_min cuts, see launch_intersect) are "long": their two solve chains (curve << 4 |
+// piece << 1 | side, non-empty only) are listed, and the piece for the wave-parallel merge.  Shorter pieces are listed for
 // one thread that solves and walks both sides.  Chains and short pieces are grouped by
 // (cubic or closed-form solve, length bin), longest first, so the lanes of a wave run
 // loops of the same kind and about the same trip count and the long sequential walks
@@ -506,9 +508,10 @@ __device__ __forceinline__ CurvePieces curve_pieces(const SceneDev &sc, uint32_t
 }
 
 // the classes of piece k's entries: x chain, y chain (-1 when not listed), piece
-__device__ __forceinline__ void piece_classes(const CurvePieces &cp, int k, int &qx, int &qy, int &qp) {
+__device__ __forceinline__ void piece_classes(const CurvePieces &cp, int k, uint32_t cubic_min, int &qx, int &qy,
+                                              int &qp) {
     const uint32_t nx = cp.pc[k] & 0xFFFFu, ny = cp.pc[k] >> 16, L = nx + ny + 1;
-    if (L >= kLongPiece) {
+    if (L >= (cp.cb ? kLongPiece : cubic_min)) {
         qx = nx ? cp.cb + len_bin(nx) : -1;
         qy = ny ? cp.cb + len_bin(ny) : -1;
         qp = kLongPieceClass;
@@ -521,7 +524,8 @@ __device__ __forceinline__ void piece_classes(const CurvePieces &cp, int k, int 
 // class counts (cnt[kListClasses])
 __global__ void __launch_bounds__(kChainListThreads) k_list_count(SceneDev sc, uint32_t C,
                                                                   const uint32_t *__restrict__ nchain,
-                                                                  const uint32_t *__restrict__ pcnt, uint32_t *cnt) {
+                                                                  const uint32_t *__restrict__ pcnt, uint32_t cubic_min,
+                                                                  uint32_t *cnt) {
     __shared__ uint32_t h[kListClasses];
     for (int q = threadIdx.x; q < kListClasses; q += blockDim.x) h[q] = 0u;
     __syncthreads();
@@ -530,7 +534,7 @@ __global__ void __launch_bounds__(kChainListThreads) k_list_count(SceneDev sc, u
     for (int k = 0; k < 5; ++k) {
         if (k >= cp.np) break;
         int qx, qy, qp;
-        piece_classes(cp, k, qx, qy, qp);
+        piece_classes(cp, k, cubic_min, qx, qy, qp);
         if (qx >= 0) atomicAdd(&h[qx], 1u);
         if (qy >= 0) atomicAdd(&h[qy], 1u);
         atomicAdd(&h[qp], 1u);
@@ -544,7 +548,7 @@ __global__ void __launch_bounds__(kChainListThreads) k_list_count(SceneDev sc, u
 __global__ void __launch_bounds__(kChainListThreads) k_list_place(SceneDev sc, uint32_t C,
                                                                   const uint32_t *__restrict__ nchain,
                                                                   const uint32_t *__restrict__ pcnt,
-                                                                  const uint32_t *__restrict__ coff,
+                                                                  const uint32_t *__restrict__ coff, uint32_t cubic_min,
                                                                   const uint32_t *__restrict__ cnt, uint32_t *cursor,
                                                                   uint4 *clist, uint4 *plist) {
     __shared__ uint32_t h[kListClasses], base[kListClasses];
@@ -564,7 +568,7 @@ __global__ void __launch_bounds__(kChainListThreads) k_list_place(SceneDev sc, u
     for (int k = 0; k < 5; ++k) {
         if (k >= cp.np) break;
         int qx, qy, qp;
-        piece_classes(cp, k, qx, qy, qp);
+        piece_classes(cp, k, cubic_min, qx, qy, qp);
         rk[3 * k] = qx >= 0 ? atomicAdd(&h[qx], 1u) : 0u;
         rk[3 * k + 1] = qy >= 0 ? atomicAdd(&h[qy], 1u) : 0u;
         rk[3 * k + 2] = atomicAdd(&h[qp], 1u);
@@ -578,7 +582,7 @@ __global__ void __launch_bounds__(kChainListThreads) k_list_place(SceneDev sc, u
     for (int k = 0; k < 5; ++k) {
         if (k >= cp.np) break;
         int qx, qy, qp;
-        piece_classes(cp, k, qx, qy, qp);
+        piece_classes(cp, k, cubic_min, qx, qy, qp);
         // each entry carries its piece's ts offset and cut counts, so that the intersection
         // passes read only the curve's record besides it
         const uint32_t pb = off, pw = cp.pc[k];
@@ -611,20 +615,20 @@ __device__ __forceinline__ float solve_cut(int type, float w, float a0, float a1
     if (type == CT_LINEAR) return tmin(tmax((cc - a0) * safe_rcp(a1 - a0), t_min), t1);
     if (type == CT_QUAD) return solve_quad_bezier(a0, a1, a2, cc, t_min, t1);
     if (type == CT_RATIONAL) return solve_quad_bezier(a0 - cc, (a1 - cc) * w, a2 - cc, 0.f, t_min, t1);
-    // 24 bisection steps.  lo moves only to a midpoint whose f - cc has the sign bit of
-    // f(lo) - cc, so that sign bit stays the one of f(t_min) - cc.
-    float lo = t_min, hi = t1;
-    const float vlo = curve_eval(CT_CUBIC, 0.f, a0, a1, a2, a3, lo);
-    float t_solve = lo;
+    // 24 bisection steps.  An end moves only to a midpoint whose f - cc has the sign bit of its
+    // own (f - cc is negative exactly when f < cc), so the ends are kept by their side of cc:
+    // the midpoint of the two is the same whichever is the lower one.
+    const float vlo = curve_eval(CT_CUBIC, 0.f, a0, a1, a2, a3, t_min);
+    float t_solve = t_min;
     if (vlo != cc) {
-        const uint32_t s0 = fb(vlo - cc) >> 31;
+        float p = vlo < cc ? t_min : t1, q = vlo < cc ? t1 : t_min;
         float last_v = 0.f;
         for (int it = 0; it < 24; ++it) {
-            const float tm = (lo + hi) * .5f;
+            const float tm = (p + q) * .5f;
             const float vm = curve_eval(CT_CUBIC, 0.f, a0, a1, a2, a3, tm);
-            const bool up = (fb(vm - cc) >> 31) == s0;
-            lo = up ? tm : lo;
-            hi = up ? hi : tm;
+            const bool low = vm < cc;
+            p = low ? tm : p;
+            q = low ? q : tm;
             t_solve = tm;
             last_v = vm;
         }
@@ -732,6 +736,193 @@ __device__ __forceinline__ void solve_chain(const SceneDev &sc, const float4 *__
     }
 }
 
+// Cubic chains of frames that leave the GPU idle.  A chain is serial: every cut's bisection
+// starts from the previous cut's t, and its 24 steps depend on each other, so one lane needs
+// about 1.5 us a cut and a frame's longest chain sets the pass's time whatever the size of
+// the GPU.  Here 2^K lanes share a chain: lane l follows the bits of l through K halvings,
+// computing the interval ends exactly as the serial steps would, evaluates the curve at its
+// lower end T[l] (T[1] .. T[2^K - 1] are the 2^K - 1 midpoints the next K steps can visit), and
+// the steps' outcome is read from all lanes' signs at once.  Along a monotone piece the signs
+// change once, and the interval left is the one between the last T on the lower side and the
+// first on the upper; where rounding makes them change more often, the K steps are walked
+// through the sign bits one by one.  Either way the result is the serial bisection's, bit for bit.
+struct WideChain {
+    float a0, a1, a2, a3, d01, d12, d23;
+    __device__ __forceinline__ float eval(float t) const {  // curve_eval of a cubic, its first differences at hand
+        const float q0 = a0 + t * d01, q1 = a1 + t * d12, q2 = a2 + t * d23;
+        const float l0 = q0 + t * (q1 - q0), l1 = q1 + t * (q2 - q1);
+        return l0 + t * (l1 - l0);
+    }
+};
+
+template <int CTRL> __device__ __forceinline__ uint32_t dpp_u32(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, CTRL, 0xf, 0xf, false);
+}
+// row-wide (16 lanes) maximum / minimum in every lane of the row
+__device__ __forceinline__ uint32_t row_max(uint32_t x) {
+    x = tmax(x, dpp_u32<0x128>(x));  // row_ror:8, 4, 2, 1
+    x = tmax(x, dpp_u32<0x124>(x));
+    x = tmax(x, dpp_u32<0x122>(x));
+    return tmax(x, dpp_u32<0x121>(x));
+}
+__device__ __forceinline__ uint32_t row_min(uint32_t x) {
+    x = tmin(x, dpp_u32<0x128>(x));
+    x = tmin(x, dpp_u32<0x124>(x));
+    x = tmin(x, dpp_u32<0x122>(x));
+    return tmin(x, dpp_u32<0x121>(x));
+}
+
+// T[l] of the next K steps from the interval [lo, hi], 0 <= lo <= hi.  The interval is kept
+// scaled by 2^k at step k, so a midpoint is a plain sum S = A + B (its rounding does not depend
+// on the scale) and the next one S + 2 X, X being the end the step keeps: one fma a step on the
+// critical path.
+template <int K> __device__ __forceinline__ float wide_node(float lo, float hi, int l) {
+    float S = lo + hi, A = lo, X = (l >> (K - 1)) & 1 ? hi : lo;
+#pragma unroll
+    for (int k = K - 1; k >= 0; --k) {
+        const bool up = (l >> k) & 1;
+        const float A2 = A + A;
+        if (k > 0) {
+            const bool same = ((l >> k) & 1) == ((l >> (k - 1)) & 1);
+            const float S2 = __builtin_fmaf(X, 2.f, S), X2 = X + X;
+            X = same ? X2 : S;
+            A = up ? S : A2;
+            S = S2;
+        } else {
+            A = up ? S : A2;
+        }
+    }
+    return A * (1.f / (float)(1 << K));
+}
+
+// One cut by a whole wave, four rounds of six steps; `odd` is set where the signs changed more
+// than once (the result is then not to be used).
+__device__ __forceinline__ float wide_cut64(const WideChain &w, float cc, float t_min, float t1, bool &odd) {
+    const int lane = threadIdx.x & 63;
+    float lo = t_min, hi = t1;
+    uint64_t flip = 0ull, spread = 0ull, eq = 0ull, far = 0ull;
+    uint32_t leaf = 0u;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float T = wide_node<6>(lo, hi, lane);
+        const float Th = lane == 0 ? hi : T;  // the upper end of leaf 63 is the interval's
+        const float v = w.eval(T);
+        uint64_t m = __ballot(v < cc);
+        if (r == 0) {
+            eq = __ballot(v == cc) & 1ull;       // lane 0 is at t_min
+            flip = (m & 1ull) ? 0ull : ~0ull;    // lanes on t_min's side get a 1
+        }
+        m = (m ^ flip) | 1ull;
+        spread |= m & (m + 1ull);
+        leaf = (uint32_t)__popcll(m) - 1u;
+        if (r == 3) far = __ballot(fabsf(v - cc) > 1.f);
+        lo = bf((uint32_t)__builtin_amdgcn_readlane((int)fb(T), leaf));
+        hi = bf((uint32_t)__builtin_amdgcn_readlane((int)fb(Th), (leaf + 1u) & 63u));
+    }
+    odd = spread != 0ull;
+    const float t = (leaf & 1u) ? lo : hi;  // the last midpoint
+    return (eq || ((far >> (leaf | 1u)) & 1ull)) ? t_min : t;
+}
+
+// One cut by each of the wave's four rows of 16 lanes: six rounds of four steps.
+__device__ __forceinline__ float wide_cut16(const WideChain &w, float cc, float t_min, float t1, bool &odd) {
+    const int lane = threadIdx.x & 63, sub = lane & 15;
+    float lo = t_min, hi = t1;
+    bool below = false, exact = false;
+    uint32_t rows = 0u, far = 0u;
+    odd = false;
+#pragma unroll
+    for (int r = 0; r < 6; ++r) {
+        const float T = wide_node<4>(lo, hi, sub);
+        const float v = w.eval(T);
+        if (r == 0) {
+            const float v0 = bf(dpp_u32<0x150>(fb(v)));  // row_newbcast:0, at t_min
+            exact = v0 == cc;
+            below = v0 < cc;
+        }
+        const bool up = (v < cc) == below || sub == 0;
+        // t >= 0: the bits order like the values
+        const uint32_t cl = row_max(up ? fb(T) : fb(lo)), ch = row_min(up ? fb(hi) : fb(T));
+        odd |= cl > ch;
+        if (r == 5) {
+            // the row's sign bits give the last midpoint: the lower end left after an up step
+            const uint64_t mu = __ballot(up), mf = __ballot(fabsf(v - cc) > 1.f);
+            const int sh = lane & 16;
+            rows = (((lane & 32) ? (uint32_t)(mu >> 32) : (uint32_t)mu) >> sh) & 0xFFFFu;
+            far = (((lane & 32) ? (uint32_t)(mf >> 32) : (uint32_t)mf) >> sh) & 0xFFFFu;
+        }
+        lo = bf(cl);
+        hi = bf(ch);
+    }
+    const uint32_t leaf = (uint32_t)__popc(rows) - 1u;
+    return (exact || ((far >> (leaf | 1u)) & 1u)) ? t_min : ((leaf & 1u) ? lo : hi);
+}
+
+// Chains [0, n) of the list (cubic, longest first) over the waves of `blocks` blocks: the
+// first n64 of them a wave each, the others four to a wave, the long ones at a raised wave
+// priority, since the last of them ends the pass.  The t's of a chain are stored a row or a
+// wave at a time.  Bound by the instructions of a chain's own wave (about 250 a cut with 64
+// lanes, 300 with 16, against 528 with one lane).  Rows of 16 lanes with four nodes a lane
+// (four rounds of six steps) were slower: 1.27 us a cut for 1.06.
+__device__ __forceinline__ void wide_chains(const SceneDev &sc, const float4 *__restrict__ crec,
+                                            const uint4 *__restrict__ clist, uint32_t n, uint32_t blocks,
+                                            int W, int H, float *__restrict__ chain_t) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t waves = blocks * (blockDim.x >> 6);
+    const uint32_t wave = (threadIdx.x >> 6) * blocks + blockIdx.x;  // neighbours in the list go to other CUs
+    // with few chains, the longest of them a wave each: 0.67 us a cut against 1.06 us
+    const uint32_t n64 = n <= 8192u ? tmin(512u, n) : 0u;
+    const uint32_t units = n64 + (n - n64 + 3u) / 4u;
+    for (uint32_t u = wave; u < units; u += waves) {
+        const bool whole = u < n64;
+        const uint32_t i = whole ? u : n64 + 4u * (u - n64) + (uint32_t)(lane >> 4);
+        const bool live = i < n;
+        const uint4 e = clist[live ? i : 0u];
+        const int side = (int)(e.x & 1u);
+        const PieceSetup p = piece_setup(sc, crec, e.x >> 4, (int)((e.x >> 1) & 7u), e, W, H);
+        const SideSolver sv = side ? p.sy : p.sx;
+        const uint32_t cnt = live ? (side ? p.ny : p.nx) : 0u;
+        float *out = chain_t + p.base + (side ? p.nx : 0u);
+        const WideChain w{sv.a0, sv.a1, sv.a2, sv.a3, sv.a1 - sv.a0, sv.a2 - sv.a1, sv.a3 - sv.a2};
+        const bool tiny = !(sv.t1m >= 1e-30f);  // scaled sums would round subnormals differently
+        float cc = sv.cc, t = sv.t_min, keep = 0.f;
+        if (whole) {
+            __builtin_amdgcn_s_setprio(3);
+            for (uint32_t j = 0; j < cnt; ++j) {
+                bool odd;
+                float r = wide_cut64(w, cc, t, sv.t1m, odd);
+                if (odd || tiny) r = solve_cut(CT_CUBIC, 0.f, sv.a0, sv.a1, sv.a2, sv.a3, cc, t, sv.t1m);
+                t = bf((fb(r) & 0xFFFFFFFCu) | sv.side);
+                cc += sv.dd;
+                keep = (j & 63u) == (uint32_t)lane ? t : keep;
+                if ((j & 63u) == 63u || j + 1 == cnt) {
+                    const uint32_t j0 = j & ~63u;
+                    if (j0 + lane <= j) out[j0 + lane] = keep;
+                }
+            }
+        } else {
+            const uint32_t most = (uint32_t)wave_reduce((int)cnt, 0, OpMaxU());
+            const uint32_t sub = (uint32_t)(lane & 15);
+            if (most > 64u) __builtin_amdgcn_s_setprio(2);
+            else __builtin_amdgcn_s_setprio(1);
+            for (uint32_t j = 0; j < most; ++j) {
+                bool odd;
+                float r = wide_cut16(w, cc, t, sv.t1m, odd);
+                if (__ballot(odd || tiny)) {
+                    const float q = solve_cut(CT_CUBIC, 0.f, sv.a0, sv.a1, sv.a2, sv.a3, cc, t, sv.t1m);
+                    r = odd || tiny ? q : r;
+                }
+                t = bf((fb(r) & 0xFFFFFFFCu) | sv.side);
+                cc += sv.dd;
+                keep = (j & 15u) == sub ? t : keep;
+                const uint32_t k = (j & ~15u) + sub;
+                if (((j & 15u) == 15u || j + 1 == most) && k <= j && k < cnt) out[k] = keep;
+            }
+        }
+        __builtin_amdgcn_s_setprio(0);
+    }
+}
+
 // Intersection pass 2 replays the reference's slot walk (ras_cut.h:910-1000) per
 // monotone piece over the piece's solved chains: pick the x slot when x <= y, emit its t,
 // refill it from the chain or with the exhausted marker 2 | side; equal consecutive t's
@@ -817,7 +1008,10 @@ __device__ __forceinline__ void walk_piece(const PieceRef &r, const float *__res
 
 // Short and medium pieces (nx + ny + 1 < 128): one thread solves both sides and replays
 // the slot walk as it goes, each slot refilled by the next cut of its side -- the same
-// sequence walk_piece reads from the stored chains, without storing them.  The output is
+// sequence walk_piece reads from the stored chains, without storing them.  A step's lanes
+// take cuts of both sides in one solve, in a loop that stays rolled: with a solve per side,
+// unrolled 16 times, the kernel's 80 KB of code did not fit the instruction cache and a
+// 64x64 drawing's k_chains took 153 us for 89.  The output is
 // staged: every lane walks kStageSteps entries of its piece into an LDS column, then the
 // wave writes the chunk out 16 lanes to a piece, so each piece's run of up to 128 bytes
 // goes out in one store instead of one 8-byte store a step (lines left partly written by
@@ -835,26 +1029,34 @@ __device__ __forceinline__ void walk_pieces_staged(PieceSetup &p, bool live, int
     const float two = 2.f, two1 = bf(fb(2.f) | 1u);
     float xs = two, ys = two1;
     uint32_t rx = 0, ry = 0;
+    float ccx = p.sx.cc, ccy = p.sy.cc;
+    const int type = p.sx.type;
+    const float w = p.sx.w, t1m = p.sx.t1m;
     if (live) {
         if (nx == 0) { xs = two; ys = p.t0m; rx = 0; ry = ny; }
         else if (ny == 0) { xs = p.t0m; ys = two1; rx = nx; ry = 0; }
-        else { xs = p.sx.next(); rx = nx - 1; ys = p.t0m; ry = ny; }
+        else { xs = p.sx.next(); ccx = p.sx.cc; rx = nx - 1; ys = p.t0m; ry = ny; }
     }
     const uint32_t nmax = (uint32_t)wave_reduce((int)n_loop, 0, OpMaxU());
     uint32_t last = fb(-1.f);
     for (uint32_t it0 = 0; it0 < nmax; it0 += kStageSteps) {
-#pragma unroll
+#pragma unroll 1
         for (int j = 0; j < kStageSteps; ++j) {
             const uint32_t it = it0 + j;
             if (it < n_loop) {
-                float v;
-                if (xs <= ys) {
-                    v = xs;
-                    if (rx > 0) { xs = p.sx.next(); rx--; } else { xs = two; }
-                } else {
-                    v = ys;
-                    if (ry > 0) { ys = p.sy.next(); ry--; } else { ys = two1; }
+                // the slot taken is refilled by its side's next cut, solved from the t just
+                // taken; the lanes of both sides share one solve
+                const bool tx = xs <= ys;
+                const float v = tx ? xs : ys;
+                float nv = tx ? two : two1;
+                if ((tx ? rx : ry) > 0) {
+                    const float t = solve_cut(type, w, tx ? p.sx.a0 : p.sy.a0, tx ? p.sx.a1 : p.sy.a1,
+                                              tx ? p.sx.a2 : p.sy.a2, tx ? p.sx.a3 : p.sy.a3, tx ? ccx : ccy, v, t1m);
+                    nv = bf((fb(t) & 0xFFFFFFFCu) | (tx ? 0u : 1u));
+                    if (tx) { ccx += p.sx.dd; rx--; } else { ccy += p.sy.dd; ry--; }
                 }
+                xs = tx ? nv : xs;
+                ys = tx ? ys : nv;
                 uint32_t o = fb(v);
                 if ((o & 0xFFFFFFFCu) == (last & 0xFFFFFFFCu)) {
                     o |= last;
@@ -883,20 +1085,28 @@ __device__ __forceinline__ void walk_pieces_staged(PieceSetup &p, bool live, int
     }
 }
 
-// Intersection pass 1.  Blocks [0, chain_blocks) solve the listed chains of long pieces,
-// longest first; the blocks after them each take 256 short pieces and walk them while
-// solving, so the short pieces fill the GPU while the long chains run.
+// Intersection pass 1.  Blocks [0, wide_blocks) solve the cubic chains of the first wide_bins
+// length bins with several lanes each; the next chain_blocks solve the other listed chains
+// of long pieces, longest first; the blocks after them each take 256 short pieces and walk
+// them while solving, so the short pieces fill the GPU while the long chains run.
 __global__ void __launch_bounds__(256) k_chains(SceneDev sc, const float4 *__restrict__ crec, const uint4 *__restrict__ clist,
                                                  const uint4 *__restrict__ plist, const uint32_t *__restrict__ cnt,
-                                                 uint32_t chain_blocks, int W, int H, float *chain_t, int2 *ts) {
-    if (blockIdx.x < chain_blocks) {
-        const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+                                                 uint32_t wide_blocks, int wide_bins, uint32_t chain_blocks, int W, int H,
+                                                 float *chain_t, int2 *ts) {
+    if (blockIdx.x < wide_blocks) {
+        wide_chains(sc, crec, clist, class_total(cnt, 0, wide_bins), wide_blocks, W, H, chain_t);
+        return;
+    }
+    const uint32_t blk = blockIdx.x - wide_blocks;
+    if (blk < chain_blocks) {
+        // the chains after those of the wide blocks
+        const uint32_t i = blk * blockDim.x + threadIdx.x + class_total(cnt, 0, wide_bins);
         if (i >= class_total(cnt, 0, kChainClasses)) return;
         solve_chain(sc, crec, clist[i], W, H, chain_t);
         return;
     }
     __shared__ uint32_t stage[4][kStageSteps * 64];
-    const uint32_t g = (blockIdx.x - chain_blocks) * blockDim.x + threadIdx.x;
+    const uint32_t g = (blk - chain_blocks) * blockDim.x + threadIdx.x;
     const bool live = g < class_total(cnt, kShortClass0, kListClasses);
     if (!__ballot(live)) return;  // whole wave past the list
     PieceSetup p;
@@ -1053,17 +1263,35 @@ void launch_intersect(const SceneDev &sc, Frame &f, hipStream_t s) {
     if (!sc.C) return;
     uint32_t *cnt = f.lcount, *cursor = f.lcount + kListClasses;
     launch_fill_u32(f.lcount, 0u, 2 * kListClasses, s);
+    // Cubic chains of the first wide_bins length bins take several lanes each (wide_chains): one
+    // lane's 1.5 us a cut makes the longest chains the pass's time in frames of every size, but
+    // the lanes cost up to 20 times the issue slots, so the more cuts a frame has, the fewer
+    // chains pay.  Pieces of cubic_min cuts are listed as chains; shorter ones are walked by one
+    // lane.  Intersection stage, one lane a chain / the rule, us: 3.5 k cuts 111 / 67, 0.45 M
+    // 415 / 219, 2.1 M 515 / 385, 2.9 M 528 / 296, 5 M 483 / 300, 6.2 M 712 / 380, 12.8 M
+    // 782 / 484, 26 M 840 / 566, 51 M 985 / 719.  Neighbouring settings at each limit: 5 M with
+    // three bins 341, 6.2 M with four 387 and two 458, 12.8 M with four 570, 26 M with three 698,
+    // 51 M with three 1115; 2.1 M with 128-cut pieces and four bins 439.
+    const struct { int64_t cuts; uint32_t cubic_min; int bins; uint32_t blocks; } rule[] = {
+        {1 << 18, 24u, kLenBins, 2048u},  {1 << 21, 64u, kLenBins, 2048u}, {5 << 20, kLongPiece, 4, 512u},
+        {1 << 24, kLongPiece, 3, 256u},   {INT64_MAX, kLongPiece, 2, 256u}};
+    int at = 0;
+    while (f.F > rule[at].cuts) ++at;
+    const uint32_t cubic_min = rule[at].cubic_min;
+    const int wide_bins = rule[at].bins;
     const dim3 gl(blocks_for(sc.C, kChainListThreads)), bl(kChainListThreads);
-    hipLaunchKernelGGL(k_list_count, gl, bl, 0, s, sc, sc.C, (const uint32_t *)f.nchain, (const uint32_t *)f.pcnt, cnt);
+    hipLaunchKernelGGL(k_list_count, gl, bl, 0, s, sc, sc.C, (const uint32_t *)f.nchain, (const uint32_t *)f.pcnt, cubic_min,
+                       cnt);
     hipLaunchKernelGGL(k_list_place, gl, bl, 0, s, sc, sc.C, (const uint32_t *)f.nchain, (const uint32_t *)f.pcnt,
-                       (const uint32_t *)f.coff, (const uint32_t *)cnt, cursor, f.chains, f.plist);
+                       (const uint32_t *)f.coff, cubic_min, (const uint32_t *)cnt, cursor, f.chains, f.plist);
     // chain blocks: enough for every chain; piece blocks: enough for every piece
     const uint32_t npieces = (uint32_t)(f.NCH / 2);
     const uint32_t chain_blocks = blocks_for(f.NCH, 256), piece_blocks = blocks_for(npieces, 256);
+    const uint32_t wide_blocks = std::min<uint32_t>(rule[at].blocks, blocks_for(f.NCH, 4));
     if (f.NCH)
-        hipLaunchKernelGGL(k_chains, dim3(chain_blocks + piece_blocks), dim3(256), 0, s, sc, (const float4 *)f.crec,
+        hipLaunchKernelGGL(k_chains, dim3(wide_blocks + chain_blocks + piece_blocks), dim3(256), 0, s, sc, (const float4 *)f.crec,
                            (const uint4 *)f.chains, (const uint4 *)f.plist,
-                           (const uint32_t *)cnt, chain_blocks, f.W, f.H, f.chain_t, f.ts);
+                           (const uint32_t *)cnt, wide_blocks, wide_bins, chain_blocks, f.W, f.H, f.chain_t, f.ts);
     // one block per long piece up to 32768 blocks: the pieces' sizes vary widely, and
     // blocks that find no piece exit at once
     if (npieces)
