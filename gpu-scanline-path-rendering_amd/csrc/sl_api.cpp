@@ -89,7 +89,7 @@ struct sl_handle {
     size_t stage_cap = 0;
     // tables (device)
     DevBuf ptable[3];
-    DevBuf ctab[2];  // [srgb] : dec_c, thr_c, dec_a, thr_a, lut_c, lut_a packed
+    DevBuf ctab[2];  // [srgb]: a ColorBlock
     // per-frame arena
     Arena A;
     // debug host copies
@@ -228,9 +228,8 @@ int spp_slot(int spp) { return spp == 8 ? 0 : (spp == 16 ? 1 : 2); }
 
 // colour table block layout in one device buffer
 struct ColorBlock {
-    float step_c[256][4];  // {thr[k+1], dec[k], dec[k+1], 0} of the colour encoding
+    sl::ColorTables::Step step_c[sl::kQuantSteps];  // steps of the colour encoding
     float dec_c[256], thr_c[256], dec_a[256], thr_a[256];
-    uint8_t lut_c[4096], lut_a[4096];
 };
 
 int ensure_tables(sl_handle *h) {
@@ -245,20 +244,13 @@ int ensure_tables(sl_handle *h) {
     if (!ct.p) {
         sl::ColorTables c, a;
         if (!sl::build_color_tables(h->srgb, c) || !sl::build_color_tables(0, a))
-            return fail(h, SL_E_UNSUPPORTED, "colour encode table has two thresholds in one LUT bucket");
+            return fail(h, SL_E_UNSUPPORTED, "colour encode table has two thresholds in one interval");
         ColorBlock blk;
         std::memcpy(blk.dec_c, c.dec, sizeof blk.dec_c);
         std::memcpy(blk.thr_c, c.thr, sizeof blk.thr_c);
-        std::memcpy(blk.lut_c, c.lut, sizeof blk.lut_c);
         std::memcpy(blk.dec_a, a.dec, sizeof blk.dec_a);
         std::memcpy(blk.thr_a, a.thr, sizeof blk.thr_a);
-        std::memcpy(blk.lut_a, a.lut, sizeof blk.lut_a);
-        for (int k = 0; k < 256; ++k) {
-            blk.step_c[k][0] = k < 255 ? c.thr[k + 1] : INFINITY;
-            blk.step_c[k][1] = c.dec[k];
-            blk.step_c[k][2] = c.dec[k < 255 ? k + 1 : 255];
-            blk.step_c[k][3] = 0.f;
-        }
+        std::memcpy(blk.step_c, c.step, sizeof blk.step_c);
         int rc = upload(h, ct, &blk, sizeof blk);
         if (rc) return rc;
     }
@@ -275,8 +267,8 @@ sl::Tables tables_view(sl_handle *h) {
     t.words = words_for(h->spp);
     t.pixel = P_<uint32_t>(h->ptable[spp_slot(h->spp)]);
     ColorBlock *cb = P_<ColorBlock>(h->ctab[h->srgb ? 1 : 0]);
-    t.dec_c = cb->dec_c; t.thr_c = cb->thr_c; t.lut_c = cb->lut_c;
-    t.dec_a = cb->dec_a; t.thr_a = cb->thr_a; t.lut_a = cb->lut_a;
+    t.dec_c = cb->dec_c; t.thr_c = cb->thr_c;
+    t.dec_a = cb->dec_a; t.thr_a = cb->thr_a;
     t.step_c = (const float4 *)cb->step_c;
     t.srgb = h->srgb;
     return t;

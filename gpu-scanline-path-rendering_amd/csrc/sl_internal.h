@@ -51,11 +51,9 @@ struct Tables {
     const uint32_t *pixel;   // [65536 * words] line -> sample mask table
     const float *dec_c;      // [256] colour decode (sRGB or UNORM)
     const float *thr_c;      // [256] colour encode thresholds
-    const uint8_t *lut_c;    // [4096] encode LUT
     const float *dec_a;      // [256] alpha decode (UNORM)
     const float *thr_a;      // [256]
-    const uint8_t *lut_a;    // [4096]
-    const float4 *step_c;    // [256] sRGB steps {thr[k+1], dec[k], dec[k+1], 0}
+    const float4 *step_c;    // [kQuantSteps] {thr, dec, dec_next, code bits} (sl_tables.h)
 };
 
 // Gradient paint of a frame (output_32.vert.glsl:55-97, output_32.frag.glsl:45-51).  A

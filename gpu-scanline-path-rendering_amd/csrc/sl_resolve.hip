@@ -14,6 +14,7 @@
 //              the same slot of `imask`).
 #include "sl_device.h"
 #include "sl_internal.h"
+#include "sl_tables.h"
 
 #include <algorithm>
 
@@ -984,61 +985,73 @@ __device__ __forceinline__ void wave_sync_lds() {
 //   UNORM8: code = largest k with v >= (k - 0.5) / 255, i.e. with 510 v - (2k - 1) >= 0 --
 //           one fma gives that sign exactly, applied to an estimate that is never too
 //           small; decode = RN(k / 255) by a corrected product.
-//   sRGB8:  a 4096-entry table gives the code k0 of the interval start floor(4096 v)/4096;
-//           no interval holds two thresholds, so the code is k0 or k0 + 1, and one 16-byte
-//           step entry {thr[k0+1], dec[k0], dec[k0+1]} decides and decodes.
+//   sRGB8:  the top bits of v + 2^-5 name one of 645 intervals that grow with v like the
+//           thresholds' distances; none holds two thresholds, so the code is the interval's
+//           first or the next, and one 16-byte entry {thr, dec, dec_next, code} decides and
+//           decodes.  (4096 equal intervals naming a step took a second, dependent LDS read:
+//           headline composite 2.20 ms for 2.01, a 1024x768 gradient scene's 0.43 for 0.32.)
 // ---------------------------------------------------------------------------------
-// The code is m = floor(255 v + 0.5) (clamped).  The estimate trunc(RN(255 v + 0.5)) is m or
-// m + 1: rounding is monotone and the integers m, m + 1 are floats, so RN never crosses below
-// m.  One exact sign test, RN(510 v + 1 - 2k) < 0 iff v < thr[k], takes the extra one back.
-__device__ __forceinline__ int unorm_code(float v) {
-    int k = tmin(tmax((int)__builtin_fmaf(v, 255.f, 0.5f), 0), 255);
-    k -= (__builtin_fmaf(v, 510.f, (float)(1 - 2 * k)) < 0.f) ? 1 : 0;  // v < thr[k]
-    return tmax(k, 0);
-}
+// v clamped to [0, 1], NaN to 0
+__device__ __forceinline__ float unit(float v) { return __builtin_amdgcn_fmed3f(v, 0.f, 1.f); }
 
-__device__ __forceinline__ float unorm_dec(int k) {
-    const float fk = (float)k, r = 1.f / 255.f;
+// The code is m = floor(255 v + 0.5).  The estimate floor(RN(255 v + 0.5)) is m or m + 1:
+// rounding is monotone and the integers m, m + 1 are floats, so RN never crosses below m.
+// One exact sign test, RN(510 v + 1 - 2k) < 0 iff v < thr[k], takes the extra one back.
+__device__ __forceinline__ float unorm_codef(float v) {
+    const float u = unit(v);
+    const float k = floorf(__builtin_fmaf(u, 255.f, 0.5f));
+    return __builtin_fmaf(u, 510.f, __builtin_fmaf(k, -2.f, 1.f)) < 0.f ? k - 1.f : k;  // u < thr[k]
+}
+__device__ __forceinline__ int unorm_code(float v) { return (int)unorm_codef(v); }
+
+__device__ __forceinline__ float unorm_decf(float fk) {
+    const float r = 1.f / 255.f;
     const float q = fk * r;
     return __builtin_fmaf(__builtin_fmaf(-q, 255.f, fk), r, q);
 }
+__device__ __forceinline__ float unorm_dec(int k) { return unorm_decf((float)k); }
 
-// lut[i] is the code of i/4096; at most one threshold lies in each 1/4096 interval, so the
-// code of v is lut[i] or lut[i] + 1 for i = floor(4096 v).
-__device__ __forceinline__ int srgb_code(const float4 *step, const uint8_t *lut, float v, float &dec) {
-    const int i = tmin(tmax((int)(v * 4096.f), 0), 4095);
-    const int k0 = lut[i];
-    const float4 st = step[k0];
+// the step entry of v's interval (v below 0 or NaN takes the first, above 1 the last)
+__device__ __forceinline__ float4 srgb_step(const float4 *step, float v) {
+    const float u = __builtin_amdgcn_fmed3f(v + kQuantShift, kQuantShift, 1.f + kQuantShift);
+    return step[(__float_as_uint(u) >> 16) - kQuantBase];
+}
+__device__ __forceinline__ float srgb_dec(const float4 *step, float v) {
+    const float4 st = srgb_step(step, v);
+    return v >= st.x ? st.z : st.y;
+}
+__device__ __forceinline__ int srgb_code(const float4 *step, float v, float &dec) {
+    const float4 st = srgb_step(step, v);
     const bool up = v >= st.x;
     dec = up ? st.z : st.y;
-    return k0 + (up ? 1 : 0);
+    return (int)__float_as_uint(st.w) + (up ? 1 : 0);
 }
 
 template <bool SRGB>
-__device__ __forceinline__ void blend_dec(const float4 *step, const uint8_t *lut, float *d, const float4 &src, float a) {
+__device__ __forceinline__ void blend_dec(const float4 *step, float *d, const float4 &src, float a) {
     const float oma = 1.f - a;
     const float v0 = src.x * a + d[0] * oma;
     const float v1 = src.y * a + d[1] * oma;
     const float v2 = src.z * a + d[2] * oma;
     const float va = a * a + d[3] * oma;
     if (SRGB) {
-        srgb_code(step, lut, v0, d[0]);
-        srgb_code(step, lut, v1, d[1]);
-        srgb_code(step, lut, v2, d[2]);
+        d[0] = srgb_dec(step, v0);
+        d[1] = srgb_dec(step, v1);
+        d[2] = srgb_dec(step, v2);
     } else {
-        d[0] = unorm_dec(unorm_code(v0));
-        d[1] = unorm_dec(unorm_code(v1));
-        d[2] = unorm_dec(unorm_code(v2));
+        d[0] = unorm_decf(unorm_codef(v0));
+        d[1] = unorm_decf(unorm_codef(v1));
+        d[2] = unorm_decf(unorm_codef(v2));
     }
-    d[3] = unorm_dec(unorm_code(va));
+    d[3] = unorm_decf(unorm_codef(va));
 }
 
 template <bool SRGB>
-__device__ __forceinline__ uint32_t pack_dec(const float4 *step, const uint8_t *lut, const float *d) {
+__device__ __forceinline__ uint32_t pack_dec(const float4 *step, const float *d) {
     uint32_t o = 0u;
     float t;
 #pragma unroll
-    for (int ch = 0; ch < 3; ++ch) o |= (uint32_t)(SRGB ? srgb_code(step, lut, d[ch], t) : unorm_code(d[ch])) << (8 * ch);
+    for (int ch = 0; ch < 3; ++ch) o |= (uint32_t)(SRGB ? srgb_code(step, d[ch], t) : unorm_code(d[ch])) << (8 * ch);
     return o | ((uint32_t)unorm_code(d[3]) << 24);
 }
 
@@ -1053,8 +1066,7 @@ struct CovArgs {
     const uint32_t *ptab;       // per-path blend tables (multisample output)
     const float *dec_c;         // [256] colour decode, for the paint colours
     const float *dec_a;         // [256] alpha decode (gradient ramp texels)
-    const float4 *step_c;       // [256] sRGB steps {thr[k+1], dec[k], dec[k+1], 0}
-    const uint8_t *lut_c;       // [4096] sRGB code of i/4096
+    const float4 *step_c;       // [kQuantSteps] sRGB steps {thr, dec, dec_next, code}
     uint8_t *image;
     int pitch;
     GradDev G;
@@ -1094,19 +1106,17 @@ __device__ __noinline__ void scatter_big(const uint32_t *items, uint32_t ib, int
 // on the 4096-scene batch: 32.7 ms a render against 35.5 ms when capped at four).
 template <int SPP, bool SRGB, int kCovGroup, bool BATCH, bool GRAD>
 __global__ void __launch_bounds__(256, (kCovGroup == 4 || !SRGB) ? 8 : 6) k_composite_cov(CovArgs A) {
-    __shared__ float4 s_step[SRGB ? 256 : 1];
-    __shared__ uint8_t s_lut[SRGB ? 4096 : 4];
+    __shared__ float4 s_step[SRGB ? kQuantSteps : 1];
     __shared__ float s_dec[256];
     __shared__ float s_deca[GRAD ? 256 : 1];
     __shared__ float4 l_src[4][kCovList];
     __shared__ uint2 l_ref[4][kCovList];
     __shared__ uint32_t slot[4][kCovGroup][64];
     for (int i = threadIdx.x; i < 256; i += 256) {
-        if (SRGB) s_step[i] = A.step_c[i];
         s_dec[i] = A.dec_c[i];
         if (GRAD) s_deca[i] = A.dec_a[i];
     }
-    for (int i = threadIdx.x; i < (SRGB ? 1024 : 0); i += 256) ((uint32_t *)s_lut)[i] = ((const uint32_t *)A.lut_c)[i];
+    for (int i = threadIdx.x; i < (SRGB ? kQuantSteps : 0); i += 256) s_step[i] = A.step_c[i];
     __syncthreads();
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     int W = A.W, H = A.H, tiles_x = A.tiles_x, row0 = 0, pitch = A.pitch;
@@ -1229,11 +1239,11 @@ __global__ void __launch_bounds__(256, (kCovGroup == 4 || !SRGB) ? 8 : 6) k_comp
                         const int ix0 = (int)(ent2[j] & 0xFFFFu), iw = (int)(ent2[j] >> 16);
                         const float4 p0 = grad_color(A.G, c, ix0, iw, x, 2 * r, s_dec, s_deca);
                         const float4 p1 = grad_color(A.G, c, ix0, iw, x, 2 * r + 1, s_dec, s_deca);
-                        blend_dec<SRGB>(s_step, s_lut, d0, p0, p0.w * ((float)(e & 63u) / (float)SPP));
-                        blend_dec<SRGB>(s_step, s_lut, d1, p1, p1.w * ((float)((e >> 8) & 63u) / (float)SPP));
+                        blend_dec<SRGB>(s_step, d0, p0, p0.w * ((float)(e & 63u) / (float)SPP));
+                        blend_dec<SRGB>(s_step, d1, p1, p1.w * ((float)((e >> 8) & 63u) / (float)SPP));
                     } else {
-                        blend_dec<SRGB>(s_step, s_lut, d0, src, src.w * ((float)(e & 63u) / (float)SPP));
-                        blend_dec<SRGB>(s_step, s_lut, d1, src, src.w * ((float)((e >> 8) & 63u) / (float)SPP));
+                        blend_dec<SRGB>(s_step, d0, src, src.w * ((float)(e & 63u) / (float)SPP));
+                        blend_dec<SRGB>(s_step, d1, src, src.w * ((float)((e >> 8) & 63u) / (float)SPP));
                     }
                 }
             }
@@ -1274,8 +1284,8 @@ __global__ void __launch_bounds__(256, (kCovGroup == 4 || !SRGB) ? 8 : 6) k_comp
 
     if (x >= W) return;
     const int y0 = 2 * r;
-    *(uint32_t *)(image + (size_t)y0 * pitch + (size_t)x * 4) = pack_dec<SRGB>(s_step, s_lut, d0);
-    if (y0 + 1 < H) *(uint32_t *)(image + (size_t)(y0 + 1) * pitch + (size_t)x * 4) = pack_dec<SRGB>(s_step, s_lut, d1);
+    *(uint32_t *)(image + (size_t)y0 * pitch + (size_t)x * 4) = pack_dec<SRGB>(s_step, d0);
+    if (y0 + 1 < H) *(uint32_t *)(image + (size_t)(y0 + 1) * pitch + (size_t)x * 4) = pack_dec<SRGB>(s_step, d1);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1408,7 +1418,7 @@ template <> struct SampleRegs<16> {
 template <bool SRGB>
 __global__ void __launch_bounds__(256) k_paint_tables(uint32_t P, const uint32_t *__restrict__ finfo,
                                                       const float *__restrict__ dec, const float4 *__restrict__ step,
-                                                      const uint8_t *__restrict__ lut, uint32_t *__restrict__ ptab) {
+                                                      uint32_t *__restrict__ ptab) {
     const uint32_t path = blockIdx.x * 4u + (threadIdx.x >> 6);
     if (path >= P) return;
     const uint32_t c = finfo[path];
@@ -1427,9 +1437,9 @@ __global__ void __launch_bounds__(256) k_paint_tables(uint32_t P, const uint32_t
         const float v2 = src.z * a + dk * oma;
         const float va = a * a + unorm_dec(k) * oma;
         float t;
-        const uint32_t c0 = SRGB ? (uint32_t)srgb_code(step, lut, v0, t) : (uint32_t)unorm_code(v0);
-        const uint32_t c1 = SRGB ? (uint32_t)srgb_code(step, lut, v1, t) : (uint32_t)unorm_code(v1);
-        const uint32_t c2 = SRGB ? (uint32_t)srgb_code(step, lut, v2, t) : (uint32_t)unorm_code(v2);
+        const uint32_t c0 = SRGB ? (uint32_t)srgb_code(step, v0, t) : (uint32_t)unorm_code(v0);
+        const uint32_t c1 = SRGB ? (uint32_t)srgb_code(step, v1, t) : (uint32_t)unorm_code(v1);
+        const uint32_t c2 = SRGB ? (uint32_t)srgb_code(step, v2, t) : (uint32_t)unorm_code(v2);
         e[0] |= c0 << (8 * j);
         e[1] |= c1 << (8 * j);
         e[2] |= c2 << (8 * j);
@@ -1451,7 +1461,7 @@ __device__ __forceinline__ uint32_t table_code(const uint32_t *T, uint32_t st) {
 // One sample's framebuffer code blended with paint src (decoded colour, alpha a) and
 // re-quantised: the arithmetic of blend_dec on the decoded code.
 template <bool SRGB>
-__device__ __forceinline__ uint32_t blend_code(const float4 *step, const uint8_t *lut, const float *dec, uint32_t code,
+__device__ __forceinline__ uint32_t blend_code(const float4 *step, const float *dec, uint32_t code,
                                                const float4 &src, float a) {
     const float oma = 1.f - a;
     const uint32_t k0 = code & 0xFFu, k1 = (code >> 8) & 0xFFu, k2 = (code >> 16) & 0xFFu;
@@ -1464,9 +1474,9 @@ __device__ __forceinline__ uint32_t blend_code(const float4 *step, const uint8_t
     const float v2 = src.z * a + d2 * oma;
     const float va = a * a + da * oma;
     float t;
-    const uint32_t c0 = SRGB ? (uint32_t)srgb_code(step, lut, v0, t) : (uint32_t)unorm_code(v0);
-    const uint32_t c1 = SRGB ? (uint32_t)srgb_code(step, lut, v1, t) : (uint32_t)unorm_code(v1);
-    const uint32_t c2 = SRGB ? (uint32_t)srgb_code(step, lut, v2, t) : (uint32_t)unorm_code(v2);
+    const uint32_t c0 = SRGB ? (uint32_t)srgb_code(step, v0, t) : (uint32_t)unorm_code(v0);
+    const uint32_t c1 = SRGB ? (uint32_t)srgb_code(step, v1, t) : (uint32_t)unorm_code(v1);
+    const uint32_t c2 = SRGB ? (uint32_t)srgb_code(step, v2, t) : (uint32_t)unorm_code(v2);
     return c0 | (c1 << 8) | (c2 << 16) | ((uint32_t)unorm_code(va) << 24);
 }
 
@@ -1522,8 +1532,7 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
     constexpr int NREG = 64 / CPR;
     constexpr int G = GRAD ? 4 : 2;
     constexpr uint32_t FULL = SPP == 8 ? 0xFFFFu : 0xFFFFFFFFu;  // both rows' bits (N = 32: each row)
-    __shared__ float4 s_step[SRGB ? 256 : 1];
-    __shared__ uint8_t s_lut[SRGB ? 4096 : 4];
+    __shared__ float4 s_step[SRGB ? kQuantSteps : 1];
     __shared__ float s_dec[256];
     __shared__ float s_deca[GRAD ? 256 : 1];
     __shared__ float4 l_src[4][kCovList];
@@ -1532,11 +1541,10 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
     __shared__ uint32_t slot[4][G][64];
     __shared__ uint32_t tbl[4][G][256];
     for (int i = threadIdx.x; i < 256; i += 256) {
-        if (SRGB) s_step[i] = A.step_c[i];
         s_dec[i] = A.dec_c[i];
         if (GRAD) s_deca[i] = A.dec_a[i];
     }
-    for (int i = threadIdx.x; i < (SRGB ? 1024 : 0); i += 256) ((uint32_t *)s_lut)[i] = ((const uint32_t *)A.lut_c)[i];
+    for (int i = threadIdx.x; i < (SRGB ? kQuantSteps : 0); i += 256) s_step[i] = A.step_c[i];
     __syncthreads();
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int W = A.W, H = A.H, tiles_x = A.tiles_x;
@@ -1663,7 +1671,7 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
                         const uint32_t e = (uint32_t)__shfl((int)ceg, c, 64);
                         const float4 pa = grad_color(A.G, __float_as_uint(src.x), (int)(e & 0xFFFFu), (int)(e >> 16),
                                                      tx0 + c, 2 * r + dy, s_dec, s_deca);
-                        const uint32_t nst = blend_code<SRGB>(s_step, s_lut, s_dec, st, pa, pa.w);
+                        const uint32_t nst = blend_code<SRGB>(s_step, s_dec, st, pa, pa.w);
                         return covers(p) ? nst : st;
                     });
                 }
@@ -1731,7 +1739,7 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
             }
             const float avg = sum / (float)SPP;
             float tmp;
-            const uint32_t code = (SRGB && ch < 3) ? (uint32_t)srgb_code(s_step, s_lut, avg, tmp) : (uint32_t)unorm_code(avg);
+            const uint32_t code = (SRGB && ch < 3) ? (uint32_t)srgb_code(s_step, avg, tmp) : (uint32_t)unorm_code(avg);
             uint32_t word = code << (8 * ch);
             word |= (uint32_t)__shfl_xor((int)word, 1, 64);
             word |= (uint32_t)__shfl_xor((int)word, 2, 64);
@@ -1762,13 +1770,13 @@ __global__ void k_row_records(int64_t NB, const uint32_t *__restrict__ n_ptr, co
 // decoded values of the codes.
 template <bool SRGB>
 __global__ void k_encode_values(int64_t n, const float *__restrict__ v, const float4 *__restrict__ step,
-                                const uint8_t *__restrict__ lut, uint8_t *__restrict__ code, float *__restrict__ dec) {
+                                uint8_t *__restrict__ code, float *__restrict__ dec) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     float d;
     int k;
     if (SRGB) {
-        k = srgb_code(step, lut, v[i], d);
+        k = srgb_code(step, v[i], d);
     } else {
         k = unorm_code(v[i]);
         d = unorm_dec(k);
@@ -1780,7 +1788,7 @@ __global__ void k_encode_values(int64_t n, const float *__restrict__ v, const fl
 // Exhaustive comparison of the device requantisation with the threshold tables over every
 // float bit pattern in [lo, hi): counts disagreements of code or decoded value.
 template <bool SRGB>
-__global__ void k_encode_sweep(uint32_t lo, uint32_t hi, const float4 *__restrict__ step, const uint8_t *__restrict__ lut,
+__global__ void k_encode_sweep(uint32_t lo, uint32_t hi, const float4 *__restrict__ step,
                                const float *__restrict__ thr, const float *__restrict__ dec, unsigned long long *bad) {
     unsigned long long nbad = 0;
     for (uint64_t b = (uint64_t)lo + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; b < hi;
@@ -1793,7 +1801,7 @@ __global__ void k_encode_sweep(uint32_t lo, uint32_t hi, const float4 *__restric
         float d;
         int k;
         if (SRGB) {
-            k = srgb_code(step, lut, v, d);
+            k = srgb_code(step, v, d);
         } else {
             k = unorm_code(v);
             d = unorm_dec(k);
@@ -1956,7 +1964,7 @@ void launch_composite(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t
         CovArgs C;
         C.W = f.W; C.H = f.H; C.tiles_x = tiles_x;
         C.rowbeg = f.rowbeg; C.rowend = f.rowend; C.rrec = f.rrec; C.rtile = f.rtile;
-        C.items = f.items; C.icov = f.icov; C.imask = nullptr; C.rpath = nullptr; C.ptab = nullptr; C.dec_c = t.dec_c; C.dec_a = t.dec_a; C.step_c = t.step_c; C.lut_c = t.lut_c;
+        C.items = f.items; C.icov = f.icov; C.imask = nullptr; C.rpath = nullptr; C.ptab = nullptr; C.dec_c = t.dec_c; C.dec_a = t.dec_a; C.step_c = t.step_c;
         C.image = f.image; C.pitch = f.pitch;
         C.G = f.grad;
         C.nscenes = f.nscenes; C.ntiles = ntiles; C.stile = f.stile; C.simg = f.simg;
@@ -1990,17 +1998,17 @@ void launch_composite(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t
     C.W = f.W; C.H = f.H; C.tiles_x = tiles_x;
     C.rowbeg = f.rowbeg; C.rowend = f.rowend; C.rrec = f.rrec; C.rtile = f.rtile;
     C.items = f.items; C.icov = f.icov; C.imask = f.imask; C.rpath = f.rpath; C.ptab = f.ptab;
-    C.dec_c = t.dec_c; C.dec_a = t.dec_a; C.step_c = t.step_c; C.lut_c = t.lut_c;
+    C.dec_c = t.dec_c; C.dec_a = t.dec_a; C.step_c = t.step_c;
     C.image = f.image; C.pitch = f.pitch;
     C.G = f.grad;
     C.nscenes = 0; C.ntiles = ntiles; C.stile = nullptr; C.simg = nullptr;
     if (sc.P) {
         if (f.srgb)
             hipLaunchKernelGGL(k_paint_tables<true>, dim3(blocks_for(sc.P, 4)), dim3(256), 0, s, (uint32_t)sc.P, sc.finfo,
-                               t.dec_c, t.step_c, t.lut_c, f.ptab);
+                               t.dec_c, t.step_c, f.ptab);
         else
             hipLaunchKernelGGL(k_paint_tables<false>, dim3(blocks_for(sc.P, 4)), dim3(256), 0, s, (uint32_t)sc.P, sc.finfo,
-                               t.dec_c, t.step_c, t.lut_c, f.ptab);
+                               t.dec_c, t.step_c, f.ptab);
     }
     dim3 g(8u * blocks_for((int64_t)tiles_x * ((R + 7) / 8), 4)), b(256);
 #define SL_LAUNCH(N)                                                                                    \
@@ -2024,9 +2032,9 @@ void launch_encode_values(const Tables &t, int channel, const float *v, int64_t 
     if (n <= 0) return;
     dim3 g(blocks_for(n, 256)), b(256);
     if (channel == 0 && t.srgb)
-        hipLaunchKernelGGL(k_encode_values<true>, g, b, 0, s, n, v, t.step_c, t.lut_c, code, dec);
+        hipLaunchKernelGGL(k_encode_values<true>, g, b, 0, s, n, v, t.step_c, code, dec);
     else
-        hipLaunchKernelGGL(k_encode_values<false>, g, b, 0, s, n, v, t.step_c, t.lut_c, code, dec);
+        hipLaunchKernelGGL(k_encode_values<false>, g, b, 0, s, n, v, t.step_c, code, dec);
 }
 
 void launch_encode_sweep(const Tables &t, int channel, uint32_t lo, uint32_t hi, unsigned long long *bad,
@@ -2036,9 +2044,9 @@ void launch_encode_sweep(const Tables &t, int channel, uint32_t lo, uint32_t hi,
     const float *thr = channel == 0 ? t.thr_c : t.thr_a;
     const float *dec = channel == 0 ? t.dec_c : t.dec_a;
     if (srgb)
-        hipLaunchKernelGGL(k_encode_sweep<true>, dim3(8192), dim3(256), 0, s, lo, hi, t.step_c, t.lut_c, thr, dec, bad);
+        hipLaunchKernelGGL(k_encode_sweep<true>, dim3(8192), dim3(256), 0, s, lo, hi, t.step_c, thr, dec, bad);
     else
-        hipLaunchKernelGGL(k_encode_sweep<false>, dim3(8192), dim3(256), 0, s, lo, hi, t.step_c, t.lut_c, thr, dec, bad);
+        hipLaunchKernelGGL(k_encode_sweep<false>, dim3(8192), dim3(256), 0, s, lo, hi, t.step_c, thr, dec, bad);
 }
 
 void launch_debug_draw_list(const SceneDev &sc, const Tables &t, Frame &f, const uint32_t *moff, const uint32_t *ioff,

@@ -106,22 +106,29 @@ bool build_color_tables(int srgb, ColorTables &t) {
             t.thr[k] = smallest_float_at_least(srgb ? srgb_to_linear(mid) : mid);
         }
     }
-    // lut[i] = code of i/4096; valid only if no bucket (i/4096, (i+1)/4096) holds more
-    // than one threshold, which the check below enforces.
-    int k = 0;
-    for (int i = 0; i < 4096; ++i) {
-        const float lo = (float)i / 4096.f;
-        while (k < 255 && lo >= t.thr[k + 1]) ++k;
-        t.lut[i] = (uint8_t)k;
-        const float hi = (float)(i + 1) / 4096.f;
-        int inside = 0;
-        for (int j = k + 1; j < 256; ++j) {
-            if (t.thr[j] > lo && t.thr[j] < hi) ++inside;
-            if (t.thr[j] >= hi) break;
-        }
-        if (inside > 1) return false;
+    if (!srgb) {  // UNORM codes are computed, not looked up
+        std::memset(t.step, 0, sizeof t.step);
+        return true;
     }
-    return true;
+    // the interval of a threshold, by the float operations of the device
+    auto interval = [](float v) {
+        const float u = v + kQuantShift;
+        uint32_t b;
+        std::memcpy(&b, &u, 4);
+        return (int)(b >> 16) - (int)kQuantBase;
+    };
+    int k = 0;
+    for (int i = 0; i < kQuantSteps; ++i) {
+        // k: the code at the interval's start, one more after each earlier interval's threshold
+        const bool in = k < 255 && interval(t.thr[k + 1]) == i;
+        t.step[i].thr = in ? t.thr[k + 1] : INFINITY;
+        t.step[i].dec = t.dec[k];
+        t.step[i].dec_next = t.dec[k < 255 ? k + 1 : 255];
+        t.step[i].code = (uint32_t)k;
+        if (in) ++k;
+        if (k < 255 && interval(t.thr[k + 1]) <= i) return false;  // two thresholds in one interval
+    }
+    return k == 255;
 }
 
 }  // namespace sl
