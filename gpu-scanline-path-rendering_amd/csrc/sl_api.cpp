@@ -36,9 +36,8 @@ struct DevBuf {
 struct Arena {
     DevBuf b_pcnt, b_nchain, b_choff, b_chains, b_chain_t;
     DevBuf b_tvtx, b_pflags, b_prow, b_crec, b_cfrag, b_coff, b_ts, b_pnb, b_pbase, b_binfo, b_bcount,
-        b_boff, b_bwsum, b_bcarry, b_rec_meta, b_rec_mask, b_scratch, b_items, b_imask, b_icov, b_bicnt, b_bmcnt,
-        b_bext, b_big_list, b_small, b_nz_flag, b_nz_off, b_nzk0, b_nzk1, b_nzv0, b_nzv1, b_rs_hist, b_rs_hoff,
-        b_rowbeg, b_rowend, b_rrec, b_btile, b_rtile, b_rpath, b_ptab, b_image, b_scan_tmp, b_lcount;
+        b_boff, b_bwsum, b_bcarry, b_rec_meta, b_rec_mask, b_scratch, b_items, b_imask, b_icov, b_prec, b_brec, b_big_list, b_small, b_nz_flag, b_nz_off, b_nzk0, b_nzk1, b_nzv0, b_nzv1, b_rs_hist, b_rs_hoff,
+        b_rowbeg, b_rowend, b_rrec, b_rtile, b_rext, b_ptab, b_image, b_scan_tmp, b_lcount;
     // carving state: non-null base = every array comes from [base, base + cap)
     uint8_t *carve_base = nullptr;
     size_t carve_cap = 0, carve_off = 0;
@@ -523,37 +522,36 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
         (rc = ensure_in(h, A, A.b_boff, ((size_t)NB + 1) * 4)) || (rc = ensure_in(h, A, A.b_bwsum, ((size_t)NB + 1) * 4)) ||
         (rc = ensure_in(h, A, A.b_bcarry, ((size_t)NB + 1) * 4)) ||
         (rc = ensure_in(h, A, A.b_rec_meta, (size_t)F * 4)) || (rc = ensure_in(h, A, A.b_rec_mask, (size_t)F * 4 * NW)) ||
-        (rc = ensure_in(h, A, A.b_scratch, (size_t)F * 8)) || (rc = ensure_in(h, A, A.b_items, (size_t)F * 8)) ||
-        (rc = ensure_in(h, A, A.b_imask, (carved && !f.keep_masks) ? 0 : (size_t)F * 8 * NW)) || (rc = ensure_in(h, A, A.b_icov, (size_t)F * 8)) || (rc = ensure_in(h, A, A.b_bicnt, ((size_t)NB + 1) * 4)) ||
-        (rc = ensure_in(h, A, A.b_bmcnt, ((size_t)NB + 1) * 4)) || (rc = ensure_in(h, A, A.b_bext, (size_t)NB * 4)) ||
+        (rc = ensure_in(h, A, A.b_scratch, (size_t)F * 4)) || (rc = ensure_in(h, A, A.b_items, h->debug ? (size_t)F * 8 : 0)) ||
+        (rc = ensure_in(h, A, A.b_imask, f.keep_masks ? (size_t)F * 4 * NW : 0)) || (rc = ensure_in(h, A, A.b_icov, (size_t)F * 4)) ||
+        (rc = ensure_in(h, A, A.b_prec, (size_t)F * 16)) || (rc = ensure_in(h, A, A.b_brec, (size_t)NB * 32)) ||
         (rc = ensure_in(h, A, A.b_big_list, (size_t)NB * 4)) || (rc = ensure_in(h, A, A.b_nz_flag, ((size_t)NB + 1) * 4)) ||
         (rc = ensure_in(h, A, A.b_nz_off, ((size_t)NB + 1) * 4)) || (rc = ensure_in(h, A, A.b_nzk0, (size_t)NB * 4)) ||
         (rc = ensure_in(h, A, A.b_nzk1, (size_t)NB * 4)) || (rc = ensure_in(h, A, A.b_nzv0, (size_t)NB * 4)) ||
         (rc = ensure_in(h, A, A.b_nzv1, (size_t)NB * 4)) || (rc = ensure_in(h, A, A.b_rs_hist, 256 * rs_tiles * 4 + 16)) ||
         (rc = ensure_in(h, A, A.b_rs_hoff, (256 * rs_tiles + 1) * 4 + 16)) || (rc = ensure_in(h, A, A.b_rowbeg, R * 4)) ||
         (rc = ensure_in(h, A, A.b_rowend, R * 4)) || (rc = ensure_in(h, A, A.b_rrec, (size_t)NB * 16)) ||
-        (rc = ensure_in(h, A, A.b_btile, (size_t)NB * 8)) || (rc = ensure_in(h, A, A.b_rtile, (size_t)NB * 8)) ||
-        (rc = ensure_in(h, A, A.b_rpath, f.ms ? (size_t)NB * 4 : 0)) || (rc = ensure_in(h, A, A.b_ptab, f.ms ? (size_t)P * 1024 : 0)) ||
+        (rc = ensure_in(h, A, A.b_rtile, (size_t)NB * 16)) ||
+        (rc = ensure_in(h, A, A.b_rext, (size_t)NB * 4)) || (rc = ensure_in(h, A, A.b_ptab, f.ms ? (size_t)P * 1024 : 0)) ||
         (rc = ensure_in(h, A, A.b_scan_tmp, scan_need * 4)))
         return rc;
     f.binfo = P_<int2>(A.b_binfo); f.bcount = P_<uint32_t>(A.b_bcount); f.boff = P_<uint32_t>(A.b_boff);
     f.bwsum = P_<uint32_t>(A.b_bwsum); f.bcarry = P_<uint32_t>(A.b_bcarry);
     f.rec_meta = P_<uint32_t>(A.b_rec_meta); f.rec_mask = P_<uint32_t>(A.b_rec_mask);
-    f.scratch_keys = P_<uint32_t>(A.b_scratch); f.items = P_<uint32_t>(A.b_items); f.imask = P_<uint32_t>(A.b_imask);
-    f.icov = P_<uint32_t>(A.b_icov);
-    // the rank array lives in the large-bucket scratch (used only later, by the resolve);
-    // the winding scan's output lives in the item masks the resolve overwrites
+    f.scratch_keys = P_<uint32_t>(A.b_scratch); f.items = h->debug ? P_<uint32_t>(A.b_items) : nullptr;
+    f.imask = P_<uint32_t>(A.b_imask);
+    f.icov = P_<uint32_t>(A.b_icov); f.prec = P_<uint4>(A.b_prec);
+    // the rank array lives in the large-bucket scratch (used only later, by the resolve)
     f.frank = f.scratch_keys;
-    f.bicnt = P_<uint32_t>(A.b_bicnt); f.bmcnt = P_<uint32_t>(A.b_bmcnt); f.bext = P_<uint32_t>(A.b_bext);
+    f.brec = P_<uint4>(A.b_brec);
     f.big_list = P_<uint32_t>(A.b_big_list); f.nz_flag = P_<uint32_t>(A.b_nz_flag); f.nz_off = P_<uint32_t>(A.b_nz_off);
     f.nz_keys[0] = P_<uint32_t>(A.b_nzk0); f.nz_keys[1] = P_<uint32_t>(A.b_nzk1);
     f.nz_vals[0] = P_<uint32_t>(A.b_nzv0); f.nz_vals[1] = P_<uint32_t>(A.b_nzv1);
     f.rs_hist = P_<uint32_t>(A.b_rs_hist); f.rs_hoff = P_<uint32_t>(A.b_rs_hoff);
     f.rowbeg = P_<uint32_t>(A.b_rowbeg); f.rowend = P_<uint32_t>(A.b_rowend);
     f.rrec = P_<uint4>(A.b_rrec);
-    f.btile = P_<uint64_t>(A.b_btile);
-    f.rtile = P_<uint64_t>(A.b_rtile);
-    f.rpath = f.ms ? P_<uint32_t>(A.b_rpath) : nullptr;
+    f.rtile = P_<ulonglong2>(A.b_rtile);
+    f.rext = P_<uint32_t>(A.b_rext);
     f.ptab = f.ms ? P_<uint32_t>(A.b_ptab) : nullptr;
     f.scan_tmp = P_<uint32_t>(A.b_scan_tmp);
 
@@ -595,7 +593,7 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
     // element counts (M, S) and the error flag
     unsigned long long *red = (unsigned long long *)(P_<uint32_t>(A.b_small) + 4);
     sl::launch_fill_u32((uint32_t *)red, 0u, 4, s);
-    sl::launch_count_reduce(f.bmcnt, f.bicnt, NB, red, s);
+    sl::launch_count_reduce(f.brec, NB, red, s);
     if (deferred) {
         HIPCHK(h, hipMemcpyAsync(h->fstat, A.b_small.p, 32, hipMemcpyDeviceToHost, s));
         h->stat_pending = true;
@@ -638,8 +636,9 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
         if (!r2) {
             sl::launch_debug_fragments(sc, tb, f, P_<int32_t>(dyx), P_<int32_t>(dpid), P_<int8_t>(dwn),
                                        P_<uint32_t>(dmask), s);
-            sl::scan_exclusive_u32(f.bmcnt, P_<uint32_t>(dmoff), NB, f.scan_tmp, s);
-            sl::scan_exclusive_u32(f.bicnt, P_<uint32_t>(dioff), NB, f.scan_tmp, s);
+            sl::launch_debug_counts(f, f.bcount, f.bwsum, s);  // the frame is done with both arrays
+            sl::scan_exclusive_u32(f.bcount, P_<uint32_t>(dmoff), NB, f.scan_tmp, s);
+            sl::scan_exclusive_u32(f.bwsum, P_<uint32_t>(dioff), NB, f.scan_tmp, s);
             sl::launch_debug_draw_list(sc, tb, f, P_<uint32_t>(dmoff), P_<uint32_t>(dioff), P_<int4>(ddraw),
                                        P_<uint32_t>(dmm), s);
             r2 = check_launch(h, "debug");
@@ -663,8 +662,9 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
             h->d_boff.resize((size_t)NB + 1); h->d_rowkeys.resize(NZ); h->d_rowvals.resize(NZ);
             h->d_rowbeg.resize(R); h->d_rowend.resize(R);
             if (e == hipSuccess) e = hipMemcpy(h->d_binfo.data(), f.binfo, (size_t)NB * 8, hipMemcpyDeviceToHost);
-            if (e == hipSuccess) e = hipMemcpy(h->d_bicnt.data(), f.bicnt, (size_t)NB * 4, hipMemcpyDeviceToHost);
-            if (e == hipSuccess) e = hipMemcpy(h->d_bext.data(), f.bext, (size_t)NB * 4, hipMemcpyDeviceToHost);
+            if (e == hipSuccess) e = hipMemcpy2D(h->d_bicnt.data(), 4, (const uint32_t *)f.brec + 6, 32, 4, (size_t)NB, hipMemcpyDeviceToHost);
+            if (e == hipSuccess)  // the extent is the record's first word
+                e = hipMemcpy2D(h->d_bext.data(), 4, f.brec, 32, 4, (size_t)NB, hipMemcpyDeviceToHost);
             if (e == hipSuccess) e = hipMemcpy(h->d_boff.data(), f.boff, ((size_t)NB + 1) * 4, hipMemcpyDeviceToHost);
             if (e == hipSuccess && NZ) e = hipMemcpy(h->d_rowkeys.data(), f.nz_keys[0], (size_t)NZ * 4, hipMemcpyDeviceToHost);
             if (e == hipSuccess && NZ) e = hipMemcpy(h->d_rowvals.data(), f.nz_vals[0], (size_t)NZ * 4, hipMemcpyDeviceToHost);
@@ -763,10 +763,10 @@ int sl_destroy(sl_handle *h) {
                       &h->ptable[0], &h->ptable[1], &h->ptable[2], &h->ctab[0], &h->ctab[1], &h->A.b_tvtx, &h->A.b_pflags,
                       &h->A.b_prow, &h->A.b_crec, &h->A.b_cfrag, &h->A.b_coff, &h->A.b_ts, &h->A.b_pnb, &h->A.b_pbase,
                       &h->A.b_binfo, &h->A.b_bcount, &h->A.b_boff, &h->A.b_bwsum, &h->A.b_bcarry, &h->A.b_rec_meta,
-                      &h->A.b_rec_mask, &h->A.b_scratch, &h->A.b_items, &h->A.b_imask, &h->A.b_icov, &h->A.b_bicnt, &h->A.b_bmcnt, &h->A.b_bext,
+                      &h->A.b_rec_mask, &h->A.b_scratch, &h->A.b_items, &h->A.b_imask, &h->A.b_icov, &h->A.b_prec, &h->A.b_brec,
                       &h->A.b_big_list, &h->A.b_small, &h->A.b_nz_flag, &h->A.b_nz_off, &h->A.b_nzk0, &h->A.b_nzk1, &h->A.b_nzv0,
                       &h->A.b_nzv1, &h->A.b_rs_hist, &h->A.b_rs_hoff, &h->A.b_rowbeg, &h->A.b_rowend, &h->A.b_image, &h->A.b_scan_tmp,
-                      &h->A.b_rrec, &h->A.b_btile, &h->A.b_rtile, &h->A.b_rpath, &h->A.b_ptab, &h->A.b_lcount, &h->pcanvas, &h->stile, &h->simg, &h->sfirst, &h->scarry,
+                      &h->A.b_rrec, &h->A.b_rtile, &h->A.b_rext, &h->A.b_ptab, &h->A.b_lcount, &h->pcanvas, &h->stile, &h->simg, &h->sfirst, &h->scarry,
                       &h->gramp, &h->gtable, &h->chord_keys};
     for (DevBuf *b : bufs) release(*b);
     if (h->fstat) (void)hipHostFree(h->fstat);
@@ -1804,7 +1804,7 @@ int sl_batch_tune(sl_batch *b, int reps, double *best_ms) {
     // bucket group, fragment block size
     const int rg[] = {4096, 16384, 65536};
     const int cg[] = {1024, 4096};
-    const int gg[] = {4, 8};
+    const int gg[] = {4};
     const int fbk[] = {128, 256};
     hipEvent_t e0, e1;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)

@@ -113,15 +113,14 @@ struct Frame {
     uint32_t *frank;         // [F] rank of each fragment in its bucket (~0: none)
     uint32_t *rec_meta;      // [F] (valid fragments only are written)
     uint32_t *rec_mask;      // [F * words]
-    uint32_t *scratch_keys;  // [F] sort keys of large buckets
-    // resolve outputs, per bucket and per item slot (2 slots per valid fragment)
-    uint32_t *items;         // [2F]
-    uint32_t *imask;         // [2F * words]
-    uint32_t *icov;          // [2F] per merged item: sample counts of its 4 pixels
-    uint32_t *bicnt;         // [NB+1]
-    uint32_t *bmcnt;         // [NB+1]
-    uint32_t *bext;          // [NB]
-    uint64_t *btile;         // [NB] 64-pixel tiles of the row holding items
+    uint32_t *scratch_keys;  // [F] sorted fragment order of the largest buckets
+    // resolve outputs, at each bucket's stretch of the fragments (see sl_resolve.hip)
+    uint32_t *items;         // [2F] item lists (parity dumps only, else null)
+    uint32_t *imask;         // [F * words] masks of merged cells
+    uint32_t *icov;          // [F] sample counts of a merged cell's 4 pixels
+    uint4 *prec;             // [F] records of tiles holding merged cells
+    uint4 *brec;             // [2 NB] {extent, records, tiles with a record (64 bits)},
+                             //   {tiles wholly inside a span (64 bits), items, merged cells}
     uint32_t *big_list;      // [NB] buckets with more than 64 fragments
     uint32_t *big_count;     // [1]
     uint32_t *err_flag;      // [1]
@@ -145,9 +144,9 @@ struct Frame {
     int resolve_grid, class_grid, comp_group, frag_block;
     uint32_t *rowbeg;        // [R]
     uint32_t *rowend;        // [R]
-    uint4 *rrec;             // [NB] row-list records {extent, colour, items, item base}
-    uint64_t *rtile;         // [NB] row-list tile masks
-    uint32_t *rpath;         // [NB] row-list path ids (multisample output)
+    uint32_t *rext;          // [NB] row-list extents
+    uint4 *rrec;             // [NB] row-list records {colour, records, base, path}
+    ulonglong2 *rtile;       // [NB] row-list tile bitmaps {with a record, inside a span}
     uint32_t *ptab;          // [P][256] per-path blend tables (multisample output)
     uint8_t *image;          // [H * pitch]
     int pitch;
@@ -221,7 +220,8 @@ void launch_debug_fragments(const SceneDev &sc, const Tables &t, Frame &f, int32
                             int8_t *wn, uint32_t *mask4, hipStream_t s);
 void launch_debug_draw_list(const SceneDev &sc, const Tables &t, Frame &f, const uint32_t *moff,
                             const uint32_t *ioff, int4 *draw, uint32_t *mmask4, hipStream_t s);
-// out[0] += sum of a, out[1] += sum of c
-void launch_count_reduce(const uint32_t *a, const uint32_t *c, size_t n, unsigned long long *out, hipStream_t s);
+// out[0] += merged cells, out[1] += items
+void launch_count_reduce(const uint4 *brec, size_t n, unsigned long long *out, hipStream_t s);
+void launch_debug_counts(const Frame &f, uint32_t *merged, uint32_t *items, hipStream_t s);
 
 }  // namespace sl

@@ -6,12 +6,19 @@
 // k_gen_stencil_block_boundary (.cu:554-786) and k_gen_gl_merged_fragment_and_span
 // (.cu:789-868).
 //
-// Item encoding (one u32 per item; a bucket's items are disjoint and stored in x order,
-// i.e. the span that ends at a cell precedes the cell's merged fragment -- the reference's
-// draw list emits the pair the other way round, which the draw-list dump restores):
-//   bits 0-15  x of the first pixel
-//   bits 16-31 span width in pixels, 0 for a merged 2x2 fragment (its mask is stored at
-//              the same slot of `imask`).
+// What a bucket leaves for the compositors, at its own stretch of arrays indexed by fragment
+// (base = boff[bucket]; it has at most as many merged cells as fragments):
+//   icov / imask [base + m]  sample counts / mask of its m-th merged 2x2 cell, in x order;
+//   prec [base + e]          per 64-pixel tile holding merged cells, in x order: {cells
+//                            covered by a span or merged, merged cells (bit c: the tile's
+//                            c-th 2-pixel cell), merged cells before the tile, tile | a span
+//                            runs on past the tile << 31 (kept for buckets wider than 63 tiles)};
+//   brec [2 bucket, + 1]     {extent, records, tiles with a record (64 bits)}, {tiles wholly
+//                            inside a span (64 bits), items, merged cells}; bit k is the k-th
+//                            tile from the extent's first, bit 63 that tile or any beyond.
+// A column finds its covering item with two bit tests, and a merged cell's index with one
+// population count.  For the parity dumps a bucket's items are also listed (one u32 each, x
+// of the first pixel | span width << 16, 0 for a merged cell).
 #include "sl_device.h"
 #include "sl_internal.h"
 #include "sl_tables.h"
@@ -182,35 +189,68 @@ struct ResolveArgs {
     int W;
     const int4 *pcanvas;     // batched scenes: per-path canvas (W, H, row base, scene)
     const uint32_t *scarry;  // batched scenes: winding-scan carry at each scene's first bucket
-    uint32_t *items;
-    uint32_t *imask;         // null when no consumer needs the merged masks
+    uint32_t *items;         // [2F] item lists, null unless parity dumps are on
+    uint32_t *imask;         // written by the KEEP kernels only
     uint32_t *icov;
-    uint32_t *bicnt;
-    uint32_t *bmcnt;
-    uint32_t *bext;
-    uint64_t *btile;         // [NB] 64-pixel tiles holding items, bit k = the k-th tile from the
-                             // one holding the extent's start (bit 63: that tile or any beyond)
+    uint4 *prec;
+    uint4 *brec;
     uint32_t *big_list;
     uint32_t *big_count;
     uint32_t *err;
 };
 
-// 64-pixel tiles spanned by [lo, hi) as bits of a 64-bit mask (all tiles when the canvas
-// is wider than 64 tiles), OR-reduced over the wave into lane 63.
-__device__ __forceinline__ uint64_t tile_bits(int lo, int hi, int tb) {
-    if (lo >= hi) return 0ull;
-    const int t0 = tmin((lo >> 6) - tb, 63), t1 = tmin(((hi - 1) >> 6) - tb, 63);
-    return (~0ull << t0) & (~0ull >> (63 - t1));
+// bits of tiles [t0, t1] counted from tile tb (t0 <= t1), tiles from the 63rd on in bit 63
+__device__ __forceinline__ uint64_t tile_bits(int t0, int t1, int tb) {
+    return (~0ull << tmin(t0 - tb, 63)) & (~0ull >> (63 - tmin(t1 - tb, 63)));
 }
+// cells [c0, c1) of a tile, 0 <= c0 < c1 <= 32
+__device__ __forceinline__ uint32_t cell_bits(int c0, int c1) { return (~0u << c0) & (~0u >> (32 - c1)); }
 
-// The bit a tile starting at tx0 tests in the bitmap of a bucket whose extent starts at
-// exlo (tiles at or beyond the 63rd from the extent's first all test bit 63).
-__device__ __forceinline__ int tile_bit(int tx0, int exlo) { return tmax(tmin((tx0 >> 6) - (exlo >> 6), 63), 0); }
-__device__ __forceinline__ uint64_t wave_or64(uint64_t v) {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane(dpp_scan((int)(uint32_t)v, 0, OpOr()), 63);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane(dpp_scan((int)(uint32_t)(v >> 32), 0, OpOr()), 63);
-    return (uint64_t)lo | ((uint64_t)hi << 32);
-}
+constexpr int kBigStage = 16;  // chunks of 64 fragments staged in LDS
+
+// LDS of the buckets packed in a wave: their two tile bitmaps; of a chunked bucket, the group
+// heads of its chunks
+struct RecLds {
+    unsigned long long et[4], ft[4], heads[kBigStage];
+};
+
+// What a lane contributes to its bucket's records: its group head's merged cell at x (if any)
+// and the span [prev_x + 2, x) before it (if any).  prev_ok: the group before it was merged.
+// A record's run of lanes starts at its leader (the first merged cell of its tile); the cells
+// of a run are disjoint bits, so their union is a sum, taken from a plain prefix sum.
+struct Lane {
+    bool merged, span, prev_ok, leader;
+    int x, prev_x;
+    uint32_t eb;             // its merged cell
+    uint32_t co, cp;         // cells it covers in its own run's tile and (leaders) in the run's before
+    int f0, f1;              // tiles wholly inside the span: [f0, f1]
+    __device__ __forceinline__ void init(bool m, bool s, bool has_prev, int x_, int px, int W) {
+        merged = m;
+        span = s;
+        x = x_;
+        prev_x = px;
+        prev_ok = has_prev && px >= 0 && px < W;
+        leader = merged && !(prev_ok && (px >> 6) == (x >> 6));
+        eb = merged ? 1u << ((x & 63) >> 1) : 0u;
+        co = eb;
+        cp = 0u;
+        f0 = 1;
+        f1 = 0;
+        if (span) {
+            const int a = px + 2, ta = a >> 6, tb = (x - 1) >> 6;
+            const bool pr = prev_ok && (px >> 6) == ta, ow = merged && (x >> 6) == tb;
+            const uint32_t after = pr ? cell_bits((a & 63) >> 1, tmin(x - ta * 64, 64) >> 1) : 0u;
+            const uint32_t before = ow && !(pr && ta == tb) ? cell_bits(ta == tb ? (a & 63) >> 1 : 0, (x & 63) >> 1) : 0u;
+            co |= before;
+            if (leader) cp = after; else co |= after;
+            f0 = pr ? ta + 1 : ta;
+            f1 = ow ? tb - 1 : tb;
+        }
+    }
+    __device__ __forceinline__ int lo() const { return span ? prev_x + 2 : x; }   // first pixel of its items
+    __device__ __forceinline__ int hi() const { return merged ? x + 2 : x; }      // past the last
+};
+
 __device__ __forceinline__ int scan_add(int x) { return dpp_scan(x, 0, OpAdd()); }
 __device__ __forceinline__ int lane63(int x) { return __builtin_amdgcn_readlane(x, 63); }
 
@@ -232,25 +272,109 @@ __device__ __forceinline__ void group_mask(const uint32_t *order, const uint32_t
         }
         st.finish(rule, w_at, res);
     } else {
-        Stencil<NW> st;
-        st.init(w_at);
-        st.add(first, neg0);
-        for (int q = p + 1; q < e; ++q) {
-            const uint32_t iq = order[q];
-            st.add(msk + iq * NW, ((meta[iq] >> 24) & 1u) != 0u);
+        // rare: one word at a time, for eight counters instead of eight a word
+#pragma unroll
+        for (int k = 0; k < NW; ++k) {
+            Stencil<1> st;
+            st.init(w_at);
+            st.add(first + k, neg0);
+            for (int q = p + 1; q < e; ++q) {
+                const uint32_t iq = order[q];
+                st.add(msk + iq * NW + k, ((meta[iq] >> 24) & 1u) != 0u);
+            }
+            st.finish(rule, res + k);
         }
-        st.finish(rule, res);
     }
+}
+
+// A bucket walked in chunks of 64 sorted records: totals, and the cells of the last record,
+// which the next chunk may add to.
+struct Chunks {
+    int nrec = 0, merged = 0, spans = 0, xmin = INT_MAX, xmax = INT_MIN;
+    uint32_t cover = 0u, edge = 0u;
+};
+
+__device__ __forceinline__ void chunks_begin(RecLds &R) {
+    if ((threadIdx.x & 63) == 0) R.et[0] = R.ft[0] = 0ull;
+}
+
+template <int SPP, bool KEEP>
+__device__ __forceinline__ void chunk_emit(const ResolveArgs &A, uint32_t base, const Lane &L, const uint32_t *res,
+                                           RecLds &R, Chunks &K) {
+    constexpr int NW = Words<SPP>::n;
+    const int lane = threadIdx.x & 63;
+    const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+    const uint64_t mm = __ballot(L.merged), sm = __ballot(L.span), lm = __ballot(L.leader);
+    const int mi = K.merged + (int)__popcll(mm & lt), li = (int)__popcll(lm & lt);
+    const uint32_t pe = (uint32_t)scan_add((int)L.eb), pc = (uint32_t)scan_add((int)L.co);
+    uint4 *rec = A.prec + base;
+    // the open record takes the lanes before the first leader; a leader closes it
+    const int f = lm ? (int)__builtin_ctzll(lm) : 64;
+    if (f > 0) {
+        K.edge += (uint32_t)__builtin_amdgcn_readlane((int)pe, f - 1);
+        K.cover += (uint32_t)__builtin_amdgcn_readlane((int)pc, f - 1);
+    }
+    if (lm) {
+        K.cover += (uint32_t)__builtin_amdgcn_readlane((int)L.cp, f);
+        if (lane == 0 && K.nrec > 0) *(uint2 *)&rec[K.nrec - 1].x = make_uint2(K.cover, K.edge);
+        const uint64_t later = lane < 63 ? lm & (~0ull << (lane + 1)) : 0ull;
+        const int last = later ? (int)__builtin_ctzll(later) - 1 : 63;
+        const uint32_t e = (uint32_t)__shfl((int)pe, last, 64) - (pe - L.eb);
+        const uint32_t nc = (uint32_t)__shfl((int)L.cp, (last + 1) & 63, 64);
+        const uint32_t c = (uint32_t)__shfl((int)pc, last, 64) - (pc - L.co) + (later ? nc : 0u);
+        if (L.leader) rec[K.nrec + li] = make_uint4(c, e, (uint32_t)mi, (uint32_t)(L.x >> 6));
+        const int ol = 63 - (int)__builtin_clzll(lm);  // the last leader's record stays open
+        K.cover = (uint32_t)__builtin_amdgcn_readlane((int)c, ol);
+        K.edge = (uint32_t)__builtin_amdgcn_readlane((int)e, ol);
+    }
+    if (mm | sm) {
+        const int first = (int)__builtin_ctzll(mm | sm), last = 63 - (int)__builtin_clzll(mm | sm);
+        K.xmin = tmin(K.xmin, __builtin_amdgcn_readlane(L.lo(), first));
+        K.xmax = tmax(K.xmax, __builtin_amdgcn_readlane(L.hi(), last));
+        const int tb = K.xmin >> 6;
+        if (L.leader) atomicOr(&R.et[0], 1ull << tmin((L.x >> 6) - tb, 63));
+        if (L.f0 <= L.f1) atomicOr(&R.ft[0], tile_bits(L.f0, L.f1, tb));
+    }
+    const bool far = L.f0 <= L.f1 && L.prev_ok && L.f1 - (K.xmin >> 6) >= 63;
+    if (__ballot(far)) {
+        __threadfence();  // the record's tile is stored
+        if (far) atomicOr(&rec[K.nrec - 1 + li].w, 0x80000000u);
+    }
+    if (KEEP && A.items) {
+        const size_t it = 2 * (size_t)base + (size_t)(mi + K.spans + (int)__popcll(sm & lt));
+        if (L.span) A.items[it] = (uint32_t)(L.prev_x + 2) | ((uint32_t)(L.x - L.prev_x - 2) << 16);
+        if (L.merged) A.items[it + (L.span ? 1 : 0)] = (uint32_t)L.x;
+    }
+    if (L.merged) {
+        if (KEEP) store_mask<NW>(A.imask, (size_t)base + mi, res);
+        A.icov[base + mi] = cell_counts<SPP>(res);
+    }
+    K.nrec += (int)__popcll(lm);
+    K.merged += (int)__popcll(mm);
+    K.spans += (int)__popcll(sm);
+}
+
+__device__ __forceinline__ void chunks_end(const ResolveArgs &A, int64_t b, uint32_t base, RecLds &R, const Chunks &K) {
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) {
+        if (K.nrec) *(uint2 *)&A.prec[base + K.nrec - 1].x = make_uint2(K.cover, K.edge);
+        const bool any = K.merged + K.spans > 0;
+        A.brec[2 * b] = make_uint4(any ? ((uint32_t)K.xmin | ((uint32_t)K.xmax << 16)) : 0xFFFFu, (uint32_t)K.nrec,
+                               (uint32_t)R.et[0], (uint32_t)(R.et[0] >> 32));
+        A.brec[2 * b + 1] = make_uint4((uint32_t)R.ft[0], (uint32_t)(R.ft[0] >> 32), (uint32_t)(K.merged + K.spans),
+                                       (uint32_t)K.merged);
+    }
+    __syncthreads();
 }
 
 // Resolve one (path, row) bucket of n <= 64*S fragments with one wavefront: stage the
 // records in LDS, rank them by (cell x, index), then walk the sorted order in chunks of
-// 64 carrying the winding number and item count.  Per cell group, the first lane sums
+// 64 carrying the winding number and the records.  Per cell group, the first lane sums
 // the members' masks into the per-sample stencil; spans open between groups whose
 // winding passes the fill rule.
-template <int SPP, int S>
+template <int SPP, int S, bool KEEP>
 __device__ __forceinline__ void resolve_bucket(const ResolveArgs &A, int64_t b, uint32_t base, int n, uint32_t *key,
-                                               uint32_t *order, uint32_t *meta, uint32_t *msk) {
+                                               uint32_t *order, uint32_t *meta, uint32_t *msk, RecLds &R) {
     constexpr int NW = Words<SPP>::n;
     const int lane = threadIdx.x & 63;
     uint32_t mykey[S];
@@ -269,6 +393,7 @@ __device__ __forceinline__ void resolve_bucket(const ResolveArgs &A, int64_t b, 
             key[i] = mykey[s];
         }
     }
+    chunks_begin(R);
     __syncthreads();
     int rk[S];
 #pragma unroll
@@ -301,21 +426,20 @@ __device__ __forceinline__ void resolve_bucket(const ResolveArgs &A, int64_t b, 
         W = cv.x;
         wcarry -= A.scarry[cv.w];
     }
-    int icarry = 0, nmerged = 0, xmin = INT_MAX, xmax = INT_MIN;
-    uint64_t tmask = 0ull;
-    const size_t ib = 2 * (size_t)base;
+    Chunks K;
     // group heads of every chunk as wave masks: a group ends at the next head
-    uint64_t hm[S];
-#pragma unroll
-    for (int c = 0; c < S; ++c) {
+    const int nc = (n + 63) >> 6;
+#pragma unroll 1
+    for (int c = 0; c < nc; ++c) {
         const int p = c * 64 + lane;
         bool h = false;
         if (p < n) h = p == 0 || (meta[order[p]] & 0xFFFFu) != (meta[order[p - 1]] & 0xFFFFu);
-        hm[c] = __ballot(h);
+        const uint64_t hm = __ballot(h);
+        if (lane == 0) R.heads[c] = hm;
     }
-#pragma unroll
-    for (int c = 0; c < S; ++c) {
-        if (c * 64 >= n) break;
+    __syncthreads();
+#pragma unroll 1
+    for (int c = 0; c < nc; ++c) {
         const int p = c * 64 + lane;
         const bool v = p < n;
         const uint32_t i = v ? order[p] : 0u;
@@ -331,48 +455,118 @@ __device__ __forceinline__ void resolve_bucket(const ResolveArgs &A, int64_t b, 
         const bool merged = head && x >= 0 && x < W;
         uint32_t res[NW];
         if (merged) {
-            const uint64_t later = lane < 63 ? (hm[c] & (~0ull << (lane + 1))) : 0ull;
+            const uint64_t later = lane < 63 ? (R.heads[c] & (~0ull << (lane + 1))) : 0ull;
             int e = n;
             if (later) {
                 e = c * 64 + (int)__builtin_ctzll(later);
             } else {
-                for (int c2 = c + 1; c2 < S; ++c2)
-                    if (hm[c2]) { e = c2 * 64 + (int)__builtin_ctzll(hm[c2]); break; }
+                for (int c2 = c + 1; c2 < nc; ++c2)
+                    if (R.heads[c2]) { e = c2 * 64 + (int)__builtin_ctzll(R.heads[c2]); break; }
             }
             group_mask<NW>(order, meta, msk, p, e, i, m, w_at, rule, res);
         }
         const int prev_x = 2 * prev_cx - 2;
-        const bool span = head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at);
-        const int cnt = (merged ? 1 : 0) + (span ? 1 : 0);
-        const int ic = scan_add(cnt);
-        const int idx = icarry + ic - cnt;
-        icarry += lane63(ic);
-        if (span) {
-            const int x0 = prev_x + 2;
-            A.items[ib + idx] = (uint32_t)x0 | ((uint32_t)(x - x0) << 16);
-        }
-        if (merged) {
-            A.items[ib + idx + (span ? 1 : 0)] = (uint32_t)x;
-            if (A.imask) store_mask<NW>(A.imask, ib + idx + (span ? 1 : 0), res);
-            A.icov[ib + idx + (span ? 1 : 0)] = cell_counts<SPP>(res);
-        }
-        const int lo = span ? prev_x + 2 : (merged ? x : INT_MAX);
-        const int hi = merged ? x + 2 : (span ? x : INT_MIN);
-        xmin = tmin(xmin, lane63(dpp_scan(lo, INT_MAX, OpMin())));
-        xmax = tmax(xmax, lane63(dpp_scan(hi, INT_MIN, OpMax())));
-        tmask |= wave_or64(tile_bits(lo, hi, xmin >> 6));
-        nmerged += lane63(scan_add(merged ? 1 : 0));
+        Lane L;
+        L.init(merged, head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at), p > 0, x, prev_x, W);
+        chunk_emit<SPP, KEEP>(A, base, L, res, R, K);
     }
-    if (lane == 0) {
-        A.bicnt[b] = (uint32_t)icarry;
-        A.bmcnt[b] = (uint32_t)nmerged;
-        A.bext[b] = icarry ? ((uint32_t)xmin | ((uint32_t)xmax << 16)) : 0xFFFFu;
-        A.btile[b] = tmask;
+    chunks_end(A, b, base, R, K);
+}
+
+constexpr int kResolveBlocks = 65536;
+
+// A wave-wide ballot as seen by a lane of a segment of S lanes: its segment's bits, bit i the
+// segment's i-th lane.  Packed segments lie in one half of the ballot, so 32 bits do.
+template <int S> struct SegBits {
+    uint64_t m;
+    __device__ __forceinline__ SegBits(bool v) : m(__ballot(v)) {}
+    __device__ __forceinline__ int below(int i) const { return (int)__popcll(m & (i ? (~0ull >> (64 - i)) : 0ull)); }
+    __device__ __forceinline__ int count() const { return (int)__popcll(m); }
+    __device__ __forceinline__ int first() const { return (int)__builtin_ctzll(m); }
+    __device__ __forceinline__ int last() const { return 63 - (int)__builtin_clzll(m); }
+    // the first set bit after i, or S
+    __device__ __forceinline__ int after(int i) const {
+        const uint64_t l = i < 63 ? m & (~0ull << (i + 1)) : 0ull;
+        return l ? (int)__builtin_ctzll(l) : S;
+    }
+};
+template <int S> struct SegBits32 {
+    uint32_t m;
+    __device__ __forceinline__ SegBits32(bool v) {
+        const uint64_t b = __ballot(v);
+        const int lane = threadIdx.x & 63;
+        m = lane & 32 ? (uint32_t)(b >> 32) : (uint32_t)b;
+        if (S == 16) m = (m >> (lane & 16)) & 0xFFFFu;
+    }
+    __device__ __forceinline__ int below(int i) const { return __popc(m & ((1u << i) - 1u)); }
+    __device__ __forceinline__ int count() const { return __popc(m); }
+    __device__ __forceinline__ int first() const { return __ffs((int)m) - 1; }
+    __device__ __forceinline__ int last() const { return 31 - __clz((int)m); }
+    __device__ __forceinline__ int after(int i) const {
+        const uint32_t l = m & ~((2u << i) - 1u);  // i = 31: no bits
+        return l ? __ffs((int)l) - 1 : S;
+    }
+};
+template <> struct SegBits<32> : SegBits32<32> { using SegBits32<32>::SegBits32; };
+template <> struct SegBits<16> : SegBits32<16> { using SegBits32<16>::SegBits32; };
+
+// The records of the buckets in a wave's 64 / S segments, each bucket in one pass.
+template <int SPP, int S, bool KEEP>
+__device__ __forceinline__ void segment_emit(const ResolveArgs &A, bool live, int64_t b, uint32_t base, const Lane &L,
+                                             const uint32_t *res, RecLds &R) {
+    constexpr int NW = Words<SPP>::n;
+    const int lane = threadIdx.x & 63;
+    const int i = lane % S, seg = lane / S, sb = seg * S;
+    const SegBits<S> mm(L.merged), sm(L.span), lm(L.leader), any(L.merged || L.span);
+    const int mi = mm.below(i), li = lm.below(i);
+    if (L.merged) {
+        if (KEEP) store_mask<NW>(A.imask, (size_t)base + mi, res);
+        A.icov[base + mi] = cell_counts<SPP>(res);
+    }
+    // extent: the first and the last lane with an item
+    int xmin, xmax;
+    if (S == 64) {
+        xmin = __builtin_amdgcn_readlane(L.lo(), any.m ? any.first() : 0);
+        xmax = __builtin_amdgcn_readlane(L.hi(), any.m ? any.last() : 0);
+    } else {
+        xmin = __shfl(L.lo(), any.m ? sb + any.first() : lane, 64);
+        xmax = __shfl(L.hi(), any.m ? sb + any.last() : lane, 64);
+    }
+    const int tb = xmin >> 6;
+    if (L.leader) atomicOr(&R.et[seg], 1ull << tmin((L.x >> 6) - tb, 63));
+    if (L.f0 <= L.f1) atomicOr(&R.ft[seg], tile_bits(L.f0, L.f1, tb));
+    // a leader's record: the sums of its run of lanes, up to the next leader
+    const uint32_t pe = (uint32_t)dpp_scan_seg<S>((int)L.eb, 0, OpAdd()), pc = (uint32_t)dpp_scan_seg<S>((int)L.co, 0, OpAdd());
+    const int next = lm.after(i);
+    const uint32_t e = (uint32_t)__shfl((int)pe, sb + next - 1, 64) - (pe - L.eb);
+    const uint32_t nc = (uint32_t)__shfl((int)L.cp, (sb + next) & 63, 64);
+    const uint32_t c = (uint32_t)__shfl((int)pc, sb + next - 1, 64) - (pc - L.co) + (next < S ? nc : 0u);
+    uint4 *rec = A.prec + base;
+    if (L.leader) rec[li] = make_uint4(c, e, (uint32_t)mi, (uint32_t)(L.x >> 6));
+    const bool far = L.f0 <= L.f1 && L.prev_ok && L.f1 - tb >= 63;
+    if (__ballot(far)) {
+        __threadfence();  // the record's tile is stored
+        if (far) atomicOr(&rec[li - 1].w, 0x80000000u);
+    }
+    if (KEEP && A.items) {
+        const size_t it = 2 * (size_t)base + (size_t)(mi + sm.below(i));
+        if (L.span) A.items[it] = (uint32_t)(L.prev_x + 2) | ((uint32_t)(L.x - L.prev_x - 2) << 16);
+        if (L.merged) A.items[it + (L.span ? 1 : 0)] = (uint32_t)L.x;
+    }
+    __syncthreads();
+    if (live && i == 0) {
+        A.brec[2 * b] = make_uint4(any.m ? ((uint32_t)xmin | ((uint32_t)xmax << 16)) : 0xFFFFu, (uint32_t)lm.count(),
+                               (uint32_t)R.et[seg], (uint32_t)(R.et[seg] >> 32));
+        A.brec[2 * b + 1] = make_uint4((uint32_t)R.ft[seg], (uint32_t)(R.ft[seg] >> 32), (uint32_t)(mm.count() + sm.count()),
+                                       (uint32_t)mm.count());
     }
     __syncthreads();
 }
 
-constexpr int kResolveBlocks = 65536;
+__device__ __forceinline__ void segments_begin(RecLds &R) {
+    const int lane = threadIdx.x & 63;
+    if (lane < 4) R.et[lane] = R.ft[lane] = 0ull;
+}
 
 // One small bucket's records, loaded a bucket ahead of its resolve (the grid-stride loop
 // keeps the next bucket's records in flight while the current one resolves); the bucket
@@ -398,10 +592,10 @@ __device__ __forceinline__ void small_load(const ResolveArgs &A, uint32_t base, 
 }
 
 // resolve_bucket<SPP, 1> with the records already in registers
-template <int SPP>
+template <int SPP, bool KEEP>
 __device__ __forceinline__ void resolve_small(const ResolveArgs &A, int64_t b, uint32_t base, int n,
                                               const SmallIn<Words<SPP>::n> &in, uint32_t *order, uint32_t *meta,
-                                              uint32_t *msk) {
+                                              uint32_t *msk, RecLds &R) {
     constexpr int NW = Words<SPP>::n;
     const int lane = threadIdx.x & 63;
     uint32_t mykey = 0xFFFFFFFFu;
@@ -411,6 +605,7 @@ __device__ __forceinline__ void resolve_small(const ResolveArgs &A, int64_t b, u
         for (int k = 0; k < NW; ++k) msk[lane * NW + k] = in.mk[k];
         mykey = ((in.meta & 0xFFFFu) << 10) | (uint32_t)lane;
     }
+    segments_begin(R);
     int rk = 0;
 #pragma unroll 8
     for (int j = 0; j < n; ++j) {
@@ -423,7 +618,6 @@ __device__ __forceinline__ void resolve_small(const ResolveArgs &A, int64_t b, u
     const int rule = in.rule;
     uint32_t wcarry = in.carry;
     const int W = in.W;
-    const size_t ib = 2 * (size_t)base;
     const int p = lane;
     const bool v = p < n;
     const uint32_t i = v ? order[p] : 0u;
@@ -437,51 +631,23 @@ __device__ __forceinline__ void resolve_small(const ResolveArgs &A, int64_t b, u
     const int x = 2 * cx - 2;
     const bool merged = head && x >= 0 && x < W;
     // the group of a head lane ends at the next head (or the bucket end)
-    const uint64_t heads = __ballot(head);
+    const SegBits<64> heads(head);
     uint32_t res[NW];
-    if (merged) {
-        const uint64_t later = p < 63 ? (heads & (~0ull << (p + 1))) : 0ull;
-        const int e = later ? (int)__builtin_ctzll(later) : n;
-        group_mask<NW>(order, meta, msk, p, e, i, m, w_at, rule, res);
-    }
+    if (merged) group_mask<NW>(order, meta, msk, p, tmin(heads.after(p), n), i, m, w_at, rule, res);
     const int prev_x = 2 * prev_cx - 2;
-    const bool span = head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at);
-    const int cnt = (merged ? 1 : 0) + (span ? 1 : 0);
-    const int ic = scan_add(cnt);
-    const int idx = ic - cnt;
-    if (span) {
-        const int x0 = prev_x + 2;
-        A.items[ib + idx] = (uint32_t)x0 | ((uint32_t)(x - x0) << 16);
-    }
-    if (merged) {
-        A.items[ib + idx + (span ? 1 : 0)] = (uint32_t)x;
-        if (A.imask) store_mask<NW>(A.imask, ib + idx + (span ? 1 : 0), res);
-        A.icov[ib + idx + (span ? 1 : 0)] = cell_counts<SPP>(res);
-    }
-    const int lo = span ? prev_x + 2 : (merged ? x : INT_MAX);
-    const int hi = merged ? x + 2 : (span ? x : INT_MIN);
-    const int xmin = lane63(dpp_scan(lo, INT_MAX, OpMin()));
-    const int xmax = lane63(dpp_scan(hi, INT_MIN, OpMax()));
-    const int nmerged = lane63(scan_add(merged ? 1 : 0));
-    const int icnt = lane63(ic);
-    const uint64_t tmask = wave_or64(tile_bits(lo, hi, xmin >> 6));
-    if (lane == 0) {
-        A.bicnt[b] = (uint32_t)icnt;
-        A.bmcnt[b] = (uint32_t)nmerged;
-        A.bext[b] = icnt ? ((uint32_t)xmin | ((uint32_t)xmax << 16)) : 0xFFFFu;
-        A.btile[b] = tmask;
-    }
-    __syncthreads();
+    Lane L;
+    L.init(merged, head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at), p > 0, x, prev_x, W);
+    segment_emit<SPP, 64, KEEP>(A, true, b, base, L, res, R);
 }
 
 // Buckets of at most S (16 or 32) fragments, 64 / S of them in one wave: lane l works on
 // segment l / S, whose records, rank sort, scans and reductions stay inside its S lanes
 // (segmented DPP scans), so one pass resolves the whole pack.  ks[s] is the s-th bucket's
 // slot in the per-lane scalars (lane k holds bucket b0 + k G), -1 for an empty segment.
-template <int SPP, int S>
+template <int SPP, int S, bool KEEP>
 __device__ __forceinline__ void resolve_pack(const ResolveArgs &A, int64_t b0, int64_t G, const int *ks, int vbase,
                                              int vend, int vcarry, int vrule, int vW, uint32_t *order, uint32_t *meta,
-                                             uint32_t *msk) {
+                                             uint32_t *msk, RecLds &R) {
     constexpr int NW = Words<SPP>::n;
     constexpr int P = 64 / S;
     const int lane = threadIdx.x & 63;
@@ -509,6 +675,7 @@ __device__ __forceinline__ void resolve_pack(const ResolveArgs &A, int64_t b0, i
         for (int q = 0; q < NW; ++q) msk[lane * NW + q] = mk[q];
         mykey = ((m & 0xFFFFu) << 10) | (uint32_t)i;
     }
+    segments_begin(R);
     int rk = 0;
 #pragma unroll
     for (int j = 0; j < S; ++j) rk += ((uint32_t)__shfl((int)mykey, sb + j, 64) < mykey) ? 1 : 0;
@@ -528,54 +695,23 @@ __device__ __forceinline__ void resolve_pack(const ResolveArgs &A, int64_t b0, i
     const int x = 2 * cx - 2;
     const bool merged = head && x >= 0 && x < W;
     // the group of a head lane ends at the next head of its segment (or the bucket end)
-    const uint64_t heads = __ballot(head);
+    const SegBits<S> heads(head);
     uint32_t res[NW];
-    if (merged) {
-        const uint64_t segm = (S == 64) ? ~0ull : (((1ull << S) - 1ull) << sb);
-        const uint64_t later = (lane < 63 ? (heads & (~0ull << (lane + 1))) : 0ull) & segm;
-        const int e = later ? (int)__builtin_ctzll(later) - sb : n;
-        group_mask<NW>(order + sb, meta, msk, p, e, i0, m, w_at, rule, res);
-    }
+    if (merged) group_mask<NW>(order + sb, meta, msk, p, tmin(heads.after(i), n), i0, m, w_at, rule, res);
     const int prev_x = 2 * prev_cx - 2;
-    const bool span = head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at);
-    const int cnt = (merged ? 1 : 0) + (span ? 1 : 0);
-    const int ic = dpp_scan_seg<S>(cnt, 0, OpAdd());
-    const int idx = ic - cnt;
-    const size_t ib = 2 * (size_t)base;
-    if (span) {
-        const int x0 = prev_x + 2;
-        A.items[ib + idx] = (uint32_t)x0 | ((uint32_t)(x - x0) << 16);
-    }
-    if (merged) {
-        A.items[ib + idx + (span ? 1 : 0)] = (uint32_t)x;
-        if (A.imask) store_mask<NW>(A.imask, ib + idx + (span ? 1 : 0), res);
-        A.icov[ib + idx + (span ? 1 : 0)] = cell_counts<SPP>(res);
-    }
-    const int lo = span ? prev_x + 2 : (merged ? x : INT_MAX);
-    const int hi = merged ? x + 2 : (span ? x : INT_MIN);
-    const int xmin = dpp_scan_seg<S>(lo, INT_MAX, OpMin());
-    const int xmax = dpp_scan_seg<S>(hi, INT_MIN, OpMax());
-    const int nmerged = dpp_scan_seg<S>(merged ? 1 : 0, 0, OpAdd());
-    const uint64_t tb = tile_bits(lo, hi, xmin >> 6);  // a lane's prefix minimum is its segment's first item
-    const uint32_t tlo = (uint32_t)dpp_scan_seg<S>((int)(uint32_t)tb, 0, OpOr());
-    const uint32_t thi = (uint32_t)dpp_scan_seg<S>((int)(uint32_t)(tb >> 32), 0, OpOr());
-    if (k >= 0 && i == S - 1) {
-        // the segment's last lane holds its bucket's totals
-        const int64_t b = b0 + (int64_t)k * G;
-        A.bicnt[b] = (uint32_t)ic;
-        A.bmcnt[b] = (uint32_t)nmerged;
-        A.bext[b] = ic ? ((uint32_t)xmin | ((uint32_t)xmax << 16)) : 0xFFFFu;
-        A.btile[b] = (uint64_t)tlo | ((uint64_t)thi << 32);
-    }
-    __syncthreads();
+    Lane L;
+    L.init(merged, head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at), p > 0, x, prev_x, W);
+    segment_emit<SPP, S, KEEP>(A, k >= 0, b0 + (int64_t)(k < 0 ? 0 : k) * G, base, L, res, R);
 }
 
 // Every bucket: empty ones are cleared, buckets of at most 128 fragments are resolved,
-// larger ones are listed for the size-class passes below.
-template <int SPP>
-__global__ void __launch_bounds__(64, 6) k_resolve_first(ResolveArgs A) {
+// larger ones are listed for the size-class passes below.  Five waves per SIMD: the records'
+// arithmetic spills at six (1.41 ms on the 2048x2048 illustration for 1.50; four: 1.50).
+template <int SPP, bool KEEP>
+__global__ void __launch_bounds__(64, 5) k_resolve_first(ResolveArgs A) {
     constexpr int NW = Words<SPP>::n;
     __shared__ uint32_t key[128], order[128], meta[128], msk[128 * NW];
+    __shared__ RecLds R;
     const int lane = threadIdx.x;
     const int64_t G = gridDim.x;
     // Strided buckets keep the waves' loads balanced (a path's neighbouring rows have
@@ -615,7 +751,7 @@ __global__ void __launch_bounds__(64, 6) k_resolve_first(ResolveArgs A) {
                 ks[s] = m16 ? (int)__builtin_ctzll(m16) : -1;
                 m16 &= m16 - 1ull;
             }
-            resolve_pack<SPP, 16>(A, b0, G, ks, vbase, vend, vcarry, vrule, vW, order, meta, msk);
+            resolve_pack<SPP, 16, KEEP>(A, b0, G, ks, vbase, vend, vcarry, vrule, vW, order, meta, msk, R);
         }
         while (m32) {
             int ks[2];
@@ -624,7 +760,7 @@ __global__ void __launch_bounds__(64, 6) k_resolve_first(ResolveArgs A) {
                 ks[s] = m32 ? (int)__builtin_ctzll(m32) : -1;
                 m32 &= m32 - 1ull;
             }
-            resolve_pack<SPP, 32>(A, b0, G, ks, vbase, vend, vcarry, vrule, vW, order, meta, msk);
+            resolve_pack<SPP, 32, KEEP>(A, b0, G, ks, vbase, vend, vcarry, vrule, vW, order, meta, msk, R);
         }
         // the rest one by one, the next bucket's records loading during the current one
         SmallIn<NW> in0, in1;
@@ -645,16 +781,16 @@ __global__ void __launch_bounds__(64, 6) k_resolve_first(ResolveArgs A) {
                                (uint32_t)__builtin_amdgcn_readlane(vend, kn), in1);
             }
             if (n == 0) {
-                if (lane == 0) { A.bicnt[b] = 0; A.bmcnt[b] = 0; A.bext[b] = 0xFFFFu; A.btile[b] = 0ull; }
+                if (lane < 2) A.brec[2 * b + lane] = make_uint4(lane ? 0u : 0xFFFFu, 0u, 0u, 0u);
             } else if (n > 128) {
                 if (lane == 0) A.big_list[atomicAdd(A.big_count, 1u)] = (uint32_t)b;
             } else if (n > 64) {
-                resolve_bucket<SPP, 2>(A, b, base, n, key, order, meta, msk);
+                resolve_bucket<SPP, 2, KEEP>(A, b, base, n, key, order, meta, msk, R);
             } else {
                 in0.carry = (uint32_t)__builtin_amdgcn_readlane(vcarry, k);
                 in0.rule = __builtin_amdgcn_readlane(vrule, k);
                 in0.W = __builtin_amdgcn_readlane(vW, k);
-                resolve_small<SPP>(A, b, base, n, in0, order, meta, msk);
+                resolve_small<SPP, KEEP>(A, b, base, n, in0, order, meta, msk, R);
             }
             in0 = in1;
         }
@@ -663,32 +799,31 @@ __global__ void __launch_bounds__(64, 6) k_resolve_first(ResolveArgs A) {
 
 // The listed buckets (more than 128 fragments), one per block, in one launch so that the
 // few long ones overlap: up to 1024 fragments staged in LDS, more in k_resolve_huge.
-constexpr int kBigStage = 16;  // chunks of 64 fragments staged in LDS
-
-template <int SPP>
+template <int SPP, bool KEEP>
 __global__ void __launch_bounds__(64) k_resolve_big(ResolveArgs A) {
     constexpr int NW = Words<SPP>::n;
     __shared__ uint32_t key[64 * kBigStage], order[64 * kBigStage], meta[64 * kBigStage], msk[64 * kBigStage * NW];
+    __shared__ RecLds R;
     const uint32_t nbig = *A.big_count;
     for (uint32_t bi = blockIdx.x; bi < nbig; bi += gridDim.x) {
         const int64_t b = A.big_list[bi];
         const uint32_t base = A.boff[b];
         const int n = (int)(A.boff[b + 1] - base);
-        if (n <= 256) resolve_bucket<SPP, 4>(A, b, base, n, key, order, meta, msk);
-        else if (n <= 512) resolve_bucket<SPP, 8>(A, b, base, n, key, order, meta, msk);
-        else if (n <= 64 * kBigStage) resolve_bucket<SPP, kBigStage>(A, b, base, n, key, order, meta, msk);
+        if (n <= 256) resolve_bucket<SPP, 4, KEEP>(A, b, base, n, key, order, meta, msk, R);
+        else if (n <= 512) resolve_bucket<SPP, 8, KEEP>(A, b, base, n, key, order, meta, msk, R);
+        else if (n <= 64 * kBigStage) resolve_bucket<SPP, kBigStage, KEEP>(A, b, base, n, key, order, meta, msk, R);
     }
 }
 
 // Buckets of more than 1024 fragments (rare): bitonic-sort 64-bit (cell x, index) keys,
-// their high words in the bucket's stretch of the global scratch and their low words in
-// its stretch of the item array (2n words each; the padded power of two is at most 2n),
-// copy the sorted indices into the scratch (the items are written over next), then walk
-// the sorted order in chunks of 64 reading the records from global memory.  Any bucket
+// held in the bucket's stretch of the record array (4n words; the padded power of two is at
+// most 2n), copy the sorted indices into the scratch (the records are written next), then walk
+// the sorted order in chunks of 64 reading the fragments from global memory.  Any bucket
 // size works.
-template <int SPP>
+template <int SPP, bool KEEP>
 __global__ void __launch_bounds__(64) k_resolve_huge(ResolveArgs A) {
     constexpr int NW = Words<SPP>::n;
+    __shared__ RecLds R;
     const int lane = threadIdx.x;
     const uint32_t nbig = *A.big_count;
     for (uint32_t bi = blockIdx.x; bi < nbig; bi += gridDim.x) {
@@ -698,8 +833,8 @@ __global__ void __launch_bounds__(64) k_resolve_huge(ResolveArgs A) {
         if (n <= 64 * kBigStage) continue;
         int P2 = 1;
         while (P2 < n) P2 <<= 1;
-        uint32_t *khi = A.scratch + 2 * (size_t)base;
-        uint32_t *klo = A.items + 2 * (size_t)base;
+        uint32_t *khi = (uint32_t *)(A.prec + base);
+        uint32_t *klo = khi + P2;
         for (int i = lane; i < P2; i += 64) {
             khi[i] = (i < n) ? (A.rec_meta[base + i] & 0xFFFFu) : 0xFFFFFFFFu;
             klo[i] = (i < n) ? (uint32_t)i : 0xFFFFFFFFu;
@@ -722,9 +857,11 @@ __global__ void __launch_bounds__(64) k_resolve_huge(ResolveArgs A) {
                 __syncthreads();
             }
         }
-        for (int i = lane; i < n; i += 64) khi[i] = klo[i];
+        uint32_t *order = A.scratch + base;
+        for (int i = lane; i < n; i += 64) order[i] = klo[i];
+        chunks_begin(R);
         __syncthreads();
-        const uint32_t *order = khi;  // sorted fragment indices; a fragment's cell x is in its record
+        // sorted fragment indices; a fragment's cell x is in its record
         auto cell_x = [&](int q) { return (int)(A.rec_meta[base + order[q]] & 0xFFFFu); };
         const int rule = A.frule[A.binfo[b].x];
         uint32_t wcarry = A.bcarry[b];
@@ -734,9 +871,7 @@ __global__ void __launch_bounds__(64) k_resolve_huge(ResolveArgs A) {
             W = cv.x;
             wcarry -= A.scarry[cv.w];
         }
-        int icarry = 0, nmerged = 0, xmin = INT_MAX, xmax = INT_MIN;
-        uint64_t tmask = 0ull;
-        const size_t ib = 2 * (size_t)base;
+        Chunks K;
         for (int c0 = 0; c0 < n; c0 += 64) {
             const int p = c0 + lane;
             const bool v = p < n;
@@ -765,43 +900,20 @@ __global__ void __launch_bounds__(64) k_resolve_huge(ResolveArgs A) {
                 st.finish(rule, res);
             }
             const int prev_x = 2 * prev_cx - 2;
-            const bool span = head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at);
-            const int cnt = (merged ? 1 : 0) + (span ? 1 : 0);
-            const int ic = scan_add(cnt);
-            const int idx = icarry + ic - cnt;
-            icarry += lane63(ic);
-            if (span) {
-                const int x0 = prev_x + 2;
-                A.items[ib + idx] = (uint32_t)x0 | ((uint32_t)(x - x0) << 16);
-            }
-            if (merged) {
-                A.items[ib + idx + (span ? 1 : 0)] = (uint32_t)x;
-                if (A.imask) store_mask<NW>(A.imask, ib + idx + (span ? 1 : 0), res);
-                A.icov[ib + idx + (span ? 1 : 0)] = cell_counts<SPP>(res);
-            }
-            const int lo = span ? prev_x + 2 : (merged ? x : INT_MAX);
-            const int hi = merged ? x + 2 : (span ? x : INT_MIN);
-            xmin = tmin(xmin, lane63(dpp_scan(lo, INT_MAX, OpMin())));
-            xmax = tmax(xmax, lane63(dpp_scan(hi, INT_MIN, OpMax())));
-            tmask |= wave_or64(tile_bits(lo, hi, xmin >> 6));
-            nmerged += lane63(scan_add(merged ? 1 : 0));
+            Lane L;
+            L.init(merged, head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at), p > 0, x, prev_x, W);
+            chunk_emit<SPP, KEEP>(A, base, L, res, R, K);
         }
-        if (lane == 0) {
-            A.bicnt[b] = (uint32_t)icarry;
-            A.bmcnt[b] = (uint32_t)nmerged;
-            A.bext[b] = icarry ? ((uint32_t)xmin | ((uint32_t)xmax << 16)) : 0xFFFFu;
-            A.btile[b] = tmask;
-        }
-        __syncthreads();
+        chunks_end(A, b, base, R, K);
     }
 }
 
 // ---------------------------------------------------------------------------------
 // compositing order: non-empty buckets, stably sorted by cell row (path order kept)
 // ---------------------------------------------------------------------------------
-__global__ void k_nz_flags(int64_t NB, const uint32_t *__restrict__ bicnt, uint32_t *flag) {
+__global__ void k_nz_flags(int64_t NB, const uint4 *__restrict__ brec, uint32_t *flag) {
     int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < NB) flag[b] = bicnt[b] ? 1u : 0u;
+    if (b < NB) flag[b] = brec[2 * b + 1].z ? 1u : 0u;
 }
 __global__ void k_nz_compact(int64_t NB, const uint32_t *__restrict__ flag, const uint32_t *__restrict__ off,
                              const int2 *__restrict__ binfo, const int4 *__restrict__ pcanvas, uint32_t *keys,
@@ -1058,11 +1170,12 @@ __device__ __forceinline__ uint32_t pack_dec(const float4 *step, const float *d)
 struct CovArgs {
     int W, H, tiles_x;
     const uint32_t *rowbeg, *rowend;
-    const uint4 *rrec;          // per row-list entry: extent, colour, item count, item base
-    const uint64_t *rtile;      // per row-list entry: 64-pixel tiles holding items
-    const uint32_t *items, *icov;
-    const uint32_t *imask;      // merged masks (multisample output)
-    const uint32_t *rpath;      // row-list path ids (multisample output)
+    const uint32_t *rext;       // per row-list entry: extent
+    const uint4 *rrec;          //   colour, records, base, path
+    const ulonglong2 *rtile;    //   tiles with a record, tiles inside a span
+    const uint4 *prec;          // records
+    const uint32_t *icov;       // sample counts of merged cells
+    const uint32_t *imask;      // masks of merged cells (multisample output)
     const uint32_t *ptab;       // per-path blend tables (multisample output)
     const float *dec_c;         // [256] colour decode, for the paint colours
     const float *dec_a;         // [256] alpha decode (gradient ramp texels)
@@ -1079,39 +1192,210 @@ struct CovArgs {
 
 constexpr int kCovList = 64;    // per-wave list of the tile's buckets
 
-// Scatter the starts of a long bucket's items (more than 64) into the column slots.
-__device__ __noinline__ void scatter_big(const uint32_t *items, uint32_t ib, int cnt, int tx0, uint32_t *slot) {
+// A bucket's cells in one tile: those covered by a span or merged, the merged ones, and the
+// array index of the tile's first merged cell.
+struct TileCells {
+    uint32_t cover, edge, at;
+    int rec;                    // records before the tile; its own is `rec` where has_rec
+    bool has_rec;
+};
+
+// Whether the row-list entry's bucket has items in the 64-pixel tile `tile` (entry extents
+// overlap it), and where its record is.  Tiles from the 63rd of the bucket on are looked up
+// in the records themselves.
+__device__ __forceinline__ bool tile_hit(const uint4 *__restrict__ prec, uint32_t ext, const uint4 &rec,
+                                         const ulonglong2 &bits, int tile, TileCells &t) {
+    const int k = tile - (int)((ext & 0xFFFFu) >> 6);
+    t.cover = 0xFFFFFFFFu;
+    t.edge = 0u;
+    t.at = 0u;
+    if (k < 63) {
+        t.has_rec = (bits.x >> k) & 1ull;
+        t.rec = (int)__popcll(bits.x & ((1ull << k) - 1ull));
+        return t.has_rec || ((bits.y >> k) & 1ull);
+    }
+    t.has_rec = false;
+    t.rec = 0;
+    if (!((bits.x | bits.y) >> 63)) return false;
+    int lo = 0, hi = (int)rec.y;  // records of tiles up to this one
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if ((int)(prec[rec.z + mid].w & 0x7FFFFFFFu) <= tile) lo = mid + 1; else hi = mid;
+    }
+    t.rec = lo;
+    if (lo == 0) return true;  // before the first merged cell: the span from the canvas edge
+    const uint32_t w = prec[rec.z + lo - 1].w;
+    if ((int)(w & 0x7FFFFFFFu) != tile) return (w >> 31) != 0u;
+    t.has_rec = true;
+    t.rec = lo - 1;
+    return true;
+}
+
+__device__ __forceinline__ void tile_load(const uint4 *__restrict__ prec, uint32_t base, TileCells &t) {
+    if (!t.has_rec) return;
+    const uint4 r = prec[base + t.rec];
+    t.cover = r.x;
+    t.edge = r.y;
+    t.at = base + r.z;
+}
+
+// First pixel and width of the item covering cell c of a tile (gradients run along an item):
+// a merged cell, or the span between the merged cells next to it, which may lie in the
+// neighbouring records or be missing at the ends of the bucket's extent.  g: {index of the
+// record before the tile + 1 (0: none), the same of the next record, extent}.
+__device__ __forceinline__ void item_extent(const uint4 *__restrict__ prec, uint32_t edge, int c, int tx0, const uint4 &g,
+                                            int &x0, int &w) {
+    if ((edge >> c) & 1u) {
+        x0 = tx0 + 2 * c;
+        w = 2;
+        return;
+    }
+    const uint32_t below = edge & ((1u << c) - 1u), above = edge & ~((2u << c) - 1u);
+    int end;
+    if (below) {
+        x0 = tx0 + 2 * (31 - __clz((int)below)) + 2;
+    } else if (g.x) {
+        const uint4 r = prec[g.x - 1u];
+        x0 = 64 * (int)(r.w & 0x7FFFFFFFu) + 2 * (31 - __clz((int)r.y)) + 2;
+    } else {
+        x0 = (int)(g.z & 0xFFFFu);
+    }
+    if (above) {
+        end = tx0 + 2 * (__ffs((int)above) - 1);
+    } else if (g.y) {
+        const uint4 r = prec[g.y - 1u];
+        end = 64 * (int)(r.w & 0x7FFFFFFFu) + 2 * (__ffs((int)r.y) - 1);
+    } else {
+        end = (int)(g.z >> 16);
+    }
+    w = end - x0;
+}
+
+// Transposes the 32 x 32 bit matrices held by lanes 0-31 and by lanes 32-63: bit c of lane b
+// goes to bit b of lane c (c, b within the half).
+__device__ __forceinline__ uint32_t transpose32(uint32_t x) {
     const int lane = threadIdx.x & 63;
-    for (int ic = 0; ic < cnt; ic += 64) {
-        if (ic + lane < cnt) {
-            const uint32_t it = items[ib + ic + lane];
-            const int x0 = (int)(it & 0xFFFFu), iw = (int)(it >> 16);
-            const int end = x0 + (iw ? iw : 2);
-            if (end > tx0 && x0 < tx0 + 64) atomicMax(&slot[tmax(x0 - tx0, 0)], (uint32_t)(ic + lane + 1));
+#define SL_STEP(j, m, fetch)                                                                            \
+    {                                                                                                   \
+        const uint32_t p = (uint32_t)(fetch);                                                           \
+        const bool up = lane & j;                                                                       \
+        const uint32_t r = __builtin_amdgcn_alignbit(p, p, up ? j : 32 - j), k = up ? ~(m) : (m);       \
+        x = (x & k) | (r & ~k);                                                                         \
+    }
+#define SL_DPP(c, v) __builtin_amdgcn_update_dpp((int)(v), (int)(v), c, 0xf, 0xf, false)
+    SL_STEP(16, 0x0000FFFFu, __builtin_amdgcn_ds_swizzle((int)x, 0x401F))       // lane ^ 16
+    SL_STEP(8, 0x00FF00FFu, SL_DPP(0x128, x))                                   // row_ror:8
+    SL_STEP(4, 0x0F0F0F0Fu, SL_DPP(0x1B, SL_DPP(0x141, x)))                     // ^ 7, then ^ 3
+    SL_STEP(2, 0x33333333u, SL_DPP(0x4E, x))                                    // quad_perm 2,3,0,1
+    SL_STEP(1, 0x55555555u, SL_DPP(0xB1, x))                                    // quad_perm 1,0,3,2
+#undef SL_DPP
+#undef SL_STEP
+    return x;
+}
+
+// Lists the row's buckets with items in the tile, in path order, and calls flush(n) for every
+// full list and the last.  The row's extents are read first, two a lane, and the entries that
+// overlap the tile queued; 64 queued entries at a time then load their records.  (Loading
+// everything of 64 entries at once took three dependent loads for every 64 buckets of the
+// row; on a sheet of glyphs nearly all of them lie beside the tile.)
+constexpr int kRowQueue = 192;
+
+template <bool GRAD, class F>
+__device__ __forceinline__ void list_row(const CovArgs &A, uint32_t q0, uint32_t q1, int tx, int tx1, float ascale,
+                                         const float *s_dec, uint32_t *queue, float4 *l_src, uint4 *l_ent, uint4 *l_grad,
+                                         const F &flush) {
+    const int lane = threadIdx.x & 63, tx0 = tx * 64;
+    const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    int nlist = 0, nq = 0;
+    for (uint32_t qc = q0; qc < q1;) {
+        // fill the queue: two entries a lane, in order
+        const uint32_t q = qc + 2u * (uint32_t)lane;
+        const uint32_t x0 = q < q1 ? A.rext[q] : 0xFFFFu, x1 = q + 1u < q1 ? A.rext[q + 1u] : 0xFFFFu;
+        const bool h0 = (int)(x0 & 0xFFFFu) < tx1 && (int)(x0 >> 16) > tx0;
+        const bool h1 = (int)(x1 & 0xFFFFu) < tx1 && (int)(x1 >> 16) > tx0;
+        const unsigned long long m0 = __ballot(h0), m1 = __ballot(h1);
+        const int at = nq + (int)__popcll(m0 & lt) + (int)__popcll(m1 & lt);
+        if (h0) queue[at] = q;
+        if (h1) queue[at + (h0 ? 1 : 0)] = q + 1u;
+        nq += (int)__popcll(m0) + (int)__popcll(m1);
+        qc += 128u;
+        // and empty it, 64 at a time (all of it at the row's end)
+        while (nq >= 64 || (qc >= q1 && nq > 0)) {
+            wave_sync_lds();
+            const int n = tmin(nq, 64);
+            bool ov = false;
+            uint4 rec;
+            uint32_t ext = 0u;
+            TileCells tc;
+            if (lane < n) {
+                const uint32_t e = queue[lane];
+                ext = A.rext[e];
+                rec = A.rrec[e];
+                // a word without alpha paints nothing, unless it names a gradient that paints
+                const bool paints = (rec.x & 0xFF000000u) || (GRAD && rec.x != 0u && grad_paints(A.G, rec.x));
+                ov = tile_hit(A.prec, ext, rec, A.rtile[e], tx, tc) && paints;
+                if (ov) tile_load(A.prec, rec.z, tc);
+            }
+            // the queue's remainder moves to its front
+            const uint32_t r0 = n + lane < nq ? queue[n + lane] : 0u, r1 = n + 64 + lane < nq ? queue[n + 64 + lane] : 0u;
+            wave_sync_lds();
+            if (n + lane < nq) queue[lane] = r0;
+            if (n + 64 + lane < nq) queue[64 + lane] = r1;
+            nq -= n;
+            const unsigned long long om = __ballot(ov);
+            const int nov = (int)__popcll(om), rank = (int)__popcll(om & lt);
+            for (int done = 0; done < nov;) {
+                const int take = tmin(kCovList - nlist, nov - done);
+                if (ov && rank >= done && rank < done + take) {
+                    const int sl = nlist + rank - done;
+                    const uint32_t c = rec.x;
+                    if (GRAD && !(c & 0xFF000000u))
+                        l_src[sl] = make_float4(__uint_as_float(c), 0.f, 0.f, -1.f);
+                    else
+                        l_src[sl] = make_float4(s_dec[c & 0xFFu], s_dec[(c >> 8) & 0xFFu], s_dec[(c >> 16) & 0xFFu],
+                                                unorm_dec((int)(c >> 24)) * ascale);
+                    l_ent[sl] = make_uint4(tc.cover, tc.edge, tc.at, rec.w);
+                    if (GRAD) {
+                        const int nx = tc.rec + (tc.has_rec ? 1 : 0);
+                        l_grad[sl] = make_uint4(tc.rec ? rec.z + (uint32_t)tc.rec : 0u,
+                                                nx < (int)rec.y ? rec.z + (uint32_t)nx + 1u : 0u, ext, 0u);
+                    }
+                }
+                nlist += take;
+                done += take;
+                if (nlist == kCovList) {
+                    flush(nlist);
+                    nlist = 0;
+                }
+            }
         }
     }
+    if (nlist) flush(nlist);
 }
 
 // One wavefront per 64x2 pixel tile (lane = pixel column, rows 2r and 2r+1).  The cell
-// row's non-empty buckets, in path order, are filtered by extent into a per-wave list
-// (paint colour decoded, item base and count).  The list is resolved kCovGroup buckets at
-// a time: each item writes its index into the LDS slot of its first column in the tile
-// (items of a bucket are disjoint and sorted by x), an inclusive max-scan over the lanes
-// then names each column's covering candidate, and the lanes blend in path order:
-// coverage alpha = paint alpha * covered samples / N (output_{8,32}.frag.glsl).
-// The kernel is bound by VALU issue, LDS and load latency together; eight waves per SIMD
-// (registers capped at 64, a few spilled) hide the latency best.  Groups of 8 buckets with
-// the sRGB tables take about 23 KiB of LDS a workgroup, so six workgroups (six waves per
-// SIMD) fit in the CU's 160 KiB, and they get the registers of that occupancy (measured
-// on the 4096-scene batch: 32.7 ms a render against 35.5 ms when capped at four).
-template <int SPP, bool SRGB, int kCovGroup, bool BATCH, bool GRAD>
-__global__ void __launch_bounds__(256, (kCovGroup == 4 || !SRGB) ? 8 : 6) k_composite_cov(CovArgs A) {
+// row's non-empty buckets, in path order, are filtered by extent and tile bitmaps into a
+// per-wave list of up to 64 (paint colour decoded, the tile's cells).  The list's cover bits
+// are transposed, so that every lane holds the list's buckets covering its column as 64
+// bits, and the blend passes run as often as the deepest column's count, each lane taking
+// its own next bucket in path order: coverage alpha = paint alpha * covered samples / N
+// (output_{8,32}.frag.glsl).  An opaque paint over a whole column leaves its own colour
+// exactly, so a column's buckets before its last such one are dropped.
+// Bound by the passes' instructions (about 100 each for eight channels; the next pass's
+// sample counts load during them).  Seven waves per SIMD (batches six, gradients four): six
+// and eight take 1.34 and 1.40 ms for 1.27 on the 2048x2048 illustration.  Finding a column's
+// covering item by LDS slots and a max-scan per bucket, in groups of four buckets: 2.01 ms
+// there, 543 us for 325 on a 4096x4096 sheet of glyphs, 154 for 23 on a 512x512 drawing of
+// opaque cubic chains, 2.5 ms for 0.81 on 1024 such scenes in a batch.
+template <int SPP, bool SRGB, bool BATCH, bool GRAD>
+__global__ void __launch_bounds__(256, GRAD ? 4 : (BATCH ? 6 : 7)) k_composite_cov(CovArgs A) {
     __shared__ float4 s_step[SRGB ? kQuantSteps : 1];
     __shared__ float s_dec[256];
     __shared__ float s_deca[GRAD ? 256 : 1];
-    __shared__ float4 l_src[4][kCovList];
-    __shared__ uint2 l_ref[4][kCovList];
-    __shared__ uint32_t slot[4][kCovGroup][64];
+    __shared__ float4 l_src[4][kCovList];   // paint, alpha / N (a gradient's word, -1)
+    __shared__ uint4 l_ent[4][kCovList];    // {cover, edge, first merged cell, path}
+    __shared__ uint32_t l_queue[4][kRowQueue];
+    __shared__ uint4 l_grad[GRAD ? 4 : 1][GRAD ? kCovList : 1];
     for (int i = threadIdx.x; i < 256; i += 256) {
         s_dec[i] = A.dec_c[i];
         if (GRAD) s_deca[i] = A.dec_a[i];
@@ -1124,7 +1408,7 @@ __global__ void __launch_bounds__(256, (kCovGroup == 4 || !SRGB) ? 8 : 6) k_comp
     if (!BATCH) {
         // Workgroup b runs on XCD b % 8 (round-robin deal): XCD x takes the cell rows
         // x, x + 8, x + 16, ... whole, its workgroups walking them tile by tile, so each
-        // row's items are fetched into one XCD's L2 and every XCD gets rows from the whole
+        // row's records are fetched into one XCD's L2 and every XCD gets rows from the whole
         // image (the per-row work is uneven, so contiguous bands would not balance).
         const int xcd = (int)(blockIdx.x & 7u), t = (int)(blockIdx.x >> 3) * 4 + w;
         const int rr = t / tiles_x, row = xcd + 8 * rr;
@@ -1151,136 +1435,75 @@ __global__ void __launch_bounds__(256, (kCovGroup == 4 || !SRGB) ? 8 : 6) k_comp
         pitch = 4 * W;
         image = A.image + A.simg[lo];
     }
-    const int r = tile / tiles_x;
-    const int tx0 = (tile - r * tiles_x) * 64;
-    const int tx1 = tmin(tx0 + 64, W);
-    const int x = tx0 + lane;
+    const int r = tile / tiles_x, tx = tile - r * tiles_x;
+    const int tx0 = tx * 64, tx1 = tmin(tx0 + 64, W);
+    const int x = tx0 + lane, cell = lane >> 1, half = 12 * (lane & 1);
     const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    constexpr float kInvN = 1.f / (float)SPP;
+    constexpr uint32_t kFull = (uint32_t)SPP * 65u;  // both rows' counts
     float d0[4] = {1.f, 1.f, 1.f, 1.f}, d1[4] = {1.f, 1.f, 1.f, 1.f};
 
-    auto flush = [&](int nlist) {
+    auto flush = [&](int n) {
         wave_sync_lds();
-        for (int g0 = 0; g0 < nlist; g0 += kCovGroup) {
-            const int ng = tmin(kCovGroup, nlist - g0);
-            uint32_t it[kCovGroup], cv[kCovGroup];
-#pragma unroll
-            for (int g = 0; g < kCovGroup; ++g) {
-                slot[w][g][lane] = 0u;
-                const uint2 ref = g < ng ? l_ref[w][g0 + g] : make_uint2(0u, 0u);
-                const bool ld = lane < (int)ref.y;
-                it[g] = ld ? A.items[ref.x + lane] : 0u;
-                cv[g] = ld ? A.icov[ref.x + lane] : 0u;
-            }
-            wave_sync_lds();
-#pragma unroll
-            for (int g = 0; g < kCovGroup; ++g) {
-                if (g >= ng) break;
-                const uint2 ref = l_ref[w][g0 + g];
-                if (ref.y > 64u) {
-                    scatter_big(A.items, ref.x, (int)ref.y, tx0, slot[w][g]);
-                } else if (lane < (int)ref.y) {
-                    const int x0 = (int)(it[g] & 0xFFFFu), iw = (int)(it[g] >> 16);
-                    const int end = x0 + (iw ? iw : 2);
-                    if (end > tx0 && x0 < tx0 + 64) atomicMax(&slot[w][g][tmax(x0 - tx0, 0)], (uint32_t)(lane + 1));
-                }
-            }
-            wave_sync_lds();
-            uint32_t sv[kCovGroup];
-#pragma unroll
-            for (int g = 0; g < kCovGroup; ++g) sv[g] = slot[w][g][lane];
-#pragma unroll
-            for (int g = 0; g < kCovGroup; ++g) sv[g] = (uint32_t)dpp_scan((int)sv[g], 0, OpMax());
-            // Each lane lists the group's buckets covering its column, in path order, as
-            // {n0, n1, g}; the blend passes then run as many times as the deepest lane's
-            // list, each lane blending its own next entry (same per-pixel order as one
-            // pass per bucket, fewer passes where the buckets do not overlap).
-            uint32_t ent[kCovGroup], ent2[GRAD ? kCovGroup : 1];
-            int nent = 0;
-#pragma unroll
-            for (int g = 0; g < kCovGroup; ++g) {
-                ent[g] = 0u;
-                if (g >= ng) break;
-                const uint2 ref = l_ref[w][g0 + g];
-                const int p = (int)sv[g] - 1;
-                uint32_t pit, pcv;
-                if (ref.y > 64u) {
-                    pit = p >= 0 ? A.items[ref.x + p] : 0u;
-                    pcv = p >= 0 ? A.icov[ref.x + p] : 0u;
+        const uint4 mine = lane < n ? l_ent[w][lane] : make_uint4(0u, 0u, 0u, 0u);
+        const uint64_t opaque = __ballot(lane < n && l_src[w][lane].w == kInvN);
+        uint32_t t = transpose32(mine.x);
+        uint64_t L = (uint64_t)(uint32_t)__shfl((int)t, cell, 64) | ((uint64_t)(uint32_t)__shfl((int)t, 32 + cell, 64) << 32);
+        if (x >= W) L = 0ull;
+        if (opaque) {
+            t = transpose32(mine.y);
+            const uint64_t E =
+                (uint64_t)(uint32_t)__shfl((int)t, cell, 64) | ((uint64_t)(uint32_t)__shfl((int)t, 32 + cell, 64) << 32);
+            const uint64_t T = L & ~E & opaque;
+            if (T) L &= ~0ull << (63 - (int)__builtin_clzll(T));
+        }
+        // the next bucket of the lane's column and its sample counts, a pass ahead
+        int b = 0;
+        uint32_t cnt = kFull;
+        auto next = [&]() {
+            b = (int)__builtin_ctzll(L);
+            const uint2 e = *(const uint2 *)&l_ent[w][b].y;
+            cnt = kFull;
+            if ((e.x >> cell) & 1u) cnt = A.icov[e.y + (uint32_t)__popc(e.x & ((1u << cell) - 1u))] >> half;
+        };
+        if (L) next();
+        while (__ballot(L != 0ull)) {
+            // gradient paints cost several solid ones: they wait until no lane has a solid
+            // paint next, and are then blended by all lanes that hold one
+            bool turn = L != 0ull;
+            if (GRAD) {
+                const bool solid = turn && l_src[w][b].w >= 0.f;
+                if (__ballot(solid)) {
+                    turn = solid;
                 } else {
-                    pit = (uint32_t)__shfl((int)it[g], tmax(p, 0), 64);
-                    pcv = (uint32_t)__shfl((int)cv[g], tmax(p, 0), 64);
-                }
-                const int px0 = (int)(pit & 0xFFFFu), pw = (int)(pit >> 16);
-                const int pend = px0 + (pw ? pw : 2);
-                const bool covered = p >= 0 && x < pend && x < W;
-                uint32_t n0 = SPP, n1 = SPP;
-                if (pw == 0) {
-                    n0 = (pcv >> (6 * ((x - px0) * 2))) & 63u;
-                    n1 = (pcv >> (6 * ((x - px0) * 2 + 1))) & 63u;
-                }
-                const uint32_t e = n0 | (n1 << 8) | ((uint32_t)g << 16);
-                const uint32_t e2 = (uint32_t)px0 | ((uint32_t)(pw ? pw : 2) << 16);
-#pragma unroll
-                for (int j = 0; j <= g; ++j) {
-                    ent[j] = (covered && nent == j) ? e : ent[j];
-                    if (GRAD) ent2[j] = (covered && nent == j) ? e2 : ent2[j];
-                }
-                nent += covered ? 1 : 0;
-            }
-#pragma unroll
-            for (int j = 0; j < kCovGroup; ++j) {
-                if (!__ballot(nent > j)) break;
-                if (nent > j) {
-                    const uint32_t e = ent[j];
-                    const float4 src = l_src[w][g0 + (int)(e >> 16)];
-                    if (GRAD && src.w < 0.f) {
-                        // a gradient paint: its colour at each of the lane's two pixels
-                        const uint32_t c = __float_as_uint(src.x);
-                        const int ix0 = (int)(ent2[j] & 0xFFFFu), iw = (int)(ent2[j] >> 16);
+                    if (turn) {
+                        const uint32_t c = __float_as_uint(l_src[w][b].x);
+                        int ix0, iw;
+                        item_extent(A.prec, l_ent[w][b].y, cell, tx0, l_grad[w][b], ix0, iw);
                         const float4 p0 = grad_color(A.G, c, ix0, iw, x, 2 * r, s_dec, s_deca);
                         const float4 p1 = grad_color(A.G, c, ix0, iw, x, 2 * r + 1, s_dec, s_deca);
-                        blend_dec<SRGB>(s_step, d0, p0, p0.w * ((float)(e & 63u) / (float)SPP));
-                        blend_dec<SRGB>(s_step, d1, p1, p1.w * ((float)((e >> 8) & 63u) / (float)SPP));
-                    } else {
-                        blend_dec<SRGB>(s_step, d0, src, src.w * ((float)(e & 63u) / (float)SPP));
-                        blend_dec<SRGB>(s_step, d1, src, src.w * ((float)((e >> 8) & 63u) / (float)SPP));
+                        blend_dec<SRGB>(s_step, d0, p0, p0.w * ((float)(cnt & 63u) * kInvN));
+                        blend_dec<SRGB>(s_step, d1, p1, p1.w * ((float)((cnt >> 6) & 63u) * kInvN));
+                        L &= L - 1ull;
+                        if (L) next();
                     }
+                    continue;
                 }
             }
-            wave_sync_lds();
+            if (turn) {
+                const float4 src = l_src[w][b];
+                const uint32_t cc = cnt;
+                L &= L - 1ull;
+                if (L) next();
+                blend_dec<SRGB>(s_step, d0, src, src.w * (float)(cc & 63u));
+                blend_dec<SRGB>(s_step, d1, src, src.w * (float)((cc >> 6) & 63u));
+            }
         }
+        wave_sync_lds();
     };
 
     const uint32_t q0 = A.rowbeg[row0 + r], q1 = A.rowend[row0 + r];
-    int nlist = 0;
-    for (uint32_t qc = q0; qc < q1; qc += 64) {
-        const bool inq = qc + lane < q1;
-        const uint4 rec = inq ? A.rrec[qc + lane] : make_uint4(0xFFFFu, 0u, 0u, 0u);
-        const uint64_t rt = inq ? A.rtile[qc + lane] : 0ull;
-        const int exlo = (int)(rec.x & 0xFFFFu), exhi = (int)(rec.x >> 16);
-        // a word without alpha paints nothing, unless it names a gradient that paints
-        const bool paints = (rec.y & 0xFF000000u) || (GRAD && rec.y != 0u && grad_paints(A.G, rec.y));
-        const bool ov = inq && exlo < tx1 && exhi > tx0 && ((rt >> tile_bit(tx0, exlo)) & 1ull) && paints;
-        const unsigned long long om = __ballot(ov);
-        if (!om) continue;
-        const int nov = (int)__popcll(om);
-        if (nlist + nov > kCovList) {
-            flush(nlist);
-            nlist = 0;
-        }
-        if (ov) {
-            const int sl = nlist + (int)__popcll(om & lt);
-            const uint32_t c = rec.y;
-            if (GRAD && !(c & 0xFF000000u))
-                l_src[w][sl] = make_float4(__uint_as_float(c), 0.f, 0.f, -1.f);
-            else
-                l_src[w][sl] = make_float4(s_dec[c & 0xFFu], s_dec[(c >> 8) & 0xFFu], s_dec[(c >> 16) & 0xFFu],
-                                           unorm_dec((int)(c >> 24)));
-            l_ref[w][sl] = make_uint2(rec.w, rec.z);
-        }
-        nlist += nov;
-    }
-    if (nlist) flush(nlist);
+    list_row<GRAD>(A, q0, q1, tx, tx1, kInvN, s_dec, l_queue[w], l_src[w], l_ent[w], l_grad[GRAD ? w : 0], flush);
 
     if (x >= W) return;
     const int y0 = 2 * r;
@@ -1532,19 +1755,20 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
     constexpr int NREG = 64 / CPR;
     constexpr int G = GRAD ? 4 : 2;
     constexpr uint32_t FULL = SPP == 8 ? 0xFFFFu : 0xFFFFFFFFu;  // both rows' bits (N = 32: each row)
-    __shared__ float4 s_step[SRGB ? kQuantSteps : 1];
+    __shared__ float4 s_step[SRGB && GRAD ? kQuantSteps : 1];
     __shared__ float s_dec[256];
     __shared__ float s_deca[GRAD ? 256 : 1];
     __shared__ float4 l_src[4][kCovList];
-    __shared__ uint2 l_ref[4][kCovList];
-    __shared__ uint32_t l_pid[4][kCovList];
-    __shared__ uint32_t slot[4][G][64];
+    __shared__ uint4 l_ent[4][kCovList];    // {cover, edge, first merged cell, path}
+    __shared__ uint32_t l_queue[4][kRowQueue];
+    __shared__ uint4 l_grad[GRAD ? 4 : 1][GRAD ? kCovList : 1];
+    __shared__ uint32_t slot[4][G][64];     // staging of the final average
     __shared__ uint32_t tbl[4][G][256];
     for (int i = threadIdx.x; i < 256; i += 256) {
         s_dec[i] = A.dec_c[i];
         if (GRAD) s_deca[i] = A.dec_a[i];
     }
-    for (int i = threadIdx.x; i < (SRGB ? kQuantSteps : 0); i += 256) s_step[i] = A.step_c[i];
+    for (int i = threadIdx.x; i < (SRGB && GRAD ? kQuantSteps : 0); i += 256) s_step[i] = A.step_c[i];
     __syncthreads();
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int W = A.W, H = A.H, tiles_x = A.tiles_x;
@@ -1552,9 +1776,9 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
     const int xcd = (int)(blockIdx.x & 7u), t = (int)(blockIdx.x >> 3) * 4 + w;
     const int rr = t / tiles_x, r = xcd + 8 * rr;
     if (r >= (H + 1) / 2) return;
-    const int tx0 = (t - rr * tiles_x) * 64;
+    const int tx = t - rr * tiles_x, tx0 = tx * 64;
     const int tx1 = tmin(tx0 + 64, W);
-    const int x = tx0 + lane;
+    const int x = tx0 + lane, cell = lane >> 1;
     const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     // blend-phase coordinates of this lane
     const int q = lane / (2 * SPP), dy = (lane / SPP) & 1;
@@ -1565,70 +1789,31 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
         wave_sync_lds();
         for (int g0 = 0; g0 < nlist; g0 += G) {
             const int ng = tmin(G, nlist - g0);
-            uint32_t it[G], mk[G][NW];
             uint4 tv[G];
+            // per column (lane): the sample bits of both rows under each bucket's covering
+            // item, 0 where no item covers it
+            uint32_t cb[G], cbh[G];
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                slot[w][g][lane] = 0u;
-                const uint2 ref = g < ng ? l_ref[w][g0 + g] : make_uint2(0u, 0u);
-                const bool ld = lane < (int)ref.y;
-                it[g] = ld ? A.items[ref.x + lane] : 0u;
-#pragma unroll
-                for (int k = 0; k < NW; ++k) mk[g][k] = 0u;
-                if (ld) load_mask<NW>(A.imask, (size_t)ref.x + lane, mk[g]);
+                const uint4 e = g < ng ? l_ent[w][g0 + g] : make_uint4(0u, 0u, 0u, 0u);
                 // the path's blend table (solid paints; a gradient's l_src.w is negative)
                 const bool solid = g < ng && !(GRAD && l_src[w][g0 + g].w < 0.f);
-                tv[g] = solid ? *(const uint4 *)(A.ptab + (size_t)l_pid[w][g0 + g] * 256 + 4 * lane)
-                              : make_uint4(0u, 0u, 0u, 0u);
+                tv[g] = solid ? *(const uint4 *)(A.ptab + (size_t)e.w * 256 + 4 * lane) : make_uint4(0u, 0u, 0u, 0u);
+                cb[g] = cbh[g] = 0u;
+                if (((e.x >> cell) & 1u) && x < W) {
+                    uint32_t hi = FULL, lo = FULL;
+                    if ((e.y >> cell) & 1u) {
+                        uint32_t pm[NW];
+                        load_mask<NW>(A.imask, (size_t)e.z + (uint32_t)__popc(e.y & ((1u << cell) - 1u)), pm);
+                        lo = column_bits<SPP>(pm, lane & 1, hi);
+                    }
+                    cb[g] = lo;
+                    cbh[g] = SPP == 32 ? hi : 0u;
+                }
             }
 #pragma unroll
             for (int g = 0; g < G; ++g) *(uint4 *)&tbl[w][g][4 * lane] = tv[g];
             wave_sync_lds();
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                if (g >= ng) break;
-                const uint2 ref = l_ref[w][g0 + g];
-                if (ref.y > 64u) {
-                    scatter_big(A.items, ref.x, (int)ref.y, tx0, slot[w][g]);
-                } else if (lane < (int)ref.y) {
-                    const int x0 = (int)(it[g] & 0xFFFFu), iw = (int)(it[g] >> 16);
-                    const int end = x0 + (iw ? iw : 2);
-                    if (end > tx0 && x0 < tx0 + 64) atomicMax(&slot[w][g][tmax(x0 - tx0, 0)], (uint32_t)(lane + 1));
-                }
-            }
-            wave_sync_lds();
-            // per column (lane): the sample bits of both rows under each bucket's covering
-            // item, 0 where no item covers it; the covering item's extent for gradients
-            uint32_t cb[G], cbh[G], ce[GRAD ? G : 1];
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                cb[g] = 0u;
-                cbh[g] = 0u;
-                if (GRAD) ce[g] = 0u;
-                if (g >= ng) break;
-                const uint2 ref = l_ref[w][g0 + g];
-                const int p = (int)(uint32_t)dpp_scan((int)slot[w][g][lane], 0, OpMax()) - 1;
-                uint32_t pit, pm[NW];
-                if (ref.y > 64u) {
-                    pit = p >= 0 ? A.items[ref.x + p] : 0u;
-#pragma unroll
-                    for (int k = 0; k < NW; ++k) pm[k] = 0u;
-                    if (p >= 0) load_mask<NW>(A.imask, (size_t)ref.x + p, pm);
-                } else {
-                    pit = (uint32_t)__shfl((int)it[g], tmax(p, 0), 64);
-#pragma unroll
-                    for (int k = 0; k < NW; ++k) pm[k] = (uint32_t)__shfl((int)mk[g][k], tmax(p, 0), 64);
-                }
-                const int px0 = (int)(pit & 0xFFFFu), pw = (int)(pit >> 16);
-                const int pend = px0 + (pw ? pw : 2);
-                if (p >= 0 && x < pend && x < W) {
-                    uint32_t hi = FULL, lo = FULL;
-                    if (pw == 0) lo = column_bits<SPP>(pm, x - px0, hi);
-                    cb[g] = lo;
-                    cbh[g] = SPP == 32 ? hi : 0u;
-                    if (GRAD) ce[g] = (uint32_t)px0 | ((uint32_t)(pw ? pw : 2) << 16);
-                }
-            }
             // blend, bucket by bucket in path order, one wave-wide pass per state register
             // holding a covered column: four LDS reads of the path's blend table for a
             // solid paint, the blend arithmetic on the pixel's own paint for a gradient.
@@ -1639,7 +1824,6 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
                 if (!regs) continue;
                 const float4 src = l_src[w][g0 + g];
                 const bool gpaint = GRAD && src.w < 0.f;
-                const uint32_t ceg = GRAD ? ce[g] : 0u;
                 // register p's lanes are its columns' sample bits in column order (lane
                 // q * 2N + dy * N + s is bit dy * N + s of column p * CPR + q; N = 32: the
                 // rows' words cb, cbh), so the covered lanes form one wave-wide mask read
@@ -1668,9 +1852,11 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
                 } else {
                     S.apply1(regs, [&](uint32_t st, int p) -> uint32_t {
                         const int c = p * CPR + q;
-                        const uint32_t e = (uint32_t)__shfl((int)ceg, c, 64);
-                        const float4 pa = grad_color(A.G, __float_as_uint(src.x), (int)(e & 0xFFFFu), (int)(e >> 16),
-                                                     tx0 + c, 2 * r + dy, s_dec, s_deca);
+                        const uint32_t ed = l_ent[w][g0 + g].y;
+                        int ix0 = 0, iw = 1;
+                        if ((l_ent[w][g0 + g].x >> (c >> 1)) & 1u)
+                            item_extent(A.prec, ed, c >> 1, tx0, l_grad[w][g0 + g], ix0, iw);
+                        const float4 pa = grad_color(A.G, __float_as_uint(src.x), ix0, iw, tx0 + c, 2 * r + dy, s_dec, s_deca);
                         const uint32_t nst = blend_code<SRGB>(s_step, s_dec, st, pa, pa.w);
                         return covers(p) ? nst : st;
                     });
@@ -1681,35 +1867,7 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
     };
 
     const uint32_t q0 = A.rowbeg[r], q1 = A.rowend[r];
-    int nlist = 0;
-    for (uint32_t qc = q0; qc < q1; qc += 64) {
-        const bool inq = qc + lane < q1;
-        const uint4 rec = inq ? A.rrec[qc + lane] : make_uint4(0xFFFFu, 0u, 0u, 0u);
-        const uint64_t rt = inq ? A.rtile[qc + lane] : 0ull;
-        const int exlo = (int)(rec.x & 0xFFFFu), exhi = (int)(rec.x >> 16);
-        const bool paints = (rec.y & 0xFF000000u) || (GRAD && rec.y != 0u && grad_paints(A.G, rec.y));
-        const bool ov = inq && exlo < tx1 && exhi > tx0 && ((rt >> tile_bit(tx0, exlo)) & 1ull) && paints;
-        const unsigned long long om = __ballot(ov);
-        if (!om) continue;
-        const int nov = (int)__popcll(om);
-        if (nlist + nov > kCovList) {
-            flush(nlist);
-            nlist = 0;
-        }
-        if (ov) {
-            const int sl = nlist + (int)__popcll(om & lt);
-            const uint32_t c = rec.y;
-            if (GRAD && !(c & 0xFF000000u))
-                l_src[w][sl] = make_float4(__uint_as_float(c), 0.f, 0.f, -1.f);
-            else
-                l_src[w][sl] = make_float4(s_dec[c & 0xFFu], s_dec[(c >> 8) & 0xFFu], s_dec[(c >> 16) & 0xFFu],
-                                           unorm_dec((int)(c >> 24)));
-            l_ref[w][sl] = make_uint2(rec.w, rec.z);
-            l_pid[w][sl] = A.rpath[qc + lane];
-        }
-        nlist += nov;
-    }
-    if (nlist) flush(nlist);
+    list_row<GRAD>(A, q0, q1, tx, tx1, 1.f, s_dec, l_queue[w], l_src[w], l_ent[w], l_grad[GRAD ? w : 0], flush);
 
     // resolve: G registers at a time are staged in this wave's slot rows (G x 64 words);
     // lane (pixel, channel) sums the pixel's decoded samples in sample order, divides by N
@@ -1739,7 +1897,7 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
             }
             const float avg = sum / (float)SPP;
             float tmp;
-            const uint32_t code = (SRGB && ch < 3) ? (uint32_t)srgb_code(s_step, avg, tmp) : (uint32_t)unorm_code(avg);
+            const uint32_t code = (SRGB && ch < 3) ? (uint32_t)srgb_code(GRAD ? s_step : A.step_c, avg, tmp) : (uint32_t)unorm_code(avg);
             uint32_t word = code << (8 * ch);
             word |= (uint32_t)__shfl_xor((int)word, 1, 64);
             word |= (uint32_t)__shfl_xor((int)word, 2, 64);
@@ -1750,20 +1908,20 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
     }
 }
 
-// Row-list records for the compositors: one 16-byte load per listed bucket (and its path
-// id for the multisample compositor's blend tables).
+// Row-list records for the compositors.
 __global__ void k_row_records(int64_t NB, const uint32_t *__restrict__ n_ptr, const uint32_t *__restrict__ rowvals,
-                              const uint32_t *__restrict__ bext, const int2 *__restrict__ binfo,
-                              const uint32_t *__restrict__ finfo, const uint32_t *__restrict__ bicnt,
-                              const uint32_t *__restrict__ boff, const uint64_t *__restrict__ btile,
-                              uint4 *__restrict__ rrec, uint64_t *__restrict__ rtile, uint32_t *__restrict__ rpath) {
+                              const uint4 *__restrict__ brec, const int2 *__restrict__ binfo,
+                              const uint32_t *__restrict__ finfo, const uint32_t *__restrict__ boff,
+                              uint32_t *__restrict__ rext, uint4 *__restrict__ rrec,
+                              ulonglong2 *__restrict__ rtile) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= NB || q >= (int64_t)*n_ptr) return;
     const uint32_t bb = rowvals[q];
     const uint32_t path = (uint32_t)binfo[bb].x;
-    rrec[q] = make_uint4(bext[bb], finfo[path], bicnt[bb], 2u * boff[bb]);
-    rtile[q] = btile[bb];
-    if (rpath) rpath[q] = path;
+    const uint4 br = brec[2 * (size_t)bb], bf = brec[2 * (size_t)bb + 1];
+    rext[q] = br.x;
+    rrec[q] = make_uint4(finfo[path], br.y, boff[bb], path);
+    rtile[q] = make_ulonglong2((uint64_t)br.z | ((uint64_t)br.w << 32), (uint64_t)bf.x | ((uint64_t)bf.y << 32));
 }
 
 // Device requantisation of arbitrary values (colour-table self-check): codes and the
@@ -1816,14 +1974,14 @@ __global__ void k_encode_sweep(uint32_t lo, uint32_t hi, const float4 *__restric
 // draw list + merged masks in the reference's order and layout (.cu:789-868, 1195-1266)
 template <int SPP>
 __global__ void k_debug_draw(int64_t NB, const int2 *__restrict__ binfo, const uint32_t *__restrict__ finfo,
-                             const uint32_t *__restrict__ boff, const uint32_t *__restrict__ bicnt,
+                             const uint32_t *__restrict__ boff, const uint4 *__restrict__ brec,
                              const uint32_t *__restrict__ items, const uint32_t *__restrict__ imask,
                              const uint32_t *__restrict__ moff, const uint32_t *__restrict__ ioff, int4 *draw,
                              uint32_t *mmask4) {
     constexpr int NW = Words<SPP>::n;
     int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= NB) return;
-    const uint32_t cnt = bicnt[b];
+    const uint32_t cnt = brec[2 * b + 1].z;
     if (!cnt) return;
     const int2 info = binfo[b];
     const uint32_t fill = finfo[info.x];
@@ -1832,10 +1990,11 @@ __global__ void k_debug_draw(int64_t NB, const int2 *__restrict__ binfo, const u
     uint32_t mi = moff[b];
     const uint32_t io = ioff[b];
     uint32_t o = io;
-    auto put_merged = [&](uint32_t j, int x0) {
+    size_t mj = boff[b];  // the bucket's merged cells' masks, in x order
+    auto put_merged = [&](int x0) {
         draw[o++] = make_int4((int32_t)(((uint32_t)y << 16) | (uint32_t)x0), 2, (int)fill, (int)(mi + 1));
         uint32_t mk[4] = {0u, 0u, 0u, 0u};
-        load_mask<NW>(imask, ib + j, mk);
+        load_mask<NW>(imask, mj++, mk);
         *(uint4 *)(mmask4 + 4 * (size_t)mi) = make_uint4(mk[0], mk[1], mk[2], mk[3]);
         ++mi;
     };
@@ -1843,26 +2002,27 @@ __global__ void k_debug_draw(int64_t NB, const int2 *__restrict__ binfo, const u
         const uint32_t it = items[ib + j];
         const int x0 = (int)(it & 0xFFFFu), w = (int)(it >> 16);
         if (w == 0) {
-            put_merged(j, x0);
+            put_merged(x0);
             continue;
         }
         // a span followed by the merged fragment it ends at: the reference emits that
         // fragment first (.cu:836-862)
         const bool pair = j + 1 < cnt && (items[ib + j + 1] >> 16) == 0u &&
                           (int)(items[ib + j + 1] & 0xFFFFu) == x0 + w;
-        if (pair) put_merged(j + 1, x0 + w);
+        if (pair) put_merged(x0 + w);
         draw[o++] = make_int4((int32_t)(((uint32_t)y << 16) | (uint32_t)x0), w, (int)fill, 0);
         if (pair) ++j;
     }
 }
 
-__global__ void __launch_bounds__(256) k_count_reduce(const uint32_t *__restrict__ a, const uint32_t *__restrict__ c,
-                                                      size_t n, unsigned long long *out) {
+// out[0] += merged cells, out[1] += items
+__global__ void __launch_bounds__(256) k_count_reduce(const uint4 *__restrict__ brec, size_t n, unsigned long long *out) {
     __shared__ unsigned long long part[2][4];
     unsigned long long sa = 0, sc = 0;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        sa += a[i];
-        sc += c[i];
+        const uint2 c = *(const uint2 *)&brec[2 * i + 1].z;
+        sa += c.y;
+        sc += c.x;
     }
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) {
@@ -1880,6 +2040,13 @@ __global__ void __launch_bounds__(256) k_count_reduce(const uint32_t *__restrict
     }
 }
 
+__global__ void k_debug_counts(int64_t NB, const uint4 *__restrict__ brec, uint32_t *merged, uint32_t *items) {
+    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= NB) return;
+    merged[b] = brec[2 * b + 1].w;
+    items[b] = brec[2 * b + 1].z;
+}
+
 inline unsigned blocks_for(int64_t n, unsigned t) { return (unsigned)((n + t - 1) / t); }
 
 }  // namespace
@@ -1892,18 +2059,21 @@ void launch_resolve(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t s
     A.pcanvas = sc.pcanvas; A.scarry = f.scarry;
     // the merged masks feed the multisample compositor and the debug draw list; the
     // coverage compositor reads only the per-pixel sample counts
-    A.items = f.items; A.imask = f.keep_masks ? f.imask : nullptr; A.icov = f.icov; A.bicnt = f.bicnt;
-    A.bmcnt = f.bmcnt; A.bext = f.bext;
-    A.btile = f.btile;
+    A.items = f.items; A.imask = f.imask; A.icov = f.icov; A.prec = f.prec; A.brec = f.brec;
     A.big_list = f.big_list; A.big_count = f.big_count; A.err = f.err_flag;  // cleared at the frame's start
     const unsigned g1 = (unsigned)std::min<int64_t>(f.NB, f.resolve_grid > 0 ? f.resolve_grid : kResolveBlocks);
     const unsigned gc = f.class_grid > 0 ? (unsigned)f.class_grid : 4096u;
     dim3 b64(64);
+#define SL_LAUNCH2(N, K)                                                              \
+    do {                                                                              \
+        hipLaunchKernelGGL((k_resolve_first<N, K>), dim3(g1), b64, 0, s, A);          \
+        hipLaunchKernelGGL((k_resolve_big<N, K>), dim3(gc), b64, 0, s, A);            \
+        hipLaunchKernelGGL((k_resolve_huge<N, K>), dim3(1024), b64, 0, s, A);         \
+    } while (0)
 #define SL_LAUNCH(N)                                                                  \
     do {                                                                              \
-        hipLaunchKernelGGL(k_resolve_first<N>, dim3(g1), b64, 0, s, A);               \
-        hipLaunchKernelGGL(k_resolve_big<N>, dim3(gc), b64, 0, s, A);                  \
-        hipLaunchKernelGGL(k_resolve_huge<N>, dim3(1024), b64, 0, s, A);              \
+        if (f.keep_masks) SL_LAUNCH2(N, true);                                        \
+        else SL_LAUNCH2(N, false);                                                    \
     } while (0)
     if (t.spp == 8) SL_LAUNCH(8);
     else if (t.spp == 16) SL_LAUNCH(16);
@@ -1922,7 +2092,7 @@ void launch_order_rows(const SceneDev &sc, Frame &f, hipStream_t s) {
     const int64_t R = f.R;
     launch_fill2_u32(f.rowbeg, f.rowend, 0u, (size_t)R, s);
     if (!f.NB) return;
-    hipLaunchKernelGGL(k_nz_flags, dim3(blocks_for(f.NB, 256)), dim3(256), 0, s, f.NB, (const uint32_t *)f.bicnt, f.nz_flag);
+    hipLaunchKernelGGL(k_nz_flags, dim3(blocks_for(f.NB, 256)), dim3(256), 0, s, f.NB, (const uint4 *)f.brec, f.nz_flag);
     scan_exclusive_u32(f.nz_flag, f.nz_off, (size_t)f.NB, f.scan_tmp, s);
     hipLaunchKernelGGL(k_nz_compact, dim3(blocks_for(f.NB, 256)), dim3(256), 0, s, f.NB, (const uint32_t *)f.nz_flag,
                        (const uint32_t *)f.nz_off, (const int2 *)f.binfo, sc.pcanvas, f.nz_keys[0], f.nz_vals[0]);
@@ -1951,9 +2121,8 @@ void launch_order_rows(const SceneDev &sc, Frame &f, hipStream_t s) {
     hipLaunchKernelGGL(k_row_bounds, dim3(blocks_for(f.NB, 256)), dim3(256), 0, s, (const uint32_t *)f.nz_keys[0], n_ptr,
                        f.rowbeg, f.rowend);
     hipLaunchKernelGGL(k_row_records, dim3(blocks_for(f.NB, 256)), dim3(256), 0, s, f.NB, n_ptr,
-                           (const uint32_t *)f.nz_vals[0], (const uint32_t *)f.bext, (const int2 *)f.binfo, sc.finfo,
-                           (const uint32_t *)f.bicnt, (const uint32_t *)f.boff, (const uint64_t *)f.btile, f.rrec,
-                           f.rtile, f.rpath);
+                           (const uint32_t *)f.nz_vals[0], (const uint4 *)f.brec, (const int2 *)f.binfo, sc.finfo,
+                           (const uint32_t *)f.boff, f.rext, f.rrec, f.rtile);
 }
 
 void launch_composite(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t s) {
@@ -1963,8 +2132,8 @@ void launch_composite(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t
     if (!f.ms) {
         CovArgs C;
         C.W = f.W; C.H = f.H; C.tiles_x = tiles_x;
-        C.rowbeg = f.rowbeg; C.rowend = f.rowend; C.rrec = f.rrec; C.rtile = f.rtile;
-        C.items = f.items; C.icov = f.icov; C.imask = nullptr; C.rpath = nullptr; C.ptab = nullptr; C.dec_c = t.dec_c; C.dec_a = t.dec_a; C.step_c = t.step_c;
+        C.rowbeg = f.rowbeg; C.rowend = f.rowend; C.rext = f.rext; C.rrec = f.rrec; C.rtile = f.rtile;
+        C.prec = f.prec; C.icov = f.icov; C.imask = nullptr; C.ptab = nullptr; C.dec_c = t.dec_c; C.dec_a = t.dec_a; C.step_c = t.step_c;
         C.image = f.image; C.pitch = f.pitch;
         C.G = f.grad;
         C.nscenes = f.nscenes; C.ntiles = ntiles; C.stile = f.stile; C.simg = f.simg;
@@ -1972,15 +2141,9 @@ void launch_composite(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t
         dim3 g(f.nscenes ? blocks_for(ntiles, 4) : 8u * blocks_for((int64_t)tiles_x * ((R + 7) / 8), 4)), b(256);
 #define SL_LAUNCH(N, SR)                                                                   \
     do {                                                                                   \
-        if (f.nscenes) {                                                                   \
-            if (f.comp_group == 4) hipLaunchKernelGGL((k_composite_cov<N, SR, 4, true, false>), g, b, 0, s, C); \
-            else hipLaunchKernelGGL((k_composite_cov<N, SR, 8, true, false>), g, b, 0, s, C);               \
-        } else if (f.has_grad) {                                                           \
-            hipLaunchKernelGGL((k_composite_cov<N, SR, 4, false, true>), g, b, 0, s, C);   \
-        } else {                                                                           \
-            if (f.comp_group == 4) hipLaunchKernelGGL((k_composite_cov<N, SR, 4, false, false>), g, b, 0, s, C); \
-            else hipLaunchKernelGGL((k_composite_cov<N, SR, 8, false, false>), g, b, 0, s, C);               \
-        }                                                                                  \
+        if (f.nscenes) hipLaunchKernelGGL((k_composite_cov<N, SR, true, false>), g, b, 0, s, C);        \
+        else if (f.has_grad) hipLaunchKernelGGL((k_composite_cov<N, SR, false, true>), g, b, 0, s, C);  \
+        else hipLaunchKernelGGL((k_composite_cov<N, SR, false, false>), g, b, 0, s, C);                 \
     } while (0)
         if (f.srgb) {
             if (t.spp == 8) SL_LAUNCH(8, true);
@@ -1996,8 +2159,8 @@ void launch_composite(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t
     }
     CovArgs C;
     C.W = f.W; C.H = f.H; C.tiles_x = tiles_x;
-    C.rowbeg = f.rowbeg; C.rowend = f.rowend; C.rrec = f.rrec; C.rtile = f.rtile;
-    C.items = f.items; C.icov = f.icov; C.imask = f.imask; C.rpath = f.rpath; C.ptab = f.ptab;
+    C.rowbeg = f.rowbeg; C.rowend = f.rowend; C.rext = f.rext; C.rrec = f.rrec; C.rtile = f.rtile;
+    C.prec = f.prec; C.icov = f.icov; C.imask = f.imask; C.ptab = f.ptab;
     C.dec_c = t.dec_c; C.dec_a = t.dec_a; C.step_c = t.step_c;
     C.image = f.image; C.pitch = f.pitch;
     C.G = f.grad;
@@ -2055,17 +2218,21 @@ void launch_debug_draw_list(const SceneDev &sc, const Tables &t, Frame &f, const
     dim3 g(blocks_for(f.NB, 256)), b(256);
     if (t.spp == 8)
         hipLaunchKernelGGL(k_debug_draw<8>, g, b, 0, s, f.NB, (const int2 *)f.binfo, sc.finfo, (const uint32_t *)f.boff,
-                           (const uint32_t *)f.bicnt, (const uint32_t *)f.items, (const uint32_t *)f.imask, moff, ioff, draw, mmask4);
+                           (const uint4 *)f.brec, (const uint32_t *)f.items, (const uint32_t *)f.imask, moff, ioff, draw, mmask4);
     else if (t.spp == 16)
         hipLaunchKernelGGL(k_debug_draw<16>, g, b, 0, s, f.NB, (const int2 *)f.binfo, sc.finfo, (const uint32_t *)f.boff,
-                           (const uint32_t *)f.bicnt, (const uint32_t *)f.items, (const uint32_t *)f.imask, moff, ioff, draw, mmask4);
+                           (const uint4 *)f.brec, (const uint32_t *)f.items, (const uint32_t *)f.imask, moff, ioff, draw, mmask4);
     else
         hipLaunchKernelGGL(k_debug_draw<32>, g, b, 0, s, f.NB, (const int2 *)f.binfo, sc.finfo, (const uint32_t *)f.boff,
-                           (const uint32_t *)f.bicnt, (const uint32_t *)f.items, (const uint32_t *)f.imask, moff, ioff, draw, mmask4);
+                           (const uint4 *)f.brec, (const uint32_t *)f.items, (const uint32_t *)f.imask, moff, ioff, draw, mmask4);
 }
 
-void launch_count_reduce(const uint32_t *a, const uint32_t *c, size_t n, unsigned long long *out, hipStream_t s) {
-    hipLaunchKernelGGL(k_count_reduce, dim3(256), dim3(256), 0, s, a, c, n, out);
+void launch_count_reduce(const uint4 *brec, size_t n, unsigned long long *out, hipStream_t s) {
+    hipLaunchKernelGGL(k_count_reduce, dim3(256), dim3(256), 0, s, brec, n, out);
+}
+
+void launch_debug_counts(const Frame &f, uint32_t *merged, uint32_t *items, hipStream_t s) {
+    if (f.NB) hipLaunchKernelGGL(k_debug_counts, dim3(blocks_for(f.NB, 256)), dim3(256), 0, s, f.NB, (const uint4 *)f.brec, merged, items);
 }
 
 }  // namespace sl
