@@ -35,9 +35,9 @@ struct DevBuf {
 // arena whose arrays are carved out of the library's static scratch instead.
 struct Arena {
     DevBuf b_pcnt, b_nchain, b_choff, b_chains, b_chain_t;
-    DevBuf b_tvtx, b_pflags, b_prow, b_crec, b_cfrag, b_coff, b_ts, b_pnb, b_pbase, b_binfo, b_bcount,
-        b_boff, b_bwsum, b_bcarry, b_rec_meta, b_rec_mask, b_scratch, b_items, b_imask, b_icov, b_prec, b_brec, b_big_list, b_small, b_nz_flag, b_nz_off, b_nzk0, b_nzk1, b_nzv0, b_nzv1, b_rs_hist, b_rs_hoff,
-        b_rowbeg, b_rowend, b_rrec, b_rtile, b_rext, b_ptab, b_image, b_scan_tmp, b_lcount;
+    DevBuf b_tvtx, b_pflags, b_prow, b_crec, b_cfrag, b_coff, b_ts, b_pbase, b_binfo, b_bcount,
+        b_boff, b_bwsum, b_bcarry, b_rec_meta, b_rec_mask, b_scratch, b_items, b_imask, b_icov, b_prec, b_bcnt, b_big_list, b_small, b_rpos, b_rowcnt, b_rowoff,
+        b_rrec, b_rtile, b_rext, b_ptab, b_image, b_scan_tmp, b_lcount;
     // carving state: non-null base = every array comes from [base, base + cap)
     uint8_t *carve_base = nullptr;
     size_t carve_cap = 0, carve_off = 0;
@@ -111,7 +111,6 @@ struct sl_handle {
     // device address of this GPU's static scratch (the allocation-free frame)
     void *noalloc_scratch = nullptr;
     int64_t NB = 0;
-    uint32_t *nz_vals_sorted = nullptr;
     // Status of the last single-scene frame, copied back without waiting at the end of the
     // frame into pinned memory (words 0..7 of the frame's small block: big-bucket count,
     // error flags, then the merged-fragment and item totals) and read when the frame is
@@ -434,7 +433,7 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
     if ((rc = ensure_in(h, A, A.b_tvtx, (size_t)V * 8)) || (rc = ensure_in(h, A, A.b_pflags, (size_t)P * 4)) ||
         (rc = ensure_in(h, A, A.b_prow, (size_t)P * 8)) || (rc = ensure_in(h, A, A.b_crec, (size_t)C * 64)) ||
         (rc = ensure_in(h, A, A.b_cfrag, ((size_t)C + 1) * 4)) ||
-        (rc = ensure_in(h, A, A.b_coff, ((size_t)C + 1) * 4)) || (rc = ensure_in(h, A, A.b_pnb, ((size_t)P + 1) * 4)) ||
+        (rc = ensure_in(h, A, A.b_coff, ((size_t)C + 1) * 4)) ||
         (rc = ensure_in(h, A, A.b_pcnt, (size_t)C * 20)) || (rc = ensure_in(h, A, A.b_nchain, ((size_t)C + 1) * 4)) ||
         (rc = ensure_in(h, A, A.b_choff, ((size_t)C + 1) * 4)) ||
         (rc = ensure_in(h, A, A.b_pbase, ((size_t)P + 1) * 4)) || (rc = ensure_in(h, A, A.b_small, 64)) ||
@@ -444,7 +443,7 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
         return rc;
     f.tvtx = P_<float2>(A.b_tvtx); f.pflags = P_<uint32_t>(A.b_pflags); f.prow = P_<int2>(A.b_prow);
     f.crec = P_<float4>(A.b_crec); f.cfrag = P_<uint32_t>(A.b_cfrag);
-    f.coff = P_<uint32_t>(A.b_coff); f.pnb = P_<uint32_t>(A.b_pnb); f.pbase = P_<uint32_t>(A.b_pbase);
+    f.coff = P_<uint32_t>(A.b_coff); f.pbase = P_<uint32_t>(A.b_pbase);
     f.pcnt = P_<uint32_t>(A.b_pcnt); f.nchain = P_<uint32_t>(A.b_nchain); f.choff = P_<uint32_t>(A.b_choff);
     f.image = carved ? out_image : P_<uint8_t>(A.b_image);
     if (!carved) { h->img_W = h->W; h->img_H = h->H; }
@@ -456,19 +455,17 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
         if (h->timing && !replay) (void)hipEventRecord(h->ev[i], s);
     };
     mark(0);
-    sl::launch_fill_u32(f.big_count, 0u, 2, s);  // the big-bucket count and the error flag
-    sl::launch_path_init(sc, f, s);
+    f.lcount = P_<uint32_t>(A.b_lcount);
+    sl::launch_frame_init(sc, f, s);  // path ranges, the status block, the work lists' counts
     sl::launch_transform(sc, f, s);
     if ((rc = check_launch(h, "transform"))) return rc;
     mark(1);
     sl::launch_monotone(sc, f, s);
-    sl::scan_exclusive_u32(f.cfrag, f.coff, C, f.scan_tmp, s);
-    sl::scan_exclusive_u32(f.nchain, f.choff, C, f.scan_tmp, s);
+    sl::scan2_exclusive_u32(f.cfrag, f.coff, f.nchain, f.choff, C, f.scan_tmp, s);
     if ((rc = check_launch(h, "monotone"))) return rc;
     // the bucket ranges need only the paths' row ranges, final after the monotone pass, so
     // an eager frame reads its three sizes (fragments, chains, buckets) in one round trip
     sl::launch_path_buckets(sc, f, s);
-    sl::scan_exclusive_u32(f.pnb, f.pbase, P, f.scan_tmp, s);
     uint32_t F = 0, NCH = 0, NB = 0;
     if (replay) {
         F = h->last_F;
@@ -476,10 +473,13 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
         NB = h->last_NB;
     } else {
         if (!carved) h->sized = false;
-        HIPCHK(h, hipMemcpyAsync(&F, f.coff + C, 4, hipMemcpyDeviceToHost, s));
-        HIPCHK(h, hipMemcpyAsync(&NCH, f.choff + C, 4, hipMemcpyDeviceToHost, s));
-        HIPCHK(h, hipMemcpyAsync(&NB, f.pbase + P, 4, hipMemcpyDeviceToHost, s));
+        // into the status block's second half, which no queued frame writes
+        sl::launch_sizes(sc, f, h->fstat + 8, s);
+        HIPCHK(h, hipGetLastError());
         HIPCHK(h, hipStreamSynchronize(s));
+        F = h->fstat[8];
+        NCH = h->fstat[9];
+        NB = h->fstat[10];
         h->counts.path = P; h->counts.curve = C; h->counts.vertex = V;
         h->counts.curve_fragment = F;
         h->counts.merged_fragment = 0;
@@ -506,7 +506,6 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
     f.ts = P_<int2>(A.b_ts);
     f.chains = P_<uint4>(A.b_chains);
     f.plist = f.chains + (size_t)NCH;
-    f.lcount = P_<uint32_t>(A.b_lcount);
     f.chain_t = P_<float>(A.b_chain_t);
     mark(2);
     sl::launch_intersect(sc, f, s);
@@ -515,23 +514,18 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
     f.NB = NB;
     if (!replay) h->NB = NB;
     const size_t R = (size_t)f.R;
-    const size_t rs_tiles = ((size_t)NB + 2047) / 2048;
-    scan_need = sl::scan_tmp_elems_needed(
-        std::max<size_t>({(size_t)C + 1, (size_t)P + 1, (size_t)NB + 1, 256 * rs_tiles + 1, (size_t)F + 1}));
+    const size_t shares = f.rowshares = sl::row_shares(P, R, NB);
+    scan_need = sl::scan_tmp_elems_needed(std::max<size_t>({(size_t)C + 1, (size_t)P + 1, (size_t)NB + 1, R * shares + 1}));
     if ((rc = ensure_in(h, A, A.b_binfo, (size_t)NB * 8)) || (rc = ensure_in(h, A, A.b_bcount, ((size_t)NB + 1) * 4)) ||
         (rc = ensure_in(h, A, A.b_boff, ((size_t)NB + 1) * 4)) || (rc = ensure_in(h, A, A.b_bwsum, ((size_t)NB + 1) * 4)) ||
         (rc = ensure_in(h, A, A.b_bcarry, ((size_t)NB + 1) * 4)) ||
         (rc = ensure_in(h, A, A.b_rec_meta, (size_t)F * 4)) || (rc = ensure_in(h, A, A.b_rec_mask, (size_t)F * 4 * NW)) ||
         (rc = ensure_in(h, A, A.b_scratch, (size_t)F * 4)) || (rc = ensure_in(h, A, A.b_items, h->debug ? (size_t)F * 8 : 0)) ||
         (rc = ensure_in(h, A, A.b_imask, f.keep_masks ? (size_t)F * 4 * NW : 0)) || (rc = ensure_in(h, A, A.b_icov, (size_t)F * 4)) ||
-        (rc = ensure_in(h, A, A.b_prec, (size_t)F * 16)) || (rc = ensure_in(h, A, A.b_brec, (size_t)NB * 32)) ||
-        (rc = ensure_in(h, A, A.b_big_list, (size_t)NB * 4)) || (rc = ensure_in(h, A, A.b_nz_flag, ((size_t)NB + 1) * 4)) ||
-        (rc = ensure_in(h, A, A.b_nz_off, ((size_t)NB + 1) * 4)) || (rc = ensure_in(h, A, A.b_nzk0, (size_t)NB * 4)) ||
-        (rc = ensure_in(h, A, A.b_nzk1, (size_t)NB * 4)) || (rc = ensure_in(h, A, A.b_nzv0, (size_t)NB * 4)) ||
-        (rc = ensure_in(h, A, A.b_nzv1, (size_t)NB * 4)) || (rc = ensure_in(h, A, A.b_rs_hist, 256 * rs_tiles * 4 + 16)) ||
-        (rc = ensure_in(h, A, A.b_rs_hoff, (256 * rs_tiles + 1) * 4 + 16)) || (rc = ensure_in(h, A, A.b_rowbeg, R * 4)) ||
-        (rc = ensure_in(h, A, A.b_rowend, R * 4)) || (rc = ensure_in(h, A, A.b_rrec, (size_t)NB * 16)) ||
-        (rc = ensure_in(h, A, A.b_rtile, (size_t)NB * 16)) ||
+        (rc = ensure_in(h, A, A.b_prec, (size_t)F * 16)) || (rc = ensure_in(h, A, A.b_bcnt, (size_t)NB * 8)) ||
+        (rc = ensure_in(h, A, A.b_big_list, (size_t)NB * 4)) || (rc = ensure_in(h, A, A.b_rpos, (size_t)NB * 4)) ||
+        (rc = ensure_in(h, A, A.b_rowcnt, R * shares * 4)) || (rc = ensure_in(h, A, A.b_rowoff, (R * shares + 1) * 4)) ||
+        (rc = ensure_in(h, A, A.b_rrec, (size_t)NB * 16)) || (rc = ensure_in(h, A, A.b_rtile, (size_t)NB * 16)) ||
         (rc = ensure_in(h, A, A.b_rext, (size_t)NB * 4)) || (rc = ensure_in(h, A, A.b_ptab, f.ms ? (size_t)P * 1024 : 0)) ||
         (rc = ensure_in(h, A, A.b_scan_tmp, scan_need * 4)))
         return rc;
@@ -543,34 +537,27 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
     f.icov = P_<uint32_t>(A.b_icov); f.prec = P_<uint4>(A.b_prec);
     // the rank array lives in the large-bucket scratch (used only later, by the resolve)
     f.frank = f.scratch_keys;
-    f.brec = P_<uint4>(A.b_brec);
-    f.big_list = P_<uint32_t>(A.b_big_list); f.nz_flag = P_<uint32_t>(A.b_nz_flag); f.nz_off = P_<uint32_t>(A.b_nz_off);
-    f.nz_keys[0] = P_<uint32_t>(A.b_nzk0); f.nz_keys[1] = P_<uint32_t>(A.b_nzk1);
-    f.nz_vals[0] = P_<uint32_t>(A.b_nzv0); f.nz_vals[1] = P_<uint32_t>(A.b_nzv1);
-    f.rs_hist = P_<uint32_t>(A.b_rs_hist); f.rs_hoff = P_<uint32_t>(A.b_rs_hoff);
-    f.rowbeg = P_<uint32_t>(A.b_rowbeg); f.rowend = P_<uint32_t>(A.b_rowend);
+    f.bcnt = P_<uint2>(A.b_bcnt);
+    f.big_list = P_<uint32_t>(A.b_big_list); f.rpos = P_<uint32_t>(A.b_rpos);
+    f.rowcnt = P_<uint32_t>(A.b_rowcnt); f.rowoff = P_<uint32_t>(A.b_rowoff);
     f.rrec = P_<uint4>(A.b_rrec);
     f.rtile = P_<ulonglong2>(A.b_rtile);
     f.rext = P_<uint32_t>(A.b_rext);
     f.ptab = f.ms ? P_<uint32_t>(A.b_ptab) : nullptr;
     f.scan_tmp = P_<uint32_t>(A.b_scan_tmp);
 
-    sl::launch_bucket_info(sc, f, s);
-    if ((rc = check_launch(h, "bucket_info"))) return rc;
+    sl::launch_row_lists(sc, f, s);
+    if ((rc = check_launch(h, "row_lists"))) return rc;
     mark(4);
     sl::launch_frag_count(sc, tb, f, s);
-    sl::scan_exclusive_u32(f.bcount, f.boff, NB, f.scan_tmp, s);
+    sl::launch_bucket_scans(f, s);
     sl::launch_frag_scatter(sc, tb, f, s);
-    sl::launch_bucket_carry(f, s);
     sl::launch_scene_carry(sc, f, s);
     if ((rc = check_launch(h, "fragments"))) return rc;
     mark(5);
     sl::launch_resolve(sc, tb, f, s);
     if ((rc = check_launch(h, "resolve"))) return rc;
-    mark(6);
-    sl::launch_order_rows(sc, f, s);
-    if ((rc = check_launch(h, "order_rows"))) return rc;
-    if (!carved) h->nz_vals_sorted = f.nz_vals[0];
+    mark(6);  // the row order is part of bucket_setup
     mark(7);
     sl::launch_composite(sc, tb, f, s);
     if ((rc = check_launch(h, "composite"))) return rc;
@@ -592,8 +579,7 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
 
     // element counts (M, S) and the error flag
     unsigned long long *red = (unsigned long long *)(P_<uint32_t>(A.b_small) + 4);
-    sl::launch_fill_u32((uint32_t *)red, 0u, 4, s);
-    sl::launch_count_reduce(f.brec, NB, red, s);
+    sl::launch_count_reduce(f.bcnt, NB, red, s);  // cleared at the frame's start
     if (deferred) {
         HIPCHK(h, hipMemcpyAsync(h->fstat, A.b_small.p, 32, hipMemcpyDeviceToHost, s));
         h->stat_pending = true;
@@ -656,20 +642,30 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
         }
         if (!r2) {
             // internal bucket / row-order arrays for diagnosing the compositor
-            uint32_t NZ = 0;
-            hipError_t e = hipMemcpy(&NZ, f.nz_off + NB, 4, hipMemcpyDeviceToHost);
+            std::vector<uint32_t> place(NB), ext(NB), cnt(2 * (size_t)NB);
             h->d_binfo.resize((size_t)NB * 2); h->d_bicnt.resize(NB); h->d_bext.resize(NB);
-            h->d_boff.resize((size_t)NB + 1); h->d_rowkeys.resize(NZ); h->d_rowvals.resize(NZ);
-            h->d_rowbeg.resize(R); h->d_rowend.resize(R);
-            if (e == hipSuccess) e = hipMemcpy(h->d_binfo.data(), f.binfo, (size_t)NB * 8, hipMemcpyDeviceToHost);
-            if (e == hipSuccess) e = hipMemcpy2D(h->d_bicnt.data(), 4, (const uint32_t *)f.brec + 6, 32, 4, (size_t)NB, hipMemcpyDeviceToHost);
-            if (e == hipSuccess)  // the extent is the record's first word
-                e = hipMemcpy2D(h->d_bext.data(), 4, f.brec, 32, 4, (size_t)NB, hipMemcpyDeviceToHost);
+            h->d_boff.resize((size_t)NB + 1);
+            hipError_t e = hipMemcpy(h->d_binfo.data(), f.binfo, (size_t)NB * 8, hipMemcpyDeviceToHost);
+            if (e == hipSuccess) e = hipMemcpy(cnt.data(), f.bcnt, (size_t)NB * 8, hipMemcpyDeviceToHost);
+            if (e == hipSuccess) e = hipMemcpy(place.data(), f.rpos, (size_t)NB * 4, hipMemcpyDeviceToHost);
+            if (e == hipSuccess) e = hipMemcpy(ext.data(), f.rext, (size_t)NB * 4, hipMemcpyDeviceToHost);
             if (e == hipSuccess) e = hipMemcpy(h->d_boff.data(), f.boff, ((size_t)NB + 1) * 4, hipMemcpyDeviceToHost);
-            if (e == hipSuccess && NZ) e = hipMemcpy(h->d_rowkeys.data(), f.nz_keys[0], (size_t)NZ * 4, hipMemcpyDeviceToHost);
-            if (e == hipSuccess && NZ) e = hipMemcpy(h->d_rowvals.data(), f.nz_vals[0], (size_t)NZ * 4, hipMemcpyDeviceToHost);
-            if (e == hipSuccess) e = hipMemcpy(h->d_rowbeg.data(), f.rowbeg, R * 4, hipMemcpyDeviceToHost);
-            if (e == hipSuccess) e = hipMemcpy(h->d_rowend.data(), f.rowend, R * 4, hipMemcpyDeviceToHost);
+            // the non-empty buckets by (row, path): a path's buckets come in path order
+            std::vector<std::vector<uint32_t>> rows(R);
+            for (uint32_t b = 0; b < NB && e == hipSuccess; ++b) {
+                h->d_bicnt[b] = cnt[2 * (size_t)b];
+                h->d_bext[b] = place[b] == 0xFFFFFFFFu ? 0xFFFFu : ext[place[b]];
+                if (h->d_bicnt[b]) rows[h->d_binfo[2 * (size_t)b + 1]].push_back(b);
+            }
+            h->d_rowkeys.clear(); h->d_rowvals.clear();
+            h->d_rowbeg.assign(R, 0); h->d_rowend.assign(R, 0);
+            for (size_t r = 0; r < R; ++r) {
+                if (rows[r].empty()) continue;
+                h->d_rowbeg[r] = (uint32_t)h->d_rowvals.size();
+                h->d_rowvals.insert(h->d_rowvals.end(), rows[r].begin(), rows[r].end());
+                h->d_rowkeys.resize(h->d_rowvals.size(), (uint32_t)r);
+                h->d_rowend[r] = (uint32_t)h->d_rowvals.size();
+            }
             if (e != hipSuccess) r2 = fail(h, SL_E_HIP, "debug copy failed: %s", hipGetErrorString(e));
         }
         int64_t pc = 0;
@@ -759,15 +755,16 @@ int sl_destroy(sl_handle *h) {
     if (!h) return SL_OK;
     (void)hipSetDevice(h->device);
     (void)hipDeviceSynchronize();
-    DevBuf *bufs[] = {&h->A.b_pcnt, &h->A.b_nchain, &h->A.b_choff, &h->A.b_chains, &h->A.b_chain_t, &h->vtx, &h->vpath, &h->cvpos, &h->ctype, &h->cpath, &h->cw, &h->crev, &h->cinfo, &h->frule, &h->finfo,
-                      &h->ptable[0], &h->ptable[1], &h->ptable[2], &h->ctab[0], &h->ctab[1], &h->A.b_tvtx, &h->A.b_pflags,
-                      &h->A.b_prow, &h->A.b_crec, &h->A.b_cfrag, &h->A.b_coff, &h->A.b_ts, &h->A.b_pnb, &h->A.b_pbase,
-                      &h->A.b_binfo, &h->A.b_bcount, &h->A.b_boff, &h->A.b_bwsum, &h->A.b_bcarry, &h->A.b_rec_meta,
-                      &h->A.b_rec_mask, &h->A.b_scratch, &h->A.b_items, &h->A.b_imask, &h->A.b_icov, &h->A.b_prec, &h->A.b_brec,
-                      &h->A.b_big_list, &h->A.b_small, &h->A.b_nz_flag, &h->A.b_nz_off, &h->A.b_nzk0, &h->A.b_nzk1, &h->A.b_nzv0,
-                      &h->A.b_nzv1, &h->A.b_rs_hist, &h->A.b_rs_hoff, &h->A.b_rowbeg, &h->A.b_rowend, &h->A.b_image, &h->A.b_scan_tmp,
-                      &h->A.b_rrec, &h->A.b_rtile, &h->A.b_rext, &h->A.b_ptab, &h->A.b_lcount, &h->pcanvas, &h->stile, &h->simg, &h->sfirst, &h->scarry,
-                      &h->gramp, &h->gtable, &h->chord_keys};
+    DevBuf *bufs[] = {&h->vtx, &h->vpath, &h->cvpos, &h->ctype, &h->cpath, &h->cw, &h->crev, &h->cinfo, &h->frule, &h->finfo,
+                      &h->ptable[0], &h->ptable[1], &h->ptable[2], &h->ctab[0], &h->ctab[1], &h->pcanvas, &h->stile,
+                      &h->simg, &h->sfirst, &h->scarry, &h->gramp, &h->gtable, &h->chord_keys, &h->A.b_pcnt,
+                      &h->A.b_nchain, &h->A.b_choff, &h->A.b_chains, &h->A.b_chain_t, &h->A.b_tvtx, &h->A.b_pflags,
+                      &h->A.b_prow, &h->A.b_crec, &h->A.b_cfrag, &h->A.b_coff, &h->A.b_ts, &h->A.b_pbase, &h->A.b_binfo,
+                      &h->A.b_bcount, &h->A.b_boff, &h->A.b_bwsum, &h->A.b_bcarry, &h->A.b_rec_meta, &h->A.b_rec_mask,
+                      &h->A.b_scratch, &h->A.b_items, &h->A.b_imask, &h->A.b_icov, &h->A.b_prec, &h->A.b_bcnt,
+                      &h->A.b_big_list, &h->A.b_small, &h->A.b_rpos, &h->A.b_rowcnt, &h->A.b_rowoff,
+                      &h->A.b_rrec, &h->A.b_rtile, &h->A.b_rext, &h->A.b_ptab, &h->A.b_image,
+                      &h->A.b_scan_tmp, &h->A.b_lcount};
     for (DevBuf *b : bufs) release(*b);
     if (h->fstat) (void)hipHostFree(h->fstat);
     if (h->stage) (void)hipHostFree(h->stage);

@@ -150,6 +150,17 @@ __device__ __forceinline__ bool region_visible(uint32_t m) {
 
 __device__ __forceinline__ int32_t floor_even(float x) { return floor_i32(x) & (int32_t)0xFFFFFFFE; }
 
+// Buckets of a path whose fragments lie in cell rows [pr.x, pr.y] (pr.x > pr.y: none): rows 1
+// and up in order, then the out-of-canvas bucket, then row 0.
+__device__ __forceinline__ int path_first_row(int2 pr) { return tmax(pr.x, 1); }
+__device__ __forceinline__ int path_rows_above(int2 pr) {  // buckets of rows 1 and up
+    const int lo1 = path_first_row(pr);
+    return pr.y >= lo1 ? pr.y - lo1 + 1 : 0;
+}
+__device__ __forceinline__ uint32_t path_bucket_count(int2 pr) {
+    return (uint32_t)(path_rows_above(pr) + 1 + (pr.x == 0 ? 1 : 0));
+}
+
 // Texel of a point-sampled, clamped, normalized 256-wide texture.
 __device__ __forceinline__ int texel(float u) { return tmin(tmax(floor_i32(u * 256.f), 0), 255); }
 

@@ -42,18 +42,35 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t &total,
     return off + inc - v;
 }
 
-__global__ void __launch_bounds__(kScanThreads) k_scan_reduce(const uint32_t *in, size_t n, uint32_t *tile_sum) {
+// What a scan reads: up to two arrays in one launch (blockIdx.y), or the bucket count of every
+// path, worked out from its row range.
+struct ScanArrays {
+    const uint32_t *in[2];
+    __device__ __forceinline__ uint32_t operator()(int y, size_t i) const { return in[y][i]; }
+};
+struct ScanPathBuckets {
+    const int2 *prow;
+    __device__ __forceinline__ uint32_t operator()(int, size_t i) const { return path_bucket_count(prow[i]); }
+};
+struct ScanOut {
+    uint32_t *out[2];
+    uint32_t *tmp[2];  // tile totals
+};
+
+template <class In>
+__global__ void __launch_bounds__(kScanThreads) k_scan_reduce(In in, size_t n, ScanOut o) {
     __shared__ uint32_t lds[4];
+    const int y = blockIdx.y;
     size_t base = (size_t)blockIdx.x * kScanTile;
     uint32_t s = 0;
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
         size_t i = base + (size_t)k * kScanThreads + threadIdx.x;
-        if (i < n) s += in[i];
+        if (i < n) s += in(y, i);
     }
     uint32_t tot;
     block_excl_scan(s, tot, lds);
-    if (threadIdx.x == 0) tile_sum[blockIdx.x] = tot;
+    if (threadIdx.x == 0) o.tmp[y][blockIdx.x] = tot;
 }
 
 __global__ void __launch_bounds__(kScanThreads) k_scan_top(uint32_t *tile_sum, size_t ntiles, uint32_t *out_total) {
@@ -70,47 +87,32 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_top(uint32_t *tile_sum, s
     if (threadIdx.x == 0) *out_total = carry;
 }
 
-__global__ void __launch_bounds__(kScanThreads) k_scan_down(const uint32_t *in, uint32_t *out, size_t n,
-                                                             const uint32_t *tile_off) {
-    __shared__ uint32_t lds[4];
-    size_t base = (size_t)blockIdx.x * kScanTile + (size_t)threadIdx.x * kScanItems;
-    uint32_t v[kScanItems];
-    uint32_t s = 0;
-#pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-        size_t i = base + k;
-        v[k] = i < n ? in[i] : 0u;
-        s += v[k];
-    }
-    uint32_t tot;
-    uint32_t ex = block_excl_scan(s, tot, lds) + tile_off[blockIdx.x];
-#pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-        size_t i = base + k;
-        if (i < n) out[i] = ex;
-        ex += v[k];
-    }
-}
-
-// The down-sweep for scans of at most kScanDirectTiles tiles: each block sums the tile
-// totals before its own (at most 4095 L2-resident words) instead of a separate pass
+// The down-sweep.  DIRECT, for scans of at most kScanDirectTiles tiles: each block sums the
+// tile totals before its own (at most 4095 L2-resident words) instead of a separate pass
 // scanning them, and the last block writes the grand total to out[n].
 constexpr size_t kScanDirectTiles = 4096;
 
-__global__ void __launch_bounds__(kScanThreads) k_scan_down_direct(const uint32_t *in, uint32_t *out, size_t n,
-                                                                    const uint32_t *tile_sum) {
+template <bool DIRECT, class In>
+__global__ void __launch_bounds__(kScanThreads) k_scan_down(In in, size_t n, ScanOut o) {
     __shared__ uint32_t lds[4];
-    uint32_t pre = 0;
-    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kScanThreads) pre += tile_sum[i];
-    uint32_t tile_off;
-    block_excl_scan(pre, tile_off, lds);
+    const int y = blockIdx.y;
+    const uint32_t *tile = o.tmp[y];
+    uint32_t *out = o.out[y];
+    uint32_t tile_off = 0;
+    if (DIRECT) {
+        uint32_t pre = 0;
+        for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kScanThreads) pre += tile[i];
+        block_excl_scan(pre, tile_off, lds);
+    } else {
+        tile_off = tile[blockIdx.x];
+    }
     size_t base = (size_t)blockIdx.x * kScanTile + (size_t)threadIdx.x * kScanItems;
     uint32_t v[kScanItems];
     uint32_t s = 0;
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
         size_t i = base + k;
-        v[k] = i < n ? in[i] : 0u;
+        v[k] = i < n ? in(y, i) : 0u;
         s += v[k];
     }
     uint32_t tot;
@@ -121,20 +123,65 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_down_direct(const uint32_
         if (i < n) out[i] = ex;
         ex += v[k];
     }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = tile_off + tot;
+    if (DIRECT && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = tile_off + tot;
+}
+
+// A whole scan in one launch, a block an array: up to 16 values a thread.  One launch of about
+// 5 us where the two passes take 3 to 4 us each; beyond that size one block is the slower.
+constexpr int kScanSmallThreads = 1024, kScanSmallItems = 16;
+constexpr size_t kScanSmall = (size_t)kScanSmallThreads * kScanSmallItems;
+
+template <class In>
+__global__ void __launch_bounds__(kScanSmallThreads) k_scan_small(In in, size_t n, ScanOut o) {
+    __shared__ uint32_t part[kScanSmallThreads / 64];
+    const int y = blockIdx.y, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const size_t base = (size_t)threadIdx.x * kScanSmallItems;
+    uint32_t v[kScanSmallItems];
+    uint32_t s = 0;
+#pragma unroll
+    for (int k = 0; k < kScanSmallItems; ++k) {
+        v[k] = base + k < n ? in(y, base + k) : 0u;
+        s += v[k];
+    }
+    const uint32_t inc = wave_incl_scan(s);
+    if (lane == 63) part[wv] = inc;
+    __syncthreads();
+    uint32_t ex = inc - s, tot = 0;
+#pragma unroll
+    for (int w = 0; w < kScanSmallThreads / 64; ++w) {
+        if (w < wv) ex += part[w];
+        tot += part[w];
+    }
+    uint32_t *out = o.out[y];
+#pragma unroll
+    for (int k = 0; k < kScanSmallItems; ++k) {
+        if (base + k < n) out[base + k] = ex;
+        ex += v[k];
+    }
+    if (threadIdx.x == 0) out[n] = tot;
+}
+
+template <class In>
+void scan_launch(const In &in, int arrays, const ScanOut &o, size_t n, hipStream_t s) {
+    if (n <= kScanSmall) {
+        hipLaunchKernelGGL(k_scan_small<In>, dim3(1, arrays), dim3(kScanSmallThreads), 0, s, in, n, o);
+        return;
+    }
+    const size_t ntiles = (n + kScanTile - 1) / kScanTile;
+    const dim3 g((unsigned)ntiles, arrays), b(kScanThreads);
+    hipLaunchKernelGGL(k_scan_reduce<In>, g, b, 0, s, in, n, o);
+    if (ntiles <= kScanDirectTiles) {
+        hipLaunchKernelGGL((k_scan_down<true, In>), g, b, 0, s, in, n, o);
+        return;
+    }
+    for (int y = 0; y < arrays; ++y)
+        hipLaunchKernelGGL(k_scan_top, dim3(1), b, 0, s, o.tmp[y], ntiles, o.out[y] + n);
+    hipLaunchKernelGGL((k_scan_down<false, In>), g, b, 0, s, in, n, o);
 }
 
 __global__ void k_fill_u32(uint32_t *p, uint32_t v, size_t n) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
-}
-// two arrays of the same length in one launch
-__global__ void k_fill2_u32(uint32_t *p, uint32_t *q, uint32_t v, size_t n) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        p[i] = v;
-        q[i] = v;
-    }
 }
 __global__ void k_fill_u8(uint8_t *p, uint8_t v, size_t n) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -173,11 +220,23 @@ __global__ void __launch_bounds__(256) k_valu_probe(int iters, float seed, float
 // ------------------------------------------------------------------------------------
 // per-path init, vertex transform + region flags (k_transformVertex, .cu:36-105)
 // ------------------------------------------------------------------------------------
-__global__ void k_path_init(uint32_t P, uint32_t *pflags, int2 *prow) {
+__global__ void k_frame_init(uint32_t P, uint32_t *pflags, int2 *prow, uint32_t *small, uint32_t *lcount) {
     uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < kFrameStatusWords) small[p] = 0u;
+    if (p < kListCountBytes / 4) lcount[p] = 0u;
     if (p >= P) return;
     pflags[p] = 0u;
     prow[p] = make_int2(INT_MAX, INT_MIN);
+}
+
+// the three sizes a frame's host side needs, written to pinned host memory in one launch
+__global__ void k_sizes(const uint32_t *F, const uint32_t *NCH, const uint32_t *NB, uint32_t *host) {
+    if (threadIdx.x == 0) {
+        host[0] = *F;
+        host[1] = *NCH;
+        host[2] = *NB;
+        __threadfence_system();
+    }
 }
 
 struct Mat4 { float m[16]; };
@@ -1196,34 +1255,30 @@ __global__ void __launch_bounds__(kMergeThreads) k_merge_long(const float4 *__re
 
 }  // namespace
 
-size_t scan_tmp_elems_needed(size_t n) { return (n + kScanTile - 1) / kScanTile + 1; }
+// two arrays' tile totals
+size_t scan_tmp_elems_needed(size_t n) { return 2 * ((n + kScanTile - 1) / kScanTile + 1); }
 
 void scan_exclusive_u32(const uint32_t *in, uint32_t *out, size_t n, uint32_t *tmp, hipStream_t s) {
-    size_t ntiles = (n + kScanTile - 1) / kScanTile;
-    if (ntiles == 0) {
-        hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kScanThreads), 0, s, tmp, (size_t)0, out + n);
-        return;
-    }
-    hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)ntiles), dim3(kScanThreads), 0, s, in, n, tmp);
-    if (ntiles <= kScanDirectTiles) {
-        hipLaunchKernelGGL(k_scan_down_direct, dim3((unsigned)ntiles), dim3(kScanThreads), 0, s, in, out, n,
-                           (const uint32_t *)tmp);
-        return;
-    }
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kScanThreads), 0, s, tmp, ntiles, out + n);
-    hipLaunchKernelGGL(k_scan_down, dim3((unsigned)ntiles), dim3(kScanThreads), 0, s, in, out, n,
-                       (const uint32_t *)tmp);
+    scan_launch(ScanArrays{{in, nullptr}}, 1, ScanOut{{out, nullptr}, {tmp, nullptr}}, n, s);
 }
 
+void scan2_exclusive_u32(const uint32_t *in0, uint32_t *out0, const uint32_t *in1, uint32_t *out1, size_t n, uint32_t *tmp,
+                         hipStream_t s) {
+    scan_launch(ScanArrays{{in0, in1}}, 2, ScanOut{{out0, out1}, {tmp, tmp + scan_tmp_elems_needed(n) / 2}}, n, s);
+}
 
+void launch_path_buckets(const SceneDev &sc, Frame &f, hipStream_t s) {
+    scan_launch(ScanPathBuckets{f.prow}, 1, ScanOut{{f.pbase, nullptr}, {f.scan_tmp, nullptr}}, sc.P, s);
+}
+
+void launch_sizes(const SceneDev &sc, const Frame &f, uint32_t *host, hipStream_t s) {
+    hipLaunchKernelGGL(k_sizes, dim3(1), dim3(64), 0, s, (const uint32_t *)f.coff + sc.C, (const uint32_t *)f.choff + sc.C,
+                       (const uint32_t *)f.pbase + sc.P, host);
+}
 
 void launch_fill_u32(uint32_t *p, uint32_t v, size_t n, hipStream_t s) {
     if (!n) return;
     hipLaunchKernelGGL(k_fill_u32, dim3(blocks_for(n, 256)), dim3(256), 0, s, p, v, n);
-}
-void launch_fill2_u32(uint32_t *p, uint32_t *q, uint32_t v, size_t n, hipStream_t s) {
-    if (!n) return;
-    hipLaunchKernelGGL(k_fill2_u32, dim3(blocks_for(n, 256)), dim3(256), 0, s, p, q, v, n);
 }
 void launch_valu_probe(int blocks, int iters, float *out, hipStream_t s) {
     hipLaunchKernelGGL(k_valu_probe, dim3(blocks), dim3(256), 0, s, iters, 0.5f, out);
@@ -1240,9 +1295,9 @@ void launch_fill_rows_u8(uint8_t *p, uint8_t v, size_t row_bytes, size_t pitch, 
     hipLaunchKernelGGL(k_fill_rows_u8, dim3(blocks_for(n, 256)), dim3(256), 0, s, p, v, row_bytes, pitch, n);
 }
 
-void launch_path_init(const SceneDev &sc, Frame &f, hipStream_t s) {
-    if (!sc.P) return;
-    hipLaunchKernelGGL(k_path_init, dim3(blocks_for(sc.P, 256)), dim3(256), 0, s, sc.P, f.pflags, f.prow);
+void launch_frame_init(const SceneDev &sc, Frame &f, hipStream_t s) {
+    const uint32_t n = sc.P > kListCountBytes / 4 ? sc.P : (uint32_t)(kListCountBytes / 4);
+    hipLaunchKernelGGL(k_frame_init, dim3(blocks_for(n, 256)), dim3(256), 0, s, sc.P, f.pflags, f.prow, f.big_count, f.lcount);
 }
 
 void launch_transform(const SceneDev &sc, Frame &f, hipStream_t s) {
@@ -1262,7 +1317,6 @@ void launch_monotone(const SceneDev &sc, Frame &f, hipStream_t s) {
 void launch_intersect(const SceneDev &sc, Frame &f, hipStream_t s) {
     if (!sc.C) return;
     uint32_t *cnt = f.lcount, *cursor = f.lcount + kListClasses;
-    launch_fill_u32(f.lcount, 0u, 2 * kListClasses, s);
     // Cubic chains of the first wide_bins length bins take several lanes each (wide_chains): one
     // lane's 1.5 us a cut makes the longest chains the pass's time in frames of every size, but
     // the lanes cost up to 20 times the issue slots, so the more cuts a frame has, the fewer

@@ -74,6 +74,9 @@ struct GradDev {
 
 // bytes of the intersection work lists' class counts and cursors (Frame::lcount)
 constexpr size_t kListCountBytes = 1024;
+// words of the frame's status block: big-bucket count, error flags, -, -, then the 64-bit
+// merged-cell and item totals (Frame::big_count)
+constexpr uint32_t kFrameStatusWords = 8;
 
 struct Frame {
     int W, H;
@@ -102,8 +105,7 @@ struct Frame {
     // fragments
     int64_t F;
     int2 *ts;                // [F]
-    uint32_t *pnb;           // [P+1] buckets per path -> scanned to pbase
-    uint32_t *pbase;         // [P+1]
+    uint32_t *pbase;         // [P+1] first bucket of each path
     int64_t NB;
     int2 *binfo;             // [NB] (path, row or -1)
     uint32_t *bcount;        // [NB+1] -> boff
@@ -119,18 +121,15 @@ struct Frame {
     uint32_t *imask;         // [F * words] masks of merged cells
     uint32_t *icov;          // [F] sample counts of a merged cell's 4 pixels
     uint4 *prec;             // [F] records of tiles holding merged cells
-    uint4 *brec;             // [2 NB] {extent, records, tiles with a record (64 bits)},
-                             //   {tiles wholly inside a span (64 bits), items, merged cells}
+    uint2 *bcnt;             // [NB] {items, merged cells}
     uint32_t *big_list;      // [NB] buckets with more than 64 fragments
     uint32_t *big_count;     // [1]
     uint32_t *err_flag;      // [1]
-    // compositing order
-    uint32_t *nz_flag;       // [NB+1]
-    uint32_t *nz_off;        // [NB+1]
-    uint32_t *nz_keys[2];    // [NB] row keys (ping-pong)
-    uint32_t *nz_vals[2];    // [NB] bucket ids (ping-pong)
-    uint32_t *rs_hist;       // radix histogram scratch
-    uint32_t *rs_hoff;
+    // row lists (see sl_frag.hip)
+    uint32_t *rpos;          // [NB] a bucket's place in the row lists
+    uint32_t *rowcnt;        // [R * shares] paths per row and share
+    uint32_t *rowoff;        // [R * shares + 1]; row r's list: [rowoff[r shares], rowoff[(r + 1) shares])
+    uint32_t rowshares;
     int64_t R;               // cell rows (of all scenes of a batch)
     // batched scenes (nscenes > 0): per scene {W, H, first tile, first cell row}, image
     // byte offsets, first path, and the winding-scan carry at its first bucket
@@ -142,8 +141,6 @@ struct Frame {
     uint32_t *scarry;
     // launch shape (autotuned for batches; results do not depend on it)
     int resolve_grid, class_grid, comp_group, frag_block;
-    uint32_t *rowbeg;        // [R]
-    uint32_t *rowend;        // [R]
     uint32_t *rext;          // [NB] row-list extents
     uint4 *rrec;             // [NB] row-list records {colour, records, base, path}
     ulonglong2 *rtile;       // [NB] row-list tile bitmaps {with a record, inside a span}
@@ -163,18 +160,24 @@ struct Frame {
 size_t scan_tmp_elems_needed(size_t n);
 void scan_exclusive_u32(const uint32_t *in, uint32_t *out, size_t n, uint32_t *tmp, hipStream_t s);
 
-void launch_path_init(const SceneDev &sc, Frame &f, hipStream_t s);
+// two arrays of n in one launch each pass (tmp: scan_tmp_elems_needed(n))
+void scan2_exclusive_u32(const uint32_t *in0, uint32_t *out0, const uint32_t *in1, uint32_t *out1, size_t n, uint32_t *tmp,
+                         hipStream_t s);
+
+void launch_frame_init(const SceneDev &sc, Frame &f, hipStream_t s);
+void launch_sizes(const SceneDev &sc, const Frame &f, uint32_t *host, hipStream_t s);
 void launch_transform(const SceneDev &sc, Frame &f, hipStream_t s);
 void launch_monotone(const SceneDev &sc, Frame &f, hipStream_t s);
 void launch_intersect(const SceneDev &sc, Frame &f, hipStream_t s);
 void launch_path_buckets(const SceneDev &sc, Frame &f, hipStream_t s);
-void launch_bucket_info(const SceneDev &sc, Frame &f, hipStream_t s);
+// shares of the paths in the row lists' passes
+uint32_t row_shares(uint32_t P, size_t R, size_t NB);
+void launch_row_lists(const SceneDev &sc, Frame &f, hipStream_t s);
 void launch_frag_count(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t s);
 void launch_frag_scatter(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t s);
-void launch_bucket_carry(Frame &f, hipStream_t s);
+void launch_bucket_scans(Frame &f, hipStream_t s);
 void launch_resolve(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t s);
 void launch_scene_carry(const SceneDev &sc, Frame &f, hipStream_t s);
-void launch_order_rows(const SceneDev &sc, Frame &f, hipStream_t s);
 void launch_composite(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t s);
 void launch_encode_values(const Tables &t, int channel, const float *v, int64_t n, uint8_t *code, float *dec,
                           hipStream_t s);
@@ -208,7 +211,6 @@ struct ChordScene {
 float chord_ease(int time_ms);
 void launch_chord_frame(const ChordInterval *d, int n_diagrams, uint32_t P, const ChordScene &out, hipStream_t s);
 void launch_fill_u32(uint32_t *p, uint32_t v, size_t n, hipStream_t s);
-void launch_fill2_u32(uint32_t *p, uint32_t *q, uint32_t v, size_t n, hipStream_t s);
 
 // static scratch of the allocation-free frame (sl_noalloc.hip): its size, and its device
 // address on `device` (which must be current; looked up once per device)
@@ -221,7 +223,7 @@ void launch_debug_fragments(const SceneDev &sc, const Tables &t, Frame &f, int32
 void launch_debug_draw_list(const SceneDev &sc, const Tables &t, Frame &f, const uint32_t *moff,
                             const uint32_t *ioff, int4 *draw, uint32_t *mmask4, hipStream_t s);
 // out[0] += merged cells, out[1] += items
-void launch_count_reduce(const uint4 *brec, size_t n, unsigned long long *out, hipStream_t s);
+void launch_count_reduce(const uint2 *bcnt, size_t n, unsigned long long *out, hipStream_t s);
 void launch_debug_counts(const Frame &f, uint32_t *merged, uint32_t *items, hipStream_t s);
 
 }  // namespace sl

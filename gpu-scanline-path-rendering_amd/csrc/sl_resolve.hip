@@ -13,9 +13,10 @@
 //                            covered by a span or merged, merged cells (bit c: the tile's
 //                            c-th 2-pixel cell), merged cells before the tile, tile | a span
 //                            runs on past the tile << 31 (kept for buckets wider than 63 tiles)};
-//   brec [2 bucket, + 1]     {extent, records, tiles with a record (64 bits)}, {tiles wholly
-//                            inside a span (64 bits), items, merged cells}; bit k is the k-th
-//                            tile from the extent's first, bit 63 that tile or any beyond.
+//   rext, rrec, rtile [place in the row lists]  extent; {colour, records, base, path}; tiles
+//                            with a record and tiles wholly inside a span, 64 bits each, bit k
+//                            the k-th tile from the extent's first, bit 63 that or any beyond;
+//   bcnt [bucket]            {items, merged cells}.
 // A column finds its covering item with two bit tests, and a merged cell's index with one
 // population count.  For the parity dumps a bucket's items are also listed (one u32 each, x
 // of the first pixel | span width << 16, 0 for a merged cell).
@@ -193,7 +194,12 @@ struct ResolveArgs {
     uint32_t *imask;         // written by the KEEP kernels only
     uint32_t *icov;
     uint4 *prec;
-    uint4 *brec;
+    const uint32_t *rpos;    // places in the row lists
+    const uint32_t *finfo;   // fill words
+    uint32_t *rext;
+    uint4 *rrec;
+    ulonglong2 *rtile;
+    uint2 *bcnt;
     uint32_t *big_list;
     uint32_t *big_count;
     uint32_t *err;
@@ -213,6 +219,18 @@ constexpr int kBigStage = 16;  // chunks of 64 fragments staged in LDS
 struct RecLds {
     unsigned long long et[4], ft[4], heads[kBigStage];
 };
+
+// A bucket's entry in the row lists (one lane).
+__device__ __forceinline__ void put_row(const ResolveArgs &A, int64_t b, uint32_t base, uint32_t path, uint32_t ext,
+                                        int nrec, uint64_t et, uint64_t ft, int items, int merged) {
+    A.bcnt[b] = make_uint2((uint32_t)items, (uint32_t)merged);
+    const uint32_t at = A.rpos[b];
+    if (at == 0xFFFFFFFFu) return;  // the out-of-canvas bucket
+    A.rext[at] = ext;
+    if (!items) return;             // an empty extent: the rest is never read
+    A.rrec[at] = make_uint4(A.finfo[path], (uint32_t)nrec, base, path);
+    A.rtile[at] = make_ulonglong2(et, ft);
+}
 
 // What a lane contributes to its bucket's records: its group head's merged cell at x (if any)
 // and the span [prev_x + 2, x) before it (if any).  prev_ok: the group before it was merged.
@@ -359,10 +377,8 @@ __device__ __forceinline__ void chunks_end(const ResolveArgs &A, int64_t b, uint
     if ((threadIdx.x & 63) == 0) {
         if (K.nrec) *(uint2 *)&A.prec[base + K.nrec - 1].x = make_uint2(K.cover, K.edge);
         const bool any = K.merged + K.spans > 0;
-        A.brec[2 * b] = make_uint4(any ? ((uint32_t)K.xmin | ((uint32_t)K.xmax << 16)) : 0xFFFFu, (uint32_t)K.nrec,
-                               (uint32_t)R.et[0], (uint32_t)(R.et[0] >> 32));
-        A.brec[2 * b + 1] = make_uint4((uint32_t)R.ft[0], (uint32_t)(R.ft[0] >> 32), (uint32_t)(K.merged + K.spans),
-                                       (uint32_t)K.merged);
+        put_row(A, b, base, (uint32_t)A.binfo[b].x, any ? ((uint32_t)K.xmin | ((uint32_t)K.xmax << 16)) : 0xFFFFu, K.nrec,
+                R.et[0], R.ft[0], K.merged + K.spans, K.merged);
     }
     __syncthreads();
 }
@@ -512,7 +528,7 @@ template <> struct SegBits<16> : SegBits32<16> { using SegBits32<16>::SegBits32;
 
 // The records of the buckets in a wave's 64 / S segments, each bucket in one pass.
 template <int SPP, int S, bool KEEP>
-__device__ __forceinline__ void segment_emit(const ResolveArgs &A, bool live, int64_t b, uint32_t base, const Lane &L,
+__device__ __forceinline__ void segment_emit(const ResolveArgs &A, bool live, int64_t b, uint32_t base, uint32_t path, const Lane &L,
                                              const uint32_t *res, RecLds &R) {
     constexpr int NW = Words<SPP>::n;
     const int lane = threadIdx.x & 63;
@@ -555,10 +571,8 @@ __device__ __forceinline__ void segment_emit(const ResolveArgs &A, bool live, in
     }
     __syncthreads();
     if (live && i == 0) {
-        A.brec[2 * b] = make_uint4(any.m ? ((uint32_t)xmin | ((uint32_t)xmax << 16)) : 0xFFFFu, (uint32_t)lm.count(),
-                               (uint32_t)R.et[seg], (uint32_t)(R.et[seg] >> 32));
-        A.brec[2 * b + 1] = make_uint4((uint32_t)R.ft[seg], (uint32_t)(R.ft[seg] >> 32), (uint32_t)(mm.count() + sm.count()),
-                                       (uint32_t)mm.count());
+        put_row(A, b, base, path, any.m ? ((uint32_t)xmin | ((uint32_t)xmax << 16)) : 0xFFFFu, lm.count(), R.et[seg], R.ft[seg],
+                mm.count() + sm.count(), mm.count());
     }
     __syncthreads();
 }
@@ -574,7 +588,7 @@ __device__ __forceinline__ void segments_begin(RecLds &R) {
 template <int NW>
 struct SmallIn {
     uint32_t meta, mk[NW];
-    uint32_t carry;
+    uint32_t carry, path;
     int rule, W;
 };
 
@@ -637,7 +651,7 @@ __device__ __forceinline__ void resolve_small(const ResolveArgs &A, int64_t b, u
     const int prev_x = 2 * prev_cx - 2;
     Lane L;
     L.init(merged, head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at), p > 0, x, prev_x, W);
-    segment_emit<SPP, 64, KEEP>(A, true, b, base, L, res, R);
+    segment_emit<SPP, 64, KEEP>(A, true, b, base, in.path, L, res, R);
 }
 
 // Buckets of at most S (16 or 32) fragments, 64 / S of them in one wave: lane l works on
@@ -646,7 +660,7 @@ __device__ __forceinline__ void resolve_small(const ResolveArgs &A, int64_t b, u
 // slot in the per-lane scalars (lane k holds bucket b0 + k G), -1 for an empty segment.
 template <int SPP, int S, bool KEEP>
 __device__ __forceinline__ void resolve_pack(const ResolveArgs &A, int64_t b0, int64_t G, const int *ks, int vbase,
-                                             int vend, int vcarry, int vrule, int vW, uint32_t *order, uint32_t *meta,
+                                             int vend, int vcarry, int vrule, int vW, int vpath, uint32_t *order, uint32_t *meta,
                                              uint32_t *msk, RecLds &R) {
     constexpr int NW = Words<SPP>::n;
     constexpr int P = 64 / S;
@@ -664,6 +678,7 @@ __device__ __forceinline__ void resolve_pack(const ResolveArgs &A, int64_t b0, i
     const uint32_t wcarry = (uint32_t)__shfl(vcarry, src, 64);
     const int rule = __shfl(vrule, src, 64);
     const int W = __shfl(vW, src, 64);
+    const uint32_t path = (uint32_t)__shfl(vpath, src, 64);
     const int n = k < 0 ? 0 : end - (int)base;
     uint32_t mykey = 0xFFFFFFFFu;
     if (i < n) {
@@ -701,7 +716,7 @@ __device__ __forceinline__ void resolve_pack(const ResolveArgs &A, int64_t b0, i
     const int prev_x = 2 * prev_cx - 2;
     Lane L;
     L.init(merged, head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at), p > 0, x, prev_x, W);
-    segment_emit<SPP, S, KEEP>(A, k >= 0, b0 + (int64_t)(k < 0 ? 0 : k) * G, base, L, res, R);
+    segment_emit<SPP, S, KEEP>(A, k >= 0, b0 + (int64_t)(k < 0 ? 0 : k) * G, base, path, L, res, R);
 }
 
 // Every bucket: empty ones are cleared, buckets of at most 128 fragments are resolved,
@@ -722,13 +737,14 @@ __global__ void __launch_bounds__(64, 5) k_resolve_first(ResolveArgs A) {
         // vector loads, read back per bucket by readlane.  (Scalar loads would share the
         // LDS wait counter, so every LDS wait of a resolve would also wait for them.)
         const int64_t bl = b0 + (int64_t)lane * G;
-        int vbase = 0, vend = 0, vcarry = 0, vrule = 0, vW = A.W;
+        int vbase = 0, vend = 0, vcarry = 0, vrule = 0, vW = A.W, vpath = 0;
         if (bl < A.NB) {
             const int2 info = A.binfo[bl];
             vbase = (int)A.boff[bl];
             // the out-of-canvas bucket holds records only for the winding carry
             vend = info.y < 0 ? vbase : (int)A.boff[bl + 1];
             vrule = A.frule[info.x];
+            vpath = info.x;
             uint32_t carry = A.bcarry[bl];
             if (A.pcanvas) {
                 const int4 cv = A.pcanvas[info.x];
@@ -751,7 +767,7 @@ __global__ void __launch_bounds__(64, 5) k_resolve_first(ResolveArgs A) {
                 ks[s] = m16 ? (int)__builtin_ctzll(m16) : -1;
                 m16 &= m16 - 1ull;
             }
-            resolve_pack<SPP, 16, KEEP>(A, b0, G, ks, vbase, vend, vcarry, vrule, vW, order, meta, msk, R);
+            resolve_pack<SPP, 16, KEEP>(A, b0, G, ks, vbase, vend, vcarry, vrule, vW, vpath, order, meta, msk, R);
         }
         while (m32) {
             int ks[2];
@@ -760,7 +776,7 @@ __global__ void __launch_bounds__(64, 5) k_resolve_first(ResolveArgs A) {
                 ks[s] = m32 ? (int)__builtin_ctzll(m32) : -1;
                 m32 &= m32 - 1ull;
             }
-            resolve_pack<SPP, 32, KEEP>(A, b0, G, ks, vbase, vend, vcarry, vrule, vW, order, meta, msk, R);
+            resolve_pack<SPP, 32, KEEP>(A, b0, G, ks, vbase, vend, vcarry, vrule, vW, vpath, order, meta, msk, R);
         }
         // the rest one by one, the next bucket's records loading during the current one
         SmallIn<NW> in0, in1;
@@ -781,7 +797,7 @@ __global__ void __launch_bounds__(64, 5) k_resolve_first(ResolveArgs A) {
                                (uint32_t)__builtin_amdgcn_readlane(vend, kn), in1);
             }
             if (n == 0) {
-                if (lane < 2) A.brec[2 * b + lane] = make_uint4(lane ? 0u : 0xFFFFu, 0u, 0u, 0u);
+                if (lane == 0) put_row(A, b, base, 0u, 0xFFFFu, 0, 0ull, 0ull, 0, 0);
             } else if (n > 128) {
                 if (lane == 0) A.big_list[atomicAdd(A.big_count, 1u)] = (uint32_t)b;
             } else if (n > 64) {
@@ -790,6 +806,7 @@ __global__ void __launch_bounds__(64, 5) k_resolve_first(ResolveArgs A) {
                 in0.carry = (uint32_t)__builtin_amdgcn_readlane(vcarry, k);
                 in0.rule = __builtin_amdgcn_readlane(vrule, k);
                 in0.W = __builtin_amdgcn_readlane(vW, k);
+                in0.path = (uint32_t)__builtin_amdgcn_readlane(vpath, k);
                 resolve_small<SPP, KEEP>(A, b, base, n, in0, order, meta, msk, R);
             }
             in0 = in1;
@@ -798,7 +815,92 @@ __global__ void __launch_bounds__(64, 5) k_resolve_first(ResolveArgs A) {
 }
 
 // The listed buckets (more than 128 fragments), one per block, in one launch so that the
-// few long ones overlap: up to 1024 fragments staged in LDS, more in k_resolve_huge.
+// few long ones overlap: up to 1024 fragments staged in LDS, more in resolve_huge.
+// Buckets of more than 1024 fragments (rare): bitonic-sort 64-bit (cell x, index) keys,
+// held in the bucket's stretch of the record array (4n words; the padded power of two is at
+// most 2n), copy the sorted indices into the scratch (the records are written next), then walk
+// the sorted order in chunks of 64 reading the fragments from global memory.  Any bucket
+// size works.
+template <int SPP, bool KEEP>
+__device__ __noinline__ void resolve_huge(const ResolveArgs &A, int64_t b, uint32_t base, int n, RecLds &R) {
+    constexpr int NW = Words<SPP>::n;
+    const int lane = threadIdx.x;
+    int P2 = 1;
+    while (P2 < n) P2 <<= 1;
+    uint32_t *khi = (uint32_t *)(A.prec + base);
+    uint32_t *klo = khi + P2;
+    for (int i = lane; i < P2; i += 64) {
+        khi[i] = (i < n) ? (A.rec_meta[base + i] & 0xFFFFu) : 0xFFFFFFFFu;
+        klo[i] = (i < n) ? (uint32_t)i : 0xFFFFFFFFu;
+    }
+    __syncthreads();
+    for (int k = 2; k <= P2; k <<= 1) {
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            for (int i = lane; i < P2; i += 64) {
+                const int l = i ^ j;
+                if (l > i) {
+                    const uint32_t ah = khi[i], al = klo[i], ch = khi[l], cl = klo[l];
+                    const bool gt = ah > ch || (ah == ch && al > cl);
+                    const bool up = (i & k) == 0;
+                    if (gt == up) {
+                        khi[i] = ch; klo[i] = cl;
+                        khi[l] = ah; klo[l] = al;
+                    }
+                }
+            }
+            __syncthreads();
+        }
+    }
+    uint32_t *order = A.scratch + base;
+    for (int i = lane; i < n; i += 64) order[i] = klo[i];
+    chunks_begin(R);
+    __syncthreads();
+    // sorted fragment indices; a fragment's cell x is in its record
+    auto cell_x = [&](int q) { return (int)(A.rec_meta[base + order[q]] & 0xFFFFu); };
+    const int rule = A.frule[A.binfo[b].x];
+    uint32_t wcarry = A.bcarry[b];
+    int W = A.W;
+    if (A.pcanvas) {
+        const int4 cv = A.pcanvas[A.binfo[b].x];
+        W = cv.x;
+        wcarry -= A.scarry[cv.w];
+    }
+    Chunks K;
+    for (int c0 = 0; c0 < n; c0 += 64) {
+        const int p = c0 + lane;
+        const bool v = p < n;
+        const uint32_t meta = v ? A.rec_meta[base + order[p]] : 0u;
+        const int cx = (int)(meta & 0xFFFFu);
+        const int swn = v ? (int)(int8_t)(meta >> 16) : 0;
+        const int prev_cx = (v && p > 0) ? cell_x(p - 1) : -1;
+        const bool head = v && (p == 0 || cx != prev_cx);
+        const int incl = scan_add(swn);
+        const int8_t w_at = (int8_t)(int)(wcarry + (uint32_t)(incl - swn));
+        wcarry += (uint32_t)lane63(incl);
+        const int x = 2 * cx - 2;
+        const bool merged = head && x >= 0 && x < W;
+        uint32_t res[NW];
+        if (merged) {
+            Stencil<NW> st;
+            st.init(w_at);
+            for (int q = p; q < n; ++q) {
+                const uint32_t j = order[q];
+                const uint32_t mq = A.rec_meta[base + j];
+                if ((int)(mq & 0xFFFFu) != cx) break;
+                uint32_t m2[NW];
+                load_mask<NW>(A.rec_mask, (size_t)base + j, m2);
+                st.add(m2, ((A.rec_meta[base + j] >> 24) & 1u) != 0u);
+            }
+            st.finish(rule, res);
+        }
+        const int prev_x = 2 * prev_cx - 2;
+        Lane L;
+        L.init(merged, head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at), p > 0, x, prev_x, W);
+        chunk_emit<SPP, KEEP>(A, base, L, res, R, K);
+    }
+    chunks_end(A, b, base, R, K);
+}
+
 template <int SPP, bool KEEP>
 __global__ void __launch_bounds__(64) k_resolve_big(ResolveArgs A) {
     constexpr int NW = Words<SPP>::n;
@@ -812,118 +914,8 @@ __global__ void __launch_bounds__(64) k_resolve_big(ResolveArgs A) {
         if (n <= 256) resolve_bucket<SPP, 4, KEEP>(A, b, base, n, key, order, meta, msk, R);
         else if (n <= 512) resolve_bucket<SPP, 8, KEEP>(A, b, base, n, key, order, meta, msk, R);
         else if (n <= 64 * kBigStage) resolve_bucket<SPP, kBigStage, KEEP>(A, b, base, n, key, order, meta, msk, R);
+        else resolve_huge<SPP, KEEP>(A, b, base, n, R);
     }
-}
-
-// Buckets of more than 1024 fragments (rare): bitonic-sort 64-bit (cell x, index) keys,
-// held in the bucket's stretch of the record array (4n words; the padded power of two is at
-// most 2n), copy the sorted indices into the scratch (the records are written next), then walk
-// the sorted order in chunks of 64 reading the fragments from global memory.  Any bucket
-// size works.
-template <int SPP, bool KEEP>
-__global__ void __launch_bounds__(64) k_resolve_huge(ResolveArgs A) {
-    constexpr int NW = Words<SPP>::n;
-    __shared__ RecLds R;
-    const int lane = threadIdx.x;
-    const uint32_t nbig = *A.big_count;
-    for (uint32_t bi = blockIdx.x; bi < nbig; bi += gridDim.x) {
-        const int64_t b = A.big_list[bi];
-        const uint32_t base = A.boff[b];
-        const int n = (int)(A.boff[b + 1] - base);
-        if (n <= 64 * kBigStage) continue;
-        int P2 = 1;
-        while (P2 < n) P2 <<= 1;
-        uint32_t *khi = (uint32_t *)(A.prec + base);
-        uint32_t *klo = khi + P2;
-        for (int i = lane; i < P2; i += 64) {
-            khi[i] = (i < n) ? (A.rec_meta[base + i] & 0xFFFFu) : 0xFFFFFFFFu;
-            klo[i] = (i < n) ? (uint32_t)i : 0xFFFFFFFFu;
-        }
-        __syncthreads();
-        for (int k = 2; k <= P2; k <<= 1) {
-            for (int j = k >> 1; j > 0; j >>= 1) {
-                for (int i = lane; i < P2; i += 64) {
-                    const int l = i ^ j;
-                    if (l > i) {
-                        const uint32_t ah = khi[i], al = klo[i], ch = khi[l], cl = klo[l];
-                        const bool gt = ah > ch || (ah == ch && al > cl);
-                        const bool up = (i & k) == 0;
-                        if (gt == up) {
-                            khi[i] = ch; klo[i] = cl;
-                            khi[l] = ah; klo[l] = al;
-                        }
-                    }
-                }
-                __syncthreads();
-            }
-        }
-        uint32_t *order = A.scratch + base;
-        for (int i = lane; i < n; i += 64) order[i] = klo[i];
-        chunks_begin(R);
-        __syncthreads();
-        // sorted fragment indices; a fragment's cell x is in its record
-        auto cell_x = [&](int q) { return (int)(A.rec_meta[base + order[q]] & 0xFFFFu); };
-        const int rule = A.frule[A.binfo[b].x];
-        uint32_t wcarry = A.bcarry[b];
-        int W = A.W;
-        if (A.pcanvas) {
-            const int4 cv = A.pcanvas[A.binfo[b].x];
-            W = cv.x;
-            wcarry -= A.scarry[cv.w];
-        }
-        Chunks K;
-        for (int c0 = 0; c0 < n; c0 += 64) {
-            const int p = c0 + lane;
-            const bool v = p < n;
-            const uint32_t meta = v ? A.rec_meta[base + order[p]] : 0u;
-            const int cx = (int)(meta & 0xFFFFu);
-            const int swn = v ? (int)(int8_t)(meta >> 16) : 0;
-            const int prev_cx = (v && p > 0) ? cell_x(p - 1) : -1;
-            const bool head = v && (p == 0 || cx != prev_cx);
-            const int incl = scan_add(swn);
-            const int8_t w_at = (int8_t)(int)(wcarry + (uint32_t)(incl - swn));
-            wcarry += (uint32_t)lane63(incl);
-            const int x = 2 * cx - 2;
-            const bool merged = head && x >= 0 && x < W;
-            uint32_t res[NW];
-            if (merged) {
-                Stencil<NW> st;
-                st.init(w_at);
-                for (int q = p; q < n; ++q) {
-                    const uint32_t j = order[q];
-                    const uint32_t mq = A.rec_meta[base + j];
-                    if ((int)(mq & 0xFFFFu) != cx) break;
-                    uint32_t m2[NW];
-                    load_mask<NW>(A.rec_mask, (size_t)base + j, m2);
-                    st.add(m2, ((A.rec_meta[base + j] >> 24) & 1u) != 0u);
-                }
-                st.finish(rule, res);
-            }
-            const int prev_x = 2 * prev_cx - 2;
-            Lane L;
-            L.init(merged, head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at), p > 0, x, prev_x, W);
-            chunk_emit<SPP, KEEP>(A, base, L, res, R, K);
-        }
-        chunks_end(A, b, base, R, K);
-    }
-}
-
-// ---------------------------------------------------------------------------------
-// compositing order: non-empty buckets, stably sorted by cell row (path order kept)
-// ---------------------------------------------------------------------------------
-__global__ void k_nz_flags(int64_t NB, const uint4 *__restrict__ brec, uint32_t *flag) {
-    int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < NB) flag[b] = brec[2 * b + 1].z ? 1u : 0u;
-}
-__global__ void k_nz_compact(int64_t NB, const uint32_t *__restrict__ flag, const uint32_t *__restrict__ off,
-                             const int2 *__restrict__ binfo, const int4 *__restrict__ pcanvas, uint32_t *keys,
-                             uint32_t *vals) {
-    int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= NB || !flag[b]) return;
-    const uint32_t o = off[b];
-    const int2 bi = binfo[b];
-    keys[o] = (uint32_t)bi.y + (pcanvas ? (uint32_t)pcanvas[bi.x].z : 0u);
-    vals[o] = (uint32_t)b;
 }
 
 // Winding-scan carry at the first bucket of every scene of a batch.
@@ -931,88 +923,6 @@ __global__ void k_scene_carry(int n, const uint32_t *__restrict__ sfirst, const 
                               const uint32_t *__restrict__ bcarry, uint32_t *scarry) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) scarry[i] = bcarry[pbase[sfirst[i]]];
-}
-
-constexpr int kRsThreads = 256, kRsItems = 8, kRsTile = kRsThreads * kRsItems;
-
-__global__ void __launch_bounds__(kRsThreads) k_rs_hist(const uint32_t *__restrict__ keys, const uint32_t *n_ptr,
-                                                         int shift, uint32_t ntiles, uint32_t *hist) {
-    __shared__ uint32_t cnt[256];
-    cnt[threadIdx.x] = 0;
-    __syncthreads();
-    const uint32_t n = *n_ptr;
-    const size_t base = (size_t)blockIdx.x * kRsTile;
-    for (int k = 0; k < kRsItems; ++k) {
-        size_t i = base + (size_t)k * kRsThreads + threadIdx.x;
-        if (i < n) atomicAdd(&cnt[(keys[i] >> shift) & 255u], 1u);
-    }
-    __syncthreads();
-    hist[(size_t)threadIdx.x * ntiles + blockIdx.x] = cnt[threadIdx.x];
-}
-
-__global__ void __launch_bounds__(kRsThreads) k_rs_scatter(const uint32_t *__restrict__ kin, const uint32_t *__restrict__ vin,
-                                                            uint32_t *kout, uint32_t *vout, const uint32_t *n_ptr, int shift,
-                                                            uint32_t ntiles, const uint32_t *__restrict__ hoff) {
-    __shared__ uint32_t wcnt[4][256];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int d = threadIdx.x; d < 4 * 256; d += kRsThreads) (&wcnt[0][0])[d] = 0;
-    __syncthreads();
-    const uint32_t n = *n_ptr;
-    const size_t base = (size_t)blockIdx.x * kRsTile + (size_t)w * (kRsTile / 4);
-    const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    uint32_t lr[kRsItems], dg[kRsItems], kk[kRsItems], vv[kRsItems];
-#pragma unroll
-    for (int r = 0; r < kRsItems; ++r) {
-        const size_t i = base + (size_t)r * 64 + lane;
-        const bool valid = i < n;
-        kk[r] = valid ? kin[i] : 0u;
-        vv[r] = valid ? vin[i] : 0u;
-        const uint32_t d = (kk[r] >> shift) & 255u;
-        dg[r] = d;
-        unsigned long long m = __ballot(valid);
-#pragma unroll
-        for (int bit = 0; bit < 8; ++bit) {
-            const unsigned long long bb = __ballot((d >> bit) & 1u);
-            m &= ((d >> bit) & 1u) ? bb : ~bb;
-        }
-        const uint32_t before = valid ? wcnt[w][d] : 0u;
-        const int rk = __popcll(m & lt);
-        lr[r] = before + (uint32_t)rk;
-        const int tot = __popcll(m);
-        __builtin_amdgcn_wave_barrier();
-        if (valid && rk == tot - 1) wcnt[w][d] = before + (uint32_t)tot;
-        __builtin_amdgcn_wave_barrier();
-    }
-    __syncthreads();
-    {
-        const int d = threadIdx.x;
-        uint32_t run = 0;
-        for (int ww = 0; ww < 4; ++ww) {
-            uint32_t t = wcnt[ww][d];
-            wcnt[ww][d] = run;
-            run += t;
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kRsItems; ++r) {
-        const size_t i = base + (size_t)r * 64 + lane;
-        if (i < n) {
-            const uint32_t d = dg[r];
-            const uint32_t pos = hoff[(size_t)d * ntiles + blockIdx.x] + wcnt[w][d] + lr[r];
-            kout[pos] = kk[r];
-            vout[pos] = vv[r];
-        }
-    }
-}
-
-__global__ void k_row_bounds(const uint32_t *__restrict__ keys, const uint32_t *n_ptr, uint32_t *rowbeg, uint32_t *rowend) {
-    const uint32_t n = *n_ptr;
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t r = keys[i];
-    if (i == 0 || keys[i - 1] != r) rowbeg[r] = i;
-    if (i + 1 == n || keys[i + 1] != r) rowend[r] = i + 1;
 }
 
 // ---------------------------------------------------------------------------------
@@ -1169,7 +1079,8 @@ __device__ __forceinline__ uint32_t pack_dec(const float4 *step, const float *d)
 
 struct CovArgs {
     int W, H, tiles_x;
-    const uint32_t *rowbeg, *rowend;
+    const uint32_t *rowoff;  // row r: [rowoff[r shares], rowoff[(r + 1) shares])
+    uint32_t rowshares;
     const uint32_t *rext;       // per row-list entry: extent
     const uint4 *rrec;          //   colour, records, base, path
     const ulonglong2 *rtile;    //   tiles with a record, tiles inside a span
@@ -1502,7 +1413,8 @@ __global__ void __launch_bounds__(256, GRAD ? 4 : (BATCH ? 6 : 7)) k_composite_c
         wave_sync_lds();
     };
 
-    const uint32_t q0 = A.rowbeg[row0 + r], q1 = A.rowend[row0 + r];
+    const uint32_t *ro = A.rowoff + (size_t)(row0 + r) * A.rowshares;
+    const uint32_t q0 = ro[0], q1 = ro[A.rowshares];
     list_row<GRAD>(A, q0, q1, tx, tx1, kInvN, s_dec, l_queue[w], l_src[w], l_ent[w], l_grad[GRAD ? w : 0], flush);
 
     if (x >= W) return;
@@ -1866,7 +1778,8 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
         }
     };
 
-    const uint32_t q0 = A.rowbeg[r], q1 = A.rowend[r];
+    const uint32_t *ro = A.rowoff + (size_t)r * A.rowshares;
+    const uint32_t q0 = ro[0], q1 = ro[A.rowshares];
     list_row<GRAD>(A, q0, q1, tx, tx1, 1.f, s_dec, l_queue[w], l_src[w], l_ent[w], l_grad[GRAD ? w : 0], flush);
 
     // resolve: G registers at a time are staged in this wave's slot rows (G x 64 words);
@@ -1906,22 +1819,6 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
         }
         wave_sync_lds();
     }
-}
-
-// Row-list records for the compositors.
-__global__ void k_row_records(int64_t NB, const uint32_t *__restrict__ n_ptr, const uint32_t *__restrict__ rowvals,
-                              const uint4 *__restrict__ brec, const int2 *__restrict__ binfo,
-                              const uint32_t *__restrict__ finfo, const uint32_t *__restrict__ boff,
-                              uint32_t *__restrict__ rext, uint4 *__restrict__ rrec,
-                              ulonglong2 *__restrict__ rtile) {
-    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= NB || q >= (int64_t)*n_ptr) return;
-    const uint32_t bb = rowvals[q];
-    const uint32_t path = (uint32_t)binfo[bb].x;
-    const uint4 br = brec[2 * (size_t)bb], bf = brec[2 * (size_t)bb + 1];
-    rext[q] = br.x;
-    rrec[q] = make_uint4(finfo[path], br.y, boff[bb], path);
-    rtile[q] = make_ulonglong2((uint64_t)br.z | ((uint64_t)br.w << 32), (uint64_t)bf.x | ((uint64_t)bf.y << 32));
 }
 
 // Device requantisation of arbitrary values (colour-table self-check): codes and the
@@ -1974,14 +1871,14 @@ __global__ void k_encode_sweep(uint32_t lo, uint32_t hi, const float4 *__restric
 // draw list + merged masks in the reference's order and layout (.cu:789-868, 1195-1266)
 template <int SPP>
 __global__ void k_debug_draw(int64_t NB, const int2 *__restrict__ binfo, const uint32_t *__restrict__ finfo,
-                             const uint32_t *__restrict__ boff, const uint4 *__restrict__ brec,
+                             const uint32_t *__restrict__ boff, const uint2 *__restrict__ bcnt,
                              const uint32_t *__restrict__ items, const uint32_t *__restrict__ imask,
                              const uint32_t *__restrict__ moff, const uint32_t *__restrict__ ioff, int4 *draw,
                              uint32_t *mmask4) {
     constexpr int NW = Words<SPP>::n;
     int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= NB) return;
-    const uint32_t cnt = brec[2 * b + 1].z;
+    const uint32_t cnt = bcnt[b].x;
     if (!cnt) return;
     const int2 info = binfo[b];
     const uint32_t fill = finfo[info.x];
@@ -2016,11 +1913,11 @@ __global__ void k_debug_draw(int64_t NB, const int2 *__restrict__ binfo, const u
 }
 
 // out[0] += merged cells, out[1] += items
-__global__ void __launch_bounds__(256) k_count_reduce(const uint4 *__restrict__ brec, size_t n, unsigned long long *out) {
+__global__ void __launch_bounds__(256) k_count_reduce(const uint2 *__restrict__ bcnt, size_t n, unsigned long long *out) {
     __shared__ unsigned long long part[2][4];
     unsigned long long sa = 0, sc = 0;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const uint2 c = *(const uint2 *)&brec[2 * i + 1].z;
+        const uint2 c = bcnt[i];
         sa += c.y;
         sc += c.x;
     }
@@ -2040,11 +1937,11 @@ __global__ void __launch_bounds__(256) k_count_reduce(const uint4 *__restrict__ 
     }
 }
 
-__global__ void k_debug_counts(int64_t NB, const uint4 *__restrict__ brec, uint32_t *merged, uint32_t *items) {
+__global__ void k_debug_counts(int64_t NB, const uint2 *__restrict__ bcnt, uint32_t *merged, uint32_t *items) {
     const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= NB) return;
-    merged[b] = brec[2 * b + 1].w;
-    items[b] = brec[2 * b + 1].z;
+    merged[b] = bcnt[b].y;
+    items[b] = bcnt[b].x;
 }
 
 inline unsigned blocks_for(int64_t n, unsigned t) { return (unsigned)((n + t - 1) / t); }
@@ -2059,7 +1956,8 @@ void launch_resolve(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t s
     A.pcanvas = sc.pcanvas; A.scarry = f.scarry;
     // the merged masks feed the multisample compositor and the debug draw list; the
     // coverage compositor reads only the per-pixel sample counts
-    A.items = f.items; A.imask = f.imask; A.icov = f.icov; A.prec = f.prec; A.brec = f.brec;
+    A.items = f.items; A.imask = f.imask; A.icov = f.icov; A.prec = f.prec;
+    A.rpos = f.rpos; A.finfo = sc.finfo; A.rext = f.rext; A.rrec = f.rrec; A.rtile = f.rtile; A.bcnt = f.bcnt;
     A.big_list = f.big_list; A.big_count = f.big_count; A.err = f.err_flag;  // cleared at the frame's start
     const unsigned g1 = (unsigned)std::min<int64_t>(f.NB, f.resolve_grid > 0 ? f.resolve_grid : kResolveBlocks);
     const unsigned gc = f.class_grid > 0 ? (unsigned)f.class_grid : 4096u;
@@ -2068,7 +1966,6 @@ void launch_resolve(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t s
     do {                                                                              \
         hipLaunchKernelGGL((k_resolve_first<N, K>), dim3(g1), b64, 0, s, A);          \
         hipLaunchKernelGGL((k_resolve_big<N, K>), dim3(gc), b64, 0, s, A);            \
-        hipLaunchKernelGGL((k_resolve_huge<N, K>), dim3(1024), b64, 0, s, A);         \
     } while (0)
 #define SL_LAUNCH(N)                                                                  \
     do {                                                                              \
@@ -2088,43 +1985,6 @@ void launch_scene_carry(const SceneDev &sc, Frame &f, hipStream_t s) {
                        (const uint32_t *)f.pbase, (const uint32_t *)f.bcarry, f.scarry);
 }
 
-void launch_order_rows(const SceneDev &sc, Frame &f, hipStream_t s) {
-    const int64_t R = f.R;
-    launch_fill2_u32(f.rowbeg, f.rowend, 0u, (size_t)R, s);
-    if (!f.NB) return;
-    hipLaunchKernelGGL(k_nz_flags, dim3(blocks_for(f.NB, 256)), dim3(256), 0, s, f.NB, (const uint4 *)f.brec, f.nz_flag);
-    scan_exclusive_u32(f.nz_flag, f.nz_off, (size_t)f.NB, f.scan_tmp, s);
-    hipLaunchKernelGGL(k_nz_compact, dim3(blocks_for(f.NB, 256)), dim3(256), 0, s, f.NB, (const uint32_t *)f.nz_flag,
-                       (const uint32_t *)f.nz_off, (const int2 *)f.binfo, sc.pcanvas, f.nz_keys[0], f.nz_vals[0]);
-    const uint32_t *n_ptr = f.nz_off + f.NB;
-    const uint32_t ntiles = (uint32_t)((f.NB + kRsTile - 1) / kRsTile);
-    int bits = 0;
-    while ((int64_t)1 << bits < R) ++bits;
-    const int passes = bits <= 8 ? 1 : (bits + 7) / 8;
-    int cur = 0;
-    for (int pss = 0; pss < passes; ++pss) {
-        const int shift = 8 * pss;
-        hipLaunchKernelGGL(k_rs_hist, dim3(ntiles), dim3(kRsThreads), 0, s, (const uint32_t *)f.nz_keys[cur], n_ptr, shift,
-                           ntiles, f.rs_hist);
-        scan_exclusive_u32(f.rs_hist, f.rs_hoff, (size_t)256 * ntiles, f.scan_tmp, s);
-        hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(kRsThreads), 0, s, (const uint32_t *)f.nz_keys[cur],
-                           (const uint32_t *)f.nz_vals[cur], f.nz_keys[cur ^ 1], f.nz_vals[cur ^ 1], n_ptr, shift, ntiles,
-                           (const uint32_t *)f.rs_hoff);
-        cur ^= 1;
-    }
-    if (cur != 0) {
-        // keep the sorted lists in slot 0 for the compositor
-        uint32_t *k = f.nz_keys[0], *v = f.nz_vals[0];
-        f.nz_keys[0] = f.nz_keys[1]; f.nz_vals[0] = f.nz_vals[1];
-        f.nz_keys[1] = k; f.nz_vals[1] = v;
-    }
-    hipLaunchKernelGGL(k_row_bounds, dim3(blocks_for(f.NB, 256)), dim3(256), 0, s, (const uint32_t *)f.nz_keys[0], n_ptr,
-                       f.rowbeg, f.rowend);
-    hipLaunchKernelGGL(k_row_records, dim3(blocks_for(f.NB, 256)), dim3(256), 0, s, f.NB, n_ptr,
-                           (const uint32_t *)f.nz_vals[0], (const uint4 *)f.brec, (const int2 *)f.binfo, sc.finfo,
-                           (const uint32_t *)f.boff, f.rext, f.rrec, f.rtile);
-}
-
 void launch_composite(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t s) {
     const int R = (f.H + 1) / 2;
     const int tiles_x = (f.W + 63) / 64;
@@ -2132,7 +1992,7 @@ void launch_composite(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t
     if (!f.ms) {
         CovArgs C;
         C.W = f.W; C.H = f.H; C.tiles_x = tiles_x;
-        C.rowbeg = f.rowbeg; C.rowend = f.rowend; C.rext = f.rext; C.rrec = f.rrec; C.rtile = f.rtile;
+        C.rowoff = f.rowoff; C.rowshares = f.rowshares; C.rext = f.rext; C.rrec = f.rrec; C.rtile = f.rtile;
         C.prec = f.prec; C.icov = f.icov; C.imask = nullptr; C.ptab = nullptr; C.dec_c = t.dec_c; C.dec_a = t.dec_a; C.step_c = t.step_c;
         C.image = f.image; C.pitch = f.pitch;
         C.G = f.grad;
@@ -2159,7 +2019,7 @@ void launch_composite(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t
     }
     CovArgs C;
     C.W = f.W; C.H = f.H; C.tiles_x = tiles_x;
-    C.rowbeg = f.rowbeg; C.rowend = f.rowend; C.rext = f.rext; C.rrec = f.rrec; C.rtile = f.rtile;
+    C.rowoff = f.rowoff; C.rowshares = f.rowshares; C.rext = f.rext; C.rrec = f.rrec; C.rtile = f.rtile;
     C.prec = f.prec; C.icov = f.icov; C.imask = f.imask; C.ptab = f.ptab;
     C.dec_c = t.dec_c; C.dec_a = t.dec_a; C.step_c = t.step_c;
     C.image = f.image; C.pitch = f.pitch;
@@ -2218,21 +2078,21 @@ void launch_debug_draw_list(const SceneDev &sc, const Tables &t, Frame &f, const
     dim3 g(blocks_for(f.NB, 256)), b(256);
     if (t.spp == 8)
         hipLaunchKernelGGL(k_debug_draw<8>, g, b, 0, s, f.NB, (const int2 *)f.binfo, sc.finfo, (const uint32_t *)f.boff,
-                           (const uint4 *)f.brec, (const uint32_t *)f.items, (const uint32_t *)f.imask, moff, ioff, draw, mmask4);
+                           (const uint2 *)f.bcnt, (const uint32_t *)f.items, (const uint32_t *)f.imask, moff, ioff, draw, mmask4);
     else if (t.spp == 16)
         hipLaunchKernelGGL(k_debug_draw<16>, g, b, 0, s, f.NB, (const int2 *)f.binfo, sc.finfo, (const uint32_t *)f.boff,
-                           (const uint4 *)f.brec, (const uint32_t *)f.items, (const uint32_t *)f.imask, moff, ioff, draw, mmask4);
+                           (const uint2 *)f.bcnt, (const uint32_t *)f.items, (const uint32_t *)f.imask, moff, ioff, draw, mmask4);
     else
         hipLaunchKernelGGL(k_debug_draw<32>, g, b, 0, s, f.NB, (const int2 *)f.binfo, sc.finfo, (const uint32_t *)f.boff,
-                           (const uint4 *)f.brec, (const uint32_t *)f.items, (const uint32_t *)f.imask, moff, ioff, draw, mmask4);
+                           (const uint2 *)f.bcnt, (const uint32_t *)f.items, (const uint32_t *)f.imask, moff, ioff, draw, mmask4);
 }
 
-void launch_count_reduce(const uint4 *brec, size_t n, unsigned long long *out, hipStream_t s) {
-    hipLaunchKernelGGL(k_count_reduce, dim3(256), dim3(256), 0, s, brec, n, out);
+void launch_count_reduce(const uint2 *bcnt, size_t n, unsigned long long *out, hipStream_t s) {
+    hipLaunchKernelGGL(k_count_reduce, dim3(256), dim3(256), 0, s, bcnt, n, out);
 }
 
 void launch_debug_counts(const Frame &f, uint32_t *merged, uint32_t *items, hipStream_t s) {
-    if (f.NB) hipLaunchKernelGGL(k_debug_counts, dim3(blocks_for(f.NB, 256)), dim3(256), 0, s, f.NB, (const uint4 *)f.brec, merged, items);
+    if (f.NB) hipLaunchKernelGGL(k_debug_counts, dim3(blocks_for(f.NB, 256)), dim3(256), 0, s, f.NB, (const uint2 *)f.bcnt, merged, items);
 }
 
 }  // namespace sl
