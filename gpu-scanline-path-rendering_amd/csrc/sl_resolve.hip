@@ -91,27 +91,27 @@ struct Stencil {
 // at w * 0x01010101 and gain +/- 0x01 at set bits, so the word is sum_j c_j * 256^j
 // (mod 2^32) with c_j the sample's true count w + d_j.  While every c_j lies in
 // [-128, 127], adding 0x80808080 leaves byte j = c_j + 128 with no carry between lanes,
-// and the tests read c_j mod 128 != 0 (nonzero) or c_j & 1 (even-odd).  For g <= 7
-// members and |w| <= 120, c_j lies in [-127, 127], so it is enough to count d_j in
-// [-7, 7] in four two's-complement bit planes: nonzero is d_j != -w, even-odd is
-// d_j ^ w in plane 0.  Groups outside that range take the byte-lane stencil.
-constexpr int kSlicedMaxGroup = 7;
-constexpr int kSlicedMaxWinding = 120;
-
-__device__ __forceinline__ bool sliced_ok(int g, int8_t w) {
-    return g <= kSlicedMaxGroup && w >= -kSlicedMaxWinding && w <= kSlicedMaxWinding;
+// and the tests read c_j mod 128 != 0 (nonzero) or c_j & 1 (even-odd).  With g members and
+// |w| <= 127 - g, c_j lies in [-127, 127], so it is enough to count d_j in [-g, g] in P
+// two's-complement bit planes, g < 2^(P - 1): nonzero is d_j != -w, even-odd is d_j ^ w in
+// plane 0.  Four planes take groups of up to 7, six of up to 31 (crowded rows: a bucket with
+// one group of 8 waited for a byte-lane pass over each of its words); larger groups and
+// windings take the byte-lane stencil.
+__device__ __forceinline__ bool sliced_ok(int g, int8_t w, int planes) {
+    const int lim = (1 << (planes - 1)) - 1;
+    return g <= lim && w >= lim - 127 && w <= 127 - lim;
 }
 
-template <int NW>
+template <int NW, int P>
 struct Sliced {
-    uint32_t d[4][NW];
-    // d = +1 or -1 (1111 in four planes) at the set bits of one member
+    uint32_t d[P][NW];
+    // d = +1 or -1 (all planes set) at the set bits of one member
     __device__ __forceinline__ void init_one(const uint32_t *m, bool neg) {
 #pragma unroll
         for (int k = 0; k < NW; ++k) {
             d[0][k] = m[k];
 #pragma unroll
-            for (int p = 1; p < 4; ++p) d[p][k] = neg ? m[k] : 0u;
+            for (int p = 1; p < P; ++p) d[p][k] = neg ? m[k] : 0u;
         }
     }
     // d += 1 (or -= 1) at the set bits: ripple carry (borrow) through the planes
@@ -121,7 +121,7 @@ struct Sliced {
         for (int k = 0; k < NW; ++k) {
             uint32_t c = m[k];
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
+            for (int p = 0; p < P; ++p) {
                 const uint32_t t = (d[p][k] ^ nm) & c;
                 d[p][k] ^= c;
                 c = t;
@@ -136,15 +136,15 @@ struct Sliced {
             return;
         }
         const int t = -(int)w;
-        const bool hit = t >= -8 && t <= 7;  // d_j in [-7, 7] can equal -w only then
-        uint32_t tp[4];
+        const bool hit = t >= -(1 << (P - 1)) && t < (1 << (P - 1));  // d_j can equal -w only then
+        uint32_t tp[P];
 #pragma unroll
-        for (int p = 0; p < 4; ++p) tp[p] = ((t >> p) & 1) ? ~0u : 0u;
+        for (int p = 0; p < P; ++p) tp[p] = ((t >> p) & 1) ? ~0u : 0u;
 #pragma unroll
         for (int k = 0; k < NW; ++k) {
             uint32_t ne = 0u;
 #pragma unroll
-            for (int p = 0; p < 4; ++p) ne |= d[p][k] ^ tp[p];
+            for (int p = 0; p < P; ++p) ne |= d[p][k] ^ tp[p];
             out[k] = hit ? ne : ~0u;
         }
     }
@@ -176,6 +176,11 @@ __device__ __forceinline__ void load_mask(const uint32_t *p, size_t slot, uint32
     if (NW == 4) { uint4 q = *(const uint4 *)(p + slot * 4); m[0] = q.x; m[1] = q.y; m[2] = q.z; m[3] = q.w; }
     else if (NW == 2) { uint2 q = *(const uint2 *)(p + slot * 2); m[0] = q.x; m[1] = q.y; }
     else m[0] = p[slot];
+}
+
+__device__ __forceinline__ void wave_sync_lds() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+    __builtin_amdgcn_wave_barrier();
 }
 
 struct ResolveArgs {
@@ -214,22 +219,27 @@ __device__ __forceinline__ uint32_t cell_bits(int c0, int c1) { return (~0u << c
 
 constexpr int kBigStage = 16;  // chunks of 64 fragments staged in LDS
 
-// LDS of the buckets packed in a wave: their two tile bitmaps; of a chunked bucket, the group
-// heads of its chunks
-struct RecLds {
-    unsigned long long et[4], ft[4], heads[kBigStage];
+// A bucket's results, collected in LDS while it is resolved.
+struct BucketOut {
+    unsigned long long et, ft;  // tiles with a record, tiles wholly inside a span
+    uint32_t ext, nrec, items, merged;
 };
 
-// A bucket's entry in the row lists (one lane).
-__device__ __forceinline__ void put_row(const ResolveArgs &A, int64_t b, uint32_t base, uint32_t path, uint32_t ext,
-                                        int nrec, uint64_t et, uint64_t ft, int items, int merged) {
-    A.bcnt[b] = make_uint2((uint32_t)items, (uint32_t)merged);
-    const uint32_t at = A.rpos[b];
+__device__ __forceinline__ void out_clear(BucketOut &o) {
+    o.et = o.ft = 0ull;
+    o.ext = 0xFFFFu;
+    o.nrec = o.items = o.merged = 0u;
+}
+
+// A bucket's entry in the row lists, by one lane.
+__device__ __forceinline__ void put_row(const ResolveArgs &A, int64_t b, uint32_t at, uint32_t base, uint32_t path,
+                                        uint32_t colour, const BucketOut &o) {
+    A.bcnt[b] = make_uint2(o.items, o.merged);
     if (at == 0xFFFFFFFFu) return;  // the out-of-canvas bucket
-    A.rext[at] = ext;
-    if (!items) return;             // an empty extent: the rest is never read
-    A.rrec[at] = make_uint4(A.finfo[path], (uint32_t)nrec, base, path);
-    A.rtile[at] = make_ulonglong2(et, ft);
+    A.rext[at] = o.ext;
+    if (!o.items) return;           // an empty extent: the rest is never read
+    A.rrec[at] = make_uint4(colour, o.nrec, base, path);
+    A.rtile[at] = make_ulonglong2(o.et, o.ft);
 }
 
 // What a lane contributes to its bucket's records: its group head's merged cell at x (if any)
@@ -272,23 +282,34 @@ struct Lane {
 __device__ __forceinline__ int scan_add(int x) { return dpp_scan(x, 0, OpAdd()); }
 __device__ __forceinline__ int lane63(int x) { return __builtin_amdgcn_readlane(x, 63); }
 
+template <int NW, int P>
+__device__ __forceinline__ void group_sliced(const uint32_t *order, const uint32_t *meta, const uint32_t *msk, int p, int e,
+                                             const uint32_t *first, bool neg0, int8_t w_at, int rule, uint32_t *res) {
+    Sliced<NW, P> st;
+    st.init_one(first, neg0);
+    uint32_t iq = order[p + 1 < e ? p + 1 : p];
+    for (int q = p + 1; q < e; ++q) {
+        uint32_t m[NW];
+        load_mask<NW>(msk, iq, m);
+        const bool neg = ((meta[iq] >> 24) & 1u) != 0u;
+        iq = order[q + 1 < e ? q + 1 : q];  // the next member's index loads beside this one's mask
+        st.add(m, neg);
+    }
+    st.finish(rule, w_at, res);
+}
+
 // Merged mask of the cell group at sorted positions [p, e) (records staged in LDS).  The
 // first member is the head lane's own record i0 (meta m0): most groups have no other.
 template <int NW>
 __device__ __forceinline__ void group_mask(const uint32_t *order, const uint32_t *meta, const uint32_t *msk, int p,
                                            int e, uint32_t i0, uint32_t m0, int8_t w_at, int rule, uint32_t *res) {
     uint32_t first[NW];
-#pragma unroll
-    for (int k = 0; k < NW; ++k) first[k] = msk[i0 * NW + k];
+    load_mask<NW>(msk, i0, first);
     const bool neg0 = ((m0 >> 24) & 1u) != 0u;
-    if (sliced_ok(e - p, w_at)) {
-        Sliced<NW> st;
-        st.init_one(first, neg0);
-        for (int q = p + 1; q < e; ++q) {
-            const uint32_t iq = order[q];
-            st.add(msk + iq * NW, ((meta[iq] >> 24) & 1u) != 0u);
-        }
-        st.finish(rule, w_at, res);
+    if (sliced_ok(e - p, w_at, 4)) {
+        group_sliced<NW, 4>(order, meta, msk, p, e, first, neg0, w_at, rule, res);
+    } else if (sliced_ok(e - p, w_at, 6)) {
+        group_sliced<NW, 6>(order, meta, msk, p, e, first, neg0, w_at, rule, res);
     } else {
         // rare: one word at a time, for eight counters instead of eight a word
 #pragma unroll
@@ -305,6 +326,22 @@ __device__ __forceinline__ void group_mask(const uint32_t *order, const uint32_t
     }
 }
 
+// Ranks of the keys `mine` among key[0, n), n a multiple of 4 (keys are distinct; unused places
+// hold the largest value).  Four keys a read: a read a key, or a cross-lane operation a key,
+// kept the LDS pipe busier than the comparisons.
+template <int S>
+__device__ __forceinline__ void rank_keys(const uint32_t *key, int n, const uint32_t *mine, int *rk) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) rk[s] = 0;
+#pragma unroll 4
+    for (int j = 0; j < n; j += 4) {
+        const uint4 k = *(const uint4 *)(key + j);
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+            rk[s] += (k.x < mine[s] ? 1 : 0) + (k.y < mine[s] ? 1 : 0) + (k.z < mine[s] ? 1 : 0) + (k.w < mine[s] ? 1 : 0);
+    }
+}
+
 // A bucket walked in chunks of 64 sorted records: totals, and the cells of the last record,
 // which the next chunk may add to.
 struct Chunks {
@@ -312,13 +349,9 @@ struct Chunks {
     uint32_t cover = 0u, edge = 0u;
 };
 
-__device__ __forceinline__ void chunks_begin(RecLds &R) {
-    if ((threadIdx.x & 63) == 0) R.et[0] = R.ft[0] = 0ull;
-}
-
 template <int SPP, bool KEEP>
 __device__ __forceinline__ void chunk_emit(const ResolveArgs &A, uint32_t base, const Lane &L, const uint32_t *res,
-                                           RecLds &R, Chunks &K) {
+                                           BucketOut &O, Chunks &K) {
     constexpr int NW = Words<SPP>::n;
     const int lane = threadIdx.x & 63;
     const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
@@ -350,8 +383,8 @@ __device__ __forceinline__ void chunk_emit(const ResolveArgs &A, uint32_t base, 
         K.xmin = tmin(K.xmin, __builtin_amdgcn_readlane(L.lo(), first));
         K.xmax = tmax(K.xmax, __builtin_amdgcn_readlane(L.hi(), last));
         const int tb = K.xmin >> 6;
-        if (L.leader) atomicOr(&R.et[0], 1ull << tmin((L.x >> 6) - tb, 63));
-        if (L.f0 <= L.f1) atomicOr(&R.ft[0], tile_bits(L.f0, L.f1, tb));
+        if (L.leader) atomicOr(&O.et, 1ull << tmin((L.x >> 6) - tb, 63));
+        if (L.f0 <= L.f1) atomicOr(&O.ft, tile_bits(L.f0, L.f1, tb));
     }
     const bool far = L.f0 <= L.f1 && L.prev_ok && L.f1 - (K.xmin >> 6) >= 63;
     if (__ballot(far)) {
@@ -372,66 +405,63 @@ __device__ __forceinline__ void chunk_emit(const ResolveArgs &A, uint32_t base, 
     K.spans += (int)__popcll(sm);
 }
 
-__device__ __forceinline__ void chunks_end(const ResolveArgs &A, int64_t b, uint32_t base, RecLds &R, const Chunks &K) {
-    __syncthreads();
+__device__ __forceinline__ void chunks_end(const ResolveArgs &A, uint32_t base, BucketOut &O, const Chunks &K) {
     if ((threadIdx.x & 63) == 0) {
         if (K.nrec) *(uint2 *)&A.prec[base + K.nrec - 1].x = make_uint2(K.cover, K.edge);
-        const bool any = K.merged + K.spans > 0;
-        put_row(A, b, base, (uint32_t)A.binfo[b].x, any ? ((uint32_t)K.xmin | ((uint32_t)K.xmax << 16)) : 0xFFFFu, K.nrec,
-                R.et[0], R.ft[0], K.merged + K.spans, K.merged);
+        if (K.merged + K.spans > 0) O.ext = (uint32_t)K.xmin | ((uint32_t)K.xmax << 16);
+        O.nrec = (uint32_t)K.nrec;
+        O.items = (uint32_t)(K.merged + K.spans);
+        O.merged = (uint32_t)K.merged;
     }
-    __syncthreads();
+    wave_sync_lds();
 }
 
-// Resolve one (path, row) bucket of n <= 64*S fragments with one wavefront: stage the
-// records in LDS, rank them by (cell x, index), then walk the sorted order in chunks of
-// 64 carrying the winding number and the records.  Per cell group, the first lane sums
-// the members' masks into the per-sample stencil; spans open between groups whose
-// winding passes the fill rule.
-template <int SPP, int S, bool KEEP>
+// Resolve one (path, row) bucket of n <= 64*S*WAVES fragments with a block of WAVES waves: stage
+// the records in LDS, rank them by (cell x, index), then the first wave walks the sorted order
+// in chunks of 64 carrying the winding number and the records (the others return).  Per cell
+// group, the first lane sums the members' masks into the per-sample stencil; spans open between
+// groups whose winding passes the fill rule.
+template <int SPP, int S, bool KEEP, int WAVES = 1>
 __device__ __forceinline__ void resolve_bucket(const ResolveArgs &A, int64_t b, uint32_t base, int n, uint32_t *key,
-                                               uint32_t *order, uint32_t *meta, uint32_t *msk, RecLds &R) {
+                                               uint32_t *order, uint32_t *meta, uint32_t *msk,
+                                               unsigned long long *ghead, BucketOut &O) {
     constexpr int NW = Words<SPP>::n;
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, tid = threadIdx.x;
+    constexpr int T = 64 * WAVES;
     uint32_t mykey[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-        const int i = s * 64 + lane;
+        const int i = s * T + tid;
         mykey[s] = 0xFFFFFFFFu;
         if (i < n) {
             const uint32_t m = A.rec_meta[base + i];
             meta[i] = m;
             uint32_t mk[NW];
             load_mask<NW>(A.rec_mask, (size_t)base + i, mk);
-#pragma unroll
-            for (int k = 0; k < NW; ++k) msk[i * NW + k] = mk[k];
+            store_mask<NW>(msk, (size_t)i, mk);
             mykey[s] = ((m & 0xFFFFu) << 10) | (uint32_t)i;
-            key[i] = mykey[s];
         }
+        key[i] = mykey[s];
     }
-    chunks_begin(R);
     __syncthreads();
     int rk[S];
-#pragma unroll
-    for (int s = 0; s < S; ++s) rk[s] = 0;
-    if (S == 1) {
-#pragma unroll 8
-        for (int j = 0; j < n; ++j) {
-            const uint32_t kj = (uint32_t)__builtin_amdgcn_readlane((int)mykey[0], j);
-            rk[0] += (kj < mykey[0]) ? 1 : 0;
-        }
-    } else {
-#pragma unroll 8
-        for (int j = 0; j < n; ++j) {
-            const uint32_t kj = key[j];
-#pragma unroll
-            for (int s = 0; s < S; ++s) rk[s] += (kj < mykey[s]) ? 1 : 0;
-        }
-    }
+    rank_keys<S>(key, (n + 3) & ~3, mykey, rk);
 #pragma unroll
     for (int s = 0; s < S; ++s)
-        if (s * 64 + lane < n) order[rk[s]] = (uint32_t)(s * 64 + lane);
+        if (s * T + tid < n) order[rk[s]] = (uint32_t)(s * T + tid);
     __syncthreads();
+    // group heads of every chunk as wave masks: a group ends at the next head
+    const int nc = (n + 63) >> 6;
+#pragma unroll 1
+    for (int c = tid >> 6; c < nc; c += WAVES) {
+        const int p = c * 64 + lane;
+        bool h = false;
+        if (p < n) h = p == 0 || (meta[order[p]] & 0xFFFFu) != (meta[order[p - 1]] & 0xFFFFu);
+        const uint64_t hm = __ballot(h);
+        if (lane == 0) ghead[c] = hm;
+    }
+    __syncthreads();
+    if (WAVES > 1 && tid >= 64) return;
 
     const int rule = A.frule[A.binfo[b].x];
     uint32_t wcarry = A.bcarry[b];
@@ -443,17 +473,6 @@ __device__ __forceinline__ void resolve_bucket(const ResolveArgs &A, int64_t b, 
         wcarry -= A.scarry[cv.w];
     }
     Chunks K;
-    // group heads of every chunk as wave masks: a group ends at the next head
-    const int nc = (n + 63) >> 6;
-#pragma unroll 1
-    for (int c = 0; c < nc; ++c) {
-        const int p = c * 64 + lane;
-        bool h = false;
-        if (p < n) h = p == 0 || (meta[order[p]] & 0xFFFFu) != (meta[order[p - 1]] & 0xFFFFu);
-        const uint64_t hm = __ballot(h);
-        if (lane == 0) R.heads[c] = hm;
-    }
-    __syncthreads();
 #pragma unroll 1
     for (int c = 0; c < nc; ++c) {
         const int p = c * 64 + lane;
@@ -471,22 +490,22 @@ __device__ __forceinline__ void resolve_bucket(const ResolveArgs &A, int64_t b, 
         const bool merged = head && x >= 0 && x < W;
         uint32_t res[NW];
         if (merged) {
-            const uint64_t later = lane < 63 ? (R.heads[c] & (~0ull << (lane + 1))) : 0ull;
+            const uint64_t later = lane < 63 ? (ghead[c] & (~0ull << (lane + 1))) : 0ull;
             int e = n;
             if (later) {
                 e = c * 64 + (int)__builtin_ctzll(later);
             } else {
                 for (int c2 = c + 1; c2 < nc; ++c2)
-                    if (R.heads[c2]) { e = c2 * 64 + (int)__builtin_ctzll(R.heads[c2]); break; }
+                    if (ghead[c2]) { e = c2 * 64 + (int)__builtin_ctzll(ghead[c2]); break; }
             }
             group_mask<NW>(order, meta, msk, p, e, i, m, w_at, rule, res);
         }
         const int prev_x = 2 * prev_cx - 2;
         Lane L;
         L.init(merged, head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at), p > 0, x, prev_x, W);
-        chunk_emit<SPP, KEEP>(A, base, L, res, R, K);
+        chunk_emit<SPP, KEEP>(A, base, L, res, O, K);
     }
-    chunks_end(A, b, base, R, K);
+    chunks_end(A, base, O, K);
 }
 
 constexpr int kResolveBlocks = 65536;
@@ -528,8 +547,8 @@ template <> struct SegBits<16> : SegBits32<16> { using SegBits32<16>::SegBits32;
 
 // The records of the buckets in a wave's 64 / S segments, each bucket in one pass.
 template <int SPP, int S, bool KEEP>
-__device__ __forceinline__ void segment_emit(const ResolveArgs &A, bool live, int64_t b, uint32_t base, uint32_t path, const Lane &L,
-                                             const uint32_t *res, RecLds &R) {
+__device__ __forceinline__ void segment_emit(const ResolveArgs &A, bool live, uint32_t base, const Lane &L,
+                                             const uint32_t *res, BucketOut &O) {
     constexpr int NW = Words<SPP>::n;
     const int lane = threadIdx.x & 63;
     const int i = lane % S, seg = lane / S, sb = seg * S;
@@ -549,8 +568,8 @@ __device__ __forceinline__ void segment_emit(const ResolveArgs &A, bool live, in
         xmax = __shfl(L.hi(), any.m ? sb + any.last() : lane, 64);
     }
     const int tb = xmin >> 6;
-    if (L.leader) atomicOr(&R.et[seg], 1ull << tmin((L.x >> 6) - tb, 63));
-    if (L.f0 <= L.f1) atomicOr(&R.ft[seg], tile_bits(L.f0, L.f1, tb));
+    if (L.leader) atomicOr(&O.et, 1ull << tmin((L.x >> 6) - tb, 63));
+    if (L.f0 <= L.f1) atomicOr(&O.ft, tile_bits(L.f0, L.f1, tb));
     // a leader's record: the sums of its run of lanes, up to the next leader
     const uint32_t pe = (uint32_t)dpp_scan_seg<S>((int)L.eb, 0, OpAdd()), pc = (uint32_t)dpp_scan_seg<S>((int)L.co, 0, OpAdd());
     const int next = lm.after(i);
@@ -569,17 +588,13 @@ __device__ __forceinline__ void segment_emit(const ResolveArgs &A, bool live, in
         if (L.span) A.items[it] = (uint32_t)(L.prev_x + 2) | ((uint32_t)(L.x - L.prev_x - 2) << 16);
         if (L.merged) A.items[it + (L.span ? 1 : 0)] = (uint32_t)L.x;
     }
-    __syncthreads();
     if (live && i == 0) {
-        put_row(A, b, base, path, any.m ? ((uint32_t)xmin | ((uint32_t)xmax << 16)) : 0xFFFFu, lm.count(), R.et[seg], R.ft[seg],
-                mm.count() + sm.count(), mm.count());
+        if (any.m) O.ext = (uint32_t)xmin | ((uint32_t)xmax << 16);
+        O.nrec = (uint32_t)lm.count();
+        O.items = (uint32_t)(mm.count() + sm.count());
+        O.merged = (uint32_t)mm.count();
     }
     __syncthreads();
-}
-
-__device__ __forceinline__ void segments_begin(RecLds &R) {
-    const int lane = threadIdx.x & 63;
-    if (lane < 4) R.et[lane] = R.ft[lane] = 0ull;
 }
 
 // One small bucket's records, loaded a bucket ahead of its resolve (the grid-stride loop
@@ -588,7 +603,7 @@ __device__ __forceinline__ void segments_begin(RecLds &R) {
 template <int NW>
 struct SmallIn {
     uint32_t meta, mk[NW];
-    uint32_t carry, path;
+    uint32_t carry;
     int rule, W;
 };
 
@@ -607,25 +622,21 @@ __device__ __forceinline__ void small_load(const ResolveArgs &A, uint32_t base, 
 
 // resolve_bucket<SPP, 1> with the records already in registers
 template <int SPP, bool KEEP>
-__device__ __forceinline__ void resolve_small(const ResolveArgs &A, int64_t b, uint32_t base, int n,
-                                              const SmallIn<Words<SPP>::n> &in, uint32_t *order, uint32_t *meta,
-                                              uint32_t *msk, RecLds &R) {
+__device__ __forceinline__ void resolve_small(const ResolveArgs &A, uint32_t base, int n,
+                                              const SmallIn<Words<SPP>::n> &in, uint32_t *key, uint32_t *order, uint32_t *meta,
+                                              uint32_t *msk, BucketOut &O) {
     constexpr int NW = Words<SPP>::n;
     const int lane = threadIdx.x & 63;
     uint32_t mykey = 0xFFFFFFFFu;
     if (lane < n) {
         meta[lane] = in.meta;
-#pragma unroll
-        for (int k = 0; k < NW; ++k) msk[lane * NW + k] = in.mk[k];
+        store_mask<NW>(msk, (size_t)lane, in.mk);
         mykey = ((in.meta & 0xFFFFu) << 10) | (uint32_t)lane;
     }
-    segments_begin(R);
-    int rk = 0;
-#pragma unroll 8
-    for (int j = 0; j < n; ++j) {
-        const uint32_t kj = (uint32_t)__builtin_amdgcn_readlane((int)mykey, j);
-        rk += (kj < mykey) ? 1 : 0;
-    }
+    key[lane] = mykey;
+    __syncthreads();
+    int rk;
+    rank_keys<1>(key, (n + 3) & ~3, &mykey, &rk);
     if (lane < n) order[rk] = (uint32_t)lane;
     __syncthreads();
 
@@ -651,7 +662,7 @@ __device__ __forceinline__ void resolve_small(const ResolveArgs &A, int64_t b, u
     const int prev_x = 2 * prev_cx - 2;
     Lane L;
     L.init(merged, head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at), p > 0, x, prev_x, W);
-    segment_emit<SPP, 64, KEEP>(A, true, b, base, in.path, L, res, R);
+    segment_emit<SPP, 64, KEEP>(A, true, base, L, res, O);
 }
 
 // Buckets of at most S (16 or 32) fragments, 64 / S of them in one wave: lane l works on
@@ -659,9 +670,9 @@ __device__ __forceinline__ void resolve_small(const ResolveArgs &A, int64_t b, u
 // (segmented DPP scans), so one pass resolves the whole pack.  ks[s] is the s-th bucket's
 // slot in the per-lane scalars (lane k holds bucket b0 + k G), -1 for an empty segment.
 template <int SPP, int S, bool KEEP>
-__device__ __forceinline__ void resolve_pack(const ResolveArgs &A, int64_t b0, int64_t G, const int *ks, int vbase,
-                                             int vend, int vcarry, int vrule, int vW, int vpath, uint32_t *order, uint32_t *meta,
-                                             uint32_t *msk, RecLds &R) {
+__device__ __forceinline__ void resolve_pack(const ResolveArgs &A, const int *ks, int vbase, int vend, int vcarry,
+                                             int vrule, int vW, uint32_t *key, uint32_t *order, uint32_t *meta, uint32_t *msk,
+                                             BucketOut *out) {
     constexpr int NW = Words<SPP>::n;
     constexpr int P = 64 / S;
     const int lane = threadIdx.x & 63;
@@ -678,7 +689,6 @@ __device__ __forceinline__ void resolve_pack(const ResolveArgs &A, int64_t b0, i
     const uint32_t wcarry = (uint32_t)__shfl(vcarry, src, 64);
     const int rule = __shfl(vrule, src, 64);
     const int W = __shfl(vW, src, 64);
-    const uint32_t path = (uint32_t)__shfl(vpath, src, 64);
     const int n = k < 0 ? 0 : end - (int)base;
     uint32_t mykey = 0xFFFFFFFFu;
     if (i < n) {
@@ -686,14 +696,13 @@ __device__ __forceinline__ void resolve_pack(const ResolveArgs &A, int64_t b0, i
         uint32_t mk[NW];
         load_mask<NW>(A.rec_mask, (size_t)base + i, mk);
         meta[lane] = m;
-#pragma unroll
-        for (int q = 0; q < NW; ++q) msk[lane * NW + q] = mk[q];
+        store_mask<NW>(msk, (size_t)lane, mk);
         mykey = ((m & 0xFFFFu) << 10) | (uint32_t)i;
     }
-    segments_begin(R);
-    int rk = 0;
-#pragma unroll
-    for (int j = 0; j < S; ++j) rk += ((uint32_t)__shfl((int)mykey, sb + j, 64) < mykey) ? 1 : 0;
+    key[lane] = mykey;
+    __syncthreads();
+    int rk;
+    rank_keys<1>(key + sb, S, &mykey, &rk);
     if (i < n) order[sb + rk] = (uint32_t)lane;  // LDS index of the record
     __syncthreads();
 
@@ -716,17 +725,22 @@ __device__ __forceinline__ void resolve_pack(const ResolveArgs &A, int64_t b0, i
     const int prev_x = 2 * prev_cx - 2;
     Lane L;
     L.init(merged, head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at), p > 0, x, prev_x, W);
-    segment_emit<SPP, S, KEEP>(A, k >= 0, b0 + (int64_t)(k < 0 ? 0 : k) * G, base, path, L, res, R);
+    segment_emit<SPP, S, KEEP>(A, k >= 0, base, L, res, out[src]);
 }
 
 // Every bucket: empty ones are cleared, buckets of at most 128 fragments are resolved,
 // larger ones are listed for the size-class passes below.  Five waves per SIMD: the records'
-// arithmetic spills at six (1.41 ms on the 2048x2048 illustration for 1.50; four: 1.50).
+// arithmetic spills at six.  On the 2048x2048 illustration (1.8 M buckets) 1.33 ms; writing each
+// bucket's results as it ends, 1.57, ranking by cross-lane reads, 1.37.
 template <int SPP, bool KEEP>
 __global__ void __launch_bounds__(64, 5) k_resolve_first(ResolveArgs A) {
     constexpr int NW = Words<SPP>::n;
-    __shared__ uint32_t key[128], order[128], meta[128], msk[128 * NW];
-    __shared__ RecLds R;
+    __shared__ __align__(16) uint32_t key[128], msk[128 * NW];
+    __shared__ uint32_t order[128], meta[128];
+    __shared__ unsigned long long ghead[2];
+    // results of the wave's 64 buckets, written together at the end: 64 lanes wait for their
+    // buckets' places and colours at once, where a lane a bucket would wait at each
+    __shared__ BucketOut out[64];
     const int lane = threadIdx.x;
     const int64_t G = gridDim.x;
     // Strided buckets keep the waves' loads balanced (a path's neighbouring rows have
@@ -737,14 +751,13 @@ __global__ void __launch_bounds__(64, 5) k_resolve_first(ResolveArgs A) {
         // vector loads, read back per bucket by readlane.  (Scalar loads would share the
         // LDS wait counter, so every LDS wait of a resolve would also wait for them.)
         const int64_t bl = b0 + (int64_t)lane * G;
-        int vbase = 0, vend = 0, vcarry = 0, vrule = 0, vW = A.W, vpath = 0;
+        int vbase = 0, vend = 0, vcarry = 0, vrule = 0, vW = A.W;
         if (bl < A.NB) {
             const int2 info = A.binfo[bl];
             vbase = (int)A.boff[bl];
             // the out-of-canvas bucket holds records only for the winding carry
             vend = info.y < 0 ? vbase : (int)A.boff[bl + 1];
             vrule = A.frule[info.x];
-            vpath = info.x;
             uint32_t carry = A.bcarry[bl];
             if (A.pcanvas) {
                 const int4 cv = A.pcanvas[info.x];
@@ -757,9 +770,12 @@ __global__ void __launch_bounds__(64, 5) k_resolve_first(ResolveArgs A) {
         const int nk = (int)(left < 64 ? left : 64);
         // buckets of up to 16 fragments four to a wave, of 17..32 two to a wave
         const int myn = lane < nk ? vend - vbase : -1;
+        out_clear(out[lane]);
+        __syncthreads();
+        if (myn > 128) A.big_list[atomicAdd(A.big_count, 1u)] = (uint32_t)bl;
         uint64_t m16 = __ballot(myn > 0 && myn <= 16);
         uint64_t m32 = __ballot(myn > 16 && myn <= 32);
-        uint64_t rest = __ballot(lane < nk) & ~(m16 | m32);
+        uint64_t rest = __ballot(myn > 32 && myn <= 128);
         while (m16) {
             int ks[4];
 #pragma unroll
@@ -767,7 +783,7 @@ __global__ void __launch_bounds__(64, 5) k_resolve_first(ResolveArgs A) {
                 ks[s] = m16 ? (int)__builtin_ctzll(m16) : -1;
                 m16 &= m16 - 1ull;
             }
-            resolve_pack<SPP, 16, KEEP>(A, b0, G, ks, vbase, vend, vcarry, vrule, vW, vpath, order, meta, msk, R);
+            resolve_pack<SPP, 16, KEEP>(A, ks, vbase, vend, vcarry, vrule, vW, key, order, meta, msk, out);
         }
         while (m32) {
             int ks[2];
@@ -776,7 +792,7 @@ __global__ void __launch_bounds__(64, 5) k_resolve_first(ResolveArgs A) {
                 ks[s] = m32 ? (int)__builtin_ctzll(m32) : -1;
                 m32 &= m32 - 1ull;
             }
-            resolve_pack<SPP, 32, KEEP>(A, b0, G, ks, vbase, vend, vcarry, vrule, vW, vpath, order, meta, msk, R);
+            resolve_pack<SPP, 32, KEEP>(A, ks, vbase, vend, vcarry, vrule, vW, key, order, meta, msk, out);
         }
         // the rest one by one, the next bucket's records loading during the current one
         SmallIn<NW> in0, in1;
@@ -796,125 +812,154 @@ __global__ void __launch_bounds__(64, 5) k_resolve_first(ResolveArgs A) {
                 small_load<NW>(A, (uint32_t)__builtin_amdgcn_readlane(vbase, kn),
                                (uint32_t)__builtin_amdgcn_readlane(vend, kn), in1);
             }
-            if (n == 0) {
-                if (lane == 0) put_row(A, b, base, 0u, 0xFFFFu, 0, 0ull, 0ull, 0, 0);
-            } else if (n > 128) {
-                if (lane == 0) A.big_list[atomicAdd(A.big_count, 1u)] = (uint32_t)b;
-            } else if (n > 64) {
-                resolve_bucket<SPP, 2, KEEP>(A, b, base, n, key, order, meta, msk, R);
+            if (n > 64) {
+                resolve_bucket<SPP, 2, KEEP>(A, b, base, n, key, order, meta, msk, ghead, out[k]);
             } else {
                 in0.carry = (uint32_t)__builtin_amdgcn_readlane(vcarry, k);
                 in0.rule = __builtin_amdgcn_readlane(vrule, k);
                 in0.W = __builtin_amdgcn_readlane(vW, k);
-                in0.path = (uint32_t)__builtin_amdgcn_readlane(vpath, k);
-                resolve_small<SPP, KEEP>(A, b, base, n, in0, order, meta, msk, R);
+                resolve_small<SPP, KEEP>(A, base, n, in0, key, order, meta, msk, out[k]);
             }
             in0 = in1;
         }
+        if (myn >= 0 && myn <= 128) {
+            const uint32_t path = (uint32_t)A.binfo[bl].x;
+            put_row(A, bl, A.rpos[bl], (uint32_t)vbase, path, A.finfo[path], out[lane]);
+        }
+        __syncthreads();
     }
 }
 
-// The listed buckets (more than 128 fragments), one per block, in one launch so that the
-// few long ones overlap: up to 1024 fragments staged in LDS, more in resolve_huge.
+// Waves of a block that resolves one listed bucket: they share the ranking, which compares every
+// record with every other (1024 batched scenes: 96 us a sample count, by a lone wave 121).
+constexpr int kBigWaves = 4, kBigThreads = 64 * kBigWaves;
+
 // Buckets of more than 1024 fragments (rare): bitonic-sort 64-bit (cell x, index) keys,
 // held in the bucket's stretch of the record array (4n words; the padded power of two is at
-// most 2n), copy the sorted indices into the scratch (the records are written next), then walk
-// the sorted order in chunks of 64 reading the fragments from global memory.  Any bucket
-// size works.
+// most 2n), copy the sorted indices into the scratch (the records are written next), then the
+// first wave walks the sorted order in chunks of 64 reading the fragments from global memory.
+// Any bucket size works.
 template <int SPP, bool KEEP>
-__device__ __noinline__ void resolve_huge(const ResolveArgs &A, int64_t b, uint32_t base, int n, RecLds &R) {
+__global__ void __launch_bounds__(kBigThreads) k_resolve_huge(ResolveArgs A) {
     constexpr int NW = Words<SPP>::n;
-    const int lane = threadIdx.x;
-    int P2 = 1;
-    while (P2 < n) P2 <<= 1;
-    uint32_t *khi = (uint32_t *)(A.prec + base);
-    uint32_t *klo = khi + P2;
-    for (int i = lane; i < P2; i += 64) {
-        khi[i] = (i < n) ? (A.rec_meta[base + i] & 0xFFFFu) : 0xFFFFFFFFu;
-        klo[i] = (i < n) ? (uint32_t)i : 0xFFFFFFFFu;
-    }
-    __syncthreads();
-    for (int k = 2; k <= P2; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = lane; i < P2; i += 64) {
-                const int l = i ^ j;
-                if (l > i) {
-                    const uint32_t ah = khi[i], al = klo[i], ch = khi[l], cl = klo[l];
-                    const bool gt = ah > ch || (ah == ch && al > cl);
-                    const bool up = (i & k) == 0;
-                    if (gt == up) {
-                        khi[i] = ch; klo[i] = cl;
-                        khi[l] = ah; klo[l] = al;
-                    }
-                }
-            }
-            __syncthreads();
-        }
-    }
-    uint32_t *order = A.scratch + base;
-    for (int i = lane; i < n; i += 64) order[i] = klo[i];
-    chunks_begin(R);
-    __syncthreads();
-    // sorted fragment indices; a fragment's cell x is in its record
-    auto cell_x = [&](int q) { return (int)(A.rec_meta[base + order[q]] & 0xFFFFu); };
-    const int rule = A.frule[A.binfo[b].x];
-    uint32_t wcarry = A.bcarry[b];
-    int W = A.W;
-    if (A.pcanvas) {
-        const int4 cv = A.pcanvas[A.binfo[b].x];
-        W = cv.x;
-        wcarry -= A.scarry[cv.w];
-    }
-    Chunks K;
-    for (int c0 = 0; c0 < n; c0 += 64) {
-        const int p = c0 + lane;
-        const bool v = p < n;
-        const uint32_t meta = v ? A.rec_meta[base + order[p]] : 0u;
-        const int cx = (int)(meta & 0xFFFFu);
-        const int swn = v ? (int)(int8_t)(meta >> 16) : 0;
-        const int prev_cx = (v && p > 0) ? cell_x(p - 1) : -1;
-        const bool head = v && (p == 0 || cx != prev_cx);
-        const int incl = scan_add(swn);
-        const int8_t w_at = (int8_t)(int)(wcarry + (uint32_t)(incl - swn));
-        wcarry += (uint32_t)lane63(incl);
-        const int x = 2 * cx - 2;
-        const bool merged = head && x >= 0 && x < W;
-        uint32_t res[NW];
-        if (merged) {
-            Stencil<NW> st;
-            st.init(w_at);
-            for (int q = p; q < n; ++q) {
-                const uint32_t j = order[q];
-                const uint32_t mq = A.rec_meta[base + j];
-                if ((int)(mq & 0xFFFFu) != cx) break;
-                uint32_t m2[NW];
-                load_mask<NW>(A.rec_mask, (size_t)base + j, m2);
-                st.add(m2, ((A.rec_meta[base + j] >> 24) & 1u) != 0u);
-            }
-            st.finish(rule, res);
-        }
-        const int prev_x = 2 * prev_cx - 2;
-        Lane L;
-        L.init(merged, head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at), p > 0, x, prev_x, W);
-        chunk_emit<SPP, KEEP>(A, base, L, res, R, K);
-    }
-    chunks_end(A, b, base, R, K);
-}
-
-template <int SPP, bool KEEP>
-__global__ void __launch_bounds__(64) k_resolve_big(ResolveArgs A) {
-    constexpr int NW = Words<SPP>::n;
-    __shared__ uint32_t key[64 * kBigStage], order[64 * kBigStage], meta[64 * kBigStage], msk[64 * kBigStage * NW];
-    __shared__ RecLds R;
+    __shared__ BucketOut O;
+    const int lane = threadIdx.x & 63, tid = threadIdx.x;
     const uint32_t nbig = *A.big_count;
     for (uint32_t bi = blockIdx.x; bi < nbig; bi += gridDim.x) {
         const int64_t b = A.big_list[bi];
         const uint32_t base = A.boff[b];
         const int n = (int)(A.boff[b + 1] - base);
-        if (n <= 256) resolve_bucket<SPP, 4, KEEP>(A, b, base, n, key, order, meta, msk, R);
-        else if (n <= 512) resolve_bucket<SPP, 8, KEEP>(A, b, base, n, key, order, meta, msk, R);
-        else if (n <= 64 * kBigStage) resolve_bucket<SPP, kBigStage, KEEP>(A, b, base, n, key, order, meta, msk, R);
-        else resolve_huge<SPP, KEEP>(A, b, base, n, R);
+        if (n <= 64 * kBigStage) continue;
+        if (tid == 0) out_clear(O);
+        int P2 = 1;
+        while (P2 < n) P2 <<= 1;
+        uint32_t *khi = (uint32_t *)(A.prec + base);
+        uint32_t *klo = khi + P2;
+        for (int i = tid; i < P2; i += kBigThreads) {
+            khi[i] = (i < n) ? (A.rec_meta[base + i] & 0xFFFFu) : 0xFFFFFFFFu;
+            klo[i] = (i < n) ? (uint32_t)i : 0xFFFFFFFFu;
+        }
+        __syncthreads();
+        for (int k = 2; k <= P2; k <<= 1) {
+            for (int j = k >> 1; j > 0; j >>= 1) {
+                for (int i = tid; i < P2; i += kBigThreads) {
+                    const int l = i ^ j;
+                    if (l > i) {
+                        const uint32_t ah = khi[i], al = klo[i], ch = khi[l], cl = klo[l];
+                        const bool gt = ah > ch || (ah == ch && al > cl);
+                        const bool up = (i & k) == 0;
+                        if (gt == up) {
+                            khi[i] = ch; klo[i] = cl;
+                            khi[l] = ah; klo[l] = al;
+                        }
+                    }
+                }
+                __syncthreads();
+            }
+        }
+        uint32_t *order = A.scratch + base;
+        for (int i = tid; i < n; i += kBigThreads) order[i] = klo[i];
+        __syncthreads();
+        if (tid < 64) {
+            // sorted fragment indices; a fragment's cell x is in its record
+            auto cell_x = [&](int q) { return (int)(A.rec_meta[base + order[q]] & 0xFFFFu); };
+            const int rule = A.frule[A.binfo[b].x];
+            uint32_t wcarry = A.bcarry[b];
+            int W = A.W;
+            if (A.pcanvas) {
+                const int4 cv = A.pcanvas[A.binfo[b].x];
+                W = cv.x;
+                wcarry -= A.scarry[cv.w];
+            }
+            Chunks K;
+            for (int c0 = 0; c0 < n; c0 += 64) {
+                const int p = c0 + lane;
+                const bool v = p < n;
+                const uint32_t meta = v ? A.rec_meta[base + order[p]] : 0u;
+                const int cx = (int)(meta & 0xFFFFu);
+                const int swn = v ? (int)(int8_t)(meta >> 16) : 0;
+                const int prev_cx = (v && p > 0) ? cell_x(p - 1) : -1;
+                const bool head = v && (p == 0 || cx != prev_cx);
+                const int incl = scan_add(swn);
+                const int8_t w_at = (int8_t)(int)(wcarry + (uint32_t)(incl - swn));
+                wcarry += (uint32_t)lane63(incl);
+                const int x = 2 * cx - 2;
+                const bool merged = head && x >= 0 && x < W;
+                uint32_t res[NW];
+                if (merged) {
+                    Stencil<NW> st;
+                    st.init(w_at);
+                    for (int q = p; q < n; ++q) {
+                        const uint32_t j = order[q];
+                        const uint32_t mq = A.rec_meta[base + j];
+                        if ((int)(mq & 0xFFFFu) != cx) break;
+                        uint32_t m2[NW];
+                        load_mask<NW>(A.rec_mask, (size_t)base + j, m2);
+                        st.add(m2, ((A.rec_meta[base + j] >> 24) & 1u) != 0u);
+                    }
+                    st.finish(rule, res);
+                }
+                const int prev_x = 2 * prev_cx - 2;
+                Lane L;
+                L.init(merged, head && p > 0 && (prev_x + 2 < x) && fill_test(rule, w_at), p > 0, x, prev_x, W);
+                chunk_emit<SPP, KEEP>(A, base, L, res, O, K);
+            }
+            chunks_end(A, base, O, K);
+        }
+        if (tid == 0) {
+            const uint32_t path = (uint32_t)A.binfo[b].x;
+            put_row(A, b, A.rpos[b], base, path, A.finfo[path], O);
+        }
+        __syncthreads();
+    }
+}
+
+// The listed buckets (more than 128 fragments), one per block, in one launch so that the
+// few long ones overlap: up to 1024 fragments staged in LDS, more in k_resolve_huge (a kernel of
+// its own: as a call from this one it cost 30 us of such a batch, for 4 us of a launch).
+template <int SPP, bool KEEP>
+__global__ void __launch_bounds__(kBigThreads) k_resolve_big(ResolveArgs A) {
+    constexpr int NW = Words<SPP>::n;
+    __shared__ __align__(16) uint32_t key[64 * kBigStage], msk[64 * kBigStage * NW];
+    __shared__ uint32_t order[64 * kBigStage], meta[64 * kBigStage];
+    __shared__ unsigned long long ghead[kBigStage];
+    __shared__ BucketOut out;
+    const uint32_t nbig = *A.big_count;
+    for (uint32_t bi = blockIdx.x; bi < nbig; bi += gridDim.x) {
+        const int64_t b = A.big_list[bi];
+        const uint32_t base = A.boff[b];
+        const int n = (int)(A.boff[b + 1] - base);
+        if (n > 64 * kBigStage) continue;  // k_resolve_huge's
+        if (threadIdx.x == 0) out_clear(out);
+        __syncthreads();
+        if (n <= 256) resolve_bucket<SPP, 1, KEEP, kBigWaves>(A, b, base, n, key, order, meta, msk, ghead, out);
+        else if (n <= 512) resolve_bucket<SPP, 2, KEEP, kBigWaves>(A, b, base, n, key, order, meta, msk, ghead, out);
+        else resolve_bucket<SPP, 4, KEEP, kBigWaves>(A, b, base, n, key, order, meta, msk, ghead, out);
+        if (threadIdx.x == 0) {
+            const uint32_t path = (uint32_t)A.binfo[b].x;
+            put_row(A, b, A.rpos[b], base, path, A.finfo[path], out);
+        }
+        __syncthreads();
     }
 }
 
@@ -993,11 +1038,6 @@ __device__ __forceinline__ float4 grad_color(const GradDev &G, uint32_t c, int x
     o.z = (t00.z * bu + t10.z * au) * bv + (t01.z * bu + t11.z * au) * av;
     o.w = (t00.w * bu + t10.w * au) * bv + (t01.w * bu + t11.w * au) * av;
     return o;
-}
-
-__device__ __forceinline__ void wave_sync_lds() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-    __builtin_amdgcn_wave_barrier();
 }
 
 // ---------------------------------------------------------------------------------
@@ -1965,7 +2005,8 @@ void launch_resolve(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t s
 #define SL_LAUNCH2(N, K)                                                              \
     do {                                                                              \
         hipLaunchKernelGGL((k_resolve_first<N, K>), dim3(g1), b64, 0, s, A);          \
-        hipLaunchKernelGGL((k_resolve_big<N, K>), dim3(gc), b64, 0, s, A);            \
+        hipLaunchKernelGGL((k_resolve_big<N, K>), dim3(gc), dim3(kBigThreads), 0, s, A); \
+        hipLaunchKernelGGL((k_resolve_huge<N, K>), dim3(1024), dim3(kBigThreads), 0, s, A); \
     } while (0)
 #define SL_LAUNCH(N)                                                                  \
     do {                                                                              \
