@@ -456,7 +456,7 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
     };
     mark(0);
     f.lcount = P_<uint32_t>(A.b_lcount);
-    sl::launch_frame_init(sc, f, s);  // path ranges, the status block, the work lists' counts
+    sl::launch_frame_init(sc, f, s);  // path ranges, the status block
     sl::launch_transform(sc, f, s);
     if ((rc = check_launch(h, "transform"))) return rc;
     mark(1);

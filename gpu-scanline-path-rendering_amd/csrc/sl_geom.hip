@@ -220,10 +220,9 @@ __global__ void __launch_bounds__(256) k_valu_probe(int iters, float seed, float
 // ------------------------------------------------------------------------------------
 // per-path init, vertex transform + region flags (k_transformVertex, .cu:36-105)
 // ------------------------------------------------------------------------------------
-__global__ void k_frame_init(uint32_t P, uint32_t *pflags, int2 *prow, uint32_t *small, uint32_t *lcount) {
+__global__ void k_frame_init(uint32_t P, uint32_t *pflags, int2 *prow, uint32_t *small) {
     uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p < kFrameStatusWords) small[p] = 0u;
-    if (p < kListCountBytes / 4) lcount[p] = 0u;
     if (p >= P) return;
     pflags[p] = 0u;
     prow[p] = make_int2(INT_MAX, INT_MIN);
@@ -258,9 +257,11 @@ __global__ void k_transform(uint32_t V, const float2 *__restrict__ vtx, const ui
 #pragma unroll
     for (int k = 0; k < 4; ++k)
         o[k] = M.m[4 * k + 0] * ix + M.m[4 * k + 1] * iy + M.m[4 * k + 2] * iz + M.m[4 * k + 3] * iw;
-    o[0] /= o[3];
-    o[1] /= o[3];
-    o[2] /= o[3];
+    if (o[3] != 1.f) {  // an affine transform's w: the quotients are the values themselves
+        o[0] /= o[3];
+        o[1] /= o[3];
+        o[2] /= o[3];
+    }
     const float w = (float)W, h = (float)H;
     const float z = (float)(W < H ? W : H);
     const float cutoff = -z * 0.5f;
@@ -282,11 +283,13 @@ __global__ void k_transform(uint32_t V, const float2 *__restrict__ vtx, const ui
         const uint32_t lp = (uint32_t)__builtin_amdgcn_readlane((int)p, leader);
         const bool mine = ((pend >> lane) & 1ull) && p == lp;
         const uint64_t grp = __ballot(mine);
-        // the group's OR of the eight region bits, one ballot a bit (scalar results, no
-        // cross-lane data movement)
-        uint32_t acc = 0u;
+        // the group's OR of the eight region bits: mostly the leader's own, else one ballot a
+        // bit (scalar results, no cross-lane data movement)
+        uint32_t acc = (uint32_t)__builtin_amdgcn_readlane((int)bits, leader);
+        if (__ballot(mine && bits != acc)) {
 #pragma unroll
-        for (int b = 0; b < 8; ++b) acc |= __ballot(mine && ((bits >> b) & 1u)) ? (1u << b) : 0u;
+            for (int b = 0; b < 8; ++b) acc |= __ballot(mine && ((bits >> b) & 1u)) ? (1u << b) : 0u;
+        }
         if (lane == leader) atomicOr(&pflags[lp], acc);
         pend &= ~grp;
     }
@@ -525,8 +528,11 @@ __global__ void __launch_bounds__(256) k_monotone(SceneDev sc, const float2 *__r
 // one thread that solves and walks both sides.  Chains and short pieces are grouped by
 // (cubic or closed-form solve, length bin), longest first, so the lanes of a wave run
 // loops of the same kind and about the same trip count and the long sequential walks
-// start early.  A count pass sizes the classes; the place pass puts every entry at its
-// class offset plus a rank taken per block in LDS and one reservation per class and block.
+// start early.  Blocks of a fixed number take runs of curves: a count pass leaves each block's
+// entries per class, and in the place pass every block sums the counts before its own (its
+// first place in each class) and hands out places with LDS atomics.  (With one device atomic
+// per class and block of 1024 curves instead, the two passes waited for the same hundred
+// addresses: 84 and 92 us on a sheet of 100000 glyph paths, now 40 and 61.)
 constexpr int kLenBins = 25;
 constexpr int kChainClasses = 2 * kLenBins;                     // cubic bins, then closed-form bins
 constexpr int kLongPieceClass = kChainClasses;                  // one class
@@ -534,7 +540,12 @@ constexpr int kShortClass0 = kChainClasses + 1;                 // cubic bins, t
 constexpr int kListClasses = kShortClass0 + 2 * kLenBins;
 constexpr uint32_t kLongPiece = 128;
 constexpr int kChainListThreads = 1024;
-static_assert(2 * kListClasses * sizeof(uint32_t) <= kListCountBytes, "class counts and cursors exceed their buffer");
+constexpr uint32_t kListBlocks = 512;
+// Frame::lcount: class counts, their exclusive sums over all classes (and the total), and, from
+// kListSolo, the block counts of a frame whose curves fit one block
+constexpr int kListPre = kListClasses, kListSolo = 256;
+static_assert(kListPre + kListClasses + 1 <= kListSolo && (kListSolo + kListClasses) * sizeof(uint32_t) <= kListCountBytes,
+              "class counts exceed their buffer");
 
 // Length bins, longest first.  Below 256 a bin's longest entry is at most 4/3 of its
 // shortest, so that the lanes of a wave run loops of nearly equal trip counts.  The bin
@@ -580,83 +591,97 @@ __device__ __forceinline__ void piece_classes(const CurvePieces &cp, int k, uint
     }
 }
 
-// class counts (cnt[kListClasses])
-__global__ void __launch_bounds__(kChainListThreads) k_list_count(SceneDev sc, uint32_t C,
+// blk[class * blocks + block]: the block's entries of the class; a block takes `per` curves
+__global__ void __launch_bounds__(kChainListThreads) k_list_count(SceneDev sc, uint32_t C, uint32_t per,
                                                                   const uint32_t *__restrict__ nchain,
                                                                   const uint32_t *__restrict__ pcnt, uint32_t cubic_min,
-                                                                  uint32_t *cnt) {
+                                                                  uint32_t *__restrict__ blk) {
     __shared__ uint32_t h[kListClasses];
     for (int q = threadIdx.x; q < kListClasses; q += blockDim.x) h[q] = 0u;
     __syncthreads();
-    const CurvePieces cp = curve_pieces(sc, C, blockIdx.x * blockDim.x + threadIdx.x, nchain, pcnt);
+    const uint32_t c0 = blockIdx.x * per, c1 = c0 + per < C ? c0 + per : C;
+    for (uint32_t c = c0 + threadIdx.x; c < c1; c += kChainListThreads) {
+        const CurvePieces cp = curve_pieces(sc, C, c, nchain, pcnt);
 #pragma unroll
-    for (int k = 0; k < 5; ++k) {
-        if (k >= cp.np) break;
-        int qx, qy, qp;
-        piece_classes(cp, k, cubic_min, qx, qy, qp);
-        if (qx >= 0) atomicAdd(&h[qx], 1u);
-        if (qy >= 0) atomicAdd(&h[qy], 1u);
-        atomicAdd(&h[qp], 1u);
+        for (int k = 0; k < 5; ++k) {
+            if (k >= cp.np) break;
+            int qx, qy, qp;
+            piece_classes(cp, k, cubic_min, qx, qy, qp);
+            if (qx >= 0) atomicAdd(&h[qx], 1u);
+            if (qy >= 0) atomicAdd(&h[qy], 1u);
+            atomicAdd(&h[qp], 1u);
+        }
     }
     __syncthreads();
-    for (int q = threadIdx.x; q < kListClasses; q += blockDim.x)
-        if (h[q]) atomicAdd(&cnt[q], h[q]);
+    for (int q = threadIdx.x; q < kListClasses; q += blockDim.x) blk[(size_t)q * gridDim.x + blockIdx.x] = h[q];
 }
 
-// lists from the counts; cursor[kListClasses] starts at zero
-__global__ void __launch_bounds__(kChainListThreads) k_list_place(SceneDev sc, uint32_t C,
+// lists from the block counts (at most kListBlocks); writes the class counts and their sums
+__global__ void __launch_bounds__(kChainListThreads) k_list_place(SceneDev sc, uint32_t C, uint32_t per,
                                                                   const uint32_t *__restrict__ nchain,
                                                                   const uint32_t *__restrict__ pcnt,
                                                                   const uint32_t *__restrict__ coff, uint32_t cubic_min,
-                                                                  const uint32_t *__restrict__ cnt, uint32_t *cursor,
-                                                                  uint4 *clist, uint4 *plist) {
-    __shared__ uint32_t h[kListClasses], base[kListClasses];
-    for (int q = threadIdx.x; q < kListClasses; q += blockDim.x) h[q] = 0u;
-    if (threadIdx.x == 0) {
-        // class offsets: within the chain list, and within the piece list (long pieces first)
-        uint32_t a = 0u;
-        for (int q = 0; q < kChainClasses; ++q) { base[q] = a; a += cnt[q]; }
-        a = 0u;
-        for (int q = kLongPieceClass; q < kListClasses; ++q) { base[q] = a; a += cnt[q]; }
+                                                                  const uint32_t *__restrict__ blk,
+                                                                  uint32_t *__restrict__ cnt, uint4 *clist, uint4 *plist) {
+    __shared__ uint32_t total[kListClasses], base[kListClasses];
+    constexpr int kWaves = kChainListThreads / 64;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint32_t nb = gridDim.x;
+#pragma unroll
+    for (int j = 0; j < (kListClasses + kWaves - 1) / kWaves; ++j) {
+        const int q = j * kWaves + w;
+        if (q >= kListClasses) break;
+        uint32_t tot = 0u, before = 0u;
+#pragma unroll
+        for (uint32_t i0 = 0; i0 < kListBlocks; i0 += 64) {
+            const uint32_t i = i0 + (uint32_t)lane;
+            const uint32_t v = i < nb ? blk[(size_t)q * nb + i] : 0u;
+            tot += v;
+            before += i < blockIdx.x ? v : 0u;
+        }
+        tot = (uint32_t)wave_reduce((int)tot, 0, OpAdd());
+        before = (uint32_t)wave_reduce((int)before, 0, OpAdd());
+        if (lane == 0) { total[q] = tot; base[q] = before; }
     }
     __syncthreads();
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    const CurvePieces cp = curve_pieces(sc, C, c, nchain, pcnt);
-    uint32_t rk[15];
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-        if (k >= cp.np) break;
-        int qx, qy, qp;
-        piece_classes(cp, k, cubic_min, qx, qy, qp);
-        rk[3 * k] = qx >= 0 ? atomicAdd(&h[qx], 1u) : 0u;
-        rk[3 * k + 1] = qy >= 0 ? atomicAdd(&h[qy], 1u) : 0u;
-        rk[3 * k + 2] = atomicAdd(&h[qp], 1u);
+    // class offsets: within the chain list, and within the piece list (long pieces first)
+    if (w < 2) {
+        const int q = w * kChainClasses + lane, n = w ? kListClasses - kChainClasses : kChainClasses;
+        const uint32_t v = lane < n ? total[q] : 0u, inc = wave_incl_scan(v);
+        if (lane < n) {
+            base[q] += inc - v;
+            if (blockIdx.x == 0) {
+                cnt[q] = v;
+                cnt[kListPre + q] = inc - v;
+                if (q == kListClasses - 1) cnt[kListPre + kListClasses] = inc;
+            }
+        }
     }
     __syncthreads();
-    for (int q = threadIdx.x; q < kListClasses; q += blockDim.x)
-        if (h[q]) base[q] += atomicAdd(&cursor[q], h[q]);
-    __syncthreads();
-    uint32_t off = cp.np ? coff[c] : 0u;
+    const uint32_t c0 = blockIdx.x * per, c1 = c0 + per < C ? c0 + per : C;
+    for (uint32_t c = c0 + threadIdx.x; c < c1; c += kChainListThreads) {
+        const CurvePieces cp = curve_pieces(sc, C, c, nchain, pcnt);
+        uint32_t off = cp.np ? coff[c] : 0u;
 #pragma unroll
-    for (int k = 0; k < 5; ++k) {
-        if (k >= cp.np) break;
-        int qx, qy, qp;
-        piece_classes(cp, k, cubic_min, qx, qy, qp);
-        // each entry carries its piece's ts offset and cut counts, so that the intersection
-        // passes read only the curve's record besides it
-        const uint32_t pb = off, pw = cp.pc[k];
-        off += 1u + (pw & 0xFFFFu) + (pw >> 16);
-        if (qx >= 0) clist[base[qx] + rk[3 * k]] = make_uint4((c << 4) | ((uint32_t)k << 1), pb, pw, 0u);
-        if (qy >= 0) clist[base[qy] + rk[3 * k + 1]] = make_uint4((c << 4) | ((uint32_t)k << 1) | 1u, pb, pw, 0u);
-        plist[base[qp] + rk[3 * k + 2]] = make_uint4((c << 3) | (uint32_t)k, pb, pw, 0u);
+        for (int k = 0; k < 5; ++k) {
+            if (k >= cp.np) break;
+            int qx, qy, qp;
+            piece_classes(cp, k, cubic_min, qx, qy, qp);
+            // each entry carries its piece's ts offset and cut counts, so that the intersection
+            // passes read only the curve's record besides it
+            const uint32_t pb = off, pw = cp.pc[k];
+            off += 1u + (pw & 0xFFFFu) + (pw >> 16);
+            if (qx >= 0) clist[atomicAdd(&base[qx], 1u)] = make_uint4((c << 4) | ((uint32_t)k << 1), pb, pw, 0u);
+            if (qy >= 0) clist[atomicAdd(&base[qy], 1u)] = make_uint4((c << 4) | ((uint32_t)k << 1) | 1u, pb, pw, 0u);
+            plist[atomicAdd(&base[qp], 1u)] = make_uint4((c << 3) | (uint32_t)k, pb, pw, 0u);
+        }
     }
 }
 
-// total entries of classes [q0, q1)
-__device__ __forceinline__ uint32_t class_total(const uint32_t *__restrict__ cnt, int q0, int q1) {
-    uint32_t t = 0u;
-    for (int q = q0; q < q1; ++q) t += cnt[q];
-    return t;
+// entries of the chain classes before q (q < kChainClasses), or of the piece list's before q
+__device__ __forceinline__ uint32_t class_start(const uint32_t *__restrict__ cnt, int q) { return cnt[kListPre + q]; }
+__device__ __forceinline__ uint32_t chain_total(const uint32_t *__restrict__ cnt) {
+    return cnt[kListPre + kChainClasses - 1] + cnt[kChainClasses - 1];
 }
 
 // t | flags of a monotone piece's end: low bits 2 when the end lies on an integral x,
@@ -1153,24 +1178,25 @@ __global__ void __launch_bounds__(256) k_chains(SceneDev sc, const float4 *__res
                                                  uint32_t wide_blocks, int wide_bins, uint32_t chain_blocks, int W, int H,
                                                  float *chain_t, int2 *ts) {
     if (blockIdx.x < wide_blocks) {
-        wide_chains(sc, crec, clist, class_total(cnt, 0, wide_bins), wide_blocks, W, H, chain_t);
+        wide_chains(sc, crec, clist, class_start(cnt, wide_bins), wide_blocks, W, H, chain_t);
         return;
     }
     const uint32_t blk = blockIdx.x - wide_blocks;
     if (blk < chain_blocks) {
         // the chains after those of the wide blocks
-        const uint32_t i = blk * blockDim.x + threadIdx.x + class_total(cnt, 0, wide_bins);
-        if (i >= class_total(cnt, 0, kChainClasses)) return;
+        const uint32_t i = blk * blockDim.x + threadIdx.x + class_start(cnt, wide_bins);
+        if (i >= chain_total(cnt)) return;
         solve_chain(sc, crec, clist[i], W, H, chain_t);
         return;
     }
     __shared__ uint32_t stage[4][kStageSteps * 64];
     const uint32_t g = (blk - chain_blocks) * blockDim.x + threadIdx.x;
-    const bool live = g < class_total(cnt, kShortClass0, kListClasses);
+    const uint32_t nlong = cnt[kLongPieceClass];
+    const bool live = g < cnt[kListPre + kListClasses] - nlong;
     if (!__ballot(live)) return;  // whole wave past the list
     PieceSetup p;
     if (live) {
-        const uint4 e = plist[cnt[kLongPieceClass] + g];
+        const uint4 e = plist[nlong + g];
         p = piece_setup(sc, crec, e.x >> 3, (int)(e.x & 7u), e, W, H);
     }
     walk_pieces_staged(p, live, ts, stage[threadIdx.x >> 6]);
@@ -1296,8 +1322,7 @@ void launch_fill_rows_u8(uint8_t *p, uint8_t v, size_t row_bytes, size_t pitch, 
 }
 
 void launch_frame_init(const SceneDev &sc, Frame &f, hipStream_t s) {
-    const uint32_t n = sc.P > kListCountBytes / 4 ? sc.P : (uint32_t)(kListCountBytes / 4);
-    hipLaunchKernelGGL(k_frame_init, dim3(blocks_for(n, 256)), dim3(256), 0, s, sc.P, f.pflags, f.prow, f.big_count, f.lcount);
+    hipLaunchKernelGGL(k_frame_init, dim3(std::max(1u, blocks_for(sc.P, 256))), dim3(256), 0, s, sc.P, f.pflags, f.prow, f.big_count);
 }
 
 void launch_transform(const SceneDev &sc, Frame &f, hipStream_t s) {
@@ -1316,7 +1341,7 @@ void launch_monotone(const SceneDev &sc, Frame &f, hipStream_t s) {
 
 void launch_intersect(const SceneDev &sc, Frame &f, hipStream_t s) {
     if (!sc.C) return;
-    uint32_t *cnt = f.lcount, *cursor = f.lcount + kListClasses;
+    uint32_t *cnt = f.lcount;
     // Cubic chains of the first wide_bins length bins take several lanes each (wide_chains): one
     // lane's 1.5 us a cut makes the longest chains the pass's time in frames of every size, but
     // the lanes cost up to 20 times the issue slots, so the more cuts a frame has, the fewer
@@ -1333,11 +1358,18 @@ void launch_intersect(const SceneDev &sc, Frame &f, hipStream_t s) {
     while (f.F > rule[at].cuts) ++at;
     const uint32_t cubic_min = rule[at].cubic_min;
     const int wide_bins = rule[at].bins;
-    const dim3 gl(blocks_for(sc.C, kChainListThreads)), bl(kChainListThreads);
-    hipLaunchKernelGGL(k_list_count, gl, bl, 0, s, sc, sc.C, (const uint32_t *)f.nchain, (const uint32_t *)f.pcnt, cubic_min,
-                       cnt);
-    hipLaunchKernelGGL(k_list_place, gl, bl, 0, s, sc, sc.C, (const uint32_t *)f.nchain, (const uint32_t *)f.pcnt,
-                       (const uint32_t *)f.coff, cubic_min, (const uint32_t *)cnt, cursor, f.chains, f.plist);
+    // the block counts lie in the chains' t array, written after the lists
+    const uint32_t tiles = blocks_for(sc.C, kChainListThreads);
+    uint32_t nb = std::min<uint32_t>(tiles, kListBlocks);
+    if ((int64_t)nb * kListClasses > f.F) nb = std::max<uint32_t>(1u, (uint32_t)(f.F / kListClasses));
+    const uint32_t per = (tiles + nb - 1) / nb * kChainListThreads;
+    nb = blocks_for(sc.C, per);
+    uint32_t *blk = nb == 1 ? f.lcount + kListSolo : (uint32_t *)f.chain_t;
+    const dim3 gl(nb), bl(kChainListThreads);
+    hipLaunchKernelGGL(k_list_count, gl, bl, 0, s, sc, sc.C, per, (const uint32_t *)f.nchain, (const uint32_t *)f.pcnt,
+                       cubic_min, blk);
+    hipLaunchKernelGGL(k_list_place, gl, bl, 0, s, sc, sc.C, per, (const uint32_t *)f.nchain, (const uint32_t *)f.pcnt,
+                       (const uint32_t *)f.coff, cubic_min, (const uint32_t *)blk, cnt, f.chains, f.plist);
     // chain blocks: enough for every chain; piece blocks: enough for every piece
     const uint32_t npieces = (uint32_t)(f.NCH / 2);
     const uint32_t chain_blocks = blocks_for(f.NCH, 256), piece_blocks = blocks_for(npieces, 256);
