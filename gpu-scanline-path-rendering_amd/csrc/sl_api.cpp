@@ -36,7 +36,7 @@ struct DevBuf {
 struct Arena {
     DevBuf b_pcnt, b_nchain, b_choff, b_chains, b_chain_t;
     DevBuf b_tvtx, b_pflags, b_prow, b_crec, b_cfrag, b_coff, b_ts, b_pbase, b_binfo, b_bcount,
-        b_boff, b_bwsum, b_bcarry, b_rec_meta, b_rec_mask, b_scratch, b_items, b_imask, b_icov, b_prec, b_bcnt, b_big_list, b_small, b_rpos, b_rowcnt, b_rowoff,
+        b_boff, b_bwsum, b_bcarry, b_rec, b_scratch, b_items, b_imask, b_icov, b_prec, b_bcnt, b_big_list, b_small, b_rpos, b_rowcnt, b_rowoff,
         b_rrec, b_rtile, b_rext, b_ptab, b_image, b_scan_tmp, b_lcount;
     // carving state: non-null base = every array comes from [base, base + cap)
     uint8_t *carve_base = nullptr;
@@ -514,12 +514,14 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
     f.NB = NB;
     if (!replay) h->NB = NB;
     const size_t R = (size_t)f.R;
+    // a meta word and the mask words of a fragment (Records)
+    const size_t rec_bytes = (((size_t)F + 3) & ~(size_t)3) * 4 + (size_t)F * 4 * NW;
     const size_t shares = f.rowshares = sl::row_shares(P, R, NB);
     scan_need = sl::scan_tmp_elems_needed(std::max<size_t>({(size_t)C + 1, (size_t)P + 1, (size_t)NB + 1, R * shares + 1}));
     if ((rc = ensure_in(h, A, A.b_binfo, (size_t)NB * 8)) || (rc = ensure_in(h, A, A.b_bcount, ((size_t)NB + 1) * 4)) ||
         (rc = ensure_in(h, A, A.b_boff, ((size_t)NB + 1) * 4)) || (rc = ensure_in(h, A, A.b_bwsum, ((size_t)NB + 1) * 4)) ||
         (rc = ensure_in(h, A, A.b_bcarry, ((size_t)NB + 1) * 4)) ||
-        (rc = ensure_in(h, A, A.b_rec_meta, (size_t)F * 4)) || (rc = ensure_in(h, A, A.b_rec_mask, (size_t)F * 4 * NW)) ||
+        (rc = ensure_in(h, A, A.b_rec, rec_bytes)) ||
         (rc = ensure_in(h, A, A.b_scratch, (size_t)F * 4)) || (rc = ensure_in(h, A, A.b_items, h->debug ? (size_t)F * 8 : 0)) ||
         (rc = ensure_in(h, A, A.b_imask, f.keep_masks ? (size_t)F * 4 * NW : 0)) || (rc = ensure_in(h, A, A.b_icov, (size_t)F * 4)) ||
         (rc = ensure_in(h, A, A.b_prec, (size_t)F * 16)) || (rc = ensure_in(h, A, A.b_bcnt, (size_t)NB * 8)) ||
@@ -531,7 +533,7 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
         return rc;
     f.binfo = P_<int2>(A.b_binfo); f.bcount = P_<uint32_t>(A.b_bcount); f.boff = P_<uint32_t>(A.b_boff);
     f.bwsum = P_<uint32_t>(A.b_bwsum); f.bcarry = P_<uint32_t>(A.b_bcarry);
-    f.rec_meta = P_<uint32_t>(A.b_rec_meta); f.rec_mask = P_<uint32_t>(A.b_rec_mask);
+    f.rec = P_<uint32_t>(A.b_rec);
     f.scratch_keys = P_<uint32_t>(A.b_scratch); f.items = h->debug ? P_<uint32_t>(A.b_items) : nullptr;
     f.imask = P_<uint32_t>(A.b_imask);
     f.icov = P_<uint32_t>(A.b_icov); f.prec = P_<uint4>(A.b_prec);
@@ -760,7 +762,7 @@ int sl_destroy(sl_handle *h) {
                       &h->simg, &h->sfirst, &h->scarry, &h->gramp, &h->gtable, &h->chord_keys, &h->A.b_pcnt,
                       &h->A.b_nchain, &h->A.b_choff, &h->A.b_chains, &h->A.b_chain_t, &h->A.b_tvtx, &h->A.b_pflags,
                       &h->A.b_prow, &h->A.b_crec, &h->A.b_cfrag, &h->A.b_coff, &h->A.b_ts, &h->A.b_pbase, &h->A.b_binfo,
-                      &h->A.b_bcount, &h->A.b_boff, &h->A.b_bwsum, &h->A.b_bcarry, &h->A.b_rec_meta, &h->A.b_rec_mask,
+                      &h->A.b_bcount, &h->A.b_boff, &h->A.b_bwsum, &h->A.b_bcarry, &h->A.b_rec,
                       &h->A.b_scratch, &h->A.b_items, &h->A.b_imask, &h->A.b_icov, &h->A.b_prec, &h->A.b_bcnt,
                       &h->A.b_big_list, &h->A.b_small, &h->A.b_rpos, &h->A.b_rowcnt, &h->A.b_rowoff,
                       &h->A.b_rrec, &h->A.b_rtile, &h->A.b_rext, &h->A.b_ptab, &h->A.b_image,

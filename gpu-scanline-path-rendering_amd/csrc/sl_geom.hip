@@ -307,8 +307,9 @@ struct Curve {
     float x0, x1, x2, x3, y0, y1, y2, y3;
 };
 
-// A curve and its monotone cuts from its 64-byte record (k_monotone writes it): one cache
-// line per curve for the intersection passes, whose work lists visit curves out of order.
+// A curve and its monotone cuts from its 64-byte record (k_monotone writes it): {x0, y0, x1, y1},
+// {x2, y2, x3, y3}, {cuts}, {type | cuts << 8, w, path, vertex order reversed}.  One cache line per
+// curve for the intersection passes, whose work lists visit curves out of order.
 struct CurveRec {
     Curve cu;
     float4 q;       // monotone cuts
@@ -480,7 +481,8 @@ __global__ void __launch_bounds__(256) k_monotone(SceneDev sc, const float2 *__r
         stg[4 * threadIdx.x] = make_float4(cu.x0, cu.y0, cu.x1, cu.y1);
         stg[4 * threadIdx.x + 1] = make_float4(cu.x2, cu.y2, cu.x3, cu.y3);
         stg[4 * threadIdx.x + 2] = make_float4(q0, q1, q2, q3);
-        stg[4 * threadIdx.x + 3] = make_float4(bf((uint32_t)cu.type | ((uint32_t)n << 8)), cu.w, bf(path), 0.f);
+        stg[4 * threadIdx.x + 3] = make_float4(bf((uint32_t)cu.type | ((uint32_t)n << 8)), cu.w, bf(path),
+                                               bf(sc.cinfo[c].z >> 8));
         uint32_t cnt = 0;
         uint32_t pc[5] = {0u, 0u, 0u, 0u, 0u};
         const int npieces = vis ? n + 1 : 0;

@@ -113,8 +113,7 @@ struct Frame {
     uint32_t *bwsum;         // [NB+1] per-bucket sum of scan windings -> bcarry
     uint32_t *bcarry;        // [NB+1]
     uint32_t *frank;         // [F] rank of each fragment in its bucket (~0: none)
-    uint32_t *rec_meta;      // [F] (valid fragments only are written)
-    uint32_t *rec_mask;      // [F * words]
+    uint32_t *rec;           // [F] fragment records (Records; valid fragments only are written)
     uint32_t *scratch_keys;  // [F] sorted fragment order of the largest buckets
     // resolve outputs, at each bucket's stretch of the fragments (see sl_resolve.hip)
     uint32_t *items;         // [2F] item lists (parity dumps only, else null)

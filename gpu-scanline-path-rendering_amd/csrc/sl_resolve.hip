@@ -189,8 +189,8 @@ struct ResolveArgs {
     const uint32_t *boff;
     const uint32_t *bcarry;
     const uint8_t *frule;
-    const uint32_t *rec_meta;
-    const uint32_t *rec_mask;
+    uint32_t *rec;
+    int64_t F;
     uint32_t *scratch;
     int W;
     const int4 *pcanvas;     // batched scenes: per-path canvas (W, H, row base, scene)
@@ -434,10 +434,9 @@ __device__ __forceinline__ void resolve_bucket(const ResolveArgs &A, int64_t b, 
         const int i = s * T + tid;
         mykey[s] = 0xFFFFFFFFu;
         if (i < n) {
-            const uint32_t m = A.rec_meta[base + i];
-            meta[i] = m;
             uint32_t mk[NW];
-            load_mask<NW>(A.rec_mask, (size_t)base + i, mk);
+            const uint32_t m = Records<NW>{A.rec, A.F}.load((size_t)base + i, mk);
+            meta[i] = m;
             store_mask<NW>(msk, (size_t)i, mk);
             mykey[s] = ((m & 0xFFFFu) << 10) | (uint32_t)i;
         }
@@ -615,8 +614,7 @@ __device__ __forceinline__ void small_load(const ResolveArgs &A, uint32_t base, 
 #pragma unroll
     for (int k = 0; k < NW; ++k) o.mk[k] = 0u;
     if (n > 0 && n <= 64 && lane < n) {
-        o.meta = A.rec_meta[base + lane];
-        load_mask<NW>(A.rec_mask, (size_t)base + lane, o.mk);
+        o.meta = Records<NW>{A.rec, A.F}.load((size_t)base + lane, o.mk);
     }
 }
 
@@ -692,9 +690,8 @@ __device__ __forceinline__ void resolve_pack(const ResolveArgs &A, const int *ks
     const int n = k < 0 ? 0 : end - (int)base;
     uint32_t mykey = 0xFFFFFFFFu;
     if (i < n) {
-        const uint32_t m = A.rec_meta[base + i];
         uint32_t mk[NW];
-        load_mask<NW>(A.rec_mask, (size_t)base + i, mk);
+        const uint32_t m = Records<NW>{A.rec, A.F}.load((size_t)base + i, mk);
         meta[lane] = m;
         store_mask<NW>(msk, (size_t)lane, mk);
         mykey = ((m & 0xFFFFu) << 10) | (uint32_t)i;
@@ -850,13 +847,14 @@ __global__ void __launch_bounds__(kBigThreads) k_resolve_huge(ResolveArgs A) {
         const uint32_t base = A.boff[b];
         const int n = (int)(A.boff[b + 1] - base);
         if (n <= 64 * kBigStage) continue;
+        const Records<NW> recs{A.rec, A.F};
         if (tid == 0) out_clear(O);
         int P2 = 1;
         while (P2 < n) P2 <<= 1;
         uint32_t *khi = (uint32_t *)(A.prec + base);
         uint32_t *klo = khi + P2;
         for (int i = tid; i < P2; i += kBigThreads) {
-            khi[i] = (i < n) ? (A.rec_meta[base + i] & 0xFFFFu) : 0xFFFFFFFFu;
+            khi[i] = (i < n) ? (recs.meta((size_t)base + i) & 0xFFFFu) : 0xFFFFFFFFu;
             klo[i] = (i < n) ? (uint32_t)i : 0xFFFFFFFFu;
         }
         __syncthreads();
@@ -882,7 +880,7 @@ __global__ void __launch_bounds__(kBigThreads) k_resolve_huge(ResolveArgs A) {
         __syncthreads();
         if (tid < 64) {
             // sorted fragment indices; a fragment's cell x is in its record
-            auto cell_x = [&](int q) { return (int)(A.rec_meta[base + order[q]] & 0xFFFFu); };
+            auto cell_x = [&](int q) { return (int)(recs.meta((size_t)base + order[q]) & 0xFFFFu); };
             const int rule = A.frule[A.binfo[b].x];
             uint32_t wcarry = A.bcarry[b];
             int W = A.W;
@@ -895,7 +893,7 @@ __global__ void __launch_bounds__(kBigThreads) k_resolve_huge(ResolveArgs A) {
             for (int c0 = 0; c0 < n; c0 += 64) {
                 const int p = c0 + lane;
                 const bool v = p < n;
-                const uint32_t meta = v ? A.rec_meta[base + order[p]] : 0u;
+                const uint32_t meta = v ? recs.meta((size_t)base + order[p]) : 0u;
                 const int cx = (int)(meta & 0xFFFFu);
                 const int swn = v ? (int)(int8_t)(meta >> 16) : 0;
                 const int prev_cx = (v && p > 0) ? cell_x(p - 1) : -1;
@@ -911,11 +909,10 @@ __global__ void __launch_bounds__(kBigThreads) k_resolve_huge(ResolveArgs A) {
                     st.init(w_at);
                     for (int q = p; q < n; ++q) {
                         const uint32_t j = order[q];
-                        const uint32_t mq = A.rec_meta[base + j];
-                        if ((int)(mq & 0xFFFFu) != cx) break;
                         uint32_t m2[NW];
-                        load_mask<NW>(A.rec_mask, (size_t)base + j, m2);
-                        st.add(m2, ((A.rec_meta[base + j] >> 24) & 1u) != 0u);
+                        const uint32_t mq = recs.load((size_t)base + j, m2);
+                        if ((int)(mq & 0xFFFFu) != cx) break;
+                        st.add(m2, ((mq >> 24) & 1u) != 0u);
                     }
                     st.finish(rule, res);
                 }
@@ -1992,7 +1989,7 @@ void launch_resolve(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t s
     if (!f.NB) return;
     ResolveArgs A;
     A.NB = f.NB; A.binfo = f.binfo; A.boff = f.boff; A.bcarry = f.bcarry; A.frule = sc.frule;
-    A.rec_meta = f.rec_meta; A.rec_mask = f.rec_mask; A.scratch = f.scratch_keys; A.W = f.W;
+    A.rec = f.rec; A.F = f.F; A.scratch = f.scratch_keys; A.W = f.W;
     A.pcanvas = sc.pcanvas; A.scarry = f.scarry;
     // the merged masks feed the multisample compositor and the debug draw list; the
     // coverage compositor reads only the per-pixel sample counts
