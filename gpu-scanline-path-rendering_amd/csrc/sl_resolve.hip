@@ -507,7 +507,7 @@ __device__ __forceinline__ void resolve_bucket(const ResolveArgs &A, int64_t b, 
     chunks_end(A, base, O, K);
 }
 
-constexpr int kResolveBlocks = 65536;
+constexpr int64_t kResolveWaves = 10240;  // at least this many waves (see launch_resolve)
 
 // A wave-wide ballot as seen by a lane of a segment of S lanes: its segment's bits, bit i the
 // segment's i-th lane.  Packed segments lie in one half of the ballot, so 32 bits do.
@@ -1996,7 +1996,14 @@ void launch_resolve(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t s
     A.items = f.items; A.imask = f.imask; A.icov = f.icov; A.prec = f.prec;
     A.rpos = f.rpos; A.finfo = sc.finfo; A.rext = f.rext; A.rrec = f.rrec; A.rtile = f.rtile; A.bcnt = f.bcnt;
     A.big_list = f.big_list; A.big_count = f.big_count; A.err = f.err_flag;  // cleared at the frame's start
-    const unsigned g1 = (unsigned)std::min<int64_t>(f.NB, f.resolve_grid > 0 ? f.resolve_grid : kResolveBlocks);
+    // A wave resolves up to 64 buckets of the grid's stride: with fewer its packs of four and two
+    // small buckets stay part empty and every bucket pays for a wave's start and end, but below
+    // twice the 5120 resident waves the last ones leave the chip idle.  One bucket a wave up
+    // to 65536 waves, then shared / this, us: 47 k buckets 42 / 22, 57 k (a page of text) 62 / 32,
+    // a poster 152 / 107, 1.9 M 434 / 426, 1.8 M (the illustration) 1325 / 1304; at least 5120
+    // waves 20 / 29 / 111, 15360 25 / 34 / 109, at most 96 buckets 438 and 1364.
+    const int64_t gd = std::max((f.NB + 63) / 64, kResolveWaves);
+    const unsigned g1 = (unsigned)std::min<int64_t>(f.NB, f.resolve_grid > 0 ? f.resolve_grid : gd);
     const unsigned gc = f.class_grid > 0 ? (unsigned)f.class_grid : 4096u;
     dim3 b64(64);
 #define SL_LAUNCH2(N, K)                                                              \
