@@ -119,10 +119,6 @@ __device__ __forceinline__ void emit(const ChordScene &S, uint32_t cl, uint32_t 
         S.vpath[vl + k] = path;
     }
     S.ctype[cl] = (uint8_t)nv;
-    S.cvpos[cl] = vp;
-    S.cpath[cl] = path;
-    S.cw[cl] = -1.f;
-    S.crev[cl] = rev ? 1 : 0;
     S.cinfo[cl] = make_uint4(vp, path, (uint32_t)nv | ((rev ? 1u : 0u) << 8), __float_as_uint(-1.f));
 }
 
@@ -217,10 +213,9 @@ __global__ void __launch_bounds__(64) k_chord_frame(ChordLaunch L, uint32_t P, C
     __shared__ float2 s_vtx[kGenPaths * 24];
     __shared__ uint32_t s_vpath[kGenPaths * 24];
     __shared__ uint4 s_cinfo[kGenPaths * 6];
-    __shared__ uint32_t s_cvpos[kGenPaths * 6], s_cpath[kGenPaths * 6], s_finfo[kGenPaths];
-    __shared__ float s_cw[kGenPaths * 6];
-    __shared__ uint8_t s_ctype[kGenPaths * 6], s_crev[kGenPaths * 6], s_frule[kGenPaths];
-    const ChordScene S{s_vtx, s_vpath, s_cvpos, s_cpath, s_finfo, s_ctype, s_frule, s_crev, s_cw, s_cinfo};
+    __shared__ uint32_t s_finfo[kGenPaths];
+    __shared__ uint8_t s_ctype[kGenPaths * 6], s_frule[kGenPaths];
+    const ChordScene S{s_vtx, s_vpath, s_finfo, s_ctype, s_frule, s_cinfo};
     const uint32_t p0 = blockIdx.x * kGenPaths, pl = threadIdx.x, path = p0 + pl;
     if (path < P) {
         uint32_t base = 0;
@@ -245,11 +240,7 @@ __global__ void __launch_bounds__(64) k_chord_frame(ChordLaunch L, uint32_t P, C
     for (uint32_t k = threadIdx.x; k < 6u * np; k += kGenPaths) {
         const uint32_t c = 6u * p0 + k;
         G.cinfo[c] = s_cinfo[k];
-        G.cvpos[c] = s_cvpos[k];
-        G.cpath[c] = s_cpath[k];
-        G.cw[c] = s_cw[k];
         G.ctype[c] = s_ctype[k];
-        G.crev[c] = s_crev[k];
     }
     if (pl < np) {
         G.frule[path] = s_frule[pl];

@@ -445,7 +445,7 @@ __global__ void __launch_bounds__(256) k_monotone(SceneDev sc, const float2 *__r
     uint32_t path = 0u;
     if (live) {
         Curve cu = load_curve(sc, tv, c);
-        path = sc.cpath[c];
+        path = sc.cinfo[c].y;
         vis = region_visible(pflags[path]);
         path_canvas(sc, path, W, H);
         float tq[4] = {0.f, 0.f, 0.f, 0.f};

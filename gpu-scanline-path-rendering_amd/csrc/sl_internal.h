@@ -22,13 +22,9 @@ struct SceneDev {
     uint32_t P, C, V;
     const float2 *vtx;       // [V] vertices in unified (orientation-fixed) order
     const uint32_t *vpath;   // [V] owning path of each vertex
-    const uint32_t *cvpos;   // [C]
     const uint8_t *ctype;    // [C]
-    const uint32_t *cpath;   // [C]
-    const float *cw;         // [C] rational weight (else -1)
-    const uint8_t *crev;     // [C] 1 = vertex order was reversed at upload
-    const uint4 *cinfo;      // [C] the same per curve in one record: {vertex pos, path,
-                             //     type | reversed << 8, rational weight bits}
+    const uint4 *cinfo;      // [C] {vertex pos, path, type | reversed << 8 (the vertex order was
+                             //     reversed at upload), rational weight bits (else -1)}
     const uint8_t *frule;    // [P]
     const uint32_t *finfo;   // [P] fill_info (RGBA8, alpha 0 -> 0)
     const int4 *pcanvas;     // [P] batched scenes: {W, H, first cell row, scene} of the
@@ -202,9 +198,8 @@ struct ChordInterval {
 // the scene arrays a frame writes (6 curves and 24 vertex slots per path)
 struct ChordScene {
     float2 *vtx;
-    uint32_t *vpath, *cvpos, *cpath, *finfo;
-    uint8_t *ctype, *frule, *crev;
-    float *cw;
+    uint32_t *vpath, *finfo;
+    uint8_t *ctype, *frule;
     uint4 *cinfo;
 };
 float chord_ease(int time_ms);
