@@ -72,7 +72,7 @@ struct sl_handle {
     int64_t batch_rows = 0, batch_tiles = 0, batch_image_bytes = 0;
     DevBuf pcanvas, stile, simg, sfirst, scarry;
     // launch shape (results do not depend on it)
-    int resolve_grid = 0, class_grid = 0, comp_group = 4, frag_block = 256;
+    int resolve_grid = 0, class_grid = 0, frag_block = 256;
     // sizes of the last eager render; a replay of the same scene reuses them
     bool sized = false;
     uint32_t last_F = 0, last_NCH = 0, last_NB = 0;
@@ -423,7 +423,7 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
     f.sfirst = P_<uint32_t>(h->sfirst);
     f.scarry = P_<uint32_t>(h->scarry);
     f.resolve_grid = h->resolve_grid; f.class_grid = h->class_grid;
-    f.comp_group = h->comp_group; f.frag_block = h->frag_block;
+    f.frag_block = h->frag_block;
     const size_t image_bytes = h->nscenes ? (size_t)h->batch_image_bytes : (size_t)h->H * f.pitch;
 
     size_t scan_need = sl::scan_tmp_elems_needed((size_t)std::max(C, P) + 1);
@@ -1582,7 +1582,6 @@ void apply_shape(sl_batch *b) {
     for (sl_handle *h : b->grp) {
         h->resolve_grid = b->shape[0];
         h->class_grid = b->shape[1];
-        h->comp_group = b->shape[2];
         h->frag_block = b->shape[3];
     }
 }
@@ -1794,11 +1793,11 @@ int sl_batch_tune(sl_batch *b, int reps, double *best_ms) {
     if (reps <= 0) reps = 3;
     if (hipSetDevice(b->device) != hipSuccess) return bfail(b, SL_E_HIP, "hipSetDevice failed");
     if (int rc0 = batch_settle(b)) return rc0;
-    // candidate launch shapes: per-bucket resolve grid, size-class grid, compositor
-    // bucket group, fragment block size
-    const int rg[] = {4096, 16384, 65536};
+    // candidate launch shapes: per-bucket resolve grid (0: by the bucket count), size-class
+    // grid, fragment block size; the third word, a group size that the compositors do not
+    // have any more, keeps its value
+    const int rg[] = {0, 16384, 65536};
     const int cg[] = {1024, 4096};
-    const int gg[] = {4};
     const int fbk[] = {128, 256};
     hipEvent_t e0, e1;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
@@ -1808,24 +1807,23 @@ int sl_batch_tune(sl_batch *b, int reps, double *best_ms) {
     int rc = SL_OK;
     for (int a : rg)
         for (int c : cg)
-            for (int g : gg)
-                for (int f : fbk) {
-                    if (rc) break;
-                    b->shape[0] = a; b->shape[1] = c; b->shape[2] = g; b->shape[3] = f;
-                    apply_shape(b);
-                    rc = enqueue_all(b, b->cap_stream, true);  // warm-up
-                    if (rc) break;
-                    (void)hipEventRecord(e0, b->cap_stream);
-                    for (int r = 0; r < reps && !rc; ++r) rc = enqueue_all(b, b->cap_stream, true);
-                    (void)hipEventRecord(e1, b->cap_stream);
-                    if (hipEventSynchronize(e1) != hipSuccess) rc = bfail(b, SL_E_HIP, "tuning run failed");
-                    float ms = 0.f;
-                    (void)hipEventElapsedTime(&ms, e0, e1);
-                    if (!rc && ms / reps < best) {
-                        best = ms / reps;
-                        best_shape[0] = a; best_shape[1] = c; best_shape[2] = g; best_shape[3] = f;
-                    }
+            for (int f : fbk) {
+                if (rc) break;
+                b->shape[0] = a; b->shape[1] = c; b->shape[3] = f;
+                apply_shape(b);
+                rc = enqueue_all(b, b->cap_stream, true);  // warm-up
+                if (rc) break;
+                (void)hipEventRecord(e0, b->cap_stream);
+                for (int r = 0; r < reps && !rc; ++r) rc = enqueue_all(b, b->cap_stream, true);
+                (void)hipEventRecord(e1, b->cap_stream);
+                if (hipEventSynchronize(e1) != hipSuccess) rc = bfail(b, SL_E_HIP, "tuning run failed");
+                float ms = 0.f;
+                (void)hipEventElapsedTime(&ms, e0, e1);
+                if (!rc && ms / reps < best) {
+                    best = ms / reps;
+                    best_shape[0] = a; best_shape[1] = c; best_shape[3] = f;
                 }
+            }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     for (int i = 0; i < 4; ++i) b->shape[i] = best_shape[i];

@@ -135,7 +135,7 @@ struct Frame {
     const uint32_t *sfirst;
     uint32_t *scarry;
     // launch shape (autotuned for batches; results do not depend on it)
-    int resolve_grid, class_grid, comp_group, frag_block;
+    int resolve_grid, class_grid, frag_block;
     uint32_t *rext;          // [NB] row-list extents
     uint4 *rrec;             // [NB] row-list records {colour, records, base, path}
     ulonglong2 *rtile;       // [NB] row-list tile bitmaps {with a record, inside a span}

@@ -302,9 +302,9 @@ int sl_debug_valu_probe(sl_handle *h, int blocks, int iters, double *ms, uint64_
  * sl_batch_create uploads and orients every scene (as sl_add_vg), renders one eager
  * frame to size the buffers, and captures the graph.  sl_batch_render replays it on
  * `stream`; sl_batch_render_eager issues the same kernels without the graph.
- * sl_batch_tune times candidate launch shapes {per-bucket resolve grid, size-class
- * grid, compositor bucket group, fragment block size} on this batch, keeps the fastest
- * and recaptures.  Images are read per scene.  A frame issued on another stream than the
+ * sl_batch_tune times candidate launch shapes {per-bucket resolve grid (0: by the bucket
+ * count), size-class grid, 4, fragment block size} on this batch, keeps the fastest and
+ * recaptures (the third word, 4 or 8, was a compositor's group size and selects nothing).  Images are read per scene.  A frame issued on another stream than the
  * previous one waits on the device for everything queued on that stream up to the call
  * (the previous frame and the caller's reads of its images); tuning, a shape change and
  * the read-back wait for it on the host. */
