@@ -543,11 +543,9 @@ constexpr int kListClasses = kShortClass0 + 2 * kLenBins;
 constexpr uint32_t kLongPiece = 128;
 constexpr int kChainListThreads = 1024;
 constexpr uint32_t kListBlocks = 512;
-// Frame::lcount: class counts, their exclusive sums over all classes (and the total), and, from
-// kListSolo, the block counts of a frame whose curves fit one block
-constexpr int kListPre = kListClasses, kListSolo = 256;
-static_assert(kListPre + kListClasses + 1 <= kListSolo && (kListSolo + kListClasses) * sizeof(uint32_t) <= kListCountBytes,
-              "class counts exceed their buffer");
+// Frame::lcount: class counts, then their exclusive sums over all classes and the total
+constexpr int kListPre = kListClasses;
+static_assert((kListPre + kListClasses + 1) * sizeof(uint32_t) <= kListCountBytes, "class counts exceed their buffer");
 
 // Length bins, longest first.  Below 256 a bin's longest entry is at most 4/3 of its
 // shortest, so that the lanes of a wave run loops of nearly equal trip counts.  The bin
@@ -593,15 +591,10 @@ __device__ __forceinline__ void piece_classes(const CurvePieces &cp, int k, uint
     }
 }
 
-// blk[class * blocks + block]: the block's entries of the class; a block takes `per` curves
-__global__ void __launch_bounds__(kChainListThreads) k_list_count(SceneDev sc, uint32_t C, uint32_t per,
-                                                                  const uint32_t *__restrict__ nchain,
-                                                                  const uint32_t *__restrict__ pcnt, uint32_t cubic_min,
-                                                                  uint32_t *__restrict__ blk) {
-    __shared__ uint32_t h[kListClasses];
-    for (int q = threadIdx.x; q < kListClasses; q += blockDim.x) h[q] = 0u;
-    __syncthreads();
-    const uint32_t c0 = blockIdx.x * per, c1 = c0 + per < C ? c0 + per : C;
+// adds the classes of curves [c0, c1) to h
+__device__ __forceinline__ void count_classes(const SceneDev &sc, uint32_t C, uint32_t c0, uint32_t c1,
+                                              const uint32_t *__restrict__ nchain, const uint32_t *__restrict__ pcnt,
+                                              uint32_t cubic_min, uint32_t *h) {
     for (uint32_t c = c0 + threadIdx.x; c < c1; c += kChainListThreads) {
         const CurvePieces cp = curve_pieces(sc, C, c, nchain, pcnt);
 #pragma unroll
@@ -614,11 +607,25 @@ __global__ void __launch_bounds__(kChainListThreads) k_list_count(SceneDev sc, u
             atomicAdd(&h[qp], 1u);
         }
     }
+}
+
+// blk[class * blocks + block]: the block's entries of the class; a block takes `per` curves
+__global__ void __launch_bounds__(kChainListThreads) k_list_count(SceneDev sc, uint32_t C, uint32_t per,
+                                                                  const uint32_t *__restrict__ nchain,
+                                                                  const uint32_t *__restrict__ pcnt, uint32_t cubic_min,
+                                                                  uint32_t *__restrict__ blk) {
+    __shared__ uint32_t h[kListClasses];
+    for (int q = threadIdx.x; q < kListClasses; q += blockDim.x) h[q] = 0u;
+    __syncthreads();
+    const uint32_t c0 = blockIdx.x * per, c1 = c0 + per < C ? c0 + per : C;
+    count_classes(sc, C, c0, c1, nchain, pcnt, cubic_min, h);
     __syncthreads();
     for (int q = threadIdx.x; q < kListClasses; q += blockDim.x) blk[(size_t)q * gridDim.x + blockIdx.x] = h[q];
 }
 
-// lists from the block counts (at most kListBlocks); writes the class counts and their sums
+// Lists from the block counts (at most kListBlocks); writes the class counts and their sums.
+// SOLO: one block, which counts for itself first.
+template <bool SOLO>
 __global__ void __launch_bounds__(kChainListThreads) k_list_place(SceneDev sc, uint32_t C, uint32_t per,
                                                                   const uint32_t *__restrict__ nchain,
                                                                   const uint32_t *__restrict__ pcnt,
@@ -628,22 +635,28 @@ __global__ void __launch_bounds__(kChainListThreads) k_list_place(SceneDev sc, u
     __shared__ uint32_t total[kListClasses], base[kListClasses];
     constexpr int kWaves = kChainListThreads / 64;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const uint32_t nb = gridDim.x;
+    if (SOLO) {
+        for (int q = threadIdx.x; q < kListClasses; q += kChainListThreads) total[q] = base[q] = 0u;
+        __syncthreads();
+        count_classes(sc, C, 0u, C, nchain, pcnt, cubic_min, total);
+    } else {
+        const uint32_t nb = gridDim.x;
 #pragma unroll
-    for (int j = 0; j < (kListClasses + kWaves - 1) / kWaves; ++j) {
-        const int q = j * kWaves + w;
-        if (q >= kListClasses) break;
-        uint32_t tot = 0u, before = 0u;
+        for (int j = 0; j < (kListClasses + kWaves - 1) / kWaves; ++j) {
+            const int q = j * kWaves + w;
+            if (q >= kListClasses) break;
+            uint32_t tot = 0u, before = 0u;
 #pragma unroll
-        for (uint32_t i0 = 0; i0 < kListBlocks; i0 += 64) {
-            const uint32_t i = i0 + (uint32_t)lane;
-            const uint32_t v = i < nb ? blk[(size_t)q * nb + i] : 0u;
-            tot += v;
-            before += i < blockIdx.x ? v : 0u;
+            for (uint32_t i0 = 0; i0 < kListBlocks; i0 += 64) {
+                const uint32_t i = i0 + (uint32_t)lane;
+                const uint32_t v = i < nb ? blk[(size_t)q * nb + i] : 0u;
+                tot += v;
+                before += i < blockIdx.x ? v : 0u;
+            }
+            tot = (uint32_t)wave_reduce((int)tot, 0, OpAdd());
+            before = (uint32_t)wave_reduce((int)before, 0, OpAdd());
+            if (lane == 0) { total[q] = tot; base[q] = before; }
         }
-        tot = (uint32_t)wave_reduce((int)tot, 0, OpAdd());
-        before = (uint32_t)wave_reduce((int)before, 0, OpAdd());
-        if (lane == 0) { total[q] = tot; base[q] = before; }
     }
     __syncthreads();
     // class offsets: within the chain list, and within the piece list (long pieces first)
@@ -1360,18 +1373,26 @@ void launch_intersect(const SceneDev &sc, Frame &f, hipStream_t s) {
     while (f.F > rule[at].cuts) ++at;
     const uint32_t cubic_min = rule[at].cubic_min;
     const int wide_bins = rule[at].bins;
-    // the block counts lie in the chains' t array, written after the lists
-    const uint32_t tiles = blocks_for(sc.C, kChainListThreads);
-    uint32_t nb = std::min<uint32_t>(tiles, kListBlocks);
+    // One block, for up to 1024 curves, counts and places by itself: 9.6 us for the two launches'
+    // 13.6 with 91 curves, but with 1591 25 for 21.  More blocks leave their counts in the chains'
+    // t array, written after the lists; where that is too short, fewer blocks take more curves.
+    const dim3 bl(kChainListThreads);
+    uint32_t nb = std::min<uint32_t>(blocks_for(sc.C, kChainListThreads), kListBlocks);
     if ((int64_t)nb * kListClasses > f.F) nb = std::max<uint32_t>(1u, (uint32_t)(f.F / kListClasses));
-    const uint32_t per = (tiles + nb - 1) / nb * kChainListThreads;
+    const uint32_t per = blocks_for(blocks_for(sc.C, kChainListThreads), nb) * kChainListThreads;
     nb = blocks_for(sc.C, per);
-    uint32_t *blk = nb == 1 ? f.lcount + kListSolo : (uint32_t *)f.chain_t;
-    const dim3 gl(nb), bl(kChainListThreads);
-    hipLaunchKernelGGL(k_list_count, gl, bl, 0, s, sc, sc.C, per, (const uint32_t *)f.nchain, (const uint32_t *)f.pcnt,
-                       cubic_min, blk);
-    hipLaunchKernelGGL(k_list_place, gl, bl, 0, s, sc, sc.C, per, (const uint32_t *)f.nchain, (const uint32_t *)f.pcnt,
-                       (const uint32_t *)f.coff, cubic_min, (const uint32_t *)blk, cnt, f.chains, f.plist);
+    uint32_t *blk = (uint32_t *)f.chain_t;
+    if (nb == 1) {
+        hipLaunchKernelGGL(k_list_place<true>, dim3(1), bl, 0, s, sc, sc.C, per, (const uint32_t *)f.nchain,
+                           (const uint32_t *)f.pcnt, (const uint32_t *)f.coff, cubic_min, (const uint32_t *)nullptr, cnt,
+                           f.chains, f.plist);
+    } else {
+        hipLaunchKernelGGL(k_list_count, dim3(nb), bl, 0, s, sc, sc.C, per, (const uint32_t *)f.nchain,
+                           (const uint32_t *)f.pcnt, cubic_min, blk);
+        hipLaunchKernelGGL(k_list_place<false>, dim3(nb), bl, 0, s, sc, sc.C, per, (const uint32_t *)f.nchain,
+                           (const uint32_t *)f.pcnt, (const uint32_t *)f.coff, cubic_min, (const uint32_t *)blk, cnt,
+                           f.chains, f.plist);
+    }
     // chain blocks: enough for every chain; piece blocks: enough for every piece
     const uint32_t npieces = (uint32_t)(f.NCH / 2);
     const uint32_t chain_blocks = blocks_for(f.NCH, 256), piece_blocks = blocks_for(npieces, 256);

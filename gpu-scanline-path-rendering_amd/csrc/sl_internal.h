@@ -69,7 +69,7 @@ struct GradDev {
 };
 
 // bytes of the intersection work lists' class counts (Frame::lcount)
-constexpr size_t kListCountBytes = 2048;
+constexpr size_t kListCountBytes = 1024;
 // words of the frame's status block: big-bucket count, error flags, -, -, then the 64-bit
 // merged-cell and item totals (Frame::big_count)
 constexpr uint32_t kFrameStatusWords = 8;
@@ -94,8 +94,8 @@ struct Frame {
     uint4 *plist;            // [NCH/2] pieces: long ones, then short ones grouped by class;
                              //   entries {curve << 4 | piece << 1 | side (chains) or curve << 3 |
                              //   piece, ts offset of the piece, nx | ny << 16, 0}
-    uint32_t *lcount;        // class counts (50 chain, 1 long-piece, 50 short-piece classes),
-                             //   their sums, one block's counts (see sl_geom.hip)
+    uint32_t *lcount;        // class counts (50 chain, 1 long-piece, 50 short-piece classes) and
+                             //   their sums (see sl_geom.hip)
     int64_t NCH;
     float *chain_t;          // [F] solved t | side per chain
     // fragments
