@@ -541,6 +541,7 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
     f.bcnt = P_<uint2>(A.b_bcnt);
     f.big_list = P_<uint32_t>(A.b_big_list); f.rpos = P_<uint32_t>(A.b_rpos);
     f.rowcnt = P_<uint32_t>(A.b_rowcnt); f.rowoff = P_<uint32_t>(A.b_rowoff);
+    f.rowstart = shares > 1 ? f.rowcnt : f.rowoff;
     f.rrec = P_<uint4>(A.b_rrec);
     f.rtile = P_<ulonglong2>(A.b_rtile);
     f.rext = P_<uint32_t>(A.b_rext);

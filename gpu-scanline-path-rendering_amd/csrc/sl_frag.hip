@@ -373,15 +373,22 @@ __global__ void __launch_bounds__(256) k_row_count(RowLists L, uint32_t *__restr
     if (row < L.R) cnt[(size_t)row * L.S + s] = n;
 }
 
-// Writes, per bucket: its path and row, its place in the row lists, cleared counters.
+// Writes, per bucket: its path and row, its place in the row lists, cleared counters; per row,
+// where its list starts (rowstart[R + 1], null when `off` itself is that: the compositors' waves
+// read it first, and over `off` its words would lie `shares` apart, a line a row: 428 us for 389
+// of compositing a sheet of 100000 glyph paths).
 __global__ void __launch_bounds__(256) k_row_place(RowLists L, const uint32_t *__restrict__ off,
                                                    const uint32_t *__restrict__ pbase, int2 *__restrict__ binfo,
                                                    uint32_t *__restrict__ rpos, uint32_t *__restrict__ bcount,
-                                                   uint32_t *__restrict__ bwsum) {
+                                                   uint32_t *__restrict__ bwsum, uint32_t *__restrict__ rowstart) {
     const uint32_t wave = blockIdx.x * 4u + (threadIdx.x >> 6), g = wave / L.S, s = wave - g * L.S;
     const uint32_t row = g * 64u + (threadIdx.x & 63);
     if (g * 64u >= L.R) return;
     uint32_t pos = row < L.R ? off[(size_t)row * L.S + s] : 0u;
+    if (rowstart && s == 0 && row < L.R) {
+        rowstart[row] = pos;
+        if (row == L.R - 1u) rowstart[L.R] = off[(size_t)L.R * L.S];
+    }
     for_paths<true>(L, pbase, g, s, [&](uint32_t p, int2 pr, int r, bool in, uint32_t pb) {
         if (!in) return;
         const uint32_t b = pb + (uint32_t)(r > 0 ? r - path_first_row(pr) : path_rows_above(pr) + 1);
@@ -642,7 +649,7 @@ void launch_row_lists(const SceneDev &sc, Frame &f, hipStream_t s) {
     hipLaunchKernelGGL(k_row_count, dim3(blocks), dim3(256), 0, s, L, f.rowcnt);
     scan_exclusive_u32(f.rowcnt, f.rowoff, (size_t)f.R * L.S, f.scan_tmp, s);
     hipLaunchKernelGGL(k_row_place, dim3(blocks), dim3(256), 0, s, L, (const uint32_t *)f.rowoff, (const uint32_t *)f.pbase,
-                       f.binfo, f.rpos, f.bcount, f.bwsum);
+                       f.binfo, f.rpos, f.bcount, f.bwsum, L.S > 1 ? f.rowcnt : nullptr);
 }
 
 void launch_frag_count(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t s) {

@@ -123,8 +123,9 @@ struct Frame {
     // row lists (see sl_frag.hip)
     uint32_t *rpos;          // [NB] a bucket's place in the row lists
     uint32_t *rowcnt;        // [R * shares] paths per row and share
-    uint32_t *rowoff;        // [R * shares + 1]; row r's list: [rowoff[r shares], rowoff[(r + 1) shares])
+    uint32_t *rowoff;        // [R * shares + 1] their exclusive sums
     uint32_t rowshares;
+    const uint32_t *rowstart;  // [R + 1] where the rows' lists start: over rowcnt, or rowoff if shares is 1
     int64_t R;               // cell rows (of all scenes of a batch)
     // batched scenes (nscenes > 0): per scene {W, H, first tile, first cell row}, image
     // byte offsets, first path, and the winding-scan carry at its first bucket

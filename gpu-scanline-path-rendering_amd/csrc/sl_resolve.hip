@@ -727,8 +727,9 @@ __device__ __forceinline__ void resolve_pack(const ResolveArgs &A, const int *ks
 
 // Every bucket: empty ones are cleared, buckets of at most 128 fragments are resolved,
 // larger ones are listed for the size-class passes below.  Five waves per SIMD: the records'
-// arithmetic spills at six.  On the 2048x2048 illustration (1.8 M buckets) 1.33 ms; writing each
-// bucket's results as it ends, 1.57, ranking by cross-lane reads, 1.37.
+// arithmetic spills at six.  On the 2048x2048 illustration (1.8 M buckets) 1.30 ms; writing each
+// bucket's results as it ends, 1.57, ranking by cross-lane reads, 1.37, one pack's records
+// loaded ahead of their turn, 1.52.
 template <int SPP, bool KEEP>
 __global__ void __launch_bounds__(64, 5) k_resolve_first(ResolveArgs A) {
     constexpr int NW = Words<SPP>::n;
@@ -1116,8 +1117,7 @@ __device__ __forceinline__ uint32_t pack_dec(const float4 *step, const float *d)
 
 struct CovArgs {
     int W, H, tiles_x;
-    const uint32_t *rowoff;  // row r: [rowoff[r shares], rowoff[(r + 1) shares])
-    uint32_t rowshares;
+    const uint32_t *rowstart;
     const uint32_t *rext;       // per row-list entry: extent
     const uint4 *rrec;          //   colour, records, base, path
     const ulonglong2 *rtile;    //   tiles with a record, tiles inside a span
@@ -1333,7 +1333,7 @@ __device__ __forceinline__ void list_row(const CovArgs &A, uint32_t q0, uint32_t
 // sample counts load during them).  Seven waves per SIMD (batches six, gradients four): six
 // and eight take 1.34 and 1.40 ms for 1.27 on the 2048x2048 illustration.  Finding a column's
 // covering item by LDS slots and a max-scan per bucket, in groups of four buckets: 2.01 ms
-// there, 543 us for 325 on a 4096x4096 sheet of glyphs, 154 for 23 on a 512x512 drawing of
+// there, 543 us for 389 on a 4096x4096 sheet of glyphs, 154 for 23 on a 512x512 drawing of
 // opaque cubic chains, 2.5 ms for 0.81 on 1024 such scenes in a batch.
 template <int SPP, bool SRGB, bool BATCH, bool GRAD>
 __global__ void __launch_bounds__(256, GRAD ? 4 : (BATCH ? 6 : 7)) k_composite_cov(CovArgs A) {
@@ -1450,8 +1450,7 @@ __global__ void __launch_bounds__(256, GRAD ? 4 : (BATCH ? 6 : 7)) k_composite_c
         wave_sync_lds();
     };
 
-    const uint32_t *ro = A.rowoff + (size_t)(row0 + r) * A.rowshares;
-    const uint32_t q0 = ro[0], q1 = ro[A.rowshares];
+    const uint32_t q0 = A.rowstart[row0 + r], q1 = A.rowstart[row0 + r + 1];
     list_row<GRAD>(A, q0, q1, tx, tx1, kInvN, s_dec, l_queue[w], l_src[w], l_ent[w], l_grad[GRAD ? w : 0], flush);
 
     if (x >= W) return;
@@ -1815,8 +1814,7 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
         }
     };
 
-    const uint32_t *ro = A.rowoff + (size_t)r * A.rowshares;
-    const uint32_t q0 = ro[0], q1 = ro[A.rowshares];
+    const uint32_t q0 = A.rowstart[r], q1 = A.rowstart[r + 1];
     list_row<GRAD>(A, q0, q1, tx, tx1, 1.f, s_dec, l_queue[w], l_src[w], l_ent[w], l_grad[GRAD ? w : 0], flush);
 
     // resolve: G registers at a time are staged in this wave's slot rows (G x 64 words);
@@ -2037,7 +2035,7 @@ void launch_composite(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t
     if (!f.ms) {
         CovArgs C;
         C.W = f.W; C.H = f.H; C.tiles_x = tiles_x;
-        C.rowoff = f.rowoff; C.rowshares = f.rowshares; C.rext = f.rext; C.rrec = f.rrec; C.rtile = f.rtile;
+        C.rowstart = f.rowstart; C.rext = f.rext; C.rrec = f.rrec; C.rtile = f.rtile;
         C.prec = f.prec; C.icov = f.icov; C.imask = nullptr; C.ptab = nullptr; C.dec_c = t.dec_c; C.dec_a = t.dec_a; C.step_c = t.step_c;
         C.image = f.image; C.pitch = f.pitch;
         C.G = f.grad;
@@ -2064,7 +2062,7 @@ void launch_composite(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t
     }
     CovArgs C;
     C.W = f.W; C.H = f.H; C.tiles_x = tiles_x;
-    C.rowoff = f.rowoff; C.rowshares = f.rowshares; C.rext = f.rext; C.rrec = f.rrec; C.rtile = f.rtile;
+    C.rowstart = f.rowstart; C.rext = f.rext; C.rrec = f.rrec; C.rtile = f.rtile;
     C.prec = f.prec; C.icov = f.icov; C.imask = f.imask; C.ptab = f.ptab;
     C.dec_c = t.dec_c; C.dec_a = t.dec_a; C.step_c = t.step_c;
     C.image = f.image; C.pitch = f.pitch;
