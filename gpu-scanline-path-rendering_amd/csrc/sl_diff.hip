@@ -257,7 +257,9 @@ __device__ __forceinline__ int wave_scan_add(int x) { return sl::dev::dpp_scan(x
 // its winding is the sum of the directions of the bucket's crossings before it (no sorted
 // order is stored), the fill change follows, and the area right of the crossing goes into
 // the row's pixels as a second difference -- turn (p + 1 - u) at its pixel p, the rest of
-// turn at p + 1 -- so that a running sum over x gives every pixel's coverage.  The sums are
+// turn at p + 1 -- so that a running sum over x gives every pixel's coverage.  Right of a
+// bucket's last crossing nothing is filled, also where its winding does not return to zero
+// (open contours: points that moved one segment at a time).  The sums are
 // 32-bit fixed point, 2^-25 of a sample row: the atomics' order does not matter, the two
 // parts of a crossing add to exactly one, and a pixel's sum (at most 64 rows) fits 32 bits.
 // A crossing costs one pass over its bucket and two LDS adds, where integrating every
@@ -268,9 +270,15 @@ constexpr int kFillStage = 128;   // crossings of a row staged in LDS (more are 
 constexpr int kFillPixels = 512;  // pixel columns of one pass over a row
 constexpr float kAreaScale = 33554432.f;  // 2^25
 
+// What k_d_fill keeps of a crossing: the fill's change (left - right, by the windings) for the
+// adjoint, and the coverage's (right - left, with nothing after the last crossing).
+__device__ __forceinline__ uint8_t turn_code(int change, int turn) { return (uint8_t)((change + 1) | ((turn + 1) << 2)); }
+__device__ __forceinline__ int code_change(uint8_t c) { return (int)(c & 3) - 1; }
+__device__ __forceinline__ int code_turn(uint8_t c) { return (int)(c >> 2) - 1; }
+
 __global__ void __launch_bounds__(256) k_d_fill(DiffDev D, const uint32_t *__restrict__ boff,
                                                 const uint32_t *__restrict__ order, const Cross *__restrict__ xs,
-                                                int8_t *df, float *__restrict__ cov) {
+                                                uint8_t *df, float *__restrict__ cov) {
     __shared__ uint4 s_cr[4][kFillStage];       // {x key, curve, t bits, index << 1 | dir}
     __shared__ uint32_t s_sum[4][kFillPixels];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -305,16 +313,20 @@ __global__ void __launch_bounds__(256) k_d_fill(DiffDev D, const uint32_t *__res
                 const uint32_t a0 = boff[b] - r0, a1 = boff[b + 1] - r0;
                 const uint32_t kx = order_key(c.x), kt = __float_as_uint(c.t);
                 int w = 0;
+                uint32_t left = a1 - a0 - 1u;  // crossings that come after this one
                 for (uint32_t m = a0; m < a1; ++m) {
                     const uint4 q = m < nst ? cr[m] : load(m);
-                    if (comes_before(q.x, q.y, q.z, q.w >> 1, kx, c.curve, kt, i & 0x7FFFFFFFu))
+                    if (comes_before(q.x, q.y, q.z, q.w >> 1, kx, c.curve, kt, i & 0x7FFFFFFFu)) {
                         w += (q.w & 1u) ? 1 : -1;
+                        --left;
+                    }
                 }
                 const int d = (c.row_dir & 1u) ? 1 : -1;
-                turn = (filled(rule, w + d) ? 1 : 0) - (filled(rule, w) ? 1 : 0);
-                df[i] = (int8_t)-turn;
+                const int in0 = filled(rule, w) ? 1 : 0, in1 = filled(rule, w + d) ? 1 : 0;
+                turn = (left ? in1 : 0) - in0;
+                df[i] = turn_code(in0 - in1, turn);
             } else {
-                turn = -(int)df[i];  // written by this lane in the first pass
+                turn = code_turn(df[i]);  // written by this lane in the first pass
             }
             if (!turn) continue;
             const float u = fminf(fmaxf(c.x, 0.f), Wf);
@@ -456,7 +468,7 @@ __global__ void __launch_bounds__(256) k_d_back_pixels(DiffDev D, const float *_
 // result.  861 k crossings of 384 curves: 19 us, bound by the gathers of gcov; one atomic
 // per crossing, point and coordinate took 500 us, some 2200 of them meeting at each address.
 __global__ void __launch_bounds__(64) k_d_back_cross(DiffDev D, const uint32_t *__restrict__ off,
-                                                     const Cross *__restrict__ xs, const int8_t *__restrict__ df,
+                                                     const Cross *__restrict__ xs, const uint8_t *__restrict__ df,
                                                      const float2 *__restrict__ pts, const float *__restrict__ gcov,
                                                      unsigned long long *gpts) {
     const uint32_t c = blockIdx.x;
@@ -468,7 +480,7 @@ __global__ void __launch_bounds__(64) k_d_back_cross(DiffDev D, const uint32_t *
     long long sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     const int nv = g.type & 7;
     for (uint32_t i = i0 + blockIdx.y * 64u + threadIdx.x; i < i1; i += 64u * gridDim.y) {
-        const int f = df[i];
+        const int f = code_change(df[i]);
         if (!f) continue;
         const Cross cr = xs[i];
         if (!(cr.x >= 0.f && cr.x < (float)D.W)) continue;
@@ -696,7 +708,7 @@ int sl_diff_forward(sl_diff *d, const float *points, const float *colors, float 
     }
     hipLaunchKernelGGL(k_d_fill, dim3(nblk((int64_t)d->P * d->H, 4)), dim3(256), 0, s, D,
                        (const uint32_t *)BP<uint32_t>(d->boff), (const uint32_t *)BP<uint32_t>(d->order),
-                       (const Cross *)BP<Cross>(d->xs), BP<int8_t>(d->df), BP<float>(d->cov));
+                       (const Cross *)BP<Cross>(d->xs), BP<uint8_t>(d->df), BP<float>(d->cov));
     float4 *pre = nullptr;
     if (keep_for_backward) {
         if ((rc = dens(d, d->pre, (size_t)d->P * NP * 16))) return rc;
@@ -730,7 +742,7 @@ int sl_diff_backward(sl_diff *d, const float *grad_image, float *grad_points, fl
                        BP<float>(d->gcov), fix_col);
     if (d->NX) {
         hipLaunchKernelGGL(k_d_back_cross, dim3(d->C, shares_of(d->NX, d->C)), dim3(64), 0, s, D, (const uint32_t *)BP<uint32_t>(d->off),
-                           (const Cross *)BP<Cross>(d->xs), (const int8_t *)BP<int8_t>(d->df),
+                           (const Cross *)BP<Cross>(d->xs), (const uint8_t *)BP<uint8_t>(d->df),
                            (const float2 *)d->last_points, (const float *)BP<float>(d->gcov), fix_pts);
     }
     hipLaunchKernelGGL(k_d_unfix, dim3(256), dim3(256), 0, s, (const long long *)fix_pts, grad_points, npt);
