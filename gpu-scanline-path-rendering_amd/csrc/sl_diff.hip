@@ -237,8 +237,9 @@ __global__ void k_d_scatter(uint32_t NX, const uint32_t *__restrict__ key, const
 __device__ __forceinline__ bool filled(int rule, int w) { return rule ? (w & 1) != 0 : w != 0; }
 
 // Order of a bucket's crossings: (x, curve, t, index), x as an unsigned key that orders like
-// the float (NaN last, -0 and +0 equal), so the order is total whatever the values.
+// the float (every NaN last, -0 and +0 equal), so the order is total whatever the values.
 __device__ __forceinline__ uint32_t order_key(float x) {
+    if (x != x) return 0xFFFFFFFFu;
     const uint32_t u = __float_as_uint(x + 0.f);
     return u ^ ((u >> 31) ? 0xFFFFFFFFu : 0x80000000u);
 }
@@ -329,7 +330,9 @@ __global__ void __launch_bounds__(256) k_d_fill(DiffDev D, const uint32_t *__res
                 turn = code_turn(df[i]);  // written by this lane in the first pass
             }
             if (!turn) continue;
-            const float u = fminf(fmaxf(c.x, 0.f), Wf);
+            // a crossing without a position, last in the order, lies at the right edge: the
+            // positions then never decrease along the order, and a row fills no pixel twice
+            const float u = c.x < Wf ? fmaxf(c.x, 0.f) : Wf;
             const int px = (int)floorf(u);
             const int v = (int)rintf(((float)(px + 1) - u) * kAreaScale);
             const uint32_t va = (uint32_t)(turn * v), vb = (uint32_t)(turn * ((int)kAreaScale - v));
