@@ -263,6 +263,9 @@ __device__ __forceinline__ int wave_scan_add(int x) { return sl::dev::dpp_scan(x
 // (open contours: points that moved one segment at a time).  The sums are
 // 32-bit fixed point, 2^-25 of a sample row: the atomics' order does not matter, the two
 // parts of a crossing add to exactly one, and a pixel's sum (at most 64 rows) fits 32 bits.
+// From x = 1/4 on a float's fraction is a multiple of 2^-25, so the sums are exact; what a
+// crossing left of that has below, only column 0 feels, and the lanes keep it in registers in
+// units of 2^-56 (slivers of 2^-32 of a pixel keep a float's precision).
 // A crossing costs one pass over its bucket and two LDS adds, where integrating every
 // interval over every pixel column cost each column a pass over the whole row's crossings.
 // 861 k crossings (64 paths at 256x256, 16 rows): 25 us, where sorting the buckets and the
@@ -270,6 +273,7 @@ __device__ __forceinline__ int wave_scan_add(int x) { return sl::dev::dpp_scan(x
 constexpr int kFillStage = 128;   // crossings of a row staged in LDS (more are read from memory)
 constexpr int kFillPixels = 512;  // pixel columns of one pass over a row
 constexpr float kAreaScale = 33554432.f;  // 2^25
+constexpr float kRestScale = 2147483648.f;  // 2^31: the rest's units in one of the area's
 
 // What k_d_fill keeps of a crossing: the fill's change (left - right, by the windings) for the
 // adjoint, and the coverage's (right - left, with nothing after the last crossing).
@@ -305,6 +309,7 @@ __global__ void __launch_bounds__(256) k_d_fill(DiffDev D, const uint32_t *__res
         for (int k = lane; k < kFillPixels; k += 64) sum[k] = 0u;
         __syncthreads();
         uint32_t carry = 0u;  // what lies left of this pass's columns
+        long long rest = 0;   // what column 0 has below the sums' unit, taken off
         for (uint32_t k = lane; k < n; k += 64) {
             const uint32_t i = order[r0 + k];
             const Cross c = xs[i];
@@ -334,8 +339,10 @@ __global__ void __launch_bounds__(256) k_d_fill(DiffDev D, const uint32_t *__res
             // positions then never decrease along the order, and a row fills no pixel twice
             const float u = c.x < Wf ? fmaxf(c.x, 0.f) : Wf;
             const int px = (int)floorf(u);
-            const int v = (int)rintf(((float)(px + 1) - u) * kAreaScale);
-            const uint32_t va = (uint32_t)(turn * v), vb = (uint32_t)(turn * ((int)kAreaScale - v));
+            const float at = (u - (float)px) * kAreaScale, part = rintf(at);  // exact but for the rounding
+            if (px == 0) rest += turn * __float2ll_rn((at - part) * kRestScale);
+            const int v = (int)kAreaScale - (int)part;
+            const uint32_t va = (uint32_t)(turn * v), vb = (uint32_t)(turn * (int)part);
             const int q = px - x0;
             if (q < 0) carry += va;
             else if (q < kFillPixels) atomicAdd(&sum[q], va);
@@ -345,10 +352,18 @@ __global__ void __launch_bounds__(256) k_d_fill(DiffDev D, const uint32_t *__res
         __syncthreads();
         carry = (uint32_t)__builtin_amdgcn_readlane(wave_scan_add((int)carry), 63);
         const int xe = tmn(D.W - x0, kFillPixels);
+        const bool fine = x0 == 0 && __ballot(rest != 0);
+        if (fine) {
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) rest += __shfl_xor(rest, d, 64);
+        }
         for (int k0 = 0; k0 < xe; k0 += 64) {
             const uint32_t s = (uint32_t)wave_scan_add((int)sum[k0 + lane]) + carry;
             carry = (uint32_t)__builtin_amdgcn_readlane((int)s, 63);
-            if (live && k0 + lane < xe) row[x0 + k0 + lane] = (float)s * (1.f / kAreaScale) / (float)D.S;
+            float c = (float)s * (1.f / kAreaScale);
+            if (fine && k0 + lane == 0)  // at most 2^62
+                c = (float)((long long)((unsigned long long)s << 31) - rest) * (1.f / kAreaScale / kRestScale);
+            if (live && k0 + lane < xe) row[x0 + k0 + lane] = c / (float)D.S;
         }
         __syncthreads();
     }
