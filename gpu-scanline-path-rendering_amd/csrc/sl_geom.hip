@@ -1374,14 +1374,16 @@ void launch_intersect(const SceneDev &sc, Frame &f, hipStream_t s) {
     const uint32_t cubic_min = rule[at].cubic_min;
     const int wide_bins = rule[at].bins;
     // One block, for up to 1024 curves, counts and places by itself: 9.6 us for the two launches'
-    // 13.6 with 91 curves, but with 1591 25 for 21.  More blocks leave their counts in the chains'
-    // t array, written after the lists; where that is too short, fewer blocks take more curves.
+    // 13.6 with 91 curves, but with 1591 25 for 21.  More blocks leave their counts in the curves'
+    // fragment counts, which their scan was the last to read: 101 words a block for a word a curve,
+    // so they fit however few cuts the frame has.  (With the blocks cut down to the chains' t
+    // array, a view of 154 cuts of a sheet of 6.2 M curves took 5.7 ms for the stage, now 37 us.)
     const dim3 bl(kChainListThreads);
     uint32_t nb = std::min<uint32_t>(blocks_for(sc.C, kChainListThreads), kListBlocks);
-    if ((int64_t)nb * kListClasses > f.F) nb = std::max<uint32_t>(1u, (uint32_t)(f.F / kListClasses));
     const uint32_t per = blocks_for(blocks_for(sc.C, kChainListThreads), nb) * kChainListThreads;
     nb = blocks_for(sc.C, per);
-    uint32_t *blk = (uint32_t *)f.chain_t;
+    static_assert(2 * kListClasses <= kChainListThreads, "the block counts exceed the curves' words");
+    uint32_t *blk = f.cfrag;
     if (nb == 1) {
         hipLaunchKernelGGL(k_list_place<true>, dim3(1), bl, 0, s, sc, sc.C, per, (const uint32_t *)f.nchain,
                            (const uint32_t *)f.pcnt, (const uint32_t *)f.coff, cubic_min, (const uint32_t *)nullptr, cnt,

@@ -84,8 +84,8 @@ struct Frame {
     float4 *crec;            // [4C] per curve, one 64-byte record read by the intersection
                              //   passes: {x0, y0, x1, y1}, {x2, y2, x3, y3} (transformed),
                              //   the monotone cuts {t0..t3}, {type | cut count << 8, weight
-                             //   bits, path, 0}
-    uint32_t *cfrag;         // [C+1]  -> exclusive offsets after scan
+                             //   bits, path, vertex order reversed}
+    uint32_t *cfrag;         // [C+1] fragments per curve -> coff; then the work lists' block counts
     uint32_t *coff;          // [C+1]
     uint32_t *pcnt;          // [5C] per monotone piece: x cuts | y cuts << 16
     uint32_t *nchain;        // [C+1] solve chains per curve (2 per piece)
