@@ -543,21 +543,32 @@ constexpr int kListClasses = kShortClass0 + 2 * kLenBins;
 constexpr uint32_t kLongPiece = 128;
 constexpr int kChainListThreads = 1024;
 constexpr uint32_t kListBlocks = 512;
-// Frame::lcount: class counts, then their exclusive sums over all classes and the total
+// Frame::lcount: class counts, then their exclusive sums over all classes and the total, then
+// how many chains at the list's front are solved by several lanes each
 constexpr int kListPre = kListClasses;
-static_assert((kListPre + kListClasses + 1) * sizeof(uint32_t) <= kListCountBytes, "class counts exceed their buffer");
+constexpr int kListWide = kListPre + kListClasses + 1;
+static_assert((kListWide + 1) * sizeof(uint32_t) <= kListCountBytes, "class counts exceed their buffer");
 
 // Length bins, longest first.  Below 256 a bin's longest entry is at most 4/3 of its
 // shortest, so that the lanes of a wave run loops of nearly equal trip counts.  The bin
 // of L is the number of lower bounds above L.
+#define SL_BIN_LOWER {384, 256, 192, 160, 128, 112, 96, 80, 65, 57, 49, 41, 33, 29, 25, 21, 17, 13, 9, 7, 5, 4, 3, 2, 1}
 __device__ __forceinline__ int len_bin(uint32_t L) {
-    constexpr uint32_t lower[kLenBins] = {384, 256, 192, 160, 128, 112, 96, 80, 65, 57, 49, 41, 33,
-                                          29,  25,  21,  17,  13,  9,   7,  5,  4,  3,  2,  1};
+    constexpr uint32_t lower[kLenBins] = SL_BIN_LOWER;
     int b = 0;
 #pragma unroll
     for (int i = 0; i < kLenBins; ++i) b += lower[i] > L ? 1 : 0;
     return b;
 }
+// the shortest length of bin b, 0 beyond the last
+__device__ __forceinline__ uint32_t bin_lower(int b) {
+    constexpr uint32_t lower[kLenBins] = SL_BIN_LOWER;
+    uint32_t v = 0u;
+#pragma unroll
+    for (int i = 0; i < kLenBins; ++i) v = b == i ? lower[i] : v;
+    return v;
+}
+#undef SL_BIN_LOWER
 
 struct CurvePieces {
     int np;
@@ -623,6 +634,14 @@ __global__ void __launch_bounds__(kChainListThreads) k_list_count(SceneDev sc, u
     for (int q = threadIdx.x; q < kListClasses; q += blockDim.x) blk[(size_t)q * gridDim.x + blockIdx.x] = h[q];
 }
 
+// Which cubic chains get several lanes each: those of the first `bins` length bins, as long as
+// their cuts (by the bins' shortest lengths) are no more than `load` chains of the longest bin
+// there is would have (launch_intersect has the limits).
+struct WideRule {
+    int bins;
+    uint32_t load;
+};
+
 // Lists from the block counts (at most kListBlocks); writes the class counts and their sums.
 // SOLO: one block, which counts for itself first.
 template <bool SOLO>
@@ -630,7 +649,7 @@ __global__ void __launch_bounds__(kChainListThreads) k_list_place(SceneDev sc, u
                                                                   const uint32_t *__restrict__ nchain,
                                                                   const uint32_t *__restrict__ pcnt,
                                                                   const uint32_t *__restrict__ coff, uint32_t cubic_min,
-                                                                  const uint32_t *__restrict__ blk,
+                                                                  WideRule rule, const uint32_t *__restrict__ blk,
                                                                   uint32_t *__restrict__ cnt, uint4 *clist, uint4 *plist) {
     __shared__ uint32_t total[kListClasses], base[kListClasses];
     constexpr int kWaves = kChainListThreads / 64;
@@ -671,6 +690,15 @@ __global__ void __launch_bounds__(kChainListThreads) k_list_place(SceneDev sc, u
                 if (q == kListClasses - 1) cnt[kListPre + kListClasses] = inc;
             }
         }
+    } else if (w == 2 && blockIdx.x == 0) {
+        const uint32_t v = lane < kLenBins ? total[lane] : 0u, len = bin_lower(lane);
+        const uint64_t some = __ballot(v != 0u), cuts = (uint64_t)v * len;
+        const uint32_t longest = some ? (uint32_t)__builtin_amdgcn_readlane((int)len, (int)__builtin_ctzll(some)) : 0u;
+        const uint32_t chains = wave_incl_scan(v);
+        const uint32_t sum = wave_incl_scan(cuts < (1u << 26) ? (uint32_t)cuts : 1u << 26);  // 25 of them fit
+        const int b = (int)__builtin_ctzll(~__ballot(lane < rule.bins && sum <= rule.load * longest));
+        const uint32_t wide = b ? (uint32_t)__builtin_amdgcn_readlane((int)chains, b - 1) : 0u;
+        if (lane == 0) cnt[kListWide] = wide;
     }
     __syncthreads();
     const uint32_t c0 = blockIdx.x * per, c1 = c0 + per < C ? c0 + per : C;
@@ -693,8 +721,6 @@ __global__ void __launch_bounds__(kChainListThreads) k_list_place(SceneDev sc, u
     }
 }
 
-// entries of the chain classes before q (q < kChainClasses), or of the piece list's before q
-__device__ __forceinline__ uint32_t class_start(const uint32_t *__restrict__ cnt, int q) { return cnt[kListPre + q]; }
 __device__ __forceinline__ uint32_t chain_total(const uint32_t *__restrict__ cnt) {
     return cnt[kListPre + kChainClasses - 1] + cnt[kChainClasses - 1];
 }
@@ -1184,22 +1210,22 @@ __device__ __forceinline__ void walk_pieces_staged(PieceSetup &p, bool live, int
     }
 }
 
-// Intersection pass 1.  Blocks [0, wide_blocks) solve the cubic chains of the first wide_bins
-// length bins with several lanes each; the next chain_blocks solve the other listed chains
+// Intersection pass 1.  Blocks [0, wide_blocks) solve the first cnt[kListWide] chains, cubic
+// ones, with several lanes each; the next chain_blocks solve the other listed chains
 // of long pieces, longest first; the blocks after them each take 256 short pieces and walk
 // them while solving, so the short pieces fill the GPU while the long chains run.
 __global__ void __launch_bounds__(256) k_chains(SceneDev sc, const float4 *__restrict__ crec, const uint4 *__restrict__ clist,
                                                  const uint4 *__restrict__ plist, const uint32_t *__restrict__ cnt,
-                                                 uint32_t wide_blocks, int wide_bins, uint32_t chain_blocks, int W, int H,
+                                                 uint32_t wide_blocks, uint32_t chain_blocks, int W, int H,
                                                  float *chain_t, int2 *ts) {
     if (blockIdx.x < wide_blocks) {
-        wide_chains(sc, crec, clist, class_start(cnt, wide_bins), wide_blocks, W, H, chain_t);
+        wide_chains(sc, crec, clist, cnt[kListWide], wide_blocks, W, H, chain_t);
         return;
     }
     const uint32_t blk = blockIdx.x - wide_blocks;
     if (blk < chain_blocks) {
         // the chains after those of the wide blocks
-        const uint32_t i = blk * blockDim.x + threadIdx.x + class_start(cnt, wide_bins);
+        const uint32_t i = blk * blockDim.x + threadIdx.x + cnt[kListWide];
         if (i >= chain_total(cnt)) return;
         solve_chain(sc, crec, clist[i], W, H, chain_t);
         return;
@@ -1357,7 +1383,7 @@ void launch_monotone(const SceneDev &sc, Frame &f, hipStream_t s) {
 void launch_intersect(const SceneDev &sc, Frame &f, hipStream_t s) {
     if (!sc.C) return;
     uint32_t *cnt = f.lcount;
-    // Cubic chains of the first wide_bins length bins take several lanes each (wide_chains): one
+    // Cubic chains of the first length bins take several lanes each (wide_chains): one
     // lane's 1.5 us a cut makes the longest chains the pass's time in frames of every size, but
     // the lanes cost up to 20 times the issue slots, so the more cuts a frame has, the fewer
     // chains pay.  Pieces of cubic_min cuts are listed as chains; shorter ones are walked by one
@@ -1366,13 +1392,21 @@ void launch_intersect(const SceneDev &sc, Frame &f, hipStream_t s) {
     // 782 / 484, 26 M 840 / 566, 51 M 985 / 719.  Neighbouring settings at each limit: 5 M with
     // three bins 341, 6.2 M with four 387 and two 458, 12.8 M with four 570, 26 M with three 698,
     // 51 M with three 1115; 2.1 M with 128-cut pieces and four bins 439.
-    const struct { int64_t cuts; uint32_t cubic_min; int bins; uint32_t blocks; } rule[] = {
-        {1 << 18, 24u, kLenBins, 2048u},  {1 << 21, 64u, kLenBins, 2048u}, {5 << 20, kLongPiece, 4, 512u},
-        {1 << 24, kLongPiece, 3, 256u},   {INT64_MAX, kLongPiece, 2, 256u}};
+    // The bins end earlier where their chains are too many (the loads): the lanes' work then
+    // lasts longer than the longest chain would on one lane.  Stage at the loads times 1/2, 1,
+    // 4/3, 2 and without a limit, us: 4000 curves of 500 cuts (6.4 M cuts) 745, 746, 746, 1150,
+    // 1139, a lane each 742; 3000 drawn chains seen at 1:4 (24 M) 1521, 1517, 1497, 1515, 6803,
+    // a lane each 1501; 3800 curves of 60 cuts a side (0.9 M) 107, 107, 148, 144, 145; where
+    // the lanes pay, 1000 drawn chains of 1000x1000 (4.4 M) 564, 555, 592, 776, 781, a lane
+    // each 797, and the 51 M above 857, 720, 720, 720, 719.
+    const struct { int64_t cuts; uint32_t cubic_min; WideRule wide; uint32_t blocks; } rule[] = {
+        {1 << 18, 24u, {kLenBins, 6144u}, 2048u}, {1 << 21, 64u, {kLenBins, 6144u}, 2048u},
+        {5 << 20, kLongPiece, {4, 3072u}, 512u},  {1 << 24, kLongPiece, {3, 2304u}, 256u},
+        {INT64_MAX, kLongPiece, {2, 2304u}, 256u}};
     int at = 0;
     while (f.F > rule[at].cuts) ++at;
     const uint32_t cubic_min = rule[at].cubic_min;
-    const int wide_bins = rule[at].bins;
+    const WideRule wide = rule[at].wide;
     // One block, for up to 1024 curves, counts and places by itself: 9.6 us for the two launches'
     // 13.6 with 91 curves, but with 1591 25 for 21.  More blocks leave their counts in the curves'
     // fragment counts, which their scan was the last to read: 101 words a block for a word a curve,
@@ -1386,13 +1420,13 @@ void launch_intersect(const SceneDev &sc, Frame &f, hipStream_t s) {
     uint32_t *blk = f.cfrag;
     if (nb == 1) {
         hipLaunchKernelGGL(k_list_place<true>, dim3(1), bl, 0, s, sc, sc.C, per, (const uint32_t *)f.nchain,
-                           (const uint32_t *)f.pcnt, (const uint32_t *)f.coff, cubic_min, (const uint32_t *)nullptr, cnt,
+                           (const uint32_t *)f.pcnt, (const uint32_t *)f.coff, cubic_min, wide, (const uint32_t *)nullptr, cnt,
                            f.chains, f.plist);
     } else {
         hipLaunchKernelGGL(k_list_count, dim3(nb), bl, 0, s, sc, sc.C, per, (const uint32_t *)f.nchain,
                            (const uint32_t *)f.pcnt, cubic_min, blk);
         hipLaunchKernelGGL(k_list_place<false>, dim3(nb), bl, 0, s, sc, sc.C, per, (const uint32_t *)f.nchain,
-                           (const uint32_t *)f.pcnt, (const uint32_t *)f.coff, cubic_min, (const uint32_t *)blk, cnt,
+                           (const uint32_t *)f.pcnt, (const uint32_t *)f.coff, cubic_min, wide, (const uint32_t *)blk, cnt,
                            f.chains, f.plist);
     }
     // chain blocks: enough for every chain; piece blocks: enough for every piece
@@ -1402,7 +1436,7 @@ void launch_intersect(const SceneDev &sc, Frame &f, hipStream_t s) {
     if (f.NCH)
         hipLaunchKernelGGL(k_chains, dim3(wide_blocks + chain_blocks + piece_blocks), dim3(256), 0, s, sc, (const float4 *)f.crec,
                            (const uint4 *)f.chains, (const uint4 *)f.plist,
-                           (const uint32_t *)cnt, wide_blocks, wide_bins, chain_blocks, f.W, f.H, f.chain_t, f.ts);
+                           (const uint32_t *)cnt, wide_blocks, chain_blocks, f.W, f.H, f.chain_t, f.ts);
     // one block per long piece up to 32768 blocks: the pieces' sizes vary widely, and
     // blocks that find no piece exit at once
     if (npieces)
