@@ -1189,10 +1189,11 @@ __device__ __forceinline__ void tile_load(const uint4 *__restrict__ prec, uint32
 
 // First pixel and width of the item covering cell c of a tile (gradients run along an item):
 // a merged cell, or the span between the merged cells next to it, which may lie in the
-// neighbouring records or be missing at the ends of the bucket's extent.  g: {index of the
-// record before the tile + 1 (0: none), the same of the next record, extent}.
-__device__ __forceinline__ void item_extent(const uint4 *__restrict__ prec, uint32_t edge, int c, int tx0, const uint4 &g,
-                                            int &x0, int &w) {
+// neighbouring records or be missing at the ends of the bucket's extent.  src and ent: the
+// bucket's list entries (list_row).
+__device__ __forceinline__ void item_extent(const uint4 *__restrict__ prec, const float4 &src, const uint4 &ent, int c,
+                                            int tx0, int &x0, int &w) {
+    const uint32_t edge = ent.y, prev = __float_as_uint(src.y), next = __float_as_uint(src.z);
     if ((edge >> c) & 1u) {
         x0 = tx0 + 2 * c;
         w = 2;
@@ -1202,19 +1203,19 @@ __device__ __forceinline__ void item_extent(const uint4 *__restrict__ prec, uint
     int end;
     if (below) {
         x0 = tx0 + 2 * (31 - __clz((int)below)) + 2;
-    } else if (g.x) {
-        const uint4 r = prec[g.x - 1u];
+    } else if (prev) {
+        const uint4 r = prec[prev - 1u];
         x0 = 64 * (int)(r.w & 0x7FFFFFFFu) + 2 * (31 - __clz((int)r.y)) + 2;
     } else {
-        x0 = (int)(g.z & 0xFFFFu);
+        x0 = (int)(ent.w & 0xFFFFu);
     }
     if (above) {
         end = tx0 + 2 * (__ffs((int)above) - 1);
-    } else if (g.y) {
-        const uint4 r = prec[g.y - 1u];
+    } else if (next) {
+        const uint4 r = prec[next - 1u];
         end = 64 * (int)(r.w & 0x7FFFFFFFu) + 2 * (__ffs((int)r.y) - 1);
     } else {
-        end = (int)(g.z >> 16);
+        end = (int)(ent.w >> 16);
     }
     w = end - x0;
 }
@@ -1246,12 +1247,14 @@ __device__ __forceinline__ uint32_t transpose32(uint32_t x) {
 // overlap the tile queued; 64 queued entries at a time then load their records.  (Loading
 // everything of 64 entries at once took three dependent loads for every 64 buckets of the
 // row; on a sheet of glyphs nearly all of them lie beside the tile.)
+// A list entry is {paint's colour, alpha * ascale} in l_src and {cover, edge, first merged cell,
+// path} in l_ent; a gradient's {its word, the index of the bucket's record before the tile + 1
+// (0: none), the same of the next record, -1} and its extent for the path.
 constexpr int kRowQueue = 192;
 
 template <bool GRAD, class F>
 __device__ __forceinline__ void list_row(const CovArgs &A, uint32_t q0, uint32_t q1, int tx, int tx1, float ascale,
-                                         const float *s_dec, uint32_t *queue, float4 *l_src, uint4 *l_ent, uint4 *l_grad,
-                                         const F &flush) {
+                                         const float *s_dec, uint32_t *queue, float4 *l_src, uint4 *l_ent, const F &flush) {
     const int lane = threadIdx.x & 63, tx0 = tx * 64;
     const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     int nlist = 0, nq = 0;
@@ -1297,17 +1300,17 @@ __device__ __forceinline__ void list_row(const CovArgs &A, uint32_t q0, uint32_t
                 if (ov && rank >= done && rank < done + take) {
                     const int sl = nlist + rank - done;
                     const uint32_t c = rec.x;
-                    if (GRAD && !(c & 0xFF000000u))
-                        l_src[sl] = make_float4(__uint_as_float(c), 0.f, 0.f, -1.f);
-                    else
+                    uint32_t last = rec.w;
+                    if (GRAD && !(c & 0xFF000000u)) {
+                        const int nx = tc.rec + (tc.has_rec ? 1 : 0);
+                        l_src[sl] = make_float4(__uint_as_float(c), __uint_as_float(tc.rec ? rec.z + (uint32_t)tc.rec : 0u),
+                                                __uint_as_float(nx < (int)rec.y ? rec.z + (uint32_t)nx + 1u : 0u), -1.f);
+                        last = ext;
+                    } else {
                         l_src[sl] = make_float4(s_dec[c & 0xFFu], s_dec[(c >> 8) & 0xFFu], s_dec[(c >> 16) & 0xFFu],
                                                 unorm_dec((int)(c >> 24)) * ascale);
-                    l_ent[sl] = make_uint4(tc.cover, tc.edge, tc.at, rec.w);
-                    if (GRAD) {
-                        const int nx = tc.rec + (tc.has_rec ? 1 : 0);
-                        l_grad[sl] = make_uint4(tc.rec ? rec.z + (uint32_t)tc.rec : 0u,
-                                                nx < (int)rec.y ? rec.z + (uint32_t)nx + 1u : 0u, ext, 0u);
                     }
+                    l_ent[sl] = make_uint4(tc.cover, tc.edge, tc.at, last);
                 }
                 nlist += take;
                 done += take;
@@ -1340,10 +1343,9 @@ __global__ void __launch_bounds__(256, GRAD ? 4 : (BATCH ? 6 : 7)) k_composite_c
     __shared__ float4 s_step[SRGB ? kQuantSteps : 1];
     __shared__ float s_dec[256];
     __shared__ float s_deca[GRAD ? 256 : 1];
-    __shared__ float4 l_src[4][kCovList];   // paint, alpha / N (a gradient's word, -1)
-    __shared__ uint4 l_ent[4][kCovList];    // {cover, edge, first merged cell, path}
+    __shared__ float4 l_src[4][kCovList];
+    __shared__ uint4 l_ent[4][kCovList];
     __shared__ uint32_t l_queue[4][kRowQueue];
-    __shared__ uint4 l_grad[GRAD ? 4 : 1][GRAD ? kCovList : 1];
     for (int i = threadIdx.x; i < 256; i += 256) {
         s_dec[i] = A.dec_c[i];
         if (GRAD) s_deca[i] = A.dec_a[i];
@@ -1425,9 +1427,10 @@ __global__ void __launch_bounds__(256, GRAD ? 4 : (BATCH ? 6 : 7)) k_composite_c
                     turn = solid;
                 } else {
                     if (turn) {
-                        const uint32_t c = __float_as_uint(l_src[w][b].x);
+                        const float4 src = l_src[w][b];
+                        const uint32_t c = __float_as_uint(src.x);
                         int ix0, iw;
-                        item_extent(A.prec, l_ent[w][b].y, cell, tx0, l_grad[w][b], ix0, iw);
+                        item_extent(A.prec, src, l_ent[w][b], cell, tx0, ix0, iw);
                         const float4 p0 = grad_color(A.G, c, ix0, iw, x, 2 * r, s_dec, s_deca);
                         const float4 p1 = grad_color(A.G, c, ix0, iw, x, 2 * r + 1, s_dec, s_deca);
                         blend_dec<SRGB>(s_step, d0, p0, p0.w * ((float)(cnt & 63u) * kInvN));
@@ -1451,7 +1454,7 @@ __global__ void __launch_bounds__(256, GRAD ? 4 : (BATCH ? 6 : 7)) k_composite_c
     };
 
     const uint32_t q0 = A.rowstart[row0 + r], q1 = A.rowstart[row0 + r + 1];
-    list_row<GRAD>(A, q0, q1, tx, tx1, kInvN, s_dec, l_queue[w], l_src[w], l_ent[w], l_grad[GRAD ? w : 0], flush);
+    list_row<GRAD>(A, q0, q1, tx, tx1, kInvN, s_dec, l_queue[w], l_src[w], l_ent[w], flush);
 
     if (x >= W) return;
     const int y0 = 2 * r;
@@ -1693,11 +1696,17 @@ __device__ __forceinline__ uint32_t column_bits(const uint32_t *m, int dx, uint3
 // were all slower (10.2 / 10.3 / 10.6 / 10.5 / 11.7 / 15.1 ms: five waves spill 176 bytes
 // a lane); blocks of four cost 5.7 / 4.3 ms at 16 / 8 samples.  Two buckets a group with
 // registers capped for 4 / 5 / 7 waves per SIMD at 32 / 16 / 8 samples (16 bytes a lane
-// spilled at 32; six waves at 16 samples: 6.0 ms, eight at 8: 4.6 ms).  The gradient
-// variants, whose paint arithmetic would spill under those caps, keep four-bucket groups,
-// uncapped registers and the indexed loops.
+// spilled at 32; six waves at 16 samples: 6.0 ms, eight at 8: 4.6 ms).
+// The gradient variants, whose paint arithmetic would spill under those caps, take four-bucket
+// groups, the indexed loops and 3 / 4 / 4 waves.  What they read besides a pixel's own values
+// is kept out of the registers' loop: the covering item's extent is looked up once a column,
+// and the gradient's word is one for the wave, so its table comes by scalar loads.  1024x1024,
+// 800 gradient paths, 32 / 16 / 8 samples: 7.2 / 3.5 / 1.88 ms, with the look-up in the loop,
+// vector loads and 40 KB of LDS exceeded (a wave less each) 8.9 / 4.2 / 2.30; groups of two
+// 7.3 / 3.7 / 1.90 and a quarter slower on glyphs at 32 samples, of eight 8.8 / 4.7 / 2.58,
+// five waves at 16 and 8 samples 3.6 / 1.91 and a fifth slower on small canvases.
 template <int SPP, bool SRGB, bool GRAD>
-__global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 5 : 7))) k_composite_ms(CovArgs A) {
+__global__ void __launch_bounds__(256, GRAD ? (SPP == 32 ? 3 : 4) : (SPP == 32 ? 4 : (SPP == 16 ? 5 : 7))) k_composite_ms(CovArgs A) {
     constexpr int NW = Words<SPP>::n;
     constexpr int CPR = 64 / (2 * SPP);
     constexpr int NREG = 64 / CPR;
@@ -1707,11 +1716,9 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
     __shared__ float s_dec[256];
     __shared__ float s_deca[GRAD ? 256 : 1];
     __shared__ float4 l_src[4][kCovList];
-    __shared__ uint4 l_ent[4][kCovList];    // {cover, edge, first merged cell, path}
+    __shared__ uint4 l_ent[4][kCovList];
     __shared__ uint32_t l_queue[4][kRowQueue];
-    __shared__ uint4 l_grad[GRAD ? 4 : 1][GRAD ? kCovList : 1];
-    __shared__ uint32_t slot[4][G][64];     // staging of the final average
-    __shared__ uint32_t tbl[4][G][256];
+    __shared__ uint32_t tbl[4][G][256];     // the paths' blend tables; then the final average's staging
     for (int i = threadIdx.x; i < 256; i += 256) {
         s_dec[i] = A.dec_c[i];
         if (GRAD) s_deca[i] = A.dec_a[i];
@@ -1798,13 +1805,17 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
                     if (GRAD) S.apply4(regs, blend);
                     else S.template apply<SPP == 32 ? 4 : 2>(regs, blend);
                 } else {
+                    // the covering item's extent, once a column
+                    const uint4 e = l_ent[w][g0 + g];
+                    int ix0 = 0, iw = 1;
+                    if ((e.x >> cell) & 1u) item_extent(A.prec, src, e, cell, tx0, ix0, iw);
+                    const uint32_t ce = (uint32_t)ix0 | ((uint32_t)iw << 16);
+                    const uint32_t word = (uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(src.x));
                     S.apply1(regs, [&](uint32_t st, int p) -> uint32_t {
                         const int c = p * CPR + q;
-                        const uint32_t ed = l_ent[w][g0 + g].y;
-                        int ix0 = 0, iw = 1;
-                        if ((l_ent[w][g0 + g].x >> (c >> 1)) & 1u)
-                            item_extent(A.prec, ed, c >> 1, tx0, l_grad[w][g0 + g], ix0, iw);
-                        const float4 pa = grad_color(A.G, __float_as_uint(src.x), ix0, iw, tx0 + c, 2 * r + dy, s_dec, s_deca);
+                        const uint32_t ext = (uint32_t)__shfl((int)ce, c, 64);
+                        const float4 pa = grad_color(A.G, word, (int)(ext & 0xFFFFu), (int)(ext >> 16),
+                                                     tx0 + c, 2 * r + dy, s_dec, s_deca);
                         const uint32_t nst = blend_code<SRGB>(s_step, s_dec, st, pa, pa.w);
                         return covers(p) ? nst : st;
                     });
@@ -1815,13 +1826,13 @@ __global__ void __launch_bounds__(256, GRAD ? 1 : (SPP == 32 ? 4 : (SPP == 16 ? 
     };
 
     const uint32_t q0 = A.rowstart[r], q1 = A.rowstart[r + 1];
-    list_row<GRAD>(A, q0, q1, tx, tx1, 1.f, s_dec, l_queue[w], l_src[w], l_ent[w], l_grad[GRAD ? w : 0], flush);
+    list_row<GRAD>(A, q0, q1, tx, tx1, 1.f, s_dec, l_queue[w], l_src[w], l_ent[w], flush);
 
-    // resolve: G registers at a time are staged in this wave's slot rows (G x 64 words);
+    // resolve: G registers at a time are staged in this wave's tables (G x 64 words);
     // lane (pixel, channel) sums the pixel's decoded samples in sample order, divides by N
     // and re-quantises, and the four channel lanes of a pixel assemble its word
     static_assert(NREG % G == 0, "state registers are staged G at a time");
-    uint32_t *stg = &slot[w][0][0];
+    uint32_t *stg = &tbl[w][0][0];
     wave_sync_lds();
 #pragma unroll
     for (int p0 = 0; p0 < NREG; p0 += G) {
