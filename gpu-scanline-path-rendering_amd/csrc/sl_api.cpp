@@ -299,9 +299,6 @@ void collect_status(sl_handle *h) {
     if (st[1] & 1u) {
         h->frame_rc = SL_E_HIP;
         h->frame_err = "internal error: fragment row outside its path's bucket range";
-    } else if (st[1] & 2u) {
-        h->frame_rc = SL_E_UNSUPPORTED;
-        h->frame_err = "a (path, row) bucket holds more than 65536 fragments";
     }
     if (h->stat_counts) {
         unsigned long long M = 0, MS = 0;
@@ -597,7 +594,6 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
     h->counts.merged_fragment = (int64_t)M;
     h->counts.span = (int64_t)(MS - M);
     if (small[1] & 1u) return fail(h, SL_E_HIP, "internal error: fragment row outside its path's bucket range");
-    if (small[1] & 2u) return fail(h, SL_E_UNSUPPORTED, "a (path, row) bucket holds more than 65536 fragments");
     if (!carved) { h->last_F = F; h->last_NCH = NCH; h->last_NB = NB; h->sized = true; }
 
     if (h->timing) {
@@ -1526,7 +1522,7 @@ struct sl_batch {
     hipStream_t cap_stream = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    int shape[4] = {0, 0, 4, 256};        // resolve grid, class grid, compositor group, fragment block
+    int shape[4] = {0, 0, 4, 256};        // resolve grid, class grid, 4 or 8 (selects nothing), fragment block
     // the last frame issued by sl_batch_render(_eager), possibly still running
     hipEvent_t done_ev = nullptr;
     hipEvent_t switch_ev = nullptr;       // recorded on last_stream when a frame moves on

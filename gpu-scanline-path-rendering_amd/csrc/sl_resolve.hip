@@ -206,8 +206,7 @@ struct ResolveArgs {
     ulonglong2 *rtile;
     uint2 *bcnt;
     uint32_t *big_list;
-    uint32_t *big_count;
-    uint32_t *err;
+    uint32_t *big_count;     // cleared at the frame's start
 };
 
 // bits of tiles [t0, t1] counted from tile tb (t0 <= t1), tiles from the 63rd on in bit 63
@@ -1388,7 +1387,6 @@ __global__ void __launch_bounds__(256, GRAD ? 4 : (BATCH ? 6 : 7)) k_composite_c
     const int r = tile / tiles_x, tx = tile - r * tiles_x;
     const int tx0 = tx * 64, tx1 = tmin(tx0 + 64, W);
     const int x = tx0 + lane, cell = lane >> 1, half = 12 * (lane & 1);
-    const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     constexpr float kInvN = 1.f / (float)SPP;
     constexpr uint32_t kFull = (uint32_t)SPP * 65u;  // both rows' counts
     float d0[4] = {1.f, 1.f, 1.f, 1.f}, d1[4] = {1.f, 1.f, 1.f, 1.f};
@@ -1734,7 +1732,6 @@ __global__ void __launch_bounds__(256, GRAD ? (SPP == 32 ? 3 : 4) : (SPP == 32 ?
     const int tx = t - rr * tiles_x, tx0 = tx * 64;
     const int tx1 = tmin(tx0 + 64, W);
     const int x = tx0 + lane, cell = lane >> 1;
-    const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     // blend-phase coordinates of this lane
     const int q = lane / (2 * SPP), dy = (lane / SPP) & 1;
     SampleRegs<NREG> S;
@@ -2004,7 +2001,7 @@ void launch_resolve(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t s
     // coverage compositor reads only the per-pixel sample counts
     A.items = f.items; A.imask = f.imask; A.icov = f.icov; A.prec = f.prec;
     A.rpos = f.rpos; A.finfo = sc.finfo; A.rext = f.rext; A.rrec = f.rrec; A.rtile = f.rtile; A.bcnt = f.bcnt;
-    A.big_list = f.big_list; A.big_count = f.big_count; A.err = f.err_flag;  // cleared at the frame's start
+    A.big_list = f.big_list; A.big_count = f.big_count;
     // A wave resolves up to 64 buckets of the grid's stride: with fewer its packs of four and two
     // small buckets stay part empty and every bucket pays for a wave's start and end, but below
     // twice the 5120 resident waves the last ones leave the chip idle.  One bucket a wave up
