@@ -4,8 +4,9 @@
 //
 // Bucket layout: path p owns buckets [pbase[p], pbase[p+1]) in the order the reference's
 // signed int32 key (y+0x7FFF)<<16 | (x+0x7FFF) sorts a path's fragments: cell rows 1..rhi,
-// then the out-of-canvas key 0xFFFEFFFE, then row 0.  A path's rows are the exact range
-// of its fragment rows, recorded while intersecting.
+// then the out-of-canvas key 0xFFFEFFFE, then row 0.  A path's rows are those of its visible
+// curves' control hulls with a row of margin, clamped to the canvas (k_monotone): every
+// fragment row lies in the range, and rows at its ends may hold none.
 #include "sl_device.h"
 #include "sl_internal.h"
 

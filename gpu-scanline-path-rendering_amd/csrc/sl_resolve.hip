@@ -2003,11 +2003,16 @@ void launch_resolve(const SceneDev &sc, const Tables &t, Frame &f, hipStream_t s
     A.rpos = f.rpos; A.finfo = sc.finfo; A.rext = f.rext; A.rrec = f.rrec; A.rtile = f.rtile; A.bcnt = f.bcnt;
     A.big_list = f.big_list; A.big_count = f.big_count;
     // A wave resolves up to 64 buckets of the grid's stride: with fewer its packs of four and two
-    // small buckets stay part empty and every bucket pays for a wave's start and end, but below
-    // twice the 5120 resident waves the last ones leave the chip idle.  One bucket a wave up
-    // to 65536 waves, then shared / this, us: 47 k buckets 42 / 22, 57 k (a page of text) 62 / 32,
-    // a poster 152 / 107, 1.9 M 434 / 426, 1.8 M (the illustration) 1325 / 1304; at least 5120
-    // waves 20 / 29 / 111, 15360 25 / 34 / 109, at most 96 buckets 438 and 1364.
+    // small buckets stay part empty and every bucket pays for a wave's start and end.  One bucket
+    // a wave up to 65536 waves, then shared / this, us: 47 k buckets 42 / 22, 57 k (a page of
+    // text) 62 / 32, a poster 152 / 107, 1.9 M 434 / 426, 1.8 M (the illustration) 1325 / 1304;
+    // at most 96 buckets 438 and 1364.  The least number of waves weighs small frames, which
+    // lose by waves of fewer buckets, against middling ones, whose uneven buckets balance over
+    // two turns of the 5120 resident waves.  Stage with at least 5120 / 7680 / 10240, us: 512x512,
+    // 200 paths 26 / 28 / 28, the page 34 / 38 / 37, 1000x1000, 300 paths 58 / 58 / 59; 1024x768,
+    // 1500 paths 175 / 172 / 165, 1000x777, 2000 paths 300 / 309 / 276, 1279x719, 3000 paths
+    // 177 / 177 / 171, 2048x2048, 20000 glyphs 123 / 114 / 111, 1500x1500, 6000 paths
+    // 456 / 455 / 437.
     const int64_t gd = std::max((f.NB + 63) / 64, kResolveWaves);
     const unsigned g1 = (unsigned)std::min<int64_t>(f.NB, f.resolve_grid > 0 ? f.resolve_grid : gd);
     const unsigned gc = f.class_grid > 0 ? (unsigned)f.class_grid : 4096u;
