@@ -45,7 +45,7 @@ struct Arena {
 
 const char *kStageNames[] = {"transform_cull", "monotone_count", "intersect", "bucket_setup",
                              "fragments",      "resolve",        "order_rows", "composite"};
-constexpr int kStages = 8;
+constexpr int kStages = 8, kRowStage = 6;
 
 }  // namespace
 
@@ -288,6 +288,16 @@ int check_launch(sl_handle *h, const char *what) {
     return SL_OK;
 }
 
+// Stage times from a frame's events.  The row order is part of bucket_setup: its own stage has
+// no work and no event of its own, so it reads zero and the next begins where it would.
+void stage_times(sl_handle *h) {
+    for (int i = 0; i < kStages; ++i) {
+        float ms = 0.f;
+        if (i != kRowStage) (void)hipEventElapsedTime(&ms, h->ev[i == kRowStage + 1 ? kRowStage : i], h->ev[i + 1]);
+        h->stage_ms[i] = ms;
+    }
+}
+
 // The status a settled frame left in fstat: its error flags and, for an eager frame, the
 // element counts and stage times.
 void collect_status(sl_handle *h) {
@@ -309,11 +319,7 @@ void collect_status(sl_handle *h) {
         h->stat_counts = false;
     }
     if (h->timing_pending) {
-        for (int i = 0; i < kStages; ++i) {
-            float ms = 0.f;
-            (void)hipEventElapsedTime(&ms, h->ev[i], h->ev[i + 1]);
-            h->stage_ms[i] = ms;
-        }
+        stage_times(h);
         h->timing_pending = false;
     }
 }
@@ -556,8 +562,7 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
     mark(5);
     sl::launch_resolve(sc, tb, f, s);
     if ((rc = check_launch(h, "resolve"))) return rc;
-    mark(6);  // the row order is part of bucket_setup
-    mark(7);
+    mark(kRowStage);
     sl::launch_composite(sc, tb, f, s);
     if ((rc = check_launch(h, "composite"))) return rc;
     mark(8);
@@ -597,11 +602,7 @@ int render(sl_handle *h, hipStream_t s, bool replay, Arena &A, uint8_t *out_imag
     if (!carved) { h->last_F = F; h->last_NCH = NCH; h->last_NB = NB; h->sized = true; }
 
     if (h->timing) {
-        for (int i = 0; i < kStages; ++i) {
-            float ms = 0.f;
-            (void)hipEventElapsedTime(&ms, h->ev[i], h->ev[i + 1]);
-            h->stage_ms[i] = ms;
-        }
+        stage_times(h);
     }
 
     if (h->debug) {
