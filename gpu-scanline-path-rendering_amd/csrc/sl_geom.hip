@@ -690,7 +690,9 @@ __global__ void __launch_bounds__(kChainListThreads) k_list_place(SceneDev sc, u
                 if (q == kListClasses - 1) cnt[kListPre + kListClasses] = inc;
             }
         }
-    } else if (w == 2 && blockIdx.x == 0) {
+    }
+    __syncthreads();
+    if (w == kWaves - 1 && blockIdx.x == gridDim.x - 1) {  // the wave with the fewest curves
         const uint32_t v = lane < kLenBins ? total[lane] : 0u, len = bin_lower(lane);
         const uint64_t some = __ballot(v != 0u), cuts = (uint64_t)v * len;
         const uint32_t longest = some ? (uint32_t)__builtin_amdgcn_readlane((int)len, (int)__builtin_ctzll(some)) : 0u;
@@ -700,7 +702,6 @@ __global__ void __launch_bounds__(kChainListThreads) k_list_place(SceneDev sc, u
         const uint32_t wide = b ? (uint32_t)__builtin_amdgcn_readlane((int)chains, b - 1) : 0u;
         if (lane == 0) cnt[kListWide] = wide;
     }
-    __syncthreads();
     const uint32_t c0 = blockIdx.x * per, c1 = c0 + per < C ? c0 + per : C;
     for (uint32_t c = c0 + threadIdx.x; c < c1; c += kChainListThreads) {
         const CurvePieces cp = curve_pieces(sc, C, c, nchain, pcnt);
@@ -1210,22 +1211,24 @@ __device__ __forceinline__ void walk_pieces_staged(PieceSetup &p, bool live, int
     }
 }
 
-// Intersection pass 1.  Blocks [0, wide_blocks) solve the first cnt[kListWide] chains, cubic
+// Intersection pass 1.  Blocks [0, wide_blocks) solve the first cnt[wide_at] chains, cubic
 // ones, with several lanes each; the next chain_blocks solve the other listed chains
 // of long pieces, longest first; the blocks after them each take 256 short pieces and walk
-// them while solving, so the short pieces fill the GPU while the long chains run.
+// them while solving, so the short pieces fill the GPU while the long chains run.  (The word's
+// place is an argument: with it written in, the kernel's code came out differently and 1 % slower,
+// 254 us for 250 on 3000 mixed paths of 1279x719.)
 __global__ void __launch_bounds__(256) k_chains(SceneDev sc, const float4 *__restrict__ crec, const uint4 *__restrict__ clist,
                                                  const uint4 *__restrict__ plist, const uint32_t *__restrict__ cnt,
-                                                 uint32_t wide_blocks, uint32_t chain_blocks, int W, int H,
+                                                 uint32_t wide_blocks, int wide_at, uint32_t chain_blocks, int W, int H,
                                                  float *chain_t, int2 *ts) {
     if (blockIdx.x < wide_blocks) {
-        wide_chains(sc, crec, clist, cnt[kListWide], wide_blocks, W, H, chain_t);
+        wide_chains(sc, crec, clist, cnt[wide_at], wide_blocks, W, H, chain_t);
         return;
     }
     const uint32_t blk = blockIdx.x - wide_blocks;
     if (blk < chain_blocks) {
         // the chains after those of the wide blocks
-        const uint32_t i = blk * blockDim.x + threadIdx.x + cnt[kListWide];
+        const uint32_t i = blk * blockDim.x + threadIdx.x + cnt[wide_at];
         if (i >= chain_total(cnt)) return;
         solve_chain(sc, crec, clist[i], W, H, chain_t);
         return;
@@ -1436,7 +1439,7 @@ void launch_intersect(const SceneDev &sc, Frame &f, hipStream_t s) {
     if (f.NCH)
         hipLaunchKernelGGL(k_chains, dim3(wide_blocks + chain_blocks + piece_blocks), dim3(256), 0, s, sc, (const float4 *)f.crec,
                            (const uint4 *)f.chains, (const uint4 *)f.plist,
-                           (const uint32_t *)cnt, wide_blocks, chain_blocks, f.W, f.H, f.chain_t, f.ts);
+                           (const uint32_t *)cnt, wide_blocks, kListWide, chain_blocks, f.W, f.H, f.chain_t, f.ts);
     // one block per long piece up to 32768 blocks: the pieces' sizes vary widely, and
     // blocks that find no piece exit at once
     if (npieces)
