@@ -268,7 +268,7 @@ __device__ __forceinline__ int wave_scan_add(int x) { return sl::dev::dpp_scan(x
 // units of 2^-56 (slivers of 2^-32 of a pixel keep a float's precision).
 // A crossing costs one pass over its bucket and two LDS adds, where integrating every
 // interval over every pixel column cost each column a pass over the whole row's crossings.
-// 861 k crossings (64 paths at 256x256, 16 rows): 25 us, where sorting the buckets and the
+// 861 k crossings (64 paths at 256x256, 16 rows): 26 us, where sorting the buckets and the
 // column passes took 35 and 237 us.
 constexpr int kFillStage = 128;   // crossings of a row staged in LDS (more are read from memory)
 constexpr int kFillPixels = 512;  // pixel columns of one pass over a row

@@ -326,8 +326,9 @@ const char *sl_batch_last_error(sl_batch *b);
  * No reference counterpart.  Coverage is a box filter of `sample_rows` rows per pixel,
  * each integrated exactly along x (continuous in the control points); compositing is the
  * renderer's src-over onto white in path order, unquantised, into a float RGBA image.
- * Scenes of line / quadratic / cubic segments (closed contours), vertices stored per
- * curve as in sl_scene.  `points` (float [V][2]), `colors` (float [P][4], RGBA in [0,1]),
+ * Scenes of line / quadratic / cubic segments, vertices stored per curve as in sl_scene.
+ * Contours are meant to be closed; where points moved curve by curve leave one open, a
+ * sample row is filled between its first and last crossing only.  `points` (float [V][2]), `colors` (float [P][4], RGBA in [0,1]),
  * `image` (float [H][W][4]) and all gradients are DEVICE pointers; work runs on `stream`.
  * sl_diff_forward keeps what the adjoint needs when `keep_for_backward` is set (the
  * points and colours must stay unchanged until the backward).  sl_diff_backward writes
